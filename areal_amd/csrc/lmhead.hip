@@ -505,23 +505,55 @@ __global__ __launch_bounds__(256) void k_carry_factors(const float* __restrict__
 }
 
 // ---- the d_hidden product cut along K: into how many parts ---------------------------------------------------------
-// Into how many parts along K a product of `tiles` tiles and `slices` K slices is cut (1: not at all): the number of
-// parts, up to kMaxSplits, that shortens the time in rounds of tiles, ceil(tiles * parts / units) / parts, the most,
-// with 0.03 rounds charged per part for writing and adding its fp32 plane; at least 5 % have to be won, and a part
-// keeps at least 64 slices.  In whole numbers (rounds x 1200) so that the host and the device (k_compact_map, from a
-// row count that only the device holds) come to the same answer.
-constexpr int kMaxSplits = 4;
-constexpr int kRoundsUnit = 1200;  // divisible by every number of parts
-static_assert(kRoundsUnit % 2 == 0 && kRoundsUnit % 3 == 0 && kRoundsUnit % 4 == 0 && kMaxSplits <= 4, "rounds in whole numbers");
-__host__ __device__ inline int choose_splits(int64_t tiles, int64_t slices, int units) {
+// Into how many parts along K a product of `tiles` tiles and `slices` K slices is cut (1: not at all).  The time of a
+// cut, in nanoseconds: rounds of tiles, ceil(tiles * parts / units), each of its share of the slices plus what a tile
+// costs outside the main loop, and for two parts or more the fp32 planes that are written and added (a tile of a plane
+// is 256 KB each way).  The number of parts with the smallest time is taken, one part unless 5 % are won.  Up to
+// kFewSplits parts are always possible; more only while all of them run in one round (tiles * parts <= units), which
+// bounds the planes by 64 MB: a product of few tiles (a small hidden size, or few tokens) otherwise leaves most of the
+// chip idle.  Measured, d_hidden of H = 1024, V = 50 257, 1 330 rows: 24 tiles in 4 parts (96 of 256 compute units)
+// 234 us, in 10 parts 118 us.
+// In whole numbers so that the host and the device (k_compact_map, from a row count that only the device holds) come to
+// the same answer.
+constexpr int kFewSplits = 4;
+constexpr int kMaxSplits = 32;
+constexpr int kMinSplitSlices = 16;   // a part keeps at least this many slices
+constexpr int kNsPerSlice = 1400;     // 256 x 256 x 64 of a tile
+constexpr int kNsPerTile = 8000;      // prologue and epilogue of a tile
+constexpr int kNsPerPlaneTile = 105;  // one 256 x 256 fp32 tile written and read at about 5 TB/s
+constexpr int64_t kNsNever = (int64_t)1 << 62;
+__host__ __device__ inline int64_t split_ns(int tiles, int slices, int units, int parts) {
+  if (parts > 1 && (slices / parts < kMinSplitSlices || (parts > kFewSplits && tiles * parts > units))) return kNsNever;
+  const int rounds = (tiles * parts + units - 1) / units;
+  const int64_t ns = (int64_t)rounds * ((slices + parts - 1) / parts * kNsPerSlice + kNsPerTile);
+  return parts == 1 ? ns - ns / 20 : ns + (int64_t)(tiles * parts) * kNsPerPlaneTile;  // one part: less the 5 % to be won
+}
+static inline int choose_splits(int64_t tiles, int64_t slices, int units) {
   if (units <= 0 || tiles <= 0) return 1;
   int best = 1;
-  int64_t best_rounds = (tiles + units - 1) / units * (kRoundsUnit * 95 / 100);  // one part, less the 5 % to be won
-  for (int parts = 2; parts <= kMaxSplits && slices / parts >= 64; ++parts) {
-    const int64_t r = (tiles * parts + units - 1) / units * (kRoundsUnit / parts) + (kRoundsUnit * 3 / 100) * parts;
-    if (r < best_rounds) {
+  int64_t best_ns = split_ns((int)tiles, (int)slices, units, 1);
+  for (int parts = 2; parts <= kMaxSplits; ++parts) {
+    const int64_t ns = split_ns((int)tiles, (int)slices, units, parts);
+    if (ns < best_ns) {
       best = parts;
-      best_rounds = r;
+      best_ns = ns;
+    }
+  }
+  return best;
+}
+// the same by the lanes of one wave (parts = lane + 1; the smallest number of parts wins a tie)
+__device__ __forceinline__ int choose_splits_wave(int tiles, int slices, int units) {
+  if (units <= 0 || tiles <= 0) return 1;
+  const int parts = (threadIdx.x & (kWave - 1)) + 1;
+  int64_t ns = parts <= kMaxSplits ? split_ns(tiles, slices, units, parts) : kNsNever;
+  int best = parts;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int64_t ons = __shfl_xor(ns, o, kWave);
+    const int ob = __shfl_xor(best, o, kWave);
+    if (ons < ns || (ons == ns && ob < best)) {
+      ns = ons;
+      best = ob;
     }
   }
   return best;
@@ -640,6 +672,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_splitk(Operand A, Operand B, 
     tiles_n = live < tiles_n ? live : tiles_n;
     splits = bounds[kRowsSplits];
     if (splits == 1 || (int)blockIdx.x >= tiles_m * tiles_n * splits) return;  // the same in every thread
+    plane = (int64_t)tiles_n * BN * ldc;  // planes of the rows in use: there may be more of them than of all rows
   }
   const int tiles = tiles_m * tiles_n;
   const int q = xcd_contiguous(blockIdx.x, tiles * splits);
@@ -689,6 +722,7 @@ __global__ __launch_bounds__(256) void k_splitk_rows(const float* __restrict__ p
   if (bounds) {
     splits = bounds[kRowsSplits];
     if (splits == 1 || r >= bounds[kRowsTotal]) return;
+    plane = (int64_t)bounds[kRowsLive] * BN * M;  // as k_gemm_splitk lays them
   }
   const int64_t dst = c_rows ? c_rows[r] : r;
   if (dst < 0) return;
@@ -697,15 +731,26 @@ __global__ __launch_bounds__(256) void k_splitk_rows(const float* __restrict__ p
     float a[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) a[i] = 0.f;
-    for (int sp = 0; sp < splits; ++sp) {
-      const float* src = part + (int64_t)sp * plane + r * M + m;
-      const f32x4_t lo = *(const f32x4_t*)src, hi = *(const f32x4_t*)(src + 4);
+    const float* src = part + r * M + m;
+    auto add = [&](const f32x4_t lo, const f32x4_t hi) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         a[i] += lo[i];
         a[4 + i] += hi[i];
       }
+    };
+    int sp = 0;
+    for (; sp + 4 <= splits; sp += 4) {  // the loads of four planes together, added in order
+      f32x4_t lo[4], hi[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        lo[q] = *(const f32x4_t*)(src + (int64_t)(sp + q) * plane);
+        hi[q] = *(const f32x4_t*)(src + (int64_t)(sp + q) * plane + 4);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) add(lo[q], hi[q]);
     }
+    for (; sp < splits; ++sp) add(*(const f32x4_t*)(src + (int64_t)sp * plane), *(const f32x4_t*)(src + (int64_t)sp * plane + 4));
 #pragma unroll
     for (int i = 0; i < 8; ++i) a[i] = f == 0.f ? 0.f : a[i] * f;  // a zero factor gives a zero row whatever the sums hold
     store8<AA_BF16>(out + dst * ldo, m, a);
@@ -751,13 +796,16 @@ __global__ __launch_bounds__(1024) void k_compact_map(const uint8_t* __restrict_
   }
   int total = 0;
   for (int w = 0; w < 16; ++w) total += wave_sum[w];
-  if (tid == 0) {
+  if (wave == 0) {
     const int rows = total < limit ? total : limit;
     const int live = (rows + BN - 1) / BN;
-    total_out[kRowsTotal] = rows;
-    total_out[kRowsLive] = live;
-    total_out[kRowsSliced] = rows > 0 ? (rows + BK - 1) / BK * BK : BK;
-    total_out[kRowsSplits] = choose_splits((int64_t)dh_tiles_m * live, dh_slices, units);
+    const int splits = choose_splits_wave(dh_tiles_m * live, dh_slices, units);
+    if (lane == 0) {
+      total_out[kRowsTotal] = rows;
+      total_out[kRowsLive] = live;
+      total_out[kRowsSliced] = rows > 0 ? (rows + BK - 1) / BK * BK : BK;
+      total_out[kRowsSplits] = splits;
+    }
   }
   for (int p = total + tid; p < limit; p += 1024) {  // the usual case: none
     act_rows[p] = -1;
@@ -868,12 +916,14 @@ struct Workspace {
   int64_t off_panel;                    // d(logits) rows [chunk, V]
   int64_t off_hc;                       // the hidden rows of the tokens with gradient, closed up [chunk, H]
   int64_t off_dw;                       // fp32 accumulator of a bf16 d_weight when there is more than one chunk
-  int64_t off_dhp;                      // fp32 planes of a d_hidden product cut along K [kMaxSplits][chunk, H]
+  int64_t off_dhp;                      // fp32 planes of a d_hidden product cut along K [parts][rows, H]
   int64_t bytes;
 };
 
 // external_panel: the d(logits) rows live in an array of the caller's (the op that keeps them from its forward to its
 // backward), not in the workspace
+static int compute_units();
+
 static Workspace plan(int64_t T, int64_t H, int64_t V, bool external_panel = false) {
   Workspace w{};
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
@@ -897,7 +947,9 @@ static Workspace plan(int64_t T, int64_t H, int64_t V, bool external_panel = fal
   w.off_panel = off;   off += external_panel ? 0 : up(w.chunk * w.panel_ld * 2);
   w.off_hc = off;      off += up(w.chunk * H * 2);
   w.off_dw = off;      off += T > w.chunk ? up(V * H * 4) : 0;
-  w.off_dhp = off;     off += up(kMaxSplits * w.chunk * H * 4);
+  // kFewSplits parts over all rows of a chunk, or more parts of a product whose parts all run in one round
+  const int64_t few = kFewSplits * w.chunk * H, one_round = (int64_t)compute_units() * BM * BN;
+  w.off_dhp = off;     off += up((few > one_round ? few : one_round) * 4);
   w.bytes = off;
   return w;
 }

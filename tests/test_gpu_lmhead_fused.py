@@ -214,6 +214,33 @@ def test_hidden_gradient_cut_along_the_vocabulary(device, backward, T, H, V):
     assert torch.equal(dh, dh2) and torch.equal(dw, dw2) and torch.equal(loss, loss2)
 
 
+@pytest.mark.parametrize("T,active,H,V", [(1400, 40, 72, 33000), (1400, 300, 520, 16643), (1400, 40, 520, 2100)])
+def test_hidden_gradient_of_few_rows_among_many_tokens(device, T, active, H, V):
+    """Few tokens of a chunk have a gradient: their one or two tiles per 256 hidden entries are cut into more parts than
+    a product over every token of the chunk would be (32, 16 and 2 here), in planes laid for the rows in use.  Bit-equal
+    whether the host or the device counts the rows, and against the oracle."""
+    hidden, weight, labels, prox, old, adv, _ = _inputs(T, T, H, V, seed=V, w_std=0.05)
+    mask = torch.zeros(T, dtype=torch.bool)
+    mask[torch.randperm(T, generator=torch.Generator().manual_seed(1))[:active]] = True
+    args = [t.to(device) for t in (labels, prox, old, adv)]
+
+    def run(**kw):
+        h = hidden.to(device).requires_grad_(True)
+        w = weight.to(device).requires_grad_(True)
+        loss, _ = areal_amd.fused_lm_head_ppo_loss(h, w, *args, eps_clip=0.2, loss_mask=mask.to(device), **kw)
+        loss.backward()
+        return h.grad, w.grad
+
+    dh, dw = run()
+    dh_host, dw_host = run(kept_per_chunk=[active])
+    assert torch.equal(dh, dh_host) and torch.equal(dw, dw_host)
+    _, _, _, _, o_dh, o_dw = _oracle_step(hidden, weight, labels, prox, old, adv, mask, 1.0, 1.0, eps_clip=0.2)
+    assert cosine(dh.cpu().float(), o_dh) > 0.9999 and cosine(dw.cpu().float(), o_dw) > 0.9999
+    assert_same_magnitude(dh, o_dh, what="d(hidden)")
+    assert_same_magnitude(dw, o_dw, what="d(weight)")
+    assert float(dh[~mask.to(device)].float().abs().max()) == 0.0
+
+
 def test_upstream_gradient_scales_both_gradients(device):
     hidden, weight, labels, prox, old, adv, mask = _inputs(260, 260, 64, 704, seed=3)
     args = [t.to(device) for t in (labels, prox, old, adv)]
