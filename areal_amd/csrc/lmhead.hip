@@ -307,15 +307,20 @@ __global__ __launch_bounds__(256) void k_label_logit(const uint16_t* __restrict_
   if (lane == 0) xy[t] = acc;
 }
 
-// Merge of the block partials of 64 tokens by a workgroup of 1024 threads: lane = token, wave w folds blocks
-// w, w + 16, ... in order, then the 16 wave results are folded in wave order by every wave alike.  Fixed order:
-// deterministic.
+// Merge of the block partials of 32 tokens by a workgroup of 1024 threads: thread = (token, group), 32 groups; group g
+// folds blocks g, g + 32, ... in order, then the 32 group results are folded in group order by every group alike.  Fixed
+// order: deterministic.  Bound by the latency of the loads when there are few tokens (a load covers one 128-byte line of
+// a plane): 32 tokens per workgroup, not 64, so that 4 096 tokens reach 128 compute units, and the loads of four blocks
+// are issued together.  4 152 tokens x 1 188 blocks, four planes (79 MB): 54 us with 64 tokens and one block at a time,
+// 30 us so (8 000 tokens, three planes: 47 and 26 us; 16 384 tokens, bound by bandwidth: 71 and 76 us).
 struct Merged {
   float k, s, u;
   float n;  // smallest raw logit (FLT_MAX when the minimum plane was not asked for)
 };
-constexpr int kMergeWaves = 16;
-constexpr int kMergeSmemFloats = 4 * kMergeWaves * 64;
+constexpr int kMergeTokens = 32;
+constexpr int kMergeGroups = 1024 / kMergeTokens;
+constexpr int kMergeAhead = 4;  // blocks whose loads are in flight together
+constexpr int kMergeSmemFloats = 4 * 1024;
 
 __device__ __forceinline__ void merge_into(Merged& m, float bk, float bs, float bu) {
   const float nk = fmaxf(m.k, bk);
@@ -326,34 +331,53 @@ __device__ __forceinline__ void merge_into(Merged& m, float bk, float bs, float 
   m.k = nk;
 }
 
-// t: the token of this lane (may be past the end: then the result is meaningless and the caller drops it)
+// t: the token of this thread (may be past the end: then the result is meaningless and the caller drops it)
 __device__ __forceinline__ Merged merge_blocks(const float* __restrict__ pk, const float* __restrict__ ps,
                                                const float* __restrict__ pu, const float* __restrict__ pn, int blocks,
-                                               int64_t pitch_t, int64_t t, bool live, float* smem /* [4][16][64] */) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+                                               int64_t pitch_t, int64_t t, bool live, float* smem /* [4][groups][tokens] */) {
+  const int tok = threadIdx.x % kMergeTokens, group = threadIdx.x / kMergeTokens;
   Merged m{kNegBig, 0.f, 0.f, FLT_MAX};
-  if (live)
-    for (int b = wave; b < blocks; b += kMergeWaves) {
+  if (live) {
+    int b = group;
+    for (; b + (kMergeAhead - 1) * kMergeGroups < blocks; b += kMergeAhead * kMergeGroups) {
+      float k[kMergeAhead], s[kMergeAhead], u[kMergeAhead], n[kMergeAhead];
+#pragma unroll
+      for (int q = 0; q < kMergeAhead; ++q) {
+        const int64_t at = (int64_t)(b + q * kMergeGroups) * pitch_t + t;
+        k[q] = pk[at];
+        s[q] = ps[at];
+        u[q] = pu[at];
+        n[q] = pn ? pn[at] : FLT_MAX;
+      }
+#pragma unroll
+      for (int q = 0; q < kMergeAhead; ++q) {
+        merge_into(m, k[q], s[q], u[q]);
+        m.n = fminf(m.n, n[q]);
+      }
+    }
+    for (; b < blocks; b += kMergeGroups) {
       const int64_t at = (int64_t)b * pitch_t + t;
       merge_into(m, pk[at], ps[at], pu[at]);
       if (pn) m.n = fminf(m.n, pn[at]);
     }
-  smem[(0 * kMergeWaves + wave) * 64 + lane] = m.k;
-  smem[(1 * kMergeWaves + wave) * 64 + lane] = m.s;
-  smem[(2 * kMergeWaves + wave) * 64 + lane] = m.u;
-  smem[(3 * kMergeWaves + wave) * 64 + lane] = m.n;
+  }
+  const int mine = group * kMergeTokens + tok;
+  smem[mine] = m.k;
+  smem[1024 + mine] = m.s;
+  smem[2048 + mine] = m.u;
+  smem[3072 + mine] = m.n;
   __syncthreads();
   Merged r{kNegBig, 0.f, 0.f, FLT_MAX};
-#pragma unroll
-  for (int w = 0; w < kMergeWaves; ++w) {
-    merge_into(r, smem[(0 * kMergeWaves + w) * 64 + lane], smem[(1 * kMergeWaves + w) * 64 + lane],
-               smem[(2 * kMergeWaves + w) * 64 + lane]);
-    r.n = fminf(r.n, smem[(3 * kMergeWaves + w) * 64 + lane]);
+#pragma unroll 8
+  for (int g = 0; g < kMergeGroups; ++g) {
+    const int at = g * kMergeTokens + tok;
+    merge_into(r, smem[at], smem[1024 + at], smem[2048 + at]);
+    r.n = fminf(r.n, smem[3072 + at]);
   }
   return r;
 }
 
-// forward of the stand-alone op: 64 tokens per workgroup.  vmax / vmin (nullable, together): largest and smallest raw
+// forward of the stand-alone op: kMergeTokens tokens per workgroup.  vmax / vmin (nullable, together): largest and smallest raw
 // logit of the row (what FSDPEngine._get_vocab_min_max_logits takes from materialised logits,
 // areal/engine/fsdp_engine.py:1893-1906); the largest is recovered from the merged exponent k = c * max, i.e. to one
 // rounding, the smallest comes from its own plane.
@@ -364,9 +388,9 @@ __global__ __launch_bounds__(1024) void k_combine(const float* __restrict__ pk, 
                                                   float* __restrict__ row_lse, float* __restrict__ row_ez,
                                                   float* __restrict__ vmax, float* __restrict__ vmin) {
   __shared__ float smem[kMergeSmemFloats];
-  const int t = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int t = blockIdx.x * kMergeTokens + threadIdx.x % kMergeTokens;
   const Merged m = merge_blocks(pk, ps, pu, pn, blocks, pitch_t, t, t < n_tok, smem);
-  if (t >= n_tok || threadIdx.x >= 64) return;
+  if (t >= n_tok || threadIdx.x >= kMergeTokens) return;
   const float log2s = fast_log2(m.s);
   const float mean_t = m.u / m.s;
   logp[t] = (fmaf(xy[t], c, -m.k) - log2s) * kLn2;  // xy is NaN for a label outside [0, V)
@@ -414,9 +438,9 @@ __global__ __launch_bounds__(1024) void k_token_loss(const float* __restrict__ p
                                                      const int32_t* __restrict__ out_rows, float* __restrict__ g_tok,
                                                      float* __restrict__ lse_tok, CarryOut carry) {
   __shared__ float smem[kMergeSmemFloats];
-  const int t = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int t = blockIdx.x * kMergeTokens + threadIdx.x % kMergeTokens;
   const Merged m = merge_blocks(pk, ps, pu, pn, blocks, pitch_t, t, t < n_tok, smem);
-  if (t >= n_tok || threadIdx.x >= 64) return;
+  if (t >= n_tok || threadIdx.x >= kMergeTokens) return;
   const float log2s = fast_log2(m.s);
   const float lp = (fmaf(xy[t], c, -m.k) - log2s) * kLn2;
   a.logp[t] = lp;
@@ -1207,7 +1231,7 @@ extern "C" int aa_lmhead_fwd(const void* hidden, const void* weight, int64_t T, 
     hipLaunchKernelGGL(k_label_logit, dim3((unsigned)((n_tok + 3) / 4)), dim3(256), 0, st, hid, (const uint16_t*)weight,
                        labels + t0, (int)n_tok, (int)H, (int)V, a.xy, (int32_t*)nullptr);
     launch_tiles<kModeStats>(st, weight, hid, n_tok, H, V, a);
-    hipLaunchKernelGGL(k_combine, dim3((unsigned)((n_tok + 63) / 64)), dim3(1024), 0, st, a.pk, a.ps, a.pu, a.pn, a.xy,
+    hipLaunchKernelGGL(k_combine, dim3((unsigned)((n_tok + kMergeTokens - 1) / kMergeTokens)), dim3(1024), 0, st, a.pk, a.ps, a.pu, a.pn, a.xy,
                        (int)w.blocks, a.pitch_t, (int)n_tok, a.c, logp + t0, at(entropy, t0), at(row_lse, t0),
                        at(row_ez, t0), at(vocab_max, t0), at(vocab_min, t0));
   }
@@ -1281,7 +1305,7 @@ extern "C" int aa_lmhead_fwd_static(const void* hidden, const void* weight, int6
     hipLaunchKernelGGL(k_label_logit, dim3((unsigned)((n_tok + 3) / 4)), dim3(256), 0, st, hid, (const uint16_t*)weight,
                        labels + t0, (int)n_tok, (int)H, (int)V, a.xy, (int32_t*)nullptr);
     launch_tiles<kModeStats>(st, weight, hid, n_tok, H, V, a);
-    hipLaunchKernelGGL(k_combine, dim3((unsigned)((n_tok + 63) / 64)), dim3(1024), 0, st, a.pk, a.ps, a.pu,
+    hipLaunchKernelGGL(k_combine, dim3((unsigned)((n_tok + kMergeTokens - 1) / kMergeTokens)), dim3(1024), 0, st, a.pk, a.ps, a.pu,
                        (const float*)nullptr, a.xy, (int)blocks, a.pitch_t, (int)n_tok, a.c, logp + t0, at(entropy, t0),
                        at(row_lse, t0), at(row_ez, t0), (float*)nullptr, (float*)nullptr);
   }
@@ -1415,7 +1439,7 @@ extern "C" int aa_lmhead_fwd_carry(const void* hidden, const void* weight, int64
       launch_tiles<kModeStatsCarry>(st, weight, hid, n_tok, H, V, a);
     else
       launch_tiles<kModeStats>(st, weight, hid, n_tok, H, V, a);
-    hipLaunchKernelGGL(k_combine, dim3((unsigned)((n_tok + 63) / 64)), dim3(1024), 0, st, a.pk, a.ps, a.pu, a.pn, a.xy,
+    hipLaunchKernelGGL(k_combine, dim3((unsigned)((n_tok + kMergeTokens - 1) / kMergeTokens)), dim3(1024), 0, st, a.pk, a.ps, a.pu, a.pn, a.xy,
                        (int)w.blocks, a.pitch_t, (int)n_tok, a.c, logp + t0, at(entropy, t0), row_lse + t0, at(row_ez, t0),
                        at(vocab_max, t0), at(vocab_min, t0));
     row0 += rows;
@@ -1578,7 +1602,7 @@ extern "C" int aa_lmhead_ppo_fused(const void* hidden, const void* weight, int64
     // row statistics, per-token outputs, g
     TokenLossArgs la{at(prox_logp), at(adv), at(mask_eff), at(behave_w), n_valid, grad_scale, logp + t0, at(entropy),
                      at(stat_loss), at(ratio), at(flags), at(vocab_max), at(vocab_min), *params, act};
-    hipLaunchKernelGGL(k_token_loss, dim3((unsigned)((n_tok + 63) / 64)), dim3(1024), 0, st, a.pk, a.ps, a.pu, a.pn, a.xy,
+    hipLaunchKernelGGL(k_token_loss, dim3((unsigned)((n_tok + kMergeTokens - 1) / kMergeTokens)), dim3(1024), 0, st, a.pk, a.ps, a.pu, a.pn, a.xy,
                        (int)w.blocks, a.pitch_t, (int)n_tok, (int)V, a.c, inv_temperature, labels + t0, la, row_of_token,
                        g_tok, lse_tok,
                        (carry && rows > 0) ? CarryOut{row_factor, panel, w.panel_ld, redo_flag}
