@@ -500,13 +500,6 @@ __global__ __launch_bounds__(1024) void k_token_loss(const float* __restrict__ p
   }
 }
 
-// After the conditional recompute of a flagged chunk the panel holds d(logits) itself: every row factor becomes 1.
-__global__ __launch_bounds__(256) void k_unit_factors(float* __restrict__ row_factor, int rows, const int32_t* __restrict__ flag) {
-  if (*flag == 0) return;
-  const int r = blockIdx.x * 256 + threadIdx.x;
-  if (r < rows) row_factor[r] = 1.f;
-}
-
 // Backward of the stand-alone op in carry form: what k_token_loss does for the rows of the training step, for upstream
 // gradients that only exist once the forward has returned.  Per token t of the chunk with a panel row r: the row's
 // factor -(g / T) p_label from the saved log-prob, the label entry patched to 1 - 1 / p_label, and the chunk's redo
@@ -788,13 +781,14 @@ __global__ __launch_bounds__(256) void k_splitk_rows(const float* __restrict__ p
 // beyond it are dropped.  A host count larger than what the mask holds leaves positions without a token: they get
 // act_rows = -1 (the gathers then produce zero rows and the scatters skip them) and a row factor of zero when factors
 // are in use; the true count goes to total_out (the four row-count words of the chunk; dh_tiles_m, dh_slices and units
-// describe the d_hidden product for choose_splits), and k_clear_surplus_rows, launched behind this kernel, clears their
-// panel rows, which no tile writes, so that nothing stale (possibly not even finite) enters the d_weight product.
+// describe the d_hidden product for choose_splits), and k_backward_rows, ahead of the gradient GEMMs, clears their panel
+// rows, which no tile writes, so that nothing stale (possibly not even finite) enters the d_weight product.
 // One workgroup; mask has `act` entries (tokens at and after `act` have none).
 __global__ __launch_bounds__(1024) void k_compact_map(const uint8_t* __restrict__ mask, int act, int n_tok, int limit,
                                                       int32_t* __restrict__ out_rows, int32_t* __restrict__ act_rows,
                                                       float* __restrict__ row_factor, int32_t* __restrict__ total_out,
-                                                      int dh_tiles_m, int dh_slices, int units) {
+                                                      int dh_tiles_m, int dh_slices, int units,
+                                                      int32_t* __restrict__ clear_flag) {
   __shared__ int wave_sum[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int per = (n_tok + 1023) / 1024;
@@ -825,6 +819,7 @@ __global__ __launch_bounds__(1024) void k_compact_map(const uint8_t* __restrict_
     const int live = (rows + BN - 1) / BN;
     const int splits = choose_splits_wave(dh_tiles_m * live, dh_slices, units);
     if (lane == 0) {
+      if (clear_flag) *clear_flag = 0;  // the chunk's "redo by recompute" flag
       total_out[kRowsTotal] = rows;
       total_out[kRowsLive] = live;
       total_out[kRowsSliced] = rows > 0 ? (rows + BK - 1) / BK * BK : BK;
@@ -837,62 +832,70 @@ __global__ __launch_bounds__(1024) void k_compact_map(const uint8_t* __restrict_
   }
 }
 
-// Panel rows [*total, limit) are rows without a token (see k_compact_map): cleared, one workgroup per row at a time.
-// In the usual case (*total == limit) every workgroup returns at once.
-// With `bounded` the kernels that read the panel stop at *total themselves (rounded up to a K slice of the d_weight
-// product), and only the rows up to there are cleared.
-__global__ __launch_bounds__(256) void k_clear_surplus_rows(const int32_t* __restrict__ total, int limit, int bounded,
-                                                            u32x4_t* __restrict__ panel, int64_t panel_ld) {
-  const u32x4_t zero = {0u, 0u, 0u, 0u};
-  const int64_t vec = panel_ld / 8;
-  if (bounded) {
-    const int up = total[kRowsSliced];
-    limit = up < limit ? up : limit;
-  }
-  for (int64_t r = (int64_t)*total + blockIdx.x; r < limit; r += gridDim.x)
-    for (int64_t i = threadIdx.x; i < vec; i += 256) panel[r * vec + i] = zero;
-}
-
 static int compute_units();
 
-// numbering of the tokens with a panel row, and the rows without a token cleared (both kernels); H and V are those of
-// the lm_head (they shape the d_hidden product that the row-count words describe)
+// numbering of the tokens with a panel row; H and V are those of the lm_head (they shape the d_hidden product that the
+// row-count words describe)
 static void launch_compact_map(hipStream_t st, const uint8_t* mask, int64_t act, int64_t n_tok, int64_t limit,
-                               int32_t* out_rows, int32_t* act_rows, float* row_factor, int32_t* total_word,
-                               uint16_t* panel, int64_t panel_ld, int64_t H, int64_t V, bool bounded = false) {
+                               int32_t* out_rows, int32_t* act_rows, float* row_factor, int32_t* total_word, int64_t H,
+                               int64_t V, int32_t* clear_flag = nullptr) {
   hipLaunchKernelGGL(k_compact_map, dim3(1), dim3(1024), 0, st, mask, (int)act, (int)n_tok, (int)limit, out_rows, act_rows,
-                     row_factor, total_word, (int)((H + BM - 1) / BM), (int)((V + BK - 1) / BK), compute_units());
-  const int64_t blocks = bounded ? (limit < BK ? limit : BK) : (limit < 512 ? limit : 512);
-  if (blocks > 0)
-    hipLaunchKernelGGL(k_clear_surplus_rows, dim3((unsigned)blocks), dim3(256), 0, st, total_word, (int)limit,
-                       bounded ? 1 : 0, (u32x4_t*)panel, panel_ld);
+                     row_factor, total_word, (int)((H + BM - 1) / BM), (int)((V + BK - 1) / BK), compute_units(), clear_flag);
 }
 
-// dst[r, :] = scale[r] * src[rows[r], :] (H % 8 == 0); rows == nullptr: row r itself (a negative entry: a zero row);
-// scale == nullptr: 1;
-// run_if, when given: nothing happens unless *run_if != 0
-__global__ __launch_bounds__(256) void k_gather_rows(const u32x4_t* __restrict__ src, const int32_t* __restrict__ rows,
-                                                     u32x4_t* __restrict__ dst, int h_vec,
-                                                     const float* __restrict__ scale, const int32_t* __restrict__ run_if) {
-  if (run_if && *run_if == 0) return;
-  const int64_t r = blockIdx.x;
-  const int64_t t = rows ? rows[r] : r;
+// ---- everything per row that lies between the loss and the gradient GEMMs, in one launch ------------------------------
+// (each of these was a launch of its own, about 5 us on the stream and idle in the usual case: 25 us of a step)
+struct BackwardRows {
+  const u32x4_t* hidden;     // [n_tok, h_vec] of the chunk
+  u32x4_t* rows;             // [n_rows, h_vec]: the hidden rows of the panel rows, closed up
+  const int32_t* token_of_row;  // nullable: row r itself
+  const int32_t* row_of_token;  // with token_of_row
+  float* row_factor;         // nullable (1): factor per panel row
+  const int32_t* redo_flag;  // with row_factor: the chunk's redo flag
+  u32x4_t* d_hidden;         // nullable: [n_tok, h_vec], the rows of the tokens without a panel row are cleared
+  const int32_t* total;      // with token_of_row: the row-count words of the chunk
+  u32x4_t* panel;
+  int64_t panel_vec;
+  int n_tok, n_rows, h_vec;
+  int bounded;               // the GEMMs stop at the rows in use (rounded up to a K slice)
+};
+
+// Workgroup i, as token i: its d_hidden row is cleared when it has no panel row.  As row i: rows[i] = factor[i] *
+// hidden[token] (a row without a token: zeros); panel rows at and past the number of tokens that the mask really holds
+// are cleared, as far as the GEMMs read.  A chunk whose redo flag is set is about to be redone by the recompute tiles,
+// after which the panel holds d(logits) itself: its factors become 1, and the rows are the plain hidden rows that those
+// tiles multiply.
+__global__ __launch_bounds__(256) void k_backward_rows(BackwardRows a) {
+  const u32x4_t zero = {0u, 0u, 0u, 0u};
+  const int i = blockIdx.x;
+  if (a.d_hidden && i < a.n_tok && a.row_of_token[i] < 0)
+    for (int j = threadIdx.x; j < a.h_vec; j += 256) a.d_hidden[(int64_t)i * a.h_vec + j] = zero;
+  if (i >= a.n_rows) return;
+  if (a.token_of_row && i >= a.total[kRowsTotal]) {
+    const int up = a.total[kRowsSliced];
+    if (i < (a.bounded && up < a.n_rows ? up : a.n_rows))
+      for (int64_t j = threadIdx.x; j < a.panel_vec; j += 256) a.panel[(int64_t)i * a.panel_vec + j] = zero;
+  }
+  const int t = a.token_of_row ? a.token_of_row[i] : i;
+  u32x4_t* dst = a.rows + (int64_t)i * a.h_vec;
   if (t < 0) {  // a position without a token
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
-    for (int j = threadIdx.x; j < h_vec; j += 256) dst[r * h_vec + j] = zero;
+    for (int j = threadIdx.x; j < a.h_vec; j += 256) dst[j] = zero;
     return;
   }
-  if (!scale) {
-    for (int j = threadIdx.x; j < h_vec; j += 256) dst[r * h_vec + j] = src[t * h_vec + j];
+  const u32x4_t* src = a.hidden + (int64_t)t * a.h_vec;
+  const bool redo = a.row_factor && *a.redo_flag != 0;
+  if (!a.row_factor || redo) {
+    for (int j = threadIdx.x; j < a.h_vec; j += 256) dst[j] = src[j];
+    if (redo && threadIdx.x == 0) a.row_factor[i] = 1.f;
     return;
   }
-  const float f = scale[r];
-  for (int j = threadIdx.x; j < h_vec; j += 256) {
+  const float f = a.row_factor[i];
+  for (int j = threadIdx.x; j < a.h_vec; j += 256) {
     float x[8];
-    load8<AA_BF16>((const uint16_t*)(src + t * h_vec), (int64_t)j * 8, x);
+    load8<AA_BF16>((const uint16_t*)src, (int64_t)j * 8, x);
 #pragma unroll
     for (int q = 0; q < 8; ++q) x[q] *= f;
-    store8<AA_BF16>((uint16_t*)(dst + r * h_vec), (int64_t)j * 8, x);
+    store8<AA_BF16>((uint16_t*)dst, (int64_t)j * 8, x);
   }
 }
 
@@ -946,8 +949,6 @@ struct Workspace {
 
 // external_panel: the d(logits) rows live in an array of the caller's (the op that keeps them from its forward to its
 // backward), not in the workspace
-static int compute_units();
-
 static Workspace plan(int64_t T, int64_t H, int64_t V, bool external_panel = false) {
   Workspace w{};
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
@@ -1061,26 +1062,46 @@ static void launch_d_weight(hipStream_t st, const uint16_t* hid_rows, int64_t H,
                                                 bounds);
 }
 
+// The rows of a chunk made ready for the backward (k_backward_rows).  Returns the hidden rows that belong to the panel
+// rows: closed up and scaled in the workspace, or the chunk's own when every token has a row and there are no factors.
+// d_hidden_chunk: the rows of the tokens without a panel row are cleared (with a row map).
+static const uint16_t* backward_rows(hipStream_t st, const Workspace& w, char* ws, const uint16_t* hid,
+                                     const int32_t* row_of_token, const int32_t* token_of_row, float* row_factor,
+                                     const int32_t* redo_flag, int64_t n_tok, int64_t n_rows, int64_t H,
+                                     uint16_t* d_hidden_chunk, uint16_t* panel, bool bounded) {
+  if (!token_of_row && !row_factor) return hid;
+  BackwardRows a;
+  a.hidden = (const u32x4_t*)hid;
+  a.rows = (u32x4_t*)(ws + w.off_hc);
+  a.token_of_row = token_of_row;
+  a.row_of_token = row_of_token;
+  a.row_factor = row_factor;
+  a.redo_flag = redo_flag;
+  a.d_hidden = token_of_row ? (u32x4_t*)d_hidden_chunk : nullptr;
+  a.total = (const int32_t*)(ws + w.off_total);
+  a.panel = (u32x4_t*)panel;
+  a.panel_vec = w.panel_ld / 8;
+  a.n_tok = (int)n_tok;
+  a.n_rows = (int)n_rows;
+  a.h_vec = (int)(H / 8);
+  a.bounded = bounded ? 1 : 0;
+  hipLaunchKernelGGL(k_backward_rows, dim3((unsigned)(n_tok > n_rows ? n_tok : n_rows)), dim3(256), 0, st, a);
+  return (const uint16_t*)a.rows;
+}
+
 // The two GEMMs that contract the d(logits) rows ds [n_rows, V] of one token chunk, ds = row_factor[r] * panel[r, :]
 // (row_factor == nullptr: the panel holds d(logits) itself):
 //   d_hidden rows [n_rows, H] = ds . W                  contraction over V: panel K-contiguous, W [V, H] K-major;
 //                                                       the factor multiplies the fp32 sums in the epilogue
 //   d_weight [V, H] (+)= ds^T . hidden rows             contraction over the rows: both arrays K-major; the factor
-//                                                       goes into the copy of the hidden rows
-// No transposed copy of anything is made.  token_of_row, when given, lists the tokens of the chunk that the n_rows
-// rows belong to (tokens without gradient were left out): their hidden rows are closed up first, and the d_hidden rows
-// go to those tokens (the caller has cleared the others).
+//                                                       is in the hidden rows already
+// No transposed copy of anything is made.  hid_rows: what backward_rows returned.  token_of_row, when given, lists the
+// tokens of the chunk that the n_rows rows belong to (tokens without gradient were left out): the d_hidden rows go to
+// those tokens (the others have been cleared).
 static void panel_gradients(hipStream_t st, const Workspace& w, char* ws, const uint16_t* ds, const void* weight,
-                            const uint16_t* hid, const int32_t* token_of_row, const float* row_factor, int64_t n_rows,
+                            const uint16_t* hid_rows, const int32_t* token_of_row, const float* row_factor, int64_t n_rows,
                             int64_t H, int64_t V, uint16_t* d_hidden_chunk, void* d_weight, bool dw_f32, bool first,
                             const int32_t* rows_in_use = nullptr) {
-  const uint16_t* hid_rows = hid;
-  if (token_of_row || row_factor) {
-    uint16_t* hc = (uint16_t*)(ws + w.off_hc);
-    hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)n_rows), dim3(256), 0, st, (const u32x4_t*)hid, token_of_row,
-                       (u32x4_t*)hc, (int)(H / 8), row_factor, (const int32_t*)nullptr);
-    hid_rows = hc;
-  }
   const int64_t ldp = w.panel_ld;
   {
     const int tiles_m = (int)((H + BM - 1) / BM), tiles_n = (int)((n_rows + BN - 1) / BN);
@@ -1094,14 +1115,17 @@ static void panel_gradients(hipStream_t st, const Workspace& w, char* ws, const 
       // row-count words say whether the product is cut along the vocabulary and into how many parts (what the host
       // would have chosen with that count), and the form that is not in turn returns at once
       int64_t cut_groups = 0, cut_rows = 0;  // the largest grid, and the most rows, the cut product can come with
+      bool uncut = false;                    // the product can come uncut
       for (int tn = 1; tn <= tiles_n; ++tn) {
         const int parts = choose_splits((int64_t)tiles_m * tn, slices, units);
+        uncut |= parts == 1;
         if (parts == 1) continue;
         if ((int64_t)tiles_m * tn * parts > cut_groups) cut_groups = (int64_t)tiles_m * tn * parts;
         cut_rows = (int64_t)tn * BN < n_rows ? (int64_t)tn * BN : n_rows;
       }
-      launch_gemm<true, false, uint16_t, false, kBoundN>(st, (const uint16_t*)weight, H, H, ds, ldp, n_rows, V,
-                                                         d_hidden_chunk, H, token_of_row, row_factor, rows_in_use);
+      if (uncut)
+        launch_gemm<true, false, uint16_t, false, kBoundN>(st, (const uint16_t*)weight, H, H, ds, ldp, n_rows, V,
+                                                           d_hidden_chunk, H, token_of_row, row_factor, rows_in_use);
       if (cut_groups) {
         hipLaunchKernelGGL((k_gemm_splitk<true, false, true>), dim3((unsigned)cut_groups), dim3(kThreads), kLdsBytes, st, a,
                            b, (int)V, tiles_m, tiles_n, 0, part, H, plane, rows_in_use);
@@ -1128,26 +1152,18 @@ static void panel_gradients(hipStream_t st, const Workspace& w, char* ws, const 
 }
 
 // Recompute: d(logits) of the panel rows from the logits tiles formed again.  With a row map only the hidden rows that
-// have a panel row are multiplied (gathered first); `a` carries the per-token inputs of the chunk.  With run_if the
-// kernels are enqueued but do nothing unless *run_if != 0 when they start.
-static void recompute_panel(hipStream_t st, const Workspace& w, char* ws, uint16_t* panel, const void* weight,
-                            const uint16_t* hid, int64_t n_tok, const int32_t* token_of_row, int64_t rows, int64_t H,
-                            int64_t V, TileArgs a, const int32_t* run_if = nullptr, const int32_t* rows_in_use = nullptr) {
+// have a panel row are multiplied (hid_rows, closed up by backward_rows); without one, the chunk's own.  `a` carries the
+// per-token inputs of the chunk.  With run_if the kernel is enqueued but does nothing unless *run_if != 0 when it starts.
+static void recompute_panel(hipStream_t st, const Workspace& w, uint16_t* panel, const void* weight,
+                            const uint16_t* hid_rows, const int32_t* token_of_row, int64_t rows, int64_t H, int64_t V,
+                            TileArgs a, const int32_t* run_if = nullptr, const int32_t* rows_in_use = nullptr) {
   a.panel = panel;
   a.panel_ld = w.panel_ld;
   a.out_rows = nullptr;
   a.run_if = run_if;
   a.n_bound = token_of_row ? rows_in_use : nullptr;
-  if (!token_of_row) {
-    a.col_tokens = nullptr;
-    launch_tiles<kModeRecompute>(st, weight, hid, n_tok, H, V, a);
-    return;
-  }
-  uint16_t* hc = (uint16_t*)(ws + w.off_hc);
-  hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)rows), dim3(256), 0, st, (const u32x4_t*)hid, token_of_row, (u32x4_t*)hc,
-                     (int)(H / 8), (const float*)nullptr, run_if);
   a.col_tokens = token_of_row;
-  launch_tiles<kModeRecompute>(st, weight, hc, rows, H, V, a);
+  launch_tiles<kModeRecompute>(st, weight, hid_rows, rows, H, V, a);
 }
 
 // d_weight of dtype AA_F32 is accumulated in place.  A bf16 d_weight is written by the GEMM itself when there is one
@@ -1348,7 +1364,7 @@ extern "C" int aa_lmhead_bwd(const void* hidden, const void* weight, int64_t T, 
     a.g_logp = g_logp + t0;
     a.g_entropy = g_entropy ? g_entropy + t0 : nullptr;
     if (!kept_per_chunk) {
-      recompute_panel(st, w, ws, ws_panel, weight, hid, n_tok, nullptr, n_tok, H, V, a);
+      recompute_panel(st, w, ws_panel, weight, hid, nullptr, n_tok, H, V, a);
       panel_gradients(st, w, ws, ws_panel, weight, hid, nullptr, nullptr, n_tok, H, V, dh, dw.acc, dw.acc_f32, first);
       first = false;
       continue;
@@ -1363,11 +1379,11 @@ extern "C" int aa_lmhead_bwd(const void* hidden, const void* weight, int64_t T, 
     }
     int32_t* total_word = (int32_t*)(ws + w.off_total);
     const int32_t* rows_in_use = on_device ? total_word : nullptr;
-    launch_compact_map(st, row_has_gradient + t0, n_tok, n_tok, kept, out_rows, act_rows, nullptr, total_word, ws_panel,
-                       w.panel_ld, H, V, on_device);
-    recompute_panel(st, w, ws, ws_panel, weight, hid, n_tok, act_rows, kept, H, V, a, nullptr, rows_in_use);
-    launch_zero(st, dh, n_tok * H * 2);  // the rows of the other tokens
-    panel_gradients(st, w, ws, ws_panel, weight, hid, act_rows, nullptr, kept, H, V, dh, dw.acc, dw.acc_f32, first,
+    launch_compact_map(st, row_has_gradient + t0, n_tok, n_tok, kept, out_rows, act_rows, nullptr, total_word, H, V);
+    const uint16_t* hid_rows = backward_rows(st, w, ws, hid, out_rows, act_rows, nullptr, nullptr, n_tok, kept, H, dh,
+                                             ws_panel, on_device);
+    recompute_panel(st, w, ws_panel, weight, hid_rows, act_rows, kept, H, V, a, nullptr, rows_in_use);
+    panel_gradients(st, w, ws, ws_panel, weight, hid_rows, act_rows, nullptr, kept, H, V, dh, dw.acc, dw.acc_f32, first,
                     rows_in_use);
     first = false;
   }
@@ -1427,7 +1443,7 @@ extern "C" int aa_lmhead_fwd_carry(const void* hidden, const void* weight, int64
       const bool on_device = rows == AA_LMHEAD_COUNT_ON_DEVICE;  // the chunk keeps room for every token
       rows = on_device ? n_tok : (rows < 0 ? 0 : (rows > n_tok ? n_tok : rows));
       launch_compact_map(st, row_has_gradient + t0, n_tok, n_tok, rows, out_rows, act_rows, nullptr,
-                         (int32_t*)(ws + w.off_total), chunk_panel, w.panel_ld, H, V, on_device);
+                         (int32_t*)(ws + w.off_total), H, V);
     }
     TileArgs a = stats_args(w, ws, labels + t0, inv_temperature, vocab_min != nullptr);
     a.panel = chunk_panel;
@@ -1482,7 +1498,9 @@ extern "C" int aa_lmhead_bwd_carry(const void* hidden, const void* weight, int64
     const int32_t* row_of_token = nullptr;
     const int32_t* token_of_row = nullptr;
     const int32_t* rows_in_use = nullptr;  // the count of the chunk, when only the device has it
-    if (kept_per_chunk) {
+    if (!kept_per_chunk) {
+      launch_zero(st, redo_flag, 256);
+    } else {
       rows = kept_per_chunk[chunk_index];
       const bool on_device = rows == AA_LMHEAD_COUNT_ON_DEVICE;
       rows = on_device ? n_tok : (rows < 0 ? 0 : (rows > n_tok ? n_tok : rows));
@@ -1492,13 +1510,12 @@ extern "C" int aa_lmhead_bwd_carry(const void* hidden, const void* weight, int64
       }
       // the same numbering as in the forward (the mask has not changed); surplus rows get a factor of zero
       int32_t* total_word = (int32_t*)(ws + w.off_total);
-      launch_compact_map(st, row_has_gradient + t0, n_tok, n_tok, rows, out_rows, act_rows, row_factor, total_word,
-                         chunk_panel, w.panel_ld, H, V, on_device);
+      launch_compact_map(st, row_has_gradient + t0, n_tok, n_tok, rows, out_rows, act_rows, row_factor, total_word, H, V,
+                         redo_flag);
       if (on_device) rows_in_use = total_word;
       row_of_token = out_rows;
       token_of_row = act_rows;
     }
-    launch_zero(st, redo_flag, 256);
     hipLaunchKernelGGL(k_carry_factors, dim3((unsigned)((n_tok + 255) / 256)), dim3(256), 0, st, logp + t0, g_logp + t0,
                        labels + t0, row_of_token, (int)n_tok, (int)V, inv_temperature,
                        CarryOut{row_factor, chunk_panel, w.panel_ld, redo_flag});
@@ -1510,10 +1527,11 @@ extern "C" int aa_lmhead_bwd_carry(const void* hidden, const void* weight, int64
     a.row_lse = row_lse + t0;
     a.g_logp = g_logp + t0;
     a.panel_ld = w.panel_ld;
-    recompute_panel(st, w, ws, chunk_panel, weight, hid, n_tok, token_of_row, rows, H, V, a, redo_flag, rows_in_use);
-    hipLaunchKernelGGL(k_unit_factors, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, row_factor, (int)rows, redo_flag);
-    if (token_of_row) launch_zero(st, dh, n_tok * H * 2);  // the rows of the tokens without a panel row
-    panel_gradients(st, w, ws, chunk_panel, weight, hid, token_of_row, row_factor, rows, H, V, dh, dw.acc, dw.acc_f32, first,
+    const uint16_t* hid_rows = backward_rows(st, w, ws, hid, row_of_token, token_of_row, row_factor, redo_flag, n_tok, rows,
+                                             H, dh, chunk_panel, rows_in_use != nullptr);
+    recompute_panel(st, w, chunk_panel, weight, token_of_row ? hid_rows : hid, token_of_row, rows, H, V, a, redo_flag,
+                    rows_in_use);
+    panel_gradients(st, w, ws, chunk_panel, weight, hid_rows, token_of_row, row_factor, rows, H, V, dh, dw.acc, dw.acc_f32, first,
                     rows_in_use);
     first = false;
     row0 += rows;
@@ -1583,7 +1601,7 @@ extern "C" int aa_lmhead_ppo_fused(const void* hidden, const void* weight, int64
       rows = on_device ? act : (rows < 0 ? 0 : (rows > act ? act : rows));
       int32_t* total_word = (int32_t*)(ws + w.off_total);
       launch_compact_map(st, at(mask_eff), act, n_tok, rows, out_rows, act_rows, carry ? row_factor : nullptr, total_word,
-                         panel, w.panel_ld, H, V, on_device);
+                         H, V);
       if (on_device) rows_in_use = total_word;
       row_of_token = out_rows;
       token_of_row = act_rows;
@@ -1615,12 +1633,11 @@ extern "C" int aa_lmhead_ppo_fused(const void* hidden, const void* weight, int64
     // device: the kernels start and return at once otherwise), and then the row factors become 1
     a.row_lse = lse_tok;
     a.g_logp = g_tok;
-    recompute_panel(st, w, ws, panel, weight, hid, n_tok, token_of_row, rows, H, V, a, carry ? redo_flag : nullptr,
-                    rows_in_use);
-    if (carry)
-      hipLaunchKernelGGL(k_unit_factors, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, row_factor, (int)rows, redo_flag);
-    if (token_of_row) launch_zero(st, dh, n_tok * H * 2);  // the rows of the tokens without gradient
-    panel_gradients(st, w, ws, panel, weight, hid, token_of_row, carry ? row_factor : nullptr, rows, H, V, dh, dw.acc,
+    const uint16_t* hid_rows = backward_rows(st, w, ws, hid, row_of_token, token_of_row, carry ? row_factor : nullptr,
+                                             redo_flag, n_tok, rows, H, dh, panel, rows_in_use != nullptr);
+    recompute_panel(st, w, panel, weight, token_of_row ? hid_rows : hid, token_of_row, rows, H, V, a,
+                    carry ? redo_flag : nullptr, rows_in_use);
+    panel_gradients(st, w, ws, panel, weight, hid_rows, token_of_row, carry ? row_factor : nullptr, rows, H, V, dh, dw.acc,
                     dw.acc_f32, first, rows_in_use);
     first = false;
   }
