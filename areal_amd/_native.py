@@ -43,6 +43,74 @@ class PpoParams(C.Structure):
     ]
 
 
+class RsParams(C.Structure):
+    """``aa_rs_params``"""
+
+    _fields_ = [
+        ("enabled", C.c_int32),
+        ("level", C.c_int32),
+        ("action", C.c_int32),
+        ("metric", C.c_int32),
+        ("agg", C.c_int32),
+        ("has_lower", C.c_int32),
+        ("upper", C.c_float),
+        ("lower", C.c_float),
+    ]
+
+
+class LossScale(C.Structure):
+    """``aa_loss_scale``"""
+
+    _fields_ = [
+        ("factor", C.c_void_p),
+        ("total", C.c_void_p),
+        ("value", C.c_float),
+        ("total_value", C.c_float),
+        ("per_valid_token", C.c_int32),
+    ]
+
+
+STEP_WORK_BYTES = 4096  # AA_STEP_WORK_BYTES
+
+
+class PpoStep(C.Structure):
+    """``aa_ppo_step``"""
+
+    _fields_ = [
+        ("T", C.c_int64),
+        ("T_active", C.c_int64),
+        ("prox_logp", C.c_void_p),
+        ("old_logp", C.c_void_p),
+        ("adv", C.c_void_p),
+        ("mask", C.c_void_p),
+        ("cu_seqlens", C.c_void_p),
+        ("n_segments", C.c_int64),
+        ("params", PpoParams),
+        ("rs", RsParams),
+        ("scale", LossScale),
+        ("logp", C.c_void_p),
+        ("entropy", C.c_void_p),
+        ("vmax", C.c_void_p),
+        ("vmin", C.c_void_p),
+        ("stat_loss", C.c_void_p),
+        ("ratio", C.c_void_p),
+        ("flags", C.c_void_p),
+        ("approx_kl", C.c_void_p),
+        ("clip_mask", C.c_void_p),
+        ("dual_clip_mask", C.c_void_p),
+        ("behave_mask", C.c_void_p),
+        ("behave_kl", C.c_void_p),
+        ("mask_out", C.c_void_p),
+        ("behave_w", C.c_void_p),
+        ("counts", C.c_void_p),
+        ("counts_given", C.c_int32),
+        ("loss", C.c_void_p),
+        ("host_counts", C.c_void_p),
+        ("host_tag", C.c_int32),
+        ("work", C.c_void_p),
+    ]
+
+
 class NormParams(C.Structure):
     """``aa_norm_params``"""
 
@@ -73,6 +141,9 @@ SIGNATURES = {
         [_p, _i, _i64, _i64, _i64, _p, _f, _i64, _p, _p, _p, _p, C.POINTER(PpoParams), _p, _p,
          _p, _p, _p, _p, _p, _p, _p, _p, _p, _p],
     ),
+    "aa_logits_ppo_step": (_i, [C.POINTER(PpoStep), _p, _i, _i64, _i64, _p, _f, _p, _p]),
+    "aa_ppo_loss_step": (_i, [C.POINTER(PpoStep), _p, _i, _i, _p, _p]),
+    "aa_lmhead_ppo_step": (_i, [C.POINTER(PpoStep), _p, _p, _i64, _i64, _p, _f, _p, _i, _p, _p, _i, _p, _i64, _p]),
     "aa_vocab_partials_combine": (_i, [_p, _p, _p, _i, _i64, _p, _p, _p, _p, _p]),
     "aa_logits_pairs_fwd": (_i, [_p, _i, _i64, _i64, _i64, _p, _p, _i64, _f, _p, _p, _p, _p, _p]),
     "aa_logits_pairs_scatter": (_i, [_p, _i, _i64, _i64, _i64, _p, _p, _i64, _p, _f, _p]),

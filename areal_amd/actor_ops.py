@@ -10,7 +10,7 @@ from typing import Any
 import torch
 
 from . import _native as N
-from .functional import _f32, _mask_u8, _ptr, _require_gpu, _stream
+from .functional import _f32, _mask_u8, _on, _ptr, _require_gpu, _stream
 
 PROX_APPROX_METHOD_LOGLINEAR = "loglinear"
 PROX_APPROX_METHOD_LINEAR = "linear"
@@ -71,7 +71,7 @@ def apply_m2po_masking(old_logp: torch.Tensor, prox_logp: torch.Tensor, loss_mas
     ws = torch.empty(lib.aa_m2po_workspace_bytes(n), dtype=torch.uint8, device=dev)
     out = torch.empty(n, dtype=torch.bool, device=dev)
     info = torch.empty(2, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(lib.aa_m2po_mask(_ptr(lo), _ptr(lp), _ptr(m8), n, float(m2_threshold), _ptr(out), _ptr(info), _ptr(ws),
                                  ws.numel(), _stream(dev)), "aa_m2po_mask")
     return out.view(shape)
@@ -91,7 +91,7 @@ class _KdTerms(torch.autograd.Function):
         dterm = torch.empty(n, dtype=torch.float32, device=dev)
         mean = torch.empty((), dtype=torch.float32, device=dev)
         n_valid = _count_nonzero(mask_u8)
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = _stream(dev)
             N.check(lib.aa_kd_terms(_ptr(logp), _ptr(old), _ptr(teacher), _ptr(mask_u8), n, 1 if pure else 0, _ptr(term),
                                     _ptr(dterm), st), "aa_kd_terms")
@@ -178,7 +178,7 @@ def proximal_logging_stats(old_logp: torch.Tensor, logprobs: torch.Tensor, prox_
     dev = lo.device
     out = torch.empty(36, 4, dtype=torch.float32, device=dev)
     scratch = torch.empty(lib.aa_logging_stats_scratch_bytes(n), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(lib.aa_logging_stats(_ptr(lo), _ptr(ln), _ptr(gt), _ptr(ver), _ptr(m8), n,
                                      int(current_version) if have_versions else 0, methods, 1 if with_errors else 0,
                                      _ptr(out), _ptr(scratch), scratch.numel(), _stream(dev)), "aa_logging_stats")

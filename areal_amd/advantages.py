@@ -13,7 +13,7 @@ from typing import Any, Mapping
 import torch
 
 from . import _native as N
-from .functional import _f32, _mask_u8, _ptr, _require_gpu, _stream
+from .functional import _f32, _mask_u8, _on, _ptr, _require_gpu, _stream
 
 _LEVELS = {None: 0, "none": 0, "batch": 1, "group": 2}
 
@@ -66,7 +66,7 @@ class Normalization:
         n_bytes = lib.aa_normalize_scratch_bytes(bs, inner, int(self.group_size) if grouped else max(bs, 1))
         scratch = torch.empty(max(n_bytes, 32) // 8, dtype=torch.float64, device=dev)
         out = torch.empty_like(xf)
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(
                 lib.aa_normalize(_ptr(xf), _ptr(mf), bs, inner, C.byref(params), _ptr(out), _ptr(scratch),
                                  scratch.numel() * 8, _stream(dev)),
@@ -100,7 +100,7 @@ def gae_advantages(rewards: torch.Tensor, values: torch.Tensor | None, loss_mask
     adv = torch.empty_like(r)
     ret = torch.empty_like(r)
     lib = N.load()
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(
             lib.aa_gae(_ptr(r), _ptr(v), _ptr(m), _ptr(ne), bs, L, float(discount), float(gae_lambda), _ptr(adv),
                        _ptr(ret), _stream(dev)),
@@ -136,7 +136,7 @@ def masked_moments(values: Mapping[str, torch.Tensor], mask: torch.Tensor) -> di
     out = torch.empty(len(names), 4, dtype=torch.float32, device=dev)
     ptrs = (C.c_void_p * len(names))(*[t.data_ptr() for t in tensors])
     lib = N.load()
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(lib.aa_masked_moments(ptrs, len(names), _ptr(m8), n, _ptr(out), _stream(dev)), "aa_masked_moments")
     res = {}
     for i, k in enumerate(names):
@@ -170,7 +170,7 @@ def kl_regularized_rewards(old_logp: torch.Tensor, ref_logp: torch.Tensor | None
     if sl.numel() != bs or sc.numel() != bs:
         raise ValueError("seqlens and reward_score must have one entry per sequence")
     rewards, kl_rewards = torch.empty_like(lo), torch.empty_like(lo)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(
             N.load().aa_kl_rewards(_ptr(lo), _ptr(lr), _ptr(m), _ptr(sl), _ptr(sc), bs, L, float(kl_ctl),
                                    _KL_IDS[kl_estimator], int(bool(mask_no_eos_with_zero)), _ptr(rewards),
@@ -193,7 +193,7 @@ def reward_overlong_penalty(data: dict, overlong_tokens: int, overlong_penalty_f
     bs, L = mask.shape
     dev = rewards.device
     r = rewards if (rewards.dtype == torch.float32 and rewards.is_contiguous()) else _f32(rewards).contiguous()
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(
             N.load().aa_overlong_penalty(_ptr(r), _ptr(_f32(mask.to(dev)).contiguous()), bs, L, int(overlong_tokens),
                                          float(overlong_penalty_factor), int(max_response_length), _stream(dev)),
@@ -237,7 +237,7 @@ def masked_normalization(x: torch.Tensor, mask: torch.Tensor | None = None, dim=
         lib = N.load()
         dev = x.device
         scratch = torch.empty(lib.aa_masked_normalization_scratch_bytes(rows, cols), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(lib.aa_masked_normalization(_ptr(xv), _ptr(mv), rows, cols, 1 if unbiased else 0, float(eps),
                                                 _ptr(out), _ptr(scratch), scratch.numel(), _stream(dev)),
                     "aa_masked_normalization")
@@ -271,7 +271,7 @@ class KLEstimator:
             raise ValueError("log_probs and log_probs_base must have the same shape")
         a, b = _f32(log_probs), _f32(log_probs_base.to(log_probs.device))
         out = torch.empty_like(a)
-        with torch.cuda.device(a.device):
+        with _on(a.device):
             N.check(N.load().aa_kl_estimate(_ptr(a), _ptr(b), a.numel(), _KL_IDS[kl_estimator], 1 if apply_clamp else 0,
                                             _ptr(out), _stream(a.device)), "aa_kl_estimate")
         return out

@@ -24,6 +24,7 @@
 #include "device_utils.h"
 #include "gemm_tn.h"
 #include "ppo_math.h"
+#include "ppo_step.h"
 
 namespace aa {
 namespace lmhead {
@@ -415,7 +416,7 @@ struct TokenLossArgs {
   const uint8_t* mask_eff;
   const float* behave_w;
   const int32_t* n_valid;
-  const float* grad_scale;
+  aa_loss_scale scale;
   float* logp;
   float* entropy;
   float* stat_loss;
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(1024) void k_token_loss(const float* __restrict__ p
     } else {
       fn = (float)(n < 1 ? 1 : n);
     }
-    const float gscale = a.grad_scale ? *a.grad_scale : 1.f;
+    const float gscale = scale_of(a.scale, n);
     const bool on = a.mask_eff[t] != 0;
     if (a.P.loss_kind == AA_LOSS_NLL) {
       a.stat_loss[t] = on ? -lp : 0.f;
@@ -1541,11 +1542,11 @@ extern "C" int aa_lmhead_bwd_carry(const void* hidden, const void* weight, int64
   return launch_status();
 }
 
-extern "C" int aa_lmhead_ppo_fused(const void* hidden, const void* weight, int64_t T, int64_t H, int64_t V,
+static int lmhead_ppo(const void* hidden, const void* weight, int64_t T, int64_t H, int64_t V,
                                    const int64_t* labels, float inv_temperature, int64_t T_active,
                                    const float* prox_logp, const float* adv, const uint8_t* mask_eff,
                                    const float* behave_w, const aa_ppo_params* params, const int32_t* n_valid,
-                                   const float* grad_scale, const int64_t* kept_per_chunk, int backward_mode,
+                                   const aa_loss_scale& scale, const int64_t* kept_per_chunk, int backward_mode,
                                    float* logp, float* entropy, float* stat_loss, float* ratio, uint8_t* flags,
                                    float* vocab_max, float* vocab_min, void* d_hidden, void* d_weight,
                                    int d_weight_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -1618,7 +1619,7 @@ extern "C" int aa_lmhead_ppo_fused(const void* hidden, const void* weight, int64
     else
       launch_tiles<kModeStats>(st, weight, hid, n_tok, H, V, a);
     // row statistics, per-token outputs, g
-    TokenLossArgs la{at(prox_logp), at(adv), at(mask_eff), at(behave_w), n_valid, grad_scale, logp + t0, at(entropy),
+    TokenLossArgs la{at(prox_logp), at(adv), at(mask_eff), at(behave_w), n_valid, scale, logp + t0, at(entropy),
                      at(stat_loss), at(ratio), at(flags), at(vocab_max), at(vocab_min), *params, act};
     hipLaunchKernelGGL(k_token_loss, dim3((unsigned)((n_tok + kMergeTokens - 1) / kMergeTokens)), dim3(1024), 0, st, a.pk, a.ps, a.pu, a.pn, a.xy,
                        (int)w.blocks, a.pitch_t, (int)n_tok, (int)V, a.c, inv_temperature, labels + t0, la, row_of_token,
@@ -1644,4 +1645,43 @@ extern "C" int aa_lmhead_ppo_fused(const void* hidden, const void* weight, int64
   if (first) launch_zero(st, dw.acc, V * H * (dw.acc_f32 ? 4 : 2));  // no token of the batch has a gradient
   finish_weight_grad(st, dw, d_weight, V, H);
   return launch_status();
+}
+
+extern "C" int aa_lmhead_ppo_fused(const void* hidden, const void* weight, int64_t T, int64_t H, int64_t V,
+                                   const int64_t* labels, float inv_temperature, int64_t T_active,
+                                   const float* prox_logp, const float* adv, const uint8_t* mask_eff,
+                                   const float* behave_w, const aa_ppo_params* params, const int32_t* n_valid,
+                                   const float* grad_scale, const int64_t* kept_per_chunk, int backward_mode,
+                                   float* logp, float* entropy, float* stat_loss, float* ratio, uint8_t* flags,
+                                   float* vocab_max, float* vocab_min, void* d_hidden, void* d_weight,
+                                   int d_weight_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  return lmhead_ppo(hidden, weight, T, H, V, labels, inv_temperature, T_active, prox_logp, adv, mask_eff, behave_w,
+                    params, n_valid, scale_by(grad_scale), kept_per_chunk, backward_mode, logp, entropy, stat_loss,
+                    ratio, flags, vocab_max, vocab_min, d_hidden, d_weight, d_weight_dtype, workspace, workspace_bytes,
+                    stream);
+}
+
+extern "C" int aa_lmhead_ppo_step(const aa_ppo_step* step, const void* hidden, const void* weight, int64_t H, int64_t V,
+                                  const int64_t* labels, float inv_temperature, const int64_t* kept_per_chunk,
+                                  int backward_mode, void* d_hidden, void* d_weight, int d_weight_dtype, void* workspace,
+                                  int64_t workspace_bytes, void* stream) {
+  if (!step) return AA_ERR_INVALID_ARGUMENT;
+  const aa_ppo_step& p = *step;
+  // what the loss step would refuse is refused before the first launch
+  if (!hidden || !weight || !labels || !d_hidden || !d_weight || !workspace || !(inv_temperature > 0.f))
+    return AA_ERR_INVALID_ARGUMENT;
+  if ((((uintptr_t)hidden | (uintptr_t)weight | (uintptr_t)workspace | (uintptr_t)d_hidden | (uintptr_t)d_weight) & 15))
+    return AA_ERR_INVALID_ARGUMENT;
+  if (!shapes_ok(p.T, H, V) || (d_weight_dtype != AA_F32 && d_weight_dtype != AA_BF16)) return AA_ERR_UNSUPPORTED;
+  if (workspace_bytes < plan(p.T, H, V).bytes) return AA_ERR_INVALID_ARGUMENT;
+  if (backward_mode != AA_LMHEAD_RECOMPUTE && backward_mode != AA_LMHEAD_CARRY) return AA_ERR_INVALID_ARGUMENT;
+  int st = step_args_status(p);
+  if (st == AA_OK) st = step_prepare(p, stream);
+  if (st != AA_OK) return st;
+  const aa_ppo_params params = step_params(p);
+  st = lmhead_ppo(hidden, weight, p.T, H, V, labels, inv_temperature, p.T_active, p.prox_logp, p.adv, step_mask(p),
+                  params.has_behave_weight ? p.behave_w : nullptr, &params, p.counts, p.scale, kept_per_chunk, backward_mode, p.logp,
+                  p.entropy, p.stat_loss, p.ratio, p.flags, p.vmax, p.vmin, d_hidden, d_weight, d_weight_dtype, workspace,
+                  workspace_bytes, stream);
+  return st == AA_OK ? step_finish(p, stream) : st;
 }

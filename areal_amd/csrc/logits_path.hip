@@ -14,6 +14,7 @@
 // are differences of small numbers whatever the magnitude of the logits.
 #include "device_utils.h"
 #include "ppo_math.h"
+#include "ppo_step.h"
 
 namespace aa {
 
@@ -389,7 +390,7 @@ struct FusedTokenArgs {
   const uint8_t* mask_eff;
   const float* behave_w;
   const int32_t* n_valid;
-  const float* grad_scale;
+  aa_loss_scale scale;
   float* logp;
   float* entropy;
   float* vmax;
@@ -459,13 +460,13 @@ __device__ __forceinline__ uint32_t load_u16_uniform(const void* __restrict__ ro
 // d(surrogate)/d(logp) and d(scaled loss)/d(logp).
 __device__ __forceinline__ void load_loss_scale(const FusedTokenArgs& a, float& fn, float& gscale) {
   int n = *a.n_valid;
+  gscale = scale_of(a.scale, n);
   if (a.P.loss_kind == AA_LOSS_NLL) {
     fn = (float)n + 1e-5f;  // the supervised loss divides by 1e-5 + count (areal/trainer/sft/lm_engine.py:96)
   } else {
     if (n < 1) n = 1;
     fn = (float)n;
   }
-  gscale = a.grad_scale ? *a.grad_scale : 1.f;
 }
 
 // Returns g = d(scaled loss)/d(logp_t); writes the per-token outputs from one thread.
@@ -1710,13 +1711,12 @@ extern "C" int aa_logits_bwd(const void* logits, int dtype, int64_t T, int64_t V
 // register kernel measures 0.7 % slower without that) only in the instantiations that run on two distinct arrays; the
 // in-place call runs the instantiation without the qualifier.  Tests compare the in-place result bit for bit on every
 // kernel.
-extern "C" int aa_logits_ppo_fused(const void* logits, int dtype, int64_t T, int64_t V, int64_t row_stride,
-                                   const int64_t* labels, float inv_temperature, int64_t T_active,
-                                   const float* prox_logp, const float* adv, const uint8_t* mask_eff,
-                                   const float* behave_w, const aa_ppo_params* params, const int32_t* n_valid,
-                                   const float* grad_scale, float* logp, float* entropy, float* vmax, float* vmin,
-                                   float* stat_loss, float* ratio, uint8_t* flags, void* dlogits, int32_t* work,
-                                   void* stream) {
+static int launch_fused(const void* logits, int dtype, int64_t T, int64_t V, int64_t row_stride, const int64_t* labels,
+                        float inv_temperature, int64_t T_active, const float* prox_logp, const float* adv,
+                        const uint8_t* mask_eff, const float* behave_w, const aa_ppo_params* params,
+                        const int32_t* n_valid, const aa_loss_scale& scale, float* logp, float* entropy, float* vmax,
+                        float* vmin, float* stat_loss, float* ratio, uint8_t* flags, void* dlogits, int32_t* work,
+                        void* stream) {
   if (!common_args_ok(logits, dtype, T, V, row_stride, labels)) return AA_ERR_INVALID_ARGUMENT;
   if (!params || !n_valid || !logp || !dlogits) return AA_ERR_INVALID_ARGUMENT;
   if (T_active < 0 || T_active > T || !(inv_temperature > 0.f)) return AA_ERR_INVALID_ARGUMENT;
@@ -1739,7 +1739,7 @@ extern "C" int aa_logits_ppo_fused(const void* logits, int dtype, int64_t T, int
   hipStream_t st = (hipStream_t)stream;
   FusedTokenArgs a;
   a.prox_logp = prox_logp; a.adv = adv; a.mask_eff = mask_eff; a.behave_w = behave_w;
-  a.n_valid = n_valid; a.grad_scale = grad_scale;
+  a.n_valid = n_valid; a.scale = scale;
   a.logp = logp; a.entropy = entropy; a.vmax = vmax; a.vmin = vmin;
   a.stat_loss = stat_loss; a.ratio = ratio; a.flags = flags;
   a.P = *params; a.T_active = T_active;
@@ -1818,6 +1818,35 @@ extern "C" int aa_logits_ppo_fused(const void* logits, int dtype, int64_t T, int
 #undef AA_LAUNCH
 #undef AA_LAUNCH_AS
   return launch_status();
+}
+
+extern "C" int aa_logits_ppo_fused(const void* logits, int dtype, int64_t T, int64_t V, int64_t row_stride,
+                                   const int64_t* labels, float inv_temperature, int64_t T_active,
+                                   const float* prox_logp, const float* adv, const uint8_t* mask_eff,
+                                   const float* behave_w, const aa_ppo_params* params, const int32_t* n_valid,
+                                   const float* grad_scale, float* logp, float* entropy, float* vmax, float* vmin,
+                                   float* stat_loss, float* ratio, uint8_t* flags, void* dlogits, int32_t* work,
+                                   void* stream) {
+  return launch_fused(logits, dtype, T, V, row_stride, labels, inv_temperature, T_active, prox_logp, adv, mask_eff, behave_w,
+                      params, n_valid, scale_by(grad_scale), logp, entropy, vmax, vmin, stat_loss, ratio, flags, dlogits,
+                      work, stream);
+}
+
+extern "C" int aa_logits_ppo_step(const aa_ppo_step* step, const void* logits, int dtype, int64_t V, int64_t row_stride,
+                                  const int64_t* labels, float inv_temperature, void* dlogits, void* stream) {
+  if (!step) return AA_ERR_INVALID_ARGUMENT;
+  const aa_ppo_step& p = *step;
+  // what the fused kernel would refuse is refused before the first launch
+  if (!common_args_ok(logits, dtype, p.T, V, row_stride, labels) || !dlogits || !(inv_temperature > 0.f))
+    return AA_ERR_INVALID_ARGUMENT;
+  int st = step_args_status(p);
+  if (st == AA_OK) st = step_prepare(p, stream);
+  if (st != AA_OK) return st;
+  const aa_ppo_params params = step_params(p);
+  st = launch_fused(logits, dtype, p.T, V, row_stride, labels, inv_temperature, p.T_active, p.prox_logp, p.adv,
+                    step_mask(p), params.has_behave_weight ? p.behave_w : nullptr, &params, p.counts, p.scale, p.logp, p.entropy,
+                    p.vmax, p.vmin, p.stat_loss, p.ratio, p.flags, dlogits, (int32_t*)p.work, stream);
+  return st == AA_OK ? step_finish(p, stream) : st;
 }
 
 // -----------------------------------------------------------------------------

@@ -11,10 +11,12 @@
 // bandwidth.
 #include "device_utils.h"
 #include "ppo_math.h"
+#include "ppo_step.h"
 
 namespace aa {
 
 constexpr int kSegThreads = 256;
+constexpr int kFinishBlocks = 256;  // most workgroups of a launch that finishes a step
 
 struct Segments {
   const int32_t* cu;  // [B+1] or nullptr
@@ -93,10 +95,62 @@ __global__ void k_zero_i32(int32_t* p, int n) {
   if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
 }
 
+// Who takes the counts of a launch: two counters that the caller has cleared (work == nullptr), or the work buffer of a
+// step: the workgroups add up there, the last one to finish moves the sums to counts (and to host memory) and leaves the
+// buffer zero for the next launch.  One launch then does what took a clearing kernel, this one, and a copy to the host.
+struct StepWork {
+  int32_t rows[2];  // row hand-out of the fused logits kernel
+  int32_t total, hit, done;
+  int32_t finished;
+  int32_t pad[10];
+  double partial[kFinishBlocks];
+};
+static_assert(sizeof(StepWork) <= AA_STEP_WORK_BYTES, "the work buffer of a step");
+
+struct Counts {
+  int32_t* counts;
+  StepWork* work;
+  int32_t* host;
+  int32_t tag;
+};
+
+__device__ __forceinline__ void host_store(int32_t* p, int32_t v, int order_release) {
+  if (order_release) __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// one thread per workgroup
+__device__ __forceinline__ void count_up(const Counts& c, int total, int hit) {
+  if (!c.work) {
+    if (total) atomicAdd(&c.counts[0], total);
+    if (hit) atomicAdd(&c.counts[1], hit);
+    return;
+  }
+  if (gridDim.x > 1) {
+    if (total) atomicAdd(&c.work->total, total);
+    if (hit) atomicAdd(&c.work->hit, hit);
+    __threadfence();
+    if (atomicAdd(&c.work->done, 1) != (int)gridDim.x - 1) return;
+    __threadfence();
+    total = atomicExch(&c.work->total, 0);
+    hit = atomicExch(&c.work->hit, 0);
+    atomicExch(&c.work->done, 0);
+  }
+  c.counts[0] = total;
+  c.counts[1] = hit;
+  c.counts[2] = 0;
+  if (c.host) {
+    host_store(c.host + 0, total, 0);
+    host_store(c.host + 1, hit, 0);
+    host_store(c.host + 2, 0, 0);
+    host_store(c.host + 3, c.tag, 1);
+  }
+}
+
 __global__ __launch_bounds__(256) void k_rs_token(const float* __restrict__ prox, const float* __restrict__ old,
                                                   const uint8_t* __restrict__ mask, int64_t n, RsCfg c,
                                                   uint8_t* __restrict__ mask_out, float* __restrict__ w_out,
-                                                  int32_t* __restrict__ counts) {
+                                                  Counts counts) {
   __shared__ int smem[256 / kWave];
   int total = 0, hit = 0;
   const int64_t step = (int64_t)gridDim.x * 256;
@@ -121,10 +175,7 @@ __global__ __launch_bounds__(256) void k_rs_token(const float* __restrict__ prox
   }
   total = block_sum<int>(total, smem);
   hit = block_sum<int>(hit, smem);
-  if (threadIdx.x == 0) {
-    if (total) atomicAdd(&counts[0], total);
-    if (hit) atomicAdd(&counts[1], hit);
-  }
+  if (threadIdx.x == 0) count_up(counts, total, hit);
 }
 
 __global__ __launch_bounds__(kSegThreads) void k_rs_sequence(const float* __restrict__ prox,
@@ -132,7 +183,7 @@ __global__ __launch_bounds__(kSegThreads) void k_rs_sequence(const float* __rest
                                                              const uint8_t* __restrict__ mask, Segments seg, RsCfg c,
                                                              uint8_t* __restrict__ mask_out,
                                                              float* __restrict__ w_out,
-                                                             int32_t* __restrict__ counts) {
+                                                             Counts counts) {
   __shared__ double smem_d[kSegThreads / kWave];
   __shared__ float smem_f[kSegThreads / kWave];
   __shared__ int smem_i[kSegThreads / kWave];
@@ -141,6 +192,7 @@ __global__ __launch_bounds__(kSegThreads) void k_rs_sequence(const float* __rest
   seg.range(b, beg, end);
   if (b == seg.B) {  // tokens no sequence covers
     for (int64_t i = beg + threadIdx.x; i < end; i += kSegThreads) { mask_out[i] = 0; w_out[i] = 0.f; }
+    if (threadIdx.x == 0) count_up(counts, 0, 0);
     return;
   }
   const bool log_agg = c.metric == AA_RS_RATIO;
@@ -185,10 +237,23 @@ __global__ __launch_bounds__(kSegThreads) void k_rs_sequence(const float* __rest
     w_out[i] = keep ? w : 0.f;
   }
   hit = block_sum<int>(hit, smem_i);
-  if (threadIdx.x == 0) {
-    if (raw) atomicAdd(&counts[0], raw);
-    if (hit) atomicAdd(&counts[1], hit);
+  if (threadIdx.x == 0) count_up(counts, raw, hit);
+}
+
+// number of non-zero mask bytes, many workgroups (a step without rejection sampling)
+__global__ __launch_bounds__(256) void k_step_count(const uint8_t* __restrict__ mask, int64_t n, Counts counts) {
+  __shared__ int smem[256 / kWave];
+  int c = 0;
+  const int64_t step = (int64_t)gridDim.x * 256, first = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t n4 = ((((uintptr_t)mask) & 3) == 0) ? (n >> 2) : 0;  // four mask bytes per load
+  for (int64_t q = first; q < n4; q += step) {
+    const uint32_t m = ((const uint32_t*)mask)[q];
+    c += ((m & 0x000000ffu) ? 1 : 0) + ((m & 0x0000ff00u) ? 1 : 0) + ((m & 0x00ff0000u) ? 1 : 0) +
+         ((m & 0xff000000u) ? 1 : 0);
   }
+  for (int64_t i = (n4 << 2) + first; i < n; i += step) c += mask[i] != 0 ? 1 : 0;
+  c = block_sum<int>(c, smem);
+  if (threadIdx.x == 0) count_up(counts, c, 0);
 }
 
 __global__ __launch_bounds__(1024) void k_count_nonzero(const uint8_t* __restrict__ mask, int64_t n,
@@ -347,6 +412,99 @@ __global__ __launch_bounds__(256) void k_ppo_stat_outputs(const float* __restric
       behave_mask[i] = on ? 1 : 0;
       behave_kl[i] = on ? p - old[i] : 0.f;
     }
+  }
+}
+
+// ---- the end of a step: derived entries of the stat dict and the scalar loss in one launch ---------------------------
+// Bound by latency at these sizes (29 bytes per token): what counts is that it is one launch (k_masked_sum, one
+// workgroup, and k_ppo_stat_outputs were two, 9 us on the stream).  A workgroup takes a contiguous slice of the tokens
+// and leaves the fp64 sum of its masked losses; the last one to finish adds the sums in slice order: the same order in
+// every run.
+constexpr int kFinishSlice = 1024;  // tokens per workgroup, or a multiple
+
+struct FinishArgs {
+  const float* logp;
+  const float* prox;
+  const float* old;
+  const float* adv;
+  const uint8_t* mask;     // the mask the loss is summed under
+  const float* behave_w;   // nullable
+  float* stat_loss;
+  float* ratio;
+  uint8_t* flags;
+  float* g_logp;
+  float* approx_kl;        // nullable: no derived entries
+  uint8_t* clip;
+  uint8_t* dual;
+  uint8_t* behave_mask;    // nullable (with behave_kl)
+  float* behave_kl;
+  const int32_t* n_valid;
+  float* loss;
+  StepWork* work;
+  aa_loss_scale scale;
+  aa_ppo_params P;
+  int64_t n, per;          // per: tokens of a workgroup
+};
+
+// TOKEN_LOSS: the clipped surrogate and its derivative are formed here as well (log-probs that are given, token level)
+template <bool TOKEN_LOSS>
+__global__ __launch_bounds__(256) void k_step_finish(FinishArgs a) {
+  __shared__ double smem[256 / kWave];
+  __shared__ int last;
+  const int nv = *a.n_valid;
+  const float fn = a.P.loss_kind == AA_LOSS_NLL ? (float)nv + 1e-5f : (float)(nv < 1 ? 1 : nv);
+  const int64_t b = (int64_t)blockIdx.x * a.per, e = b + a.per < a.n ? b + a.per : a.n;
+  double acc = 0.0;
+  for (int64_t i = b + threadIdx.x; i < e; i += 256) {
+    const bool m = a.mask[i] != 0;
+    float l;
+    uint8_t f = 0;
+    if constexpr (TOKEN_LOSS) {
+      const float r = m ? expf(a.logp[i] - a.prox[i]) : 0.f;
+      const Surrogate s = surrogate(r, a.adv[i], a.P.has_behave_weight ? a.behave_w[i] : 1.f, a.P);
+      l = s.loss;
+      f = (uint8_t)(((s.clip && m) ? 1 : 0) | ((s.dual && m) ? 2 : 0));
+      a.stat_loss[i] = l;
+      a.ratio[i] = r;
+      a.g_logp[i] = m ? s.dloss_dr * r / fn : 0.f;
+    } else {
+      l = a.stat_loss[i];
+      if (a.approx_kl) f = a.flags[i];
+    }
+    if (m) acc += (double)l;
+    if (a.approx_kl) {
+      const float p = a.prox[i];
+      a.approx_kl[i] = a.logp[i] - p;
+      a.clip[i] = f & 1;
+      a.dual[i] = (f >> 1) & 1;
+      if (a.behave_mask) {
+        const bool on = a.behave_w[i] > 0.f && m;
+        a.behave_mask[i] = on ? 1 : 0;
+        a.behave_kl[i] = on ? p - a.old[i] : 0.f;
+      }
+    }
+  }
+  acc = block_sum<double>(acc, smem);
+  if (threadIdx.x == 0) {
+    last = 1;
+    if (gridDim.x > 1) {
+      a.work->partial[blockIdx.x] = acc;
+      __threadfence();
+      last = atomicAdd(&a.work->finished, 1) == (int)gridDim.x - 1;
+    }
+  }
+  __syncthreads();
+  if (!last) return;
+  if (gridDim.x > 1) {
+    __threadfence();
+    double part = 0.0;
+    if (threadIdx.x < gridDim.x)
+      part = __hip_atomic_load(&a.work->partial[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    acc = block_sum<double>(part, smem);
+  }
+  if (threadIdx.x == 0) {
+    a.work->finished = 0;
+    a.loss[0] = (float)acc / fn * scale_of(a.scale, nv);
   }
 }
 
@@ -544,17 +702,137 @@ extern "C" int aa_rejection_sampling(const float* prox_logp, const float* old_lo
   RsCfg c{level, action, metric, agg, has_lower, upper, lower};
   hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, counts, 3);
   if (n == 0) return launch_status();
+  const Counts cleared{counts, nullptr, nullptr, 0};
   if (level == AA_RS_LEVEL_TOKEN) {
     hipLaunchKernelGGL(k_rs_token, dim3(grid_for(n)), dim3(256), 0, st, prox_logp, old_logp, mask_in, n, c, mask_out,
-                       behave_w, counts);
+                       behave_w, cleared);
   } else {
     if (B <= 0 || B > 0x7ffffffe) return AA_ERR_INVALID_ARGUMENT;
     if (!cu_seqlens && (n % B) != 0) return AA_ERR_INVALID_ARGUMENT;
     Segments seg{cu_seqlens, B, n};
     hipLaunchKernelGGL(k_rs_sequence, dim3((unsigned)(B + 1)), dim3(kSegThreads), 0, st, prox_logp, old_logp, mask_in,
-                       seg, c, mask_out, behave_w, counts);
+                       seg, c, mask_out, behave_w, cleared);
   }
   return launch_status();
+}
+
+namespace aa {
+
+int step_args_status(const aa_ppo_step& p) {
+  if (p.T < 0 || p.T_active < 0 || p.T_active > p.T || !p.counts || !p.loss || !p.work || (((uintptr_t)p.work) & 7))
+    return AA_ERR_INVALID_ARGUMENT;
+  const bool nll = p.params.loss_kind == AA_LOSS_NLL;
+  if (!nll && p.params.loss_kind != AA_LOSS_PPO && p.params.loss_kind != AA_LOSS_SAPO) return AA_ERR_INVALID_ARGUMENT;
+  if (p.params.loss_kind == AA_LOSS_SAPO && (!(p.params.sapo_tau_pos > 0.f) || !(p.params.sapo_tau_neg > 0.f)))
+    return AA_ERR_INVALID_ARGUMENT;
+  if ((p.vmax != nullptr) != (p.vmin != nullptr)) return AA_ERR_INVALID_ARGUMENT;
+  if (p.T_active > 0 && (!p.mask || !p.stat_loss || !p.ratio || !p.flags)) return AA_ERR_INVALID_ARGUMENT;
+  if (p.T_active > 0 && !nll && (!p.prox_logp || !p.adv)) return AA_ERR_INVALID_ARGUMENT;
+  if (p.approx_kl && (!p.clip_mask || !p.dual_clip_mask || (p.T_active > 0 && !p.prox_logp))) return AA_ERR_INVALID_ARGUMENT;
+  if ((p.behave_mask != nullptr) != (p.behave_kl != nullptr)) return AA_ERR_INVALID_ARGUMENT;
+  if (p.behave_mask && (!p.behave_w || !p.old_logp || !p.approx_kl)) return AA_ERR_INVALID_ARGUMENT;
+  if (p.counts_given && p.rs.enabled) return AA_ERR_INVALID_ARGUMENT;
+  if (!p.rs.enabled && p.params.has_behave_weight && (p.params.loss_kind != AA_LOSS_PPO || (p.T_active > 0 && !p.behave_w)))
+    return AA_ERR_INVALID_ARGUMENT;
+  const aa_rs_params& r = p.rs;
+  if (r.enabled) {
+    if (p.params.loss_kind != AA_LOSS_PPO) return AA_ERR_INVALID_ARGUMENT;
+    if (p.T_active > 0 && (!p.prox_logp || !p.old_logp || !p.mask_out || !p.behave_w)) return AA_ERR_INVALID_ARGUMENT;
+    if (r.level < 0 || r.level > 1 || r.action < 0 || r.action > 1 || r.metric < 0 || r.metric > 3 || r.agg < 0 || r.agg > 2)
+      return AA_ERR_INVALID_ARGUMENT;
+    if (r.action == AA_RS_ACTION_CLAMP && r.metric != AA_RS_RATIO) return AA_ERR_INVALID_ARGUMENT;
+    if (r.level == AA_RS_LEVEL_SEQUENCE && p.T_active > 0) {
+      if (p.n_segments <= 0 || p.n_segments > 0x7ffffffe) return AA_ERR_INVALID_ARGUMENT;
+      if (!p.cu_seqlens && (p.T_active % p.n_segments) != 0) return AA_ERR_INVALID_ARGUMENT;
+    }
+  }
+  return AA_OK;
+}
+
+int step_prepare(const aa_ppo_step& p, void* stream) {
+  if (p.counts_given) return AA_OK;
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t n = p.T_active;
+  const Counts counts{p.counts, (StepWork*)p.work, p.host_counts, p.host_tag};
+  const aa_rs_params& r = p.rs;
+  if (!r.enabled || n == 0) {
+    int64_t blocks = (n + 4095) / 4096;  // 16 mask bytes per thread
+    blocks = blocks < 1 ? 1 : (blocks > 256 ? 256 : blocks);
+    hipLaunchKernelGGL(k_step_count, dim3((unsigned)blocks), dim3(256), 0, st, p.mask, n, counts);
+    return launch_status();
+  }
+  const RsCfg c{r.level, r.action, r.metric, r.agg, r.has_lower, r.upper, r.lower};
+  if (r.level == AA_RS_LEVEL_TOKEN) {
+    int64_t blocks = (n + 1023) / 1024;  // few workgroups: each ends with atomics on the same line
+    blocks = blocks > 128 ? 128 : blocks;
+    hipLaunchKernelGGL(k_rs_token, dim3((unsigned)blocks), dim3(256), 0, st, p.prox_logp, p.old_logp, p.mask, n, c, p.mask_out,
+                       p.behave_w, counts);
+  } else {
+    const Segments seg{p.cu_seqlens, p.n_segments, n};
+    hipLaunchKernelGGL(k_rs_sequence, dim3((unsigned)(p.n_segments + 1)), dim3(kSegThreads), 0, st, p.prox_logp, p.old_logp,
+                       p.mask, seg, c, p.mask_out, p.behave_w, counts);
+  }
+  return launch_status();
+}
+
+static int launch_finish(const aa_ppo_step& p, const float* logp, float* g_logp, void* stream) {
+  FinishArgs a;
+  a.logp = logp;
+  a.prox = p.prox_logp;
+  a.old = p.old_logp;
+  a.adv = p.adv;
+  a.mask = step_mask(p);
+  a.P = step_params(p);
+  a.behave_w = a.P.has_behave_weight ? p.behave_w : nullptr;
+  a.stat_loss = p.stat_loss;
+  a.ratio = p.ratio;
+  a.flags = p.flags;
+  a.g_logp = g_logp;
+  a.approx_kl = p.approx_kl;
+  a.clip = p.clip_mask;
+  a.dual = p.dual_clip_mask;
+  a.behave_mask = p.behave_mask;
+  a.behave_kl = p.behave_kl;
+  a.n_valid = p.counts;
+  a.loss = p.loss;
+  a.work = (StepWork*)p.work;
+  a.scale = p.scale;
+  a.n = p.T_active;
+  int64_t blocks = (a.n + kFinishSlice - 1) / kFinishSlice;
+  blocks = blocks < 1 ? 1 : (blocks > kFinishBlocks ? kFinishBlocks : blocks);
+  a.per = (a.n + blocks - 1) / blocks;
+  if (g_logp) hipLaunchKernelGGL(k_step_finish<true>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+  else hipLaunchKernelGGL(k_step_finish<false>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+  return launch_status();
+}
+
+int step_finish(const aa_ppo_step& p, void* stream) { return launch_finish(p, p.logp, nullptr, stream); }
+
+}  // namespace aa
+
+extern "C" int aa_ppo_loss_step(const aa_ppo_step* step, const float* logp, int sequence_level, int counts_only,
+                                float* g_logp, void* stream) {
+  if (!step) return AA_ERR_INVALID_ARGUMENT;
+  const aa_ppo_step& p = *step;
+  int st = step_args_status(p);
+  if (st == AA_OK && counts_only) return step_prepare(p, stream);
+  if (st != AA_OK) return st;
+  if (p.params.loss_kind != AA_LOSS_PPO) return AA_ERR_UNSUPPORTED;
+  if (p.T != p.T_active || (p.T > 0 && (!logp || !g_logp))) return AA_ERR_INVALID_ARGUMENT;
+  if (sequence_level && p.T > 0) {
+    if (p.n_segments <= 0 || p.n_segments > 0x7ffffffe) return AA_ERR_INVALID_ARGUMENT;
+    if (!p.cu_seqlens && (p.T % p.n_segments) != 0) return AA_ERR_INVALID_ARGUMENT;
+  }
+  st = step_prepare(p, stream);
+  if (st != AA_OK) return st;
+  if (!sequence_level || p.T == 0) return launch_finish(p, logp, p.T > 0 ? g_logp : nullptr, stream);
+  const aa_ppo_params params = step_params(p);
+  const Segments seg{p.cu_seqlens, p.n_segments, p.T};
+  hipLaunchKernelGGL(k_ppo_sequence, dim3((unsigned)(p.n_segments + 1)), dim3(kSegThreads), 0, (hipStream_t)stream, logp,
+                     p.prox_logp, p.adv, step_mask(p), params.has_behave_weight ? p.behave_w : nullptr, seg, params, p.counts,
+                     p.stat_loss, p.ratio, p.flags, g_logp);
+  st = launch_status();
+  return st == AA_OK ? launch_finish(p, logp, nullptr, stream) : st;
 }
 
 extern "C" int aa_count_nonzero_u8(const uint8_t* mask, int64_t n, int32_t* count, void* stream) {

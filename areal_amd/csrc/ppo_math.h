@@ -17,6 +17,16 @@ struct Surrogate {
   bool dual;       // pg_loss3 < max(pg_loss1, pg_loss2)
 };
 
+// The factor of a loss and its gradient; n_valid: the number of tokens with a loss (float32 throughout, in the order of
+// the tensor expression local_weight / total_loss_weight * multiplier).
+__device__ __forceinline__ float scale_of(const aa_loss_scale& s, int n_valid) {
+  float f = s.value;
+  if (s.per_valid_token) f = (float)n_valid / (s.total ? *s.total : s.total_value) * f;
+  if (s.factor) f *= *s.factor;
+  return f;
+}
+inline aa_loss_scale scale_by(const float* factor) { return aa_loss_scale{factor, nullptr, 1.f, 1.f, 0}; }
+
 // max/min that return NaN if either side is NaN (torch.max / torch.min do)
 __device__ __forceinline__ float nan_max(float a, float b) { return (a != a || b != b) ? (a + b) : fmaxf(a, b); }
 __device__ __forceinline__ float nan_min(float a, float b) { return (a != a || b != b) ? (a + b) : fminf(a, b); }

@@ -1,0 +1,28 @@
+// What the steps (logits, lm_head, given log-probs) share around their loss kernel: the launch ahead of it that counts the
+// mask or runs the rejection sampling, and the one behind it that finishes the stat dict and the scalar loss.  Defined
+// in ppo_loss.hip.
+#pragma once
+#include "device_utils.h"
+
+namespace aa {
+
+// Argument check of the parts of a step that these launches and the loss kernels use.
+int step_args_status(const aa_ppo_step& p);
+// counts (and their copy in host memory), and with rejection sampling mask_out and behave_w
+int step_prepare(const aa_ppo_step& p, void* stream);
+// approx_kl ... behave_kl (when wanted) and loss, from logp, stat_loss, flags
+int step_finish(const aa_ppo_step& p, void* stream);
+
+// the loss parameters with the behaviour weights that go with them
+inline aa_ppo_params step_params(const aa_ppo_step& p) {
+  aa_ppo_params q = p.params;
+  if (p.rs.enabled) q.has_behave_weight = 1;
+  return q;
+}
+
+// the mask the loss is summed under
+inline const uint8_t* step_mask(const aa_ppo_step& p) {
+  return p.rs.enabled && p.rs.action == AA_RS_ACTION_MASK ? p.mask_out : p.mask;
+}
+
+}  // namespace aa

@@ -10,7 +10,7 @@ from __future__ import annotations
 import torch
 
 from . import _native as N
-from .functional import _DTYPES, _f32, _mask_u8, _ptr, _require_gpu, _stream
+from .functional import _DTYPES, _f32, _mask_u8, _on, _ptr, _require_gpu, _stream
 
 _LOSS_TYPES = {"sigmoid": 0, "ipo": 1}
 
@@ -39,7 +39,7 @@ def _launch_bwd(g_sums, scale, m8, cu, n_seqs, T, dev):
     d_logp = torch.empty(T, dtype=torch.float32, device=dev)
     if T:
         lib = N.load()
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(lib.aa_dpo_seq_sums_bwd(_ptr(g_sums), _ptr(scale) if scale is not None else None, _ptr(m8),
                                             _ptr(cu), n_seqs, T, _ptr(d_logp), _stream(dev)), "aa_dpo_seq_sums_bwd")
     return d_logp
@@ -55,7 +55,7 @@ class _SeqSums(torch.autograd.Function):
         n_seqs, T = cu.numel() - 1, lp.numel()
         policy, refs, lens = torch.empty(3, n_seqs, dtype=torch.float64, device=dev).unbind(0)
         if n_seqs:
-            with torch.cuda.device(dev):
+            with _on(dev):
                 N.check(lib.aa_dpo_seq_sums(_ptr(lp), _ptr(ref), _ptr(m8), _ptr(cu), n_seqs, T, _ptr(policy),
                                             _ptr(refs), _ptr(lens), _stream(dev)), "aa_dpo_seq_sums")
         ctx.save_for_backward(m8, cu)
@@ -94,7 +94,7 @@ class _PreferenceLoss(torch.autograd.Function):
         loss = torch.empty_like(x)
         dloss = torch.empty_like(x)
         if x.numel():
-            with torch.cuda.device(dev):
+            with _on(dev):
                 N.check(lib.aa_dpo_preference_loss(_ptr(x), x.numel(), float(beta), loss_type, _ptr(loss), _ptr(dloss),
                                                    _stream(dev)), "aa_dpo_preference_loss")
         ctx.save_for_backward(dloss)
@@ -133,7 +133,7 @@ class _DpoLoss(torch.autograd.Function):
         valid = torch.empty(n_pairs, dtype=torch.bool, device=dev)
         loss = torch.empty((), dtype=torch.float32, device=dev)
         n_valid = torch.empty((), dtype=torch.int32, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = _stream(dev)
             if n_seqs:
                 N.check(lib.aa_dpo_seq_sums(_ptr(lp), _ptr(ref), _ptr(m8), _ptr(cu), n_seqs, T, _ptr(policy),
@@ -182,7 +182,7 @@ class _RwLoss(torch.autograd.Function):
         loss = torch.empty((), dtype=torch.float32, device=dev)
         n_valid = torch.empty((), dtype=torch.int32, device=dev)
         g = torch.empty(T, dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(lib.aa_rw_pair_loss(_ptr(scores), T, _ptr(cu), n_pairs, _ptr(loss), _ptr(n_valid), _ptr(pair_loss),
                                         _ptr(pos), _ptr(neg), _ptr(valid), _ptr(g), _stream(dev)), "aa_rw_pair_loss")
         ctx.save_for_backward(g)
@@ -197,7 +197,7 @@ class _RwLoss(torch.autograd.Function):
         dev = g.device
         up = _f32(g_loss).reshape(1)
         if out.numel():
-            with torch.cuda.device(dev):
+            with _on(dev):
                 N.check(N.load().aa_scale_inplace(_ptr(out), _DTYPES[out.dtype], out.numel(), _ptr(up), _stream(dev)),
                         "aa_scale_inplace")
         return out, None

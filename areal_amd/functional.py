@@ -8,7 +8,11 @@ bookkeeping only.  Tensors must live on a ROCm device: there is no CPU path.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
+import itertools
+import time
+from collections import deque
 from dataclasses import dataclass
 from typing import Any
 
@@ -34,12 +38,20 @@ _DTYPES = {torch.bfloat16: N.AA_BF16, torch.float16: N.AA_F16, torch.float32: N.
 # ----------------------------------------------------------------------------
 # helpers
 # ----------------------------------------------------------------------------
-def _ptr(t: torch.Tensor | None) -> C.c_void_p:
-    return C.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """Context in which ``device`` is the current one; nothing to enter when it is already."""
+    return _SAME_DEVICE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def _require_gpu(t: torch.Tensor, name: str) -> None:
@@ -53,6 +65,13 @@ def _f32(t: torch.Tensor) -> torch.Tensor:
     return t.to(torch.float32).contiguous()
 
 
+def _f32_values(t: torch.Tensor) -> torch.Tensor:
+    """The values of ``t`` as contiguous float32 for a kernel that reads them (no autograd)."""
+    if t.dtype is torch.float32 and t.is_contiguous():
+        return t
+    return t.detach().to(torch.float32).contiguous()
+
+
 def _mask_u8(mask: torch.Tensor) -> torch.Tensor:
     """One byte per token, non-zero = valid, without a copy for bool masks."""
     m = mask.contiguous()
@@ -61,10 +80,23 @@ def _mask_u8(mask: torch.Tensor) -> torch.Tensor:
     return (m != 0).view(torch.uint8)
 
 
+def _mask_bytes(mask: torch.Tensor) -> torch.Tensor:
+    """The same for a kernel that only needs the address: a contiguous bool mask as it is."""
+    if mask.dtype is torch.bool and mask.is_contiguous():
+        return mask
+    return _mask_u8(mask)
+
+
+def _labels_i64(labels: torch.Tensor, dev: torch.device) -> torch.Tensor:
+    if labels.dtype is torch.int64 and labels.device == dev and labels.is_contiguous():
+        return labels
+    return labels.to(device=dev, dtype=torch.int64).contiguous()
+
+
 def _rows(logits: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
     """View logits as [T, V] rows with unit inner stride; returns (2-D tensor, T, V, row stride)."""
     V = logits.shape[-1]
-    x = logits.reshape(-1, V)
+    x = logits if logits.dim() == 2 else logits.reshape(-1, V)
     if x.dtype not in _DTYPES:
         x = x.float()
     if x.stride(-1) != 1 or (x.shape[0] > 1 and x.stride(0) < V):
@@ -101,12 +133,12 @@ _WORK: dict = {}
 
 
 def _work_words(dev: torch.device) -> torch.Tensor:
-    """Two zeroed int32 words per (device, stream) for the row hand-out of the fused kernel, which returns
-    them to zero at the end of every launch."""
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
+    """The work buffer of the steps on the current stream of ``dev`` (AA_STEP_WORK_BYTES, zero between launches; its
+    first two words are the row hand-out of the fused kernel): one per (device, stream), kept."""
+    key = (dev.index, _stream(dev))
     buf = _WORK.get(key)
     if buf is None:
-        buf = _WORK[key] = torch.zeros(2, dtype=torch.int32, device=dev)
+        buf = _WORK[key] = torch.zeros(N.STEP_WORK_BYTES // 4, dtype=torch.int32, device=dev)
     return buf
 
 
@@ -143,7 +175,7 @@ class _LogprobsEntropy(torch.autograd.Function):
         row_ez = torch.empty(T, **kw) if (need_bwd and want_entropy) else None
         vmax = torch.empty(T, **kw) if want_minmax else None
         vmin = torch.empty(T, **kw) if want_minmax else None
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(
                 lib.aa_logits_fwd(
                     _ptr(logits2d), _DTYPES[logits2d.dtype], T, V, stride, _ptr(labels1d),
@@ -175,7 +207,7 @@ class _LogprobsEntropy(torch.autograd.Function):
             dlogits = logits2d.detach()
         else:  # the row stride of the input, so that both buffers are walked alike
             dlogits = _empty_rows_like(logits2d, ctx.stride)
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(
                 lib.aa_logits_bwd(
                     _ptr(logits2d), _DTYPES[logits2d.dtype], T, V, ctx.stride, _ptr(labels1d),
@@ -308,7 +340,7 @@ def _rejection_sampling_device(prox, old, mask_u8, shape, cu_seqlens, cfg):
     w = torch.empty(n, dtype=torch.float32, device=dev)
     counts = torch.empty(3, dtype=torch.int32, device=dev)
     lower = cfg.lower
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(
             lib.aa_rejection_sampling(
                 _ptr(prox), _ptr(old), _ptr(mask_u8), n, _ptr(cu), B,
@@ -334,7 +366,7 @@ class _HostCounts:
 
     def __init__(self, counts: torch.Tensor):
         self._host = torch.empty(counts.shape, dtype=counts.dtype, pin_memory=True)
-        with torch.cuda.device(counts.device):
+        with _on(counts.device):
             self._host.copy_(counts, non_blocking=True)
             self._event = torch.cuda.Event()
             self._event.record()
@@ -399,44 +431,189 @@ def apply_rejection_sampling(
 
 
 # ----------------------------------------------------------------------------
+# what the steps share: per-token arrays, loss scale, counters on the host
+# ----------------------------------------------------------------------------
+class _HostSlot:
+    """Four words of pinned host memory that the first kernel of a step writes the counts of the mask to, the tag last.
+
+    Reading them (``filtered_fraction`` is a Python float, as in the reference, and a micro-batch without a token is
+    found out on the host) waits for that kernel only, not for the long ones queued after it, and needs no copy and no
+    event of its own.  Slots are taken from and given back to a bounded pool (any thread, any stream): the tag tells a
+    use from the ones before it.  A slot that nobody read is not given back."""
+
+    __slots__ = ("_memory", "_words", "address", "tag", "_device", "_got")
+    _pool: deque = deque(maxlen=64)
+    _tags = itertools.count(1)
+    _unread: list = []  # memory that a kernel may still write to
+    _SPINS = 20000  # about a millisecond, then short sleeps: other threads run
+
+    def __init__(self, device: torch.device):
+        try:
+            self._memory, self._words = _HostSlot._pool.pop()
+        except IndexError:
+            self._memory = torch.empty(4, dtype=torch.int32, pin_memory=True)
+            self._words = (C.c_int32 * 4).from_address(self._memory.data_ptr())
+            self._words[3] = 0
+        self.address = self._memory.data_ptr()
+        self.tag = next(_HostSlot._tags) & 0x7FFFFFFF or next(_HostSlot._tags)
+        self._device = device
+        self._got = None
+
+    def read(self) -> tuple[int, int]:
+        """(non-zero entries of the loss mask, tokens filtered or clamped)"""
+        if self._got is not None:
+            return self._got
+        words, tag = self._words, self.tag
+        for _ in range(self._SPINS):
+            if words[3] == tag:
+                break
+        else:
+            done = None  # an event behind everything queued so far: the counts are there when it has passed
+            while words[3] != tag:
+                if done is None:
+                    done = torch.cuda.Event()
+                    done.record(torch.cuda.current_stream(self._device))
+                if done.query() and words[3] != tag:
+                    raise N.NativeLibraryError("the counts of a step never reached the host")
+                time.sleep(2e-5)
+        self._got = (words[0], words[1])
+        memory, self._memory = self._memory, None
+        _HostSlot._pool.append((memory, words))
+        return self._got
+
+    def __del__(self):
+        if getattr(self, "_memory", None) is not None:
+            _HostSlot._unread.append(self._memory)
+
+
+class _PerValidToken:
+    """Loss scale ``loss_mask.count_nonzero() / total * multiplier`` (fsdp_engine.py:1983-1985, 2045), formed inside the
+    kernels from the count they have anyway.  ``total`` is a number or a tensor with one element."""
+
+    __slots__ = ("total", "multiplier")
+
+    def __init__(self, total, multiplier: float):
+        self.total, self.multiplier = total, multiplier
+
+
+def _scale_struct(scale, dev: torch.device):
+    """(``aa_loss_scale``, tensors it points into)"""
+    if scale is None:
+        return N.LossScale(None, None, 1.0, 1.0, 0), None
+    if isinstance(scale, _PerValidToken):
+        total = scale.total
+        if isinstance(total, torch.Tensor) and total.is_cuda:
+            total = total.detach().to(device=dev, dtype=torch.float32).reshape(1)
+            return N.LossScale(None, total.data_ptr(), float(scale.multiplier), 1.0, 1), total
+        return N.LossScale(None, None, float(scale.multiplier), float(total), 1), None
+    if isinstance(scale, torch.Tensor) and scale.is_cuda:
+        factor = scale.detach().to(device=dev, dtype=torch.float32).reshape(1)
+        return N.LossScale(factor.data_ptr(), None, 1.0, 1.0, 0), factor
+    return N.LossScale(None, None, float(scale), 1.0, 0), None
+
+
+_NO_RS = N.RsParams()
+
+
+def _rs_struct(cfg) -> N.RsParams:
+    if cfg is None:
+        return _NO_RS
+    _validate_rs(cfg)
+    lower = cfg.lower
+    return N.RsParams(1, N.RS_LEVEL[cfg.level], N.RS_ACTION[cfg.action], N.RS_METRIC[cfg.metric], N.RS_AGG[cfg.agg],
+                      0 if lower is None else 1, float(cfg.upper), 0.0 if lower is None else float(lower))
+
+
+class _Step:
+    """One micro-batch's per-token arrays and the ``aa_ppo_step`` that describes them to the library.
+
+    The outputs are rows of two arrays (float32 and bytes), so that a step allocates three times and not sixteen."""
+
+    # floats: logp, entropy, vmax, vmin, stat_loss, ratio, approx_kl, behave_kl, behave_w, (counts)
+    # bools: (flags), mask_out, clip_mask, dual_clip_mask, behave_mask
+    __slots__ = ("T", "T_active", "device", "floats", "bools", "loss", "mask", "slot", "struct", "rs", "_keep")
+
+    def __init__(self, dev, T, T_active, mask, prox, old, adv, params, rs=None, cu=None, n_segments=0, scale=None,
+                 derived=True, host_counts=False, behave_w=None, counts=None):
+        self.T, self.T_active, self.device, self.rs, self.mask = T, T_active, dev, rs, mask
+        pitch = max(64, (T + 63) & ~63)
+        f = self.floats = torch.empty(10, pitch, dtype=torch.float32, device=dev)
+        b = self.bools = torch.empty(5, pitch, dtype=torch.bool, device=dev)
+        self.loss = torch.empty((), dtype=torch.float32, device=dev)
+        work = _work_words(dev)
+        scale_c, scale_t = _scale_struct(scale, dev)
+        self.slot = _HostSlot(dev) if (rs is not None or host_counts) else None
+        f0, b0, row = f.data_ptr(), b.data_ptr(), pitch * 4
+        c = self.struct = N.PpoStep()
+        c.T, c.T_active = T, T_active
+        c.prox_logp, c.old_logp, c.adv, c.mask = _ptr(prox), _ptr(old), _ptr(adv), _ptr(mask)
+        c.cu_seqlens, c.n_segments = _ptr(cu), n_segments
+        c.params, c.rs, c.scale = params, _rs_struct(rs), scale_c
+        c.logp, c.entropy, c.vmax, c.vmin = f0, f0 + row, f0 + 2 * row, f0 + 3 * row
+        c.stat_loss, c.ratio, c.flags = f0 + 4 * row, f0 + 5 * row, b0
+        if derived:
+            c.approx_kl, c.clip_mask, c.dual_clip_mask = f0 + 6 * row, b0 + 2 * pitch, b0 + 3 * pitch
+            if rs is not None:
+                c.behave_mask, c.behave_kl = b0 + 4 * pitch, f0 + 7 * row
+        if rs is not None:
+            c.mask_out, c.behave_w = b0 + pitch, f0 + 8 * row
+        elif behave_w is not None:
+            c.behave_w = behave_w.data_ptr()
+        if counts is not None:
+            c.counts, c.counts_given = counts.data_ptr(), 1
+        else:
+            c.counts = f0 + 9 * row
+        c.loss = self.loss.data_ptr()
+        if self.slot is not None:
+            c.host_counts, c.host_tag = self.slot.address, self.slot.tag
+        c.work = work.data_ptr()
+        self._keep = (prox, old, adv, mask, cu, scale_t, behave_w, counts, work)
+
+    @property
+    def counts_address(self) -> int:
+        """Where the device has the number of tokens with a loss (an int32)."""
+        return self.struct.counts
+
+    def rows(self) -> list:
+        """logp, entropy, vmax, vmin, stat_loss, ratio: ``[T_active]`` each."""
+        return list(self.floats[:6, : self.T_active].unbind(0))
+
+    def stats(self, rows: bool, shape=None) -> dict:
+        """The stat dict of ``ppo_actor_loss_fn`` (functional.py:505-558); ``rows``: with the per-row outputs as well."""
+        n = self.T_active
+        f = self.floats[:, :n].unbind(0)
+        b = self.bools[:, :n].unbind(0)
+        if shape is not None and len(shape) != 1:
+            f = [v.view(shape) for v in f]
+            b = [v.view(shape) for v in b]
+        stat = dict(loss=f[4], importance_weight=f[5], approx_kl=f[6], clip_mask=b[2], dual_clip_mask=b[3])
+        if rows:
+            stat.update(logprobs=f[0], entropy=f[1], vocab_min_logits=f[3], vocab_max_logits=f[2])
+        if self.rs is not None:
+            total, hit = self.slot.read()
+            stat.update(behave_approx_kl=f[7], behave_imp_weight=f[8], behave_mask=b[4],
+                        filtered_fraction=hit / max(total, 1))
+        return stat
+
+
+# ----------------------------------------------------------------------------
 # PPO actor loss on log-probs
 # ----------------------------------------------------------------------------
 class _PpoLoss(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, logp, prox, adv, mask_eff, behave_w, cu, B, seq_level, params, n_valid):
-        ctx.set_materialize_grads(False)  # no zero-filled gradients for the outputs that have none
-        lib = N.load()
-        dev = logp.device
-        n = logp.numel()
-        stat_loss = torch.empty(n, dtype=torch.float32, device=dev)
-        ratio = torch.empty(n, dtype=torch.float32, device=dev)
-        flags = torch.empty(n, dtype=torch.uint8, device=dev)
-        g_logp = torch.empty(n, dtype=torch.float32, device=dev)
-        loss = torch.empty((), dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
-            st = _stream(dev)
-            N.check(
-                lib.aa_ppo_loss(
-                    _ptr(logp), _ptr(prox), _ptr(adv), _ptr(mask_eff), _ptr(behave_w), n, _ptr(cu), B,
-                    1 if seq_level else 0, C.byref(params), _ptr(n_valid), _ptr(stat_loss), _ptr(ratio),
-                    _ptr(flags), _ptr(g_logp), st,
-                ),
-                "aa_ppo_loss",
-            )
-            N.check(
-                lib.aa_masked_sum(_ptr(stat_loss), _ptr(mask_eff), n, _ptr(n_valid), None, _ptr(loss), st),
-                "aa_masked_sum",
-            )
+    def forward(ctx, logp, step, seq_level):
+        dev = step.device
+        g_logp = torch.empty_like(logp)
+        with _on(dev):
+            N.check(N.load().aa_ppo_loss_step(step.struct, _ptr(logp), 1 if seq_level else 0, 0, _ptr(g_logp), _stream(dev)),
+                    "aa_ppo_loss_step")
         ctx.save_for_backward(g_logp)
-        ctx.mark_non_differentiable(stat_loss, ratio, flags)
-        return loss, stat_loss, ratio, flags
+        return step.loss
 
     @staticmethod
-    def backward(ctx, g_loss, *_unused):
-        if g_loss is None:  # the loss was not used (gradients are not materialised, see forward)
-            return (None,) * 10
+    def backward(ctx, g_loss):
         (g_logp,) = ctx.saved_tensors
-        return (g_logp * g_loss,) + (None,) * 9
+        return g_logp * g_loss, None, None
 
 
 def _flag_bits(flags: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
@@ -449,36 +626,9 @@ def _count_nonzero(mask_u8: torch.Tensor) -> torch.Tensor:
     lib = N.load()
     dev = mask_u8.device
     out = torch.empty(1, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(lib.aa_count_nonzero_u8(_ptr(mask_u8), mask_u8.numel(), _ptr(out), _stream(dev)), "aa_count_nonzero_u8")
     return out
-
-
-def _stat_outputs(logp, prox, old, flags, w, mask_eff_u8):
-    """The derived entries of the stat dict (functional.py:505-558) in one launch: ``approx_kl``, ``clip_mask``,
-    ``dual_clip_mask`` and, with rejection sampling (``w`` given), ``behave_mask`` and ``behave_approx_kl``
-    (None otherwise)."""
-    lib = N.load()
-    dev = logp.device
-    n = logp.numel()
-    logp = logp.detach()
-    logp = logp if logp.is_contiguous() else logp.contiguous()
-    approx_kl = torch.empty(n, dtype=torch.float32, device=dev)
-    clip = torch.empty(n, dtype=torch.uint8, device=dev)
-    dual = torch.empty(n, dtype=torch.uint8, device=dev)
-    behave_mask = behave_kl = None
-    if w is not None:
-        behave_mask = torch.empty(n, dtype=torch.uint8, device=dev)
-        behave_kl = torch.empty(n, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        N.check(
-            lib.aa_ppo_stat_outputs(_ptr(logp), _ptr(prox), _ptr(old), _ptr(flags), _ptr(w), _ptr(mask_eff_u8), n,
-                                    _ptr(approx_kl), _ptr(clip), _ptr(dual), _ptr(behave_mask), _ptr(behave_kl),
-                                    _stream(dev)),
-            "aa_ppo_stat_outputs",
-        )
-    as_bool = lambda t: None if t is None else t.view(torch.bool)
-    return approx_kl, as_bool(clip), as_bool(dual), as_bool(behave_mask), behave_kl
 
 
 def _rs_stats(stat, behave_mask, behave_kl, w, counts, shape):
@@ -519,6 +669,7 @@ def ppo_actor_loss_fn(
     _require_gpu(logprobs, "logprobs")
     shape = logprobs.shape
     seq_level = importance_sampling_level == "sequence"
+    rs = rejection_sampling
     cu, B = None, 0
     if seq_level:
         cu, B = _segments(
@@ -527,40 +678,23 @@ def ppo_actor_loss_fn(
             "cu_seqlens is required for 1D tensors (packed format). For a single sequence, use "
             "cu_seqlens=torch.tensor([0, seq_len], dtype=torch.int32).",
         )
-        if cu is not None:
-            cu = cu.to(logprobs.device)
-    params = _ppo_params(eps_clip, eps_clip_higher, c_clip, rejection_sampling is not None)
-
-    lp = _f32(logprobs).reshape(-1)
-    prox = _f32(proximal_logprobs.detach()).reshape(-1)
-    old = _f32(old_logprobs.detach()).reshape(-1)
-    adv = _f32(advantages.detach()).reshape(-1)
-    m8 = _mask_u8(loss_mask).reshape(-1)
-
-    w = counts = None
-    mask_eff = m8
-    if rejection_sampling is not None:
-        _validate_rs(rejection_sampling)
-        mask_eff, w, counts = _rejection_sampling_device(prox, old, m8, shape, cu_seqlens, rejection_sampling)
-        host_counts = _HostCounts(counts)
-        if rejection_sampling.action != "mask":
-            mask_eff = m8
-        n_valid = counts  # counts[0] is the non-zero count of the original mask
-    else:
-        n_valid = _count_nonzero(m8)
-
-    loss, stat_loss, ratio, flags = _PpoLoss.apply(lp, prox, adv, mask_eff, w, cu, B, seq_level, params, n_valid)
-    approx_kl, clip, dual, behave_mask, behave_kl = _stat_outputs(lp, prox, old, flags, w, mask_eff)
-    stat = dict(
-        loss=stat_loss.view(shape),
-        importance_weight=ratio.view(shape),
-        approx_kl=approx_kl.view(shape),
-        clip_mask=clip.view(shape),
-        dual_clip_mask=dual.view(shape),
-    )
-    if rejection_sampling is not None:
-        _rs_stats(stat, behave_mask, behave_kl, w, host_counts, shape)
-    return loss, stat
+    params = _ppo_params(eps_clip, eps_clip_higher, c_clip, rs is not None)
+    if rs is not None:
+        _validate_rs(rs)
+        if rs.level == "sequence" and not seq_level:
+            cu, B = _segments(shape, cu_seqlens,
+                              "cu_seqlens is required for 1D packed tensors in sequence-level filtering.")
+    dev = logprobs.device
+    if cu is not None:
+        cu = cu.to(dev)
+    lp = logprobs if logprobs.dtype is torch.float32 and logprobs.is_contiguous() else _f32(logprobs)
+    if lp.dim() != 1:
+        lp = lp.reshape(-1)
+    n = lp.numel()
+    step = _Step(dev, n, n, _mask_bytes(loss_mask), _f32_values(proximal_logprobs), _f32_values(old_logprobs),
+                 _f32_values(advantages), params, rs, cu, B)
+    loss = _PpoLoss.apply(lp, step, seq_level)
+    return loss, step.stats(rows=False, shape=shape)
 
 
 # ----------------------------------------------------------------------------
@@ -576,82 +710,71 @@ def _hand_out_once(ctx) -> None:
     ctx.handed_out = True
 
 
-def _finish_fused_loss(lib, params, stat_loss, logp, mask_eff, T_active, n_valid, grad_scale, loss, st) -> None:
-    """The scalar the fused kernels' per-token losses add up to: the clipped surrogate over ``max(n, 1)``, or the
-    negative log-likelihood over ``n + 1e-5`` (areal/trainer/sft/lm_engine.py:96)."""
-    if params.loss_kind == 1:
-        scratch = torch.empty(1, dtype=torch.float64, device=logp.device)
-        cnt = torch.empty(1, dtype=torch.int32, device=logp.device)
-        N.check(lib.aa_sft_loss(_ptr(logp), _ptr(mask_eff), T_active, None, 0, _ptr(n_valid), _ptr(grad_scale),
-                                _ptr(loss), None, None, _ptr(scratch), _ptr(cnt), None, st), "aa_sft_loss")
-    else:
-        N.check(lib.aa_masked_sum(_ptr(stat_loss), _ptr(mask_eff), T_active, _ptr(n_valid), _ptr(grad_scale),
-                                  _ptr(loss), st), "aa_masked_sum")
-
-
 class _FusedLogitsPpo(torch.autograd.Function):
+    """The step on logits; its per-token outputs are in ``step``."""
+
     @staticmethod
-    def forward(ctx, logits2d, labels1d, stride, temperature, T_active, prox, adv, mask_eff, behave_w, params,
-                n_valid, grad_scale, want_minmax, inplace=False):
-        ctx.set_materialize_grads(False)  # no zero-filled gradients for the outputs that have none
-        lib = N.load()
+    def forward(ctx, logits2d, step, labels1d, stride, temperature, inplace):
+        dev = step.device
         T, V = logits2d.shape
-        dev = logits2d.device
-        f32 = dict(dtype=torch.float32, device=dev)
-        logp = torch.empty(T, **f32)
-        entropy = torch.empty(T, **f32)
-        vmax = torch.empty(T, **f32) if want_minmax else None
-        vmin = torch.empty(T, **f32) if want_minmax else None
-        stat_loss = torch.empty(T_active, **f32)
-        ratio = torch.empty(T_active, **f32)
-        flags = torch.empty(T_active, dtype=torch.uint8, device=dev)
-        loss = torch.empty((), **f32)
         if inplace:
             # the gradient takes the place of the logits: every kernel reads an element for the last time before it
             # writes it, so the two arrays of the C entry point may be one
             dlogits = logits2d.detach()
         else:
             dlogits = _empty_rows_like(logits2d, stride)
-        with torch.cuda.device(dev):
-            st = _stream(dev)
+        with _on(dev):
             N.check(
-                lib.aa_logits_ppo_fused(
-                    _ptr(logits2d), _DTYPES[logits2d.dtype], T, V, stride, _ptr(labels1d), 1.0 / float(temperature),
-                    T_active, _ptr(prox), _ptr(adv), _ptr(mask_eff), _ptr(behave_w), C.byref(params),
-                    _ptr(n_valid), _ptr(grad_scale), _ptr(logp), _ptr(entropy), _ptr(vmax), _ptr(vmin),
-                    _ptr(stat_loss), _ptr(ratio), _ptr(flags), _ptr(dlogits), _ptr(_work_words(dev)), st,
-                ),
-                "aa_logits_ppo_fused",
+                N.load().aa_logits_ppo_step(step.struct, _ptr(logits2d), _DTYPES[logits2d.dtype], V, stride, _ptr(labels1d),
+                                            1.0 / temperature, _ptr(dlogits), _stream(dev)),
+                "aa_logits_ppo_step",
             )
-            _finish_fused_loss(lib, params, stat_loss, logp, mask_eff, T_active, n_valid, grad_scale, loss, st)
         if inplace:
             # written through a raw pointer: tell autograd, so that an operation that saved the logits for its own
             # backward fails loudly instead of reading gradients
             torch.autograd.graph.increment_version(logits2d)
         ctx.save_for_backward(dlogits)
-        others = [logp, entropy, stat_loss, ratio, flags] + [t for t in (vmax, vmin) if t is not None]
-        ctx.mark_non_differentiable(*others)
-        return loss, logp, entropy, vmax, vmin, stat_loss, ratio, flags
+        return step.loss
 
     @staticmethod
-    def backward(ctx, g_loss, *_unused):
-        if g_loss is None:
-            return (None,) * 14
+    def backward(ctx, g_loss):
         _hand_out_once(ctx)
-        lib = N.load()
         (dlogits,) = ctx.saved_tensors
         dev = dlogits.device
-        g = _f32(g_loss).reshape(1)
+        g = _f32_values(g_loss)
         # d(logits) was written with the loss; an upstream factor other than 1 is
         # applied in place (the kernel returns at once when the factor is 1).
         T, V = dlogits.shape
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(
-                lib.aa_scale_rows_inplace(_ptr(dlogits), _DTYPES[dlogits.dtype], T, V, dlogits.stride(0) if T > 1 else V,
-                                          _ptr(g), _stream(dev)),
+                N.load().aa_scale_rows_inplace(_ptr(dlogits), _DTYPES[dlogits.dtype], T, V,
+                                               dlogits.stride(0) if T > 1 else V, _ptr(g), _stream(dev)),
                 "aa_scale_rows_inplace",
             )
-        return (dlogits,) + (None,) * 13
+        return dlogits, None, None, None, None, None
+
+
+def _scaled(loss, scale, loss_mask):
+    """``loss`` times a loss scale, for the paths that form the loss with torch."""
+    if scale is None:
+        return loss
+    if isinstance(scale, _PerValidToken):
+        return loss * (loss_mask.count_nonzero() / scale.total * scale.multiplier)
+    return loss * torch.as_tensor(scale, dtype=torch.float32, device=loss.device).reshape(())
+
+
+def _ppo_step(dev, T, T_active, loss_mask, prox, old, adv, eps_clip, eps_clip_higher, c_clip, rs, cu_seqlens, loss_scale):
+    """The ``_Step`` of a token-level PPO loss on a packed micro-batch."""
+    params = _ppo_params(eps_clip, eps_clip_higher, c_clip, rs is not None)
+    cu, B = None, 0
+    if rs is not None:
+        _validate_rs(rs)
+        if rs.level == "sequence":
+            cu, B = _segments(loss_mask.shape, cu_seqlens,
+                              "cu_seqlens is required for 1D packed tensors in sequence-level filtering.")
+            cu = cu.to(dev)
+    return _Step(dev, T, T_active, _mask_bytes(loss_mask), _f32_values(prox), _f32_values(old), _f32_values(adv), params,
+                 rs, cu, B, loss_scale)
 
 
 def fused_logprobs_ppo_loss(
@@ -718,10 +841,6 @@ def fused_logprobs_ppo_loss(
         if t.shape != loss_mask.shape:
             raise ValueError(f"{name} shape {tuple(t.shape)} != loss_mask shape {tuple(loss_mask.shape)}")
     dev = logits.device
-    scale_t = None
-    if loss_scale is not None:
-        scale_t = torch.as_tensor(loss_scale, dtype=torch.float32, device=dev).reshape(1)
-
     # Without a gradient to produce (evaluation, torch.no_grad) the step is the forward kernel (one read of the logits,
     # no [T, V] gradient buffer) followed by the loss on log-probs.
     forward_only = not (torch.is_grad_enabled() and logits.requires_grad)
@@ -733,49 +852,15 @@ def fused_logprobs_ppo_loss(
             logp, proximal_logprobs, old_logprobs, advantages, eps_clip, loss_mask, eps_clip_higher, c_clip,
             rejection_sampling, importance_sampling_level, cu_seqlens,
         )
-        if scale_t is not None:
-            loss = loss * scale_t.squeeze(0)
+        loss = _scaled(loss, loss_scale, loss_mask)
         stat.update(logprobs=logp.detach(), entropy=entropy.detach(), vocab_min_logits=vmin, vocab_max_logits=vmax)
         return loss, stat
 
     x, T, V, stride = _rows(logits)
-    y = labels.to(device=dev, dtype=torch.int64).contiguous()
-    prox = _f32(proximal_logprobs.detach())
-    old = _f32(old_logprobs.detach())
-    adv = _f32(advantages.detach())
-    m8 = _mask_u8(loss_mask)
-    params = _ppo_params(eps_clip, eps_clip_higher, c_clip, rejection_sampling is not None)
-    w = counts = None
-    mask_eff = m8
-    if rejection_sampling is not None:
-        _validate_rs(rejection_sampling)
-        mask_eff, w, counts = _rejection_sampling_device(prox, old, m8, loss_mask.shape, cu_seqlens, rejection_sampling)
-        host_counts = _HostCounts(counts)
-        if rejection_sampling.action != "mask":
-            mask_eff = m8
-        n_valid = counts
-    else:
-        n_valid = _count_nonzero(m8)
-    loss, logp, entropy, vmax, vmin, stat_loss, ratio, flags = _FusedLogitsPpo.apply(
-        x, y, stride, float(temperature), T_active, prox, adv, mask_eff, w, params, n_valid, scale_t, True,
-        bool(inplace_backward),
-    )
-    logp_a = logp[:T_active]
-    approx_kl, clip, dual, behave_mask, behave_kl = _stat_outputs(logp_a, prox, old, flags, w, mask_eff)
-    stat = dict(
-        loss=stat_loss,
-        importance_weight=ratio,
-        approx_kl=approx_kl,
-        clip_mask=clip,
-        dual_clip_mask=dual,
-        logprobs=logp_a,
-        entropy=entropy[:T_active],
-        vocab_min_logits=vmin[:T_active],
-        vocab_max_logits=vmax[:T_active],
-    )
-    if rejection_sampling is not None:
-        _rs_stats(stat, behave_mask, behave_kl, w, host_counts, loss_mask.shape)
-    return loss, stat
+    step = _ppo_step(dev, T, T_active, loss_mask, proximal_logprobs, old_logprobs, advantages, eps_clip, eps_clip_higher,
+                     c_clip, rejection_sampling, cu_seqlens, loss_scale)
+    loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
+    return loss, step.stats(rows=True)
 
 
 # ----------------------------------------------------------------------------
@@ -815,7 +900,7 @@ class _LmHeadLogprobsEntropy(torch.autograd.Function):
         vmax = torch.empty(T, **f32) if want_minmax else None
         vmin = torch.empty(T, **f32) if want_minmax else None
         ws = _lmhead_workspace(T, H, V, dev, forward_only=True, extrema=want_minmax)  # partials only: nothing of size T x V
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(
                 lib.aa_lmhead_fwd(
                     _ptr(hidden), _ptr(weight), T, H, V, _ptr(labels), 1.0 / float(temperature), _ptr(logp),
@@ -857,7 +942,7 @@ def _lmhead_recompute_backward(hidden, weight, labels, temperature, row_lse, row
     chunk = int(lib.aa_lmhead_chunk_tokens())
     n_chunks = (T + chunk - 1) // chunk
     kept = (C.c_int64 * n_chunks)(*([N.AA_LMHEAD_COUNT_ON_DEVICE] * n_chunks))
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(
             lib.aa_lmhead_bwd(
                 _ptr(hidden), _ptr(weight), T, H, V, _ptr(labels), 1.0 / temperature, _ptr(row_lse),
@@ -898,7 +983,7 @@ class _LmHeadCarry(torch.autograd.Function):
             raise N.NativeLibraryError(
                 f"the lm_head path needs a hidden size that is a multiple of 8, and sizes below 2^22 (got H={H}, V={V})")
         ws = torch.empty(n, dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(
                 lib.aa_lmhead_fwd_carry(
                     _ptr(hidden), _ptr(weight), T, H, V, _ptr(labels), 1.0 / float(temperature), _ptr(grad_mask), kept,
@@ -938,7 +1023,7 @@ class _LmHeadCarry(torch.autograd.Function):
         d_hidden = torch.empty_like(hidden)
         d_weight = torch.empty_like(weight)
         ws = torch.empty(lib.aa_lmhead_carry_workspace_bytes(T, H, V), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             N.check(
                 lib.aa_lmhead_bwd_carry(
                     _ptr(hidden), _ptr(weight), T, H, V, _ptr(labels), 1.0 / ctx.temperature, _ptr(logp), _ptr(row_lse),
@@ -1104,7 +1189,7 @@ def lm_head_logprobs_entropy_static(
     for t in out:
         if t.dtype != torch.float32 or tuple(t.shape) != (T,) or not t.is_contiguous() or t.device != dev:
             raise ValueError("out must hold two contiguous float32 tensors of shape [T] on the device of hidden")
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(
             lib.aa_lmhead_fwd_static(_ptr(hidden), _ptr(weight), T, H, V, _ptr(labels), 1.0 / float(temperature), _ptr(logp),
                                      _ptr(entropy), None, None, _stream(dev)),
@@ -1114,58 +1199,42 @@ def lm_head_logprobs_entropy_static(
 
 
 class _FusedLmHeadPpo(torch.autograd.Function):
+    """The step on hidden states; its per-token outputs are in ``step``."""
+
     @staticmethod
-    def forward(ctx, hidden, weight, labels, temperature, T_active, prox, adv, mask_eff, behave_w, params, n_valid,
-                grad_scale, kept_per_chunk, backward_mode):
-        ctx.set_materialize_grads(False)  # no zero-filled gradients for the outputs that have none
+    def forward(ctx, hidden, weight, step, labels, temperature, kept_per_chunk, backward_mode):
         lib = N.load()
         kept = None if kept_per_chunk is None else (C.c_int64 * len(kept_per_chunk))(*kept_per_chunk)
         T, H = hidden.shape
         V = weight.shape[0]
-        dev = hidden.device
-        f32 = dict(dtype=torch.float32, device=dev)
-        logp = torch.empty(T, **f32)
-        entropy = torch.empty(T, **f32)
-        vmax = torch.empty(T, **f32)
-        vmin = torch.empty(T, **f32)
-        stat_loss = torch.empty(T_active, **f32)
-        ratio = torch.empty(T_active, **f32)
-        flags = torch.empty(T_active, dtype=torch.uint8, device=dev)
-        loss = torch.empty((), **f32)
+        dev = step.device
         d_hidden = torch.empty_like(hidden)
         d_weight = torch.empty_like(weight)  # bf16: rounded once, after fp32 accumulation over the chunks
         ws = _lmhead_workspace(T, H, V, dev)
-        with torch.cuda.device(dev):
-            st = _stream(dev)
+        with _on(dev):
             N.check(
-                lib.aa_lmhead_ppo_fused(
-                    _ptr(hidden), _ptr(weight), T, H, V, _ptr(labels), 1.0 / float(temperature), T_active, _ptr(prox),
-                    _ptr(adv), _ptr(mask_eff), _ptr(behave_w), C.byref(params), _ptr(n_valid), _ptr(grad_scale), kept,
-                    int(backward_mode), _ptr(logp), _ptr(entropy), _ptr(stat_loss), _ptr(ratio), _ptr(flags),
-                    _ptr(vmax), _ptr(vmin), _ptr(d_hidden), _ptr(d_weight), _DTYPES[d_weight.dtype], _ptr(ws),
-                    ws.numel(), st,
+                lib.aa_lmhead_ppo_step(
+                    step.struct, _ptr(hidden), _ptr(weight), H, V, _ptr(labels), 1.0 / temperature, kept,
+                    int(backward_mode), _ptr(d_hidden), _ptr(d_weight), _DTYPES[d_weight.dtype], _ptr(ws), ws.numel(),
+                    _stream(dev),
                 ),
-                "aa_lmhead_ppo_fused",
+                "aa_lmhead_ppo_step",
             )
-            _finish_fused_loss(lib, params, stat_loss, logp, mask_eff, T_active, n_valid, grad_scale, loss, st)
         ctx.save_for_backward(d_hidden, d_weight)
-        ctx.mark_non_differentiable(logp, entropy, stat_loss, ratio, flags, vmax, vmin)
-        return loss, logp, entropy, stat_loss, ratio, flags, vmax, vmin
+        return step.loss
 
     @staticmethod
-    def backward(ctx, g_loss, *_unused):
-        if g_loss is None:
-            return (None,) * 14
+    def backward(ctx, g_loss):
         _hand_out_once(ctx)
         lib = N.load()
         d_hidden, d_weight = ctx.saved_tensors
         dev = d_hidden.device
-        g = _f32(g_loss).reshape(1)
-        with torch.cuda.device(dev):  # both gradients were written with the loss; a factor of 1 is a no-op
+        g = _f32_values(g_loss)
+        with _on(dev):  # both gradients were written with the loss; a factor of 1 is a no-op
             for t in (d_hidden, d_weight):
                 N.check(lib.aa_scale_inplace(_ptr(t), _DTYPES[t.dtype], t.numel(), _ptr(g), _stream(dev)),
                         "aa_scale_inplace")
-        return (d_hidden, d_weight) + (None,) * 12
+        return (d_hidden, d_weight) + (None,) * 5
 
 
 def fused_lm_head_ppo_loss(
@@ -1259,10 +1328,7 @@ def fused_lm_head_ppo_loss(
         if t.shape != loss_mask.shape:
             raise ValueError(f"{name} shape {tuple(t.shape)} != loss_mask shape {tuple(loss_mask.shape)}")
     dev = hidden.device
-    scale_t = None
-    if loss_scale is not None:
-        scale_t = torch.as_tensor(loss_scale, dtype=torch.float32, device=dev).reshape(1)
-    y = labels.to(device=dev, dtype=torch.int64).contiguous()
+    y = _labels_i64(labels, dev)
 
     forward_only = not (torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad))
     if importance_sampling_level == "sequence" or forward_only:
@@ -1291,29 +1357,25 @@ def fused_lm_head_ppo_loss(
             logp, proximal_logprobs, old_logprobs, advantages, eps_clip, loss_mask, eps_clip_higher, c_clip,
             rejection_sampling, importance_sampling_level, cu_seqlens,
         )
-        if scale_t is not None:
-            loss = loss * scale_t.squeeze(0)
+        loss = _scaled(loss, loss_scale, loss_mask)
         stat.update(logprobs=logp.detach(), entropy=entropy.detach(), vocab_min_logits=vmin[:T_active],
                     vocab_max_logits=vmax[:T_active])
         return loss, stat
 
-    prox = _f32(proximal_logprobs.detach())
-    old = _f32(old_logprobs.detach())
-    adv = _f32(advantages.detach())
-    m8 = _mask_u8(loss_mask)
-    params = _ppo_params(eps_clip, eps_clip_higher, c_clip, rejection_sampling is not None)
-    w = counts = None
-    mask_eff = m8
-    if rejection_sampling is not None:
-        _validate_rs(rejection_sampling)
-        mask_eff, w, counts = _rejection_sampling_device(prox, old, m8, loss_mask.shape, cu_seqlens, rejection_sampling)
-        host_counts = _HostCounts(counts)
-        if rejection_sampling.action != "mask":
-            mask_eff = m8
-        n_valid = counts
-    else:
-        n_valid = _count_nonzero(m8)
+    rs = rejection_sampling
     if not forward_masked_tokens:
+        prox, old, adv = (_f32(t.detach()) for t in (proximal_logprobs, old_logprobs, advantages))
+        m8 = _mask_u8(loss_mask)
+        params = _ppo_params(eps_clip, eps_clip_higher, c_clip, rs is not None)
+        w, mask_eff = None, m8
+        if rs is not None:
+            _validate_rs(rs)
+            mask_eff, w, n_valid = _rejection_sampling_device(prox, old, m8, loss_mask.shape, cu_seqlens, rs)
+            host_counts = _HostCounts(n_valid)
+            if rs.action != "mask":
+                mask_eff = m8
+        else:
+            n_valid = _count_nonzero(m8)
         # only the tokens with a mask go through the lm_head: gather them (autograd scatters d(hidden) back), run the
         # step on the closed-up batch with an all-true mask, and put the per-token results back at their tokens
         idx = mask_eff.nonzero().squeeze(-1)
@@ -1329,51 +1391,36 @@ def fused_lm_head_ppo_loss(
             ones = torch.ones(n_kept, dtype=torch.uint8, device=dev)
             chunk = int(N.load().aa_lmhead_chunk_tokens())
             kept = [max(0, min(chunk, n_kept - c)) for c in range(0, n_kept, chunk)]
-            loss, logp, entropy, stat_loss, ratio, flags, vmax, vmin = _FusedLmHeadPpo.apply(
-                hidden.index_select(0, idx), weight.contiguous(), y.index_select(0, idx), float(temperature), n_kept,
-                prox.index_select(0, idx), adv.index_select(0, idx), ones,
-                None if w is None else w.index_select(0, idx), params, n_valid, scale_t, kept, _LMHEAD_BACKWARD[backward],
-            )
-            logp, entropy = logp[:n_kept], entropy[:n_kept]
-            clip, dual = _flag_bits(flags)
-            stat = dict(
-                loss=full(stat_loss), importance_weight=full(ratio), approx_kl=full(logp - prox.index_select(0, idx)),
-                clip_mask=full(clip, torch.bool), dual_clip_mask=full(dual, torch.bool),
-                logprobs=full(logp), entropy=full(entropy),
-                vocab_min_logits=full(vmin[:n_kept]), vocab_max_logits=full(vmax[:n_kept]),
-            )
+            step = _Step(dev, n_kept, n_kept, ones, prox.index_select(0, idx), None, adv.index_select(0, idx), params,
+                         scale=loss_scale, behave_w=None if w is None else w.index_select(0, idx), counts=n_valid)
+            loss = _FusedLmHeadPpo.apply(hidden.index_select(0, idx), weight.contiguous(), step, y.index_select(0, idx),
+                                         float(temperature), kept, _LMHEAD_BACKWARD[backward])
+            kept_stat = step.stats(rows=True)
+            stat = {k: full(v, v.dtype) for k, v in kept_stat.items()}
         if rejection_sampling is not None:
             behave_mask = (w > 0) & mask_eff.bool()
             _rs_stats(stat, behave_mask, torch.where(behave_mask, prox - old, 0.0), w, host_counts, loss_mask.shape)
         return loss, stat
+    T = hidden.shape[0]
+    step = _ppo_step(dev, T, T_active, loss_mask, proximal_logprobs, old_logprobs, advantages, eps_clip, eps_clip_higher,
+                     c_clip, rs, cu_seqlens, loss_scale)
     kept = None
     if skip_masked_tokens and kept_per_chunk is not None:
-        chunk = int(N.load().aa_lmhead_chunk_tokens())
+        chunk = lm_head_chunk_tokens()
         kept = [int(v) for v in kept_per_chunk]
-        if len(kept) != (hidden.shape[0] + chunk - 1) // chunk:
+        if len(kept) != (T + chunk - 1) // chunk:
             raise ValueError(f"kept_per_chunk needs one count per chunk of {chunk} tokens")
-    elif skip_masked_tokens:
-        kept = _device_or_read_back_counts(hidden.shape[0], T_active, mask_eff, count_on_device)
-    loss, logp, entropy, stat_loss, ratio, flags, vmax, vmin = _FusedLmHeadPpo.apply(
-        hidden.contiguous(), weight.contiguous(), y, float(temperature), T_active, prox, adv, mask_eff, w, params,
-        n_valid, scale_t, kept, _LMHEAD_BACKWARD[backward],
-    )
-    logp_a = logp[:T_active]
-    approx_kl, clip, dual, behave_mask, behave_kl = _stat_outputs(logp_a, prox, old, flags, w, mask_eff)
-    stat = dict(
-        loss=stat_loss,
-        importance_weight=ratio,
-        approx_kl=approx_kl,
-        clip_mask=clip,
-        dual_clip_mask=dual,
-        logprobs=logp_a,
-        entropy=entropy[:T_active],
-        vocab_min_logits=vmin[:T_active],
-        vocab_max_logits=vmax[:T_active],
-    )
-    if rejection_sampling is not None:
-        _rs_stats(stat, behave_mask, behave_kl, w, host_counts, loss_mask.shape)
-    return loss, stat
+    elif skip_masked_tokens and count_on_device:
+        kept = [N.AA_LMHEAD_COUNT_ON_DEVICE] * ((T + lm_head_chunk_tokens() - 1) // lm_head_chunk_tokens())
+    elif skip_masked_tokens:  # the exact counts are read back: the mask after rejection sampling first
+        mask_eff = _mask_u8(loss_mask)
+        if rs is not None and rs.action == "mask":
+            mask_eff = _rejection_sampling_device(_f32(proximal_logprobs.detach()), _f32(old_logprobs.detach()), mask_eff,
+                                                  loss_mask.shape, cu_seqlens, rs)[0]
+        kept = _device_or_read_back_counts(T, T_active, mask_eff, False)
+    loss = _FusedLmHeadPpo.apply(hidden.contiguous(), weight.contiguous(), step, y, float(temperature), kept,
+                                 _LMHEAD_BACKWARD[backward])
+    return loss, step.stats(rows=True)
 
 
 # ----------------------------------------------------------------------------
@@ -1389,7 +1436,7 @@ class _SapoLoss(torch.autograd.Function):
         stat_loss, ratio, g_logp = (torch.empty(n, **f32) for _ in range(3))
         gates = torch.empty(3, n, **f32)
         loss = torch.empty((), **f32)
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = _stream(dev)
             N.check(
                 lib.aa_sapo_loss(_ptr(logp), _ptr(old), _ptr(adv), _ptr(mask), n, _ptr(cu), B, 1 if seq_level else 0,
@@ -1471,7 +1518,7 @@ class _CriticLoss(torch.autograd.Function):
         stat_loss, g_value = torch.empty(n, **f32), torch.empty(n, **f32)
         clip = torch.empty(n, dtype=torch.uint8, device=dev)
         total = torch.empty((), **f32)
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = _stream(dev)
             N.check(
                 lib.aa_critic_loss(_ptr(value), _ptr(old), _ptr(target), _ptr(mask), n, float(eps), loss_type,

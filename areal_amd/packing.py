@@ -13,7 +13,7 @@ from typing import Any
 import torch
 
 from . import _native as N
-from .functional import _ptr, _require_gpu, _stream
+from .functional import _on, _ptr, _require_gpu, _stream
 
 N_TOKENS_PER_PAGE = 256  # areal/utils/data.py:815
 
@@ -39,7 +39,7 @@ def segment_copy(src: torch.Tensor, dst: torch.Tensor, src_starts: torch.Tensor,
     ss = src_starts.to(device=dev, dtype=torch.int64).contiguous()
     ds = dst_starts.to(device=dev, dtype=torch.int64).contiguous()
     cu = seg_cu.to(device=dev, dtype=torch.int32).contiguous()
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(N.load().aa_segment_copy(_ptr(src), _ptr(dst), row_bytes, _ptr(ss), _ptr(ds), _ptr(cu), B,
                                          int(total_rows), _stream(dev)), "aa_segment_copy")
     return dst

@@ -12,16 +12,18 @@ from . import _native as N
 from .functional import (
     _FusedLmHeadPpo,
     _FusedLogitsPpo,
-    _count_nonzero,
-    _f32,
-    _mask_u8,
+    _Step,
+    _f32_values,
+    _labels_i64,
+    _mask_bytes,
     _require_gpu,
     _rows,
+    _scaled,
     gather_logprobs_entropy_stats,
     lm_head_logprobs_entropy_stats,
     sapo_loss_fn,
 )
-from .sft import _check_fused_inputs, _scale_tensor
+from .sft import _check_fused_inputs
 
 
 def _sapo_params(tau_pos: float, tau_neg: float) -> N.PpoParams:
@@ -43,6 +45,12 @@ def _sapo_stat(stat_loss, ratio, logp, old, adv, tau_pos, tau_neg, extra):
     )
     stat.update(extra)
     return stat
+
+
+def _step_stat(step, old, adv, tau_pos, tau_neg):
+    logp, entropy, vmax, vmin, stat_loss, ratio = step.rows()
+    return _sapo_stat(stat_loss, ratio, logp, old, adv, tau_pos, tau_neg,
+                      dict(logprobs=logp, entropy=entropy, vocab_min_logits=vmin, vocab_max_logits=vmax))
 
 
 def _check_per_token(loss_mask, **tensors):
@@ -67,26 +75,17 @@ def fused_logprobs_sapo_loss(logits: torch.Tensor, labels: torch.Tensor, old_log
     T_active = _check_fused_inputs(logits, labels, loss_mask, "logits")
     _check_per_token(loss_mask, old_logprobs=old_logprobs, advantages=advantages)
     dev = logits.device
-    scale_t = _scale_tensor(loss_scale, dev)
     if not (torch.is_grad_enabled() and logits.requires_grad):
         logp, entropy, vmin, vmax = (t[:T_active] for t in gather_logprobs_entropy_stats(logits, labels, temperature))
         loss, stat = sapo_loss_fn(logp, old_logprobs, advantages, tau_pos, tau_neg, loss_mask)
-        if scale_t is not None:
-            loss = loss * scale_t.squeeze(0)
+        loss = _scaled(loss, loss_scale, loss_mask)
         stat.update(logprobs=logp.detach(), entropy=entropy.detach(), vocab_min_logits=vmin, vocab_max_logits=vmax)
         return loss, stat
     x, T, V, stride = _rows(logits)
-    y = labels.to(device=dev, dtype=torch.int64).contiguous()
-    old, adv = _f32(old_logprobs.detach()), _f32(advantages.detach())
-    m8 = _mask_u8(loss_mask.to(dev))
-    loss, logp, entropy, vmax, vmin, stat_loss, ratio, _flags = _FusedLogitsPpo.apply(
-        x, y, stride, float(temperature), T_active, old, adv, m8, None, params, _count_nonzero(m8), scale_t, True,
-        bool(inplace_backward),
-    )
-    logp_a = logp[:T_active]
-    return loss, _sapo_stat(stat_loss, ratio, logp_a, old, adv, tau_pos, tau_neg,
-                            dict(logprobs=logp_a, entropy=entropy[:T_active], vocab_min_logits=vmin[:T_active],
-                                 vocab_max_logits=vmax[:T_active]))
+    old, adv = _f32_values(old_logprobs), _f32_values(advantages)
+    step = _Step(dev, T, T_active, _mask_bytes(loss_mask.to(dev)), old, None, adv, params, scale=loss_scale, derived=False)
+    loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
+    return loss, _step_stat(step, old, adv, tau_pos, tau_neg)
 
 
 def fused_lm_head_sapo_loss(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor,
@@ -108,17 +107,14 @@ def fused_lm_head_sapo_loss(hidden: torch.Tensor, weight: torch.Tensor, labels: 
     if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         raise TypeError("fused lm_head expects bf16 hidden states and weights")
     dev = hidden.device
-    scale_t = _scale_tensor(loss_scale, dev)
-    y = labels.to(device=dev, dtype=torch.int64).contiguous()
+    y = _labels_i64(labels, dev)
     if not (torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)):
         logp, entropy, vmin, vmax = (t[:T_active] for t in lm_head_logprobs_entropy_stats(hidden, weight, y, temperature))
         loss, stat = sapo_loss_fn(logp, old_logprobs, advantages, tau_pos, tau_neg, loss_mask)
-        if scale_t is not None:
-            loss = loss * scale_t.squeeze(0)
+        loss = _scaled(loss, loss_scale, loss_mask)
         stat.update(logprobs=logp.detach(), entropy=entropy.detach(), vocab_min_logits=vmin, vocab_max_logits=vmax)
         return loss, stat
-    old, adv = _f32(old_logprobs.detach()), _f32(advantages.detach())
-    m8 = _mask_u8(loss_mask.to(dev))
+    old, adv = _f32_values(old_logprobs), _f32_values(advantages)
     kept = None
     if skip_masked_tokens:
         chunk = int(N.load().aa_lmhead_chunk_tokens())
@@ -129,11 +125,8 @@ def fused_lm_head_sapo_loss(hidden: torch.Tensor, weight: torch.Tensor, labels: 
                 raise ValueError(f"kept_per_chunk needs one count per chunk of {chunk} tokens")
         else:  # the device counts the tokens with a mask itself: nothing is read back
             kept = [N.AA_LMHEAD_COUNT_ON_DEVICE] * n_chunks
-    loss, logp, entropy, stat_loss, ratio, _flags, vmax, vmin = _FusedLmHeadPpo.apply(
-        hidden.contiguous(), weight.contiguous(), y, float(temperature), T_active, old, adv, m8, None, params,
-        _count_nonzero(m8), scale_t, kept, 1 if backward == "carry" else 0,
-    )
-    logp_a = logp[:T_active]
-    return loss, _sapo_stat(stat_loss, ratio, logp_a, old, adv, tau_pos, tau_neg,
-                            dict(logprobs=logp_a, entropy=entropy[:T_active], vocab_min_logits=vmin[:T_active],
-                                 vocab_max_logits=vmax[:T_active]))
+    step = _Step(dev, hidden.shape[0], T_active, _mask_bytes(loss_mask.to(dev)), old, None, adv, params, scale=loss_scale,
+                 derived=False)
+    loss = _FusedLmHeadPpo.apply(hidden.contiguous(), weight.contiguous(), step, y, float(temperature), kept,
+                                 1 if backward == "carry" else 0)
+    return loss, _step_stat(step, old, adv, tau_pos, tau_neg)

@@ -5,7 +5,6 @@ with the log-prob op (one pass over the logits that also writes their gradient) 
 """
 from __future__ import annotations
 
-import ctypes as C
 
 import torch
 
@@ -14,9 +13,13 @@ from .functional import (
     _DTYPES,
     _FusedLmHeadPpo,
     _FusedLogitsPpo,
+    _Step,
     _count_nonzero,
     _f32,
+    _labels_i64,
+    _mask_bytes,
     _mask_u8,
+    _on,
     _ptr,
     _require_gpu,
     _rows,
@@ -38,7 +41,8 @@ def _cu_i32(cu_seqlens, dev):
 
 
 def _launch(logp, m8, cu, n_seqs, n_valid, scale, want_grad, want_stat):
-    """``aa_sft_loss``: returns (loss, g_logp, stat_loss, seq_logp, seq_count, seq_ppl)."""
+    """``aa_sft_loss``: returns (loss, g_logp, stat_loss, seq_logp, seq_count, seq_ppl); ``n_valid``: the address of the
+    count on the device."""
     lib = N.load()
     dev = logp.device
     T = logp.numel()
@@ -49,8 +53,8 @@ def _launch(logp, m8, cu, n_seqs, n_valid, scale, want_grad, want_stat):
     seq_logp = torch.empty(n_seqs + 1, dtype=torch.float64, device=dev)
     seq_count = torch.empty(n_seqs + 1, dtype=torch.int32, device=dev)
     seq_ppl = torch.empty(n_seqs, **f32)
-    with torch.cuda.device(dev):
-        N.check(lib.aa_sft_loss(_ptr(logp), _ptr(m8), T, _ptr(cu), n_seqs, _ptr(n_valid), _ptr(scale), _ptr(loss),
+    with _on(dev):
+        N.check(lib.aa_sft_loss(_ptr(logp), _ptr(m8), T, _ptr(cu), n_seqs, n_valid, _ptr(scale), _ptr(loss),
                                 _ptr(g), _ptr(stat_loss), _ptr(seq_logp), _ptr(seq_count), _ptr(seq_ppl),
                                 _stream(dev)), "aa_sft_loss")
     return loss, g, stat_loss, seq_logp, seq_count, seq_ppl
@@ -59,7 +63,7 @@ def _launch(logp, m8, cu, n_seqs, n_valid, scale, want_grad, want_stat):
 class _SftLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logp, m8, cu, n_seqs, n_valid, scale):
-        loss, g, stat_loss, seq_logp, seq_count, seq_ppl = _launch(logp, m8, cu, n_seqs, n_valid, scale, True, True)
+        loss, g, stat_loss, seq_logp, seq_count, seq_ppl = _launch(logp, m8, cu, n_seqs, _ptr(n_valid), scale, True, True)
         ctx.save_for_backward(g)
         ctx.mark_non_differentiable(stat_loss, seq_logp, seq_count, seq_ppl)
         return loss, stat_loss, seq_logp, seq_count, seq_ppl
@@ -72,7 +76,7 @@ class _SftLoss(torch.autograd.Function):
         dev = g.device
         up = _f32(g_loss).reshape(1)
         if out.numel():
-            with torch.cuda.device(dev):
+            with _on(dev):
                 N.check(N.load().aa_scale_inplace(_ptr(out), _DTYPES[out.dtype], out.numel(), _ptr(up), _stream(dev)),
                         "aa_scale_inplace")
         return out, None, None, None, None, None
@@ -111,6 +115,21 @@ def sft_loss_fn(logprobs: torch.Tensor, loss_mask: torch.Tensor, cu_seqlens: tor
     return loss, _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs)
 
 
+def _nll_step(dev, T, T_active, loss_mask, loss_scale, host_counts=False):
+    return _Step(dev, T, T_active, _mask_bytes(loss_mask.to(dev)), None, None, None, _nll_params(), scale=loss_scale,
+                 derived=False, host_counts=host_counts)
+
+
+def _step_stat(step, cu, n_seqs, extrema):
+    """The stat dict of a fused step: that of ``sft_loss_fn`` plus the per-token outputs."""
+    logp, entropy, vmax, vmin, stat_loss, _ratio = step.rows()
+    _, _, _, seq_logp, seq_count, seq_ppl = _launch(logp, step.mask, cu, n_seqs, step.counts_address, None, False, False)
+    extra = dict(logprobs=logp, entropy=entropy)
+    if extrema:
+        extra.update(vocab_min_logits=vmin, vocab_max_logits=vmax)
+    return _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs, extra)
+
+
 def _check_fused_inputs(rows: torch.Tensor, labels: torch.Tensor, loss_mask: torch.Tensor, what: str) -> int:
     if rows.ndim != 2 or labels.ndim != 1 or labels.shape[0] != rows.shape[0]:
         raise ValueError(f"expected {what} [T, .] and labels [T], got {tuple(rows.shape)} and {tuple(labels.shape)}")
@@ -135,7 +154,6 @@ def fused_logprobs_sft_loss(logits: torch.Tensor, labels: torch.Tensor, loss_mas
     _require_gpu(logits, "logits")
     T_active = _check_fused_inputs(logits, labels, loss_mask, "logits")
     dev = logits.device
-    scale_t = _scale_tensor(loss_scale, dev)
     cu, n_seqs = _cu_i32(cu_seqlens, dev)
     if not (torch.is_grad_enabled() and logits.requires_grad):
         logp, entropy, vmin, vmax = (t[:T_active] for t in gather_logprobs_entropy_stats(logits, labels, temperature))
@@ -143,18 +161,9 @@ def fused_logprobs_sft_loss(logits: torch.Tensor, labels: torch.Tensor, loss_mas
         stat.update(logprobs=logp.detach(), entropy=entropy.detach(), vocab_min_logits=vmin, vocab_max_logits=vmax)
         return loss, stat
     x, T, V, stride = _rows(logits)
-    y = labels.to(device=dev, dtype=torch.int64).contiguous()
-    m8 = _mask_u8(loss_mask.to(dev))
-    n_valid = _count_nonzero(m8)
-    loss, logp, entropy, vmax, vmin, stat_loss, _ratio, _flags = _FusedLogitsPpo.apply(
-        x, y, stride, float(temperature), T_active, None, None, m8, None, _nll_params(), n_valid, scale_t, True,
-        bool(inplace_backward),
-    )
-    logp_a = logp[:T_active]
-    _, _, _, seq_logp, seq_count, seq_ppl = _launch(logp_a, m8, cu, n_seqs, n_valid, None, False, False)
-    return loss, _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs,
-                       dict(logprobs=logp_a, entropy=entropy[:T_active], vocab_min_logits=vmin[:T_active],
-                            vocab_max_logits=vmax[:T_active]))
+    step = _nll_step(dev, T, T_active, loss_mask, loss_scale)
+    loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
+    return loss, _step_stat(step, cu, n_seqs, extrema=True)
 
 
 def fused_lm_head_sft_loss(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, loss_mask: torch.Tensor,
@@ -172,17 +181,14 @@ def fused_lm_head_sft_loss(hidden: torch.Tensor, weight: torch.Tensor, labels: t
     if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         raise TypeError("fused lm_head expects bf16 hidden states and weights")
     dev = hidden.device
-    scale_t = _scale_tensor(loss_scale, dev)
     cu, n_seqs = _cu_i32(cu_seqlens, dev)
-    y = labels.to(device=dev, dtype=torch.int64).contiguous()
+    y = _labels_i64(labels, dev)
     if not (torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)):
         logp, entropy = lm_head_logprobs_entropy(hidden, weight, y, temperature)
         logp, entropy = logp[:T_active], entropy[:T_active]
         loss, stat = sft_loss_fn(logp, loss_mask, cu_seqlens, loss_scale)
         stat.update(logprobs=logp.detach(), entropy=entropy.detach())
         return loss, stat
-    m8 = _mask_u8(loss_mask.to(dev))
-    n_valid = _count_nonzero(m8)
     kept = None
     if skip_masked_tokens:
         chunk = int(N.load().aa_lmhead_chunk_tokens())
@@ -193,11 +199,7 @@ def fused_lm_head_sft_loss(hidden: torch.Tensor, weight: torch.Tensor, labels: t
                 raise ValueError(f"kept_per_chunk needs one count per chunk of {chunk} tokens")
         else:  # the device counts the tokens with a mask itself: nothing is read back
             kept = [N.AA_LMHEAD_COUNT_ON_DEVICE] * n_chunks
-    loss, logp, entropy, stat_loss, _ratio, _flags, _vmax, _vmin = _FusedLmHeadPpo.apply(
-        hidden.contiguous(), weight.contiguous(), y, float(temperature), T_active, None, None, m8, None, _nll_params(),
-        n_valid, scale_t, kept, 1,  # aa_lmhead_backward_mode: carry
-    )
-    logp_a = logp[:T_active]
-    _, _, _, seq_logp, seq_count, seq_ppl = _launch(logp_a, m8, cu, n_seqs, n_valid, None, False, False)
-    return loss, _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs,
-                       dict(logprobs=logp_a, entropy=entropy[:T_active]))
+    step = _nll_step(dev, hidden.shape[0], T_active, loss_mask, loss_scale)
+    loss = _FusedLmHeadPpo.apply(hidden.contiguous(), weight.contiguous(), step, y, float(temperature), kept,
+                                 1)  # aa_lmhead_backward_mode: carry
+    return loss, _step_stat(step, cu, n_seqs, extrema=False)

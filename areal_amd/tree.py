@@ -15,7 +15,7 @@ from typing import Any
 import torch
 
 from . import _native as N
-from .functional import _DTYPES, _f32, _ptr, _require_gpu, _rows, _stream
+from .functional import _DTYPES, _f32, _on, _ptr, _require_gpu, _rows, _stream
 
 
 class _PairLogprobs(torch.autograd.Function):
@@ -35,7 +35,7 @@ class _PairLogprobs(torch.autograd.Function):
         logp = torch.empty(K, **f32)
         entropy = torch.empty(K, **f32) if want_entropy else None
         inv_t = 1.0 / float(temperature)
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = _stream(dev)
             N.check(lib.aa_logits_fwd(_ptr(logits2d), _DTYPES[logits2d.dtype], T, V, stride, _ptr(none_label), inv_t,
                                       _ptr(scratch), _ptr(row_ent), _ptr(row_lse), _ptr(row_ez), None, None, st),
@@ -64,7 +64,7 @@ class _PairLogprobs(torch.autograd.Function):
             dlogits = torch.empty_like(logits2d, memory_format=torch.contiguous_format)
         else:
             dlogits = torch.empty_strided((T, V), (ctx.stride, 1), dtype=logits2d.dtype, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = _stream(dev)
             N.check(lib.aa_logits_bwd(_ptr(logits2d), _DTYPES[logits2d.dtype], T, V, ctx.stride, _ptr(none_label),
                                       ctx.inv_t, _ptr(row_lse), _ptr(row_ez), _ptr(G), _ptr(H), T, _ptr(dlogits), st),
@@ -175,7 +175,7 @@ def gather_packed_tree_vocab_stats(logits: torch.Tensor, trie: Any) -> tuple[tor
     f32 = dict(dtype=torch.float32, device=dev)
     vmax, vmin, scratch = torch.empty(T, **f32), torch.empty(T, **f32), torch.empty(T, **f32)
     none_label = torch.full((T,), -1, dtype=torch.int64, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(N.load().aa_logits_fwd(_ptr(x), _DTYPES[x.dtype], T, V, stride, _ptr(none_label), 1.0, _ptr(scratch),
                                        None, None, None, _ptr(vmax), _ptr(vmin), _stream(dev)), "aa_logits_fwd")
     sel = torch.tensor(positions, dtype=torch.int64, device=dev)

@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from . import _native as N
-from .functional import _DTYPES, _f32, _ptr, _require_gpu, _rows, _stream
+from .functional import _DTYPES, _f32, _on, _ptr, _require_gpu, _rows, _stream
 
 
 def shard_statistics(logits_shard: torch.Tensor, labels: torch.Tensor, vocab_start: int, temperature: float = 1.0):
@@ -26,7 +26,7 @@ def shard_statistics(logits_shard: torch.Tensor, labels: torch.Tensor, vocab_sta
     y = torch.where((y >= 0) & (y < V), y, torch.full_like(y, -1)).contiguous()
     f32 = dict(dtype=torch.float32, device=dev)
     logp, lse, ez = torch.empty(T, **f32), torch.empty(T, **f32), torch.empty(T, **f32)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(N.load().aa_logits_fwd(_ptr(x), _DTYPES[x.dtype], T, V, stride, _ptr(y), 1.0 / float(temperature),
                                        _ptr(logp), None, _ptr(lse), _ptr(ez), None, None, _stream(dev)), "aa_logits_fwd")
     return lse, ez, logp, y
@@ -39,7 +39,7 @@ def combine_shard_statistics(lse: torch.Tensor, ez: torch.Tensor, logp_local: to
     dev = lse.device
     f32 = dict(dtype=torch.float32, device=dev)
     logp, entropy, row_lse, row_ez = (torch.empty(T, **f32) for _ in range(4))
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(N.load().aa_vocab_partials_combine(_ptr(_f32(lse)), _ptr(_f32(ez)), _ptr(_f32(logp_local)), S, T,
                                                    _ptr(logp), _ptr(entropy), _ptr(row_lse), _ptr(row_ez),
                                                    _stream(dev)), "aa_vocab_partials_combine")
@@ -59,7 +59,7 @@ def shard_backward(logits_shard: torch.Tensor, labels_local: torch.Tensor, row_l
         out = torch.empty_like(x, memory_format=torch.contiguous_format)
     else:
         out = torch.empty_strided((T, V), (stride, 1), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(N.load().aa_logits_bwd(_ptr(x), _DTYPES[x.dtype], T, V, stride, _ptr(labels_local),
                                        1.0 / float(temperature), _ptr(row_lse), _ptr(row_ez), _ptr(gl), _ptr(gh), T,
                                        _ptr(out), _stream(dev)), "aa_logits_bwd")

@@ -74,6 +74,76 @@ typedef struct {
   float sapo_tau_neg;
 } aa_ppo_params;
 
+/* Rejection-sampling switches of a step (the arguments of
+ * aa_rejection_sampling). */
+typedef struct {
+  int32_t enabled;  /* 0: no rejection sampling, the rest is ignored */
+  int32_t level, action, metric, agg;  /* aa_rs_* */
+  int32_t has_lower;
+  float upper, lower;
+} aa_rs_params;
+
+/* The factor a loss and its gradient are multiplied by:
+ *   value, times *factor when factor is given, and, with per_valid_token != 0,
+ *   times (number of non-zero entries of the loss mask) / (*total or, when
+ *   total is NULL, total_value): the engine's local_weight /
+ *   total_loss_weight * multiplier (fsdp_engine.py:2045) without a launch or a
+ *   copy of its own. */
+typedef struct {
+  const float* factor; /* device pointer or NULL */
+  const float* total;  /* device pointer or NULL */
+  float value;
+  float total_value;
+  int32_t per_valid_token;
+} aa_loss_scale;
+
+/* Bytes of the work buffer of a step: zero before the first launch that uses
+ * it, left zero by every launch; one per stream. */
+#define AA_STEP_WORK_BYTES 4096
+
+/* The per-token side of one micro-batch's loss, for the aa_*_step entry
+ * points: inputs and outputs of aa_rejection_sampling, aa_count_nonzero_u8,
+ * the loss itself, aa_ppo_stat_outputs and aa_masked_sum, which a step runs as
+ * part of one call.  All arrays are [T_active] unless stated. */
+typedef struct {
+  int64_t T;          /* rows of logits or hidden states */
+  int64_t T_active;   /* tokens with a loss; the rows past them are padding */
+  const float* prox_logp;    /* not used by AA_LOSS_NLL (may be NULL) */
+  const float* old_logp;     /* with rejection sampling */
+  const float* adv;          /* not used by AA_LOSS_NLL (may be NULL) */
+  const uint8_t* mask;       /* loss mask, one byte per token */
+  const int32_t* cu_seqlens; /* segments, as in aa_rejection_sampling */
+  int64_t n_segments;
+  aa_ppo_params params;      /* has_behave_weight: taken as 1 with rejection
+                                sampling; without it behave_w is an input */
+  aa_rs_params rs;
+  aa_loss_scale scale;
+  /* outputs */
+  float* logp;     /* [T] */
+  float* entropy;  /* [T] nullable */
+  float* vmax;     /* [T] nullable (together with vmin) */
+  float* vmin;     /* [T] */
+  float* stat_loss;
+  float* ratio;
+  uint8_t* flags;
+  float* approx_kl;      /* these five (the last two with rejection           */
+  uint8_t* clip_mask;    /* sampling only) as in aa_ppo_stat_outputs; all      */
+  uint8_t* dual_clip_mask; /* NULL: not wanted                                 */
+  uint8_t* behave_mask;
+  float* behave_kl;
+  uint8_t* mask_out;     /* with rejection sampling: the updated mask ...      */
+  float* behave_w;       /* ... and the importance weights                     */
+  int32_t* counts;       /* [3] device, as in aa_rejection_sampling            */
+  int32_t counts_given;  /* non-zero (without rejection sampling): counts is an
+                            input, the mask is not counted                     */
+  float* loss;           /* the scaled scalar loss                             */
+  int32_t* host_counts;  /* NULL, or 4 words of pinned host memory: {counts[0],
+                            counts[1], 0, host_tag}, written as soon as the
+                            counts are known, the tag last                     */
+  int32_t host_tag;
+  void* work;            /* AA_STEP_WORK_BYTES */
+} aa_ppo_step;
+
 /* Library version (major * 10000 + minor * 100 + patch). */
 int aa_version(void);
 
@@ -179,6 +249,16 @@ int aa_logits_ppo_fused(const void* logits, int dtype, int64_t T, int64_t V,
                         int32_t* work, void* stream);
 
 /*
+ * One micro-batch from logits to gradient in one call: rejection sampling (or
+ * the count of the mask), aa_logits_ppo_fused, the derived entries of the stat
+ * dict and the scalar loss; three launches.  Arguments as in
+ * aa_logits_ppo_fused; step->T is the number of rows.
+ */
+int aa_logits_ppo_step(const aa_ppo_step* step, const void* logits, int dtype,
+                       int64_t V, int64_t row_stride, const int64_t* labels,
+                       float inv_temperature, void* dlogits, void* stream);
+
+/*
  * The reduction step of the vocabulary-parallel op
  * (areal/utils/functional/vocab_parallel.py:84-372), for n_shards slices
  * [T, V_i] of one [T, V] logits tensor that each went through aa_logits_fwd
@@ -266,6 +346,20 @@ int aa_ppo_loss(const float* logp, const float* prox_logp, const float* adv,
                 const aa_ppo_params* params, const int32_t* n_valid,
                 float* stat_loss, float* ratio, uint8_t* flags, float* g_logp,
                 void* stream);
+
+/*
+ * ppo_actor_loss_fn on log-probs that are given, in one call: rejection
+ * sampling (or the count of the mask), the loss with its closed-form backward,
+ * the derived entries of the stat dict and the scalar loss; two launches at
+ * token level, three at sequence level.  step->T == step->T_active; logp (an
+ * input here) and g_logp [T], the other arrays as in aa_ppo_step (step->logp,
+ * entropy, vmax, vmin are not used).  AA_LOSS_PPO only.  With counts_only != 0
+ * the call ends behind the first launch: counts, and with rejection sampling
+ * mask_out and behave_w.
+ */
+int aa_ppo_loss_step(const aa_ppo_step* step, const float* logp,
+                     int sequence_level, int counts_only, float* g_logp,
+                     void* stream);
 
 /*
  * The derived entries of the stat dict of ppo_actor_loss_fn
@@ -917,6 +1011,18 @@ int aa_mfma_only_loop(int form, int random_operands, int workgroups, int iters,
  * any product path. */
 int aa_hbm_stream_probe(int kind, int nt_policy, const void* src, void* dst,
                         int64_t bytes, int workgroups, void* stream);
+
+/*
+ * aa_lmhead_ppo_fused as a step (see aa_ppo_step): with rejection sampling or
+ * the count of the mask ahead of it, and the derived entries of the stat dict
+ * and the scalar loss behind it.
+ */
+int aa_lmhead_ppo_step(const aa_ppo_step* step, const void* hidden,
+                       const void* weight, int64_t H, int64_t V,
+                       const int64_t* labels, float inv_temperature,
+                       const int64_t* kept_per_chunk, int backward_mode,
+                       void* d_hidden, void* d_weight, int d_weight_dtype,
+                       void* workspace, int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -207,3 +207,34 @@ def test_empty_batches_do_not_raise(device):
     adv, ret = areal_amd.gae_advantages(torch.zeros(0, 8, device=device), torch.zeros(0, 8, device=device),
                                         torch.zeros(0, 8, device=device), eb, 1.0, 0.95)
     assert adv.shape == (0, 8) and ret.shape == (0, 8)
+
+
+@pytest.mark.parametrize("n", [1, 255, 1023, 1024, 1025, 5000, 262144, 262145])
+@pytest.mark.parametrize("rs", [None, dict(level="token", upper=1.3), dict(level="sequence", upper=1.02)])
+def test_step_launches_at_the_edges_of_their_slices(device, n, rs):
+    """One workgroup, whole and ragged slices of 1024 tokens, and more tokens than the largest grid takes one slice of:
+    counts, per-token outputs and loss of the launches around the loss, twice on one work buffer (it comes back zero).
+    Whole numbers exactly; the loss is an fp64 sum of fp32 terms rounded once (and the terms differ by a few ulps of
+    expf): 1e-5 relative to the mean absolute term."""
+    g = torch.Generator().manual_seed(n)
+    prox = -2 + 0.5 * torch.randn(n, generator=g)
+    old, lp = prox + 0.3 * torch.randn(n, generator=g), prox + 0.3 * torch.randn(n, generator=g)
+    adv, mask = torch.randn(n, generator=g), torch.rand(n, generator=g) < 0.7
+    cu = torch.tensor([0] + sorted({n // 3, n // 2, n}), dtype=torch.int32)
+    cfg = None if rs is None else RejectionSamplingConfig(action="mask", metric="ratio", **rs)
+    want_loss, want = oracle.ppo_actor_loss(lp, prox, old, adv, 0.2, mask, rejection_sampling_cfg=cfg, cu_seqlens=cu, c_clip=3.0)
+    d = _to(device, lp, prox, old, adv, mask, cu)
+    for _ in range(2):
+        x = d[0].clone().requires_grad_(True)
+        loss, stat = areal_amd.ppo_actor_loss_fn(x, d[1], d[2], d[3], 0.2, d[4], c_clip=3.0, rejection_sampling=cfg, cu_seqlens=d[5])
+        loss.backward()
+        scale = float(want["loss"].abs().mean()) + 1e-6
+        assert abs(float(loss.detach()) - float(want_loss)) <= 1e-5 * scale
+        for k in ("clip_mask", "dual_clip_mask") + (("behave_mask",) if rs else ()):
+            assert torch.equal(stat[k].cpu(), want[k]), k
+        for k in ("loss", "importance_weight", "approx_kl"):
+            assert torch.allclose(stat[k].cpu(), want[k], rtol=1e-5, atol=1e-5), k
+        if rs:
+            assert stat["filtered_fraction"] == want["filtered_fraction"]
+        kept = mask if not rs else want["behave_mask"]
+        assert float(x.grad[~kept.to(device)].abs().sum()) == 0.0
