@@ -10,7 +10,8 @@ from typing import Any
 import torch
 
 from . import _native as N
-from .functional import _f32, _mask_u8, _on, _ptr, _require_gpu, _stream
+from .advantages import _MOMENT_KEYS
+from .functional import _f32, _f32_values, _mask_bytes, _mask_u8, _on, _ptr, _require_gpu, _stream, _work_words
 
 PROX_APPROX_METHOD_LOGLINEAR = "loglinear"
 PROX_APPROX_METHOD_LINEAR = "linear"
@@ -132,16 +133,6 @@ _LOGSTAT_METHOD_KEYS = ("approx_logp", "behave_imp_weight", "importance_weight",
                         "importance_weight_abs_error", "importance_weight_rel_error")
 
 
-def _moment_rows(table: torch.Tensor) -> list[dict[str, torch.Tensor]]:
-    """``[rows, 4]`` of {sum, min, max, count} -> one dict of 0-d tensors per row, with one division for all rows."""
-    cols = torch.cat([table, (table[:, 0] / table[:, 3])[:, None]], dim=1)
-    rows = []
-    for row in cols.unbind(0):
-        s, lo, hi, c, avg = row.unbind(0)
-        rows.append(dict(sum=s, avg=avg, min=lo, max=hi, count=c))
-    return rows
-
-
 @torch.no_grad()
 def proximal_logging_stats(old_logp: torch.Tensor, logprobs: torch.Tensor, prox_logp_gt: torch.Tensor | None,
                            versions: torch.Tensor | None, current_version: int | None, mask: torch.Tensor,
@@ -160,15 +151,14 @@ def proximal_logging_stats(old_logp: torch.Tensor, logprobs: torch.Tensor, prox_
     is empty without versions.  Nothing is read back: whether any generated token is selected is the ``count``.
     """
     _require_gpu(old_logp, "old_logp")
-    lo = _f32(old_logp.detach()).reshape(-1)
-    ln = _f32(logprobs.detach()).reshape(-1)
-    m8 = _mask_u8(mask.to(lo.device)).reshape(-1)
+    lo, ln = _f32_values(old_logp), _f32_values(logprobs)
+    m8 = _mask_bytes(mask.to(lo.device))
     n = lo.numel()
     if ln.numel() != n or m8.numel() != n:
         raise ValueError("old_logp, logprobs and mask must have the same number of elements")
-    gt = _f32(prox_logp_gt.detach()).reshape(-1) if prox_logp_gt is not None else None
+    gt = _f32_values(prox_logp_gt) if prox_logp_gt is not None else None
     have_versions = versions is not None and current_version is not None
-    ver = versions.to(device=lo.device, dtype=torch.int32).contiguous().reshape(-1) if have_versions else None
+    ver = versions.to(device=lo.device, dtype=torch.int32).contiguous() if have_versions else None
     methods, with_errors = 0, False
     if have_versions and prox_logp_method == "loglinear":
         methods = 1
@@ -176,26 +166,35 @@ def proximal_logging_stats(old_logp: torch.Tensor, logprobs: torch.Tensor, prox_
         methods, with_errors = 7, True
     lib = N.load()
     dev = lo.device
-    out = torch.empty(36, 4, dtype=torch.float32, device=dev)
+    out = torch.empty(36, 5, dtype=torch.float32, device=dev)
     scratch = torch.empty(lib.aa_logging_stats_scratch_bytes(n), dtype=torch.uint8, device=dev)
     with _on(dev):
-        N.check(lib.aa_logging_stats(_ptr(lo), _ptr(ln), _ptr(gt), _ptr(ver), _ptr(m8), n,
-                                     int(current_version) if have_versions else 0, methods, 1 if with_errors else 0,
-                                     _ptr(out), _ptr(scratch), scratch.numel(), _stream(dev)), "aa_logging_stats")
-    rows = _moment_rows(out)
+        N.check(lib.aa_logging_stats_table(_ptr(lo), _ptr(ln), _ptr(gt), _ptr(ver), _ptr(m8), n,
+                                           int(current_version) if have_versions else 0, methods, 1 if with_errors else 0,
+                                           _ptr(out), _ptr(scratch), scratch.numel(), _ptr(_work_words(dev)), _stream(dev)),
+                "aa_logging_stats_table")
+    # the cells of the rows that are returned, as 0-d tensors
+    want = {}  # row of the table -> where its moments go
     compute_logp: dict[str, dict] = {}
-    if gt is not None:
-        compute_logp["prox_logp_gt"] = rows[0]
     version_stats: dict[str, Any] = {}
+    if gt is not None:
+        want[0] = (compute_logp, "prox_logp_gt")
     if have_versions:
         for m, name in enumerate(PROX_APPROX_METHODS_ALL):
             if not (methods >> m) & 1:
                 continue
             for j, key in enumerate(_LOGSTAT_METHOD_KEYS[: 10 if with_errors else 3]):
-                compute_logp[f"{name}/{key}"] = rows[4 + 10 * m + j]
+                want[4 + 10 * m + j] = (compute_logp, f"{name}/{key}")
         for j, key in enumerate(("kl_div_direct", "kl_div_taylor", "kl_div_dual")):
-            compute_logp[key] = rows[1 + j]
-        version_stats = dict(sample_staleness_proximal=rows[34],
-                             sample_staleness_theta=rows[35],
-                             v_theta=int(current_version), v_proximal=int(current_version) - 1)
+            want[1 + j] = (compute_logp, key)
+        want[34] = (version_stats, "sample_staleness_proximal")
+        want[35] = (version_stats, "sample_staleness_theta")
+    for first, last in ((0, 4), (4, 34), (34, 36)):  # one unbind for each part of the table that is in use
+        if any(first <= r < last for r in want):
+            cells = out[first:last].view(-1).unbind(0)
+            for r, (where, key) in want.items():
+                if first <= r < last:
+                    where[key] = dict(zip(_MOMENT_KEYS, cells[5 * (r - first) : 5 * (r - first) + 5]))
+    if have_versions:
+        version_stats.update(v_theta=int(current_version), v_proximal=int(current_version) - 1)
     return dict(compute_logp=compute_logp, version_stats=version_stats)

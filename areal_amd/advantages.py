@@ -13,7 +13,7 @@ from typing import Any, Mapping
 import torch
 
 from . import _native as N
-from .functional import _f32, _mask_u8, _on, _ptr, _require_gpu, _stream
+from .functional import _f32, _f32_values, _mask_bytes, _mask_u8, _on, _ptr, _require_gpu, _stream, _work_words
 
 _LEVELS = {None: 0, "none": 0, "batch": 1, "group": 2}
 
@@ -109,6 +109,51 @@ def gae_advantages(rewards: torch.Tensor, values: torch.Tensor | None, loss_mask
     return adv, ret
 
 
+_MOMENT_KEYS = ("sum", "min", "max", "count", "avg")
+_MAX_MOMENTS = 32
+
+
+def _moment_values(t: torch.Tensor) -> tuple[torch.Tensor, bool]:
+    """``t`` as the moments kernel takes it, and whether it has one byte per token."""
+    if t.dtype is torch.bool:
+        return (t if t.is_contiguous() else t.contiguous()), True
+    return _f32_values(t), False
+
+
+def moments_table(entries: list[tuple[str, torch.Tensor, torch.Tensor | None]]) -> dict[str, dict[str, torch.Tensor]]:
+    """``masked_moments`` of up to 32 tensors, each under a mask of its own (None: every element), in one launch.
+    ``entries``: (name, tensor, mask), all of the same number of elements; bool tensors count as 0 / 1."""
+    k = len(entries)
+    if k == 0:
+        return {}
+    if k > _MAX_MOMENTS:
+        raise ValueError(f"at most {_MAX_MOMENTS} tensors per call")
+    n = entries[0][1].numel()
+    dev = entries[0][1].device
+    keep, byte_values = [], 0
+    values, masks = (C.c_void_p * k)(), (C.c_void_p * k)()
+    for i, (name, t, mask) in enumerate(entries):
+        _require_gpu(t, name)
+        if t.numel() != n or (mask is not None and mask.numel() != n):
+            raise ValueError(f"{name} has {t.numel()} elements, the mask has {n if mask is None else mask.numel()}")
+        v, is_bytes = _moment_values(t)
+        byte_values |= int(is_bytes) << i
+        values[i] = v.data_ptr()
+        keep.append(v)
+        if mask is not None:
+            m = _mask_bytes(mask)
+            masks[i] = m.data_ptr()
+            keep.append(m)
+    lib = N.load()
+    out = torch.empty(k * 5, dtype=torch.float32, device=dev)
+    scratch = torch.empty(lib.aa_moments_table_scratch_bytes(k, n) // 8, dtype=torch.float64, device=dev)
+    with _on(dev):
+        N.check(lib.aa_moments_table(values, masks, byte_values, k, n, _ptr(out), _ptr(scratch), scratch.numel() * 8,
+                                     _ptr(_work_words(dev)), _stream(dev)), "aa_moments_table")
+    cells = out.unbind(0)
+    return {name: dict(zip(_MOMENT_KEYS, cells[5 * i : 5 * i + 5])) for i, (name, _, _) in enumerate(entries)}
+
+
 @torch.no_grad()
 def masked_moments(values: Mapping[str, torch.Tensor], mask: torch.Tensor) -> dict[str, dict[str, torch.Tensor]]:
     """Sum, mean, min, max and count of every tensor in ``values`` over ``mask``, in one launch.
@@ -117,32 +162,11 @@ def masked_moments(values: Mapping[str, torch.Tensor], mask: torch.Tensor) -> di
     (stats_tracker.py:227-285).  Returns ``{name: {"sum", "avg", "min", "max", "count"}}`` of 0-d device tensors;
     ``avg`` is NaN and ``min`` / ``max`` are +/-inf when the mask selects nothing.
     """
-    names = list(values)
-    if not names:
-        return {}
-    if len(names) > 16:
+    if len(values) > 16:
         raise ValueError("at most 16 tensors per call")
-    _require_gpu(mask, "mask")
-    m8 = _mask_u8(mask.reshape(-1))
-    n = m8.numel()
-    tensors = []
-    for k in names:
-        t = values[k]
-        _require_gpu(t, k)
-        if t.numel() != n:
-            raise ValueError(f"{k} has {t.numel()} elements, the mask has {n}")
-        tensors.append(_f32(t.detach()).reshape(-1))
-    dev = m8.device
-    out = torch.empty(len(names), 4, dtype=torch.float32, device=dev)
-    ptrs = (C.c_void_p * len(names))(*[t.data_ptr() for t in tensors])
-    lib = N.load()
-    with _on(dev):
-        N.check(lib.aa_masked_moments(ptrs, len(names), _ptr(m8), n, _ptr(out), _stream(dev)), "aa_masked_moments")
-    res = {}
-    for i, k in enumerate(names):
-        s, lo, hi, c = out[i, 0], out[i, 1], out[i, 2], out[i, 3]
-        res[k] = dict(sum=s, avg=s / c, min=lo, max=hi, count=c)
-    return res
+    if values:
+        _require_gpu(mask, "mask")
+    return moments_table([(name, t, mask) for name, t in values.items()])
 
 
 _KL_IDS = {"k1": 0, "k2": 1, "k3": 2}

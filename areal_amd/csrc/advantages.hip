@@ -380,54 +380,6 @@ __global__ __launch_bounds__(256) void k_overlong_penalty(float* __restrict__ re
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Masked moments of up to kMaxTensors per-token tensors under one mask: out[k] = {sum, min, max, count}
-// (min = +inf, max = -inf when nothing is selected).  One workgroup per tensor, fixed summation order.
-// ------------------------------------------------------------------------------------------------------------------
-constexpr int kMaxTensors = 16;
-struct MomentArgs {
-  const float* v[kMaxTensors];
-};
-
-__global__ __launch_bounds__(kThreads) void k_masked_moments(MomentArgs a, const uint8_t* __restrict__ mask, int64_t n,
-                                                             float* __restrict__ out) {
-  __shared__ double smem_d[kThreads / kWave];
-  __shared__ float smem_lo[kThreads / kWave], smem_hi[kThreads / kWave];
-  const float* v = a.v[blockIdx.x];
-  double s = 0.0, c = 0.0;
-  float lo = __builtin_inff(), hi = -__builtin_inff();
-  for (int64_t i = threadIdx.x; i < n; i += kThreads) {
-    if (mask[i] != 0) {
-      const float x = v[i];
-      s += (double)x;
-      c += 1.0;
-      lo = fminf(lo, x);
-      hi = fmaxf(hi, x);
-    }
-  }
-  s = block_sum<double>(s, smem_d);
-  c = block_sum<double>(c, smem_d);
-  lo = wave_min(lo);
-  hi = wave_max(hi);
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  if (lane == 0) {
-    smem_lo[wave] = lo;
-    smem_hi[wave] = hi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kThreads / kWave; ++w) {
-      lo = fminf(lo, smem_lo[w]);
-      hi = fmaxf(hi, smem_hi[w]);
-    }
-    float* o = out + 4 * blockIdx.x;
-    o[0] = (float)s;
-    o[1] = lo;
-    o[2] = hi;
-    o[3] = (float)c;
-  }
-}
-
-// ------------------------------------------------------------------------------------------------------------------
 // masked_normalization (areal/utils/functional/functional.py:16-53): every row of an [R, C] view is whitened by
 // the mean and the E[x^2] - E[x]^2 variance of its masked values.  A row is cut into `parts` slices, one workgroup
 // each; the second launch adds the slices of its row in a fixed order and writes the result.
@@ -583,21 +535,6 @@ extern "C" int aa_normalize(const float* x, const float* loss_mask, int64_t bs, 
   int64_t blocks = (a.n + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   hipLaunchKernelGGL(k_norm_apply, dim3((unsigned)blocks), dim3(256), 0, st, a, stats, out);
-  return launch_status();
-}
-
-extern "C" int aa_masked_moments(const float* const* values, int n_tensors, const uint8_t* mask, int64_t n,
-                                 float* out, void* stream) {
-  if (!values || !out || n_tensors < 0 || n_tensors > kMaxTensors || n < 0 || (n > 0 && !mask))
-    return AA_ERR_INVALID_ARGUMENT;
-  if (n_tensors == 0) return AA_OK;
-  MomentArgs a{};
-  for (int k = 0; k < n_tensors; ++k) {
-    if (!values[k] && n > 0) return AA_ERR_INVALID_ARGUMENT;
-    a.v[k] = values[k];
-  }
-  hipLaunchKernelGGL(k_masked_moments, dim3((unsigned)n_tensors), dim3(kThreads), 0, (hipStream_t)stream, a, mask, n,
-                     out);
   return launch_status();
 }
 

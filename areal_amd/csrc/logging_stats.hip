@@ -4,6 +4,7 @@
 // Reference: areal/trainer/ppo/actor.py:852-1110 (_log_proximal_approximation_stats, _log_version_staleness_stats
 // and their helpers), reduced as areal/utils/stats_tracker.py:227-285 reduces a tensor under a denominator mask.
 #include "ppo_math.h"
+#include "ppo_step.h"
 
 namespace aa {
 namespace logstats {
@@ -47,56 +48,107 @@ __device__ __forceinline__ void errors(float gt, float approx, float& abs_e, flo
   sq_e = d * d;
 }
 
-// grid = kGroups * parts; workgroup (g, part) reduces its slice of the tokens for the quantities of group g
-__global__ __launch_bounds__(kThreads) void k_partial(const float* __restrict__ old, const float* __restrict__ logp,
-                                                      const float* __restrict__ gt, const int32_t* __restrict__ versions,
-                                                      const uint8_t* __restrict__ mask, int64_t n, int current_version,
-                                                      int methods, int with_errors, int parts,
-                                                      Partial* __restrict__ partial) {
-  __shared__ double sh_sum[kWaves], sh_cnt[kWaves];
-  __shared__ float sh_lo[kWaves], sh_hi[kWaves];
-  const int g = blockIdx.x / parts, part = blockIdx.x % parts;
-  const int64_t per = (n + parts - 1) / parts;
-  const int64_t b = (int64_t)part * per, e = b + per < n ? b + per : n;
+struct Args {
+  const float* old;
+  const float* logp;
+  const float* gt;
+  const int32_t* versions;
+  const uint8_t* mask;
+  int64_t n;
+  int current_version, methods, with_errors, parts;
+  Partial* partial;
+  float* out;
+  int cols;        // 4, or 5 with the mean behind the count
+  StepWork* work;  // nullable: k_finish follows as a launch of its own
+};
+
+__device__ __forceinline__ bool active(const Args& a, int g) { return g == 0 || ((a.methods >> (g - 1)) & 1); }
+
+// One wave folds the slices of (group, quantity): lane l folds slices l, l + 64, ... in index order, then a fixed
+// butterfly folds the lanes; out[slot] = {sum, min, max, count(, mean)}
+__device__ __forceinline__ void fold(const Args& a, int g, int j) {
+  const int slot = slot_of(g, j);
+  if (slot < 0) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  double sum = 0.0, cnt = 0.0;
+  float lo = __builtin_inff(), hi = -__builtin_inff();
+  if (active(a, g)) {
+    for (int p = lane; p < a.parts; p += kWave) {
+      const Partial v = a.partial[((int64_t)g * a.parts + p) * kPerGroup + j];
+      sum += v.sum;
+      cnt += v.cnt;
+      lo = nan_min(lo, v.lo);
+      hi = nan_max(hi, v.hi);
+    }
+    sum = wave_sum(sum);
+    cnt = wave_sum(cnt);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = nan_min(lo, __shfl_xor(lo, o, kWave));
+      hi = nan_max(hi, __shfl_xor(hi, o, kWave));
+    }
+  }
+  if (lane == 0) {
+    float* o = a.out + a.cols * slot;
+    o[0] = (float)sum;
+    o[1] = lo;
+    o[2] = hi;
+    o[3] = (float)cnt;
+    if (a.cols > 4) o[4] = (float)sum / (float)cnt;
+  }
+}
+
+// Workgroup (g, part) reduces its slice of the tokens for the quantities of group g; only the groups that are asked for
+// are launched (blockIdx.x / parts counts those).  With the work buffer the last workgroup to finish folds the slices of
+// all groups; otherwise k_finish does, one launch later.
+__global__ __launch_bounds__(kThreads) void k_partial(Args a) {
+  __shared__ double sh_sum[kPerGroup][kWaves], sh_cnt[kPerGroup][kWaves];
+  __shared__ float sh_lo[kPerGroup][kWaves], sh_hi[kPerGroup][kWaves];
+  __shared__ int last;
+  int g = 0;
+  for (int left = blockIdx.x / a.parts; left > 0;) {  // the left-th active group
+    ++g;
+    if (active(a, g)) --left;
+  }
+  const int part = blockIdx.x % a.parts;
+  const int64_t per = (a.n + a.parts - 1) / a.parts;
+  const int64_t b = (int64_t)part * per, e = b + per < a.n ? b + per : a.n;
   Acc acc[kPerGroup];
-  const bool active = g == 0 || ((methods >> (g - 1)) & 1);
-  if (active) {
-    for (int64_t i = b + threadIdx.x; i < e; i += kThreads) {
-      if (mask[i] == 0) continue;
-      const float lo = old[i], ln = logp[i];
-      if (g == 0) {
-        if (gt) acc[0].add(gt[i]);
-        if (versions) {
-          const float lr = ln - lo;                       // actor.py:1049
-          acc[1].add(-lr);
-          acc[2].add(lr * lr / 2.0f);
-          acc[3].add(expf(lr) - 1.f - lr);
-          const int ver = versions[i];
-          if (ver >= 0) {                                 // actor.py:1087-1094
-            acc[4].add((float)(current_version - 1) - (float)ver);
-            acc[5].add((float)current_version - (float)ver);
-          }
+  for (int64_t i = b + threadIdx.x; i < e; i += kThreads) {
+    if (a.mask[i] == 0) continue;
+    const float lo = a.old[i], ln = a.logp[i];
+    if (g == 0) {
+      if (a.gt) acc[0].add(a.gt[i]);
+      if (a.versions) {
+        const float lr = ln - lo;                       // actor.py:1049
+        acc[1].add(-lr);
+        acc[2].add(lr * lr / 2.0f);
+        acc[3].add(expf(lr) - 1.f - lr);
+        const int ver = a.versions[i];
+        if (ver >= 0) {                                 // actor.py:1087-1094
+          acc[4].add((float)(a.current_version - 1) - (float)ver);
+          acc[5].add((float)a.current_version - (float)ver);
         }
-      } else {
-        const float ap = prox_approx_value(lo, ln, versions[i], current_version, g - 1);
-        const float bw = expf(ap - lo), iw = expf(ln - ap);     // actor.py:924-925
-        acc[0].add(ap);
-        acc[1].add(bw);
-        acc[2].add(iw);
-        if (with_errors) {                                      // actor.py:934-968
-          const float p = gt[i];
-          float a, r, s;
-          errors(p, ap, a, r, s);
-          acc[3].add(a);
-          acc[4].add(r);
-          acc[5].add(s);
-          errors(expf(p - lo), bw, a, r, s);
-          acc[6].add(a);
-          acc[7].add(r);
-          errors(expf(ln - p), iw, a, r, s);
-          acc[8].add(a);
-          acc[9].add(r);
-        }
+      }
+    } else {
+      const float ap = prox_approx_value(lo, ln, a.versions[i], a.current_version, g - 1);
+      const float bw = expf(ap - lo), iw = expf(ln - ap);     // actor.py:924-925
+      acc[0].add(ap);
+      acc[1].add(bw);
+      acc[2].add(iw);
+      if (a.with_errors) {                                      // actor.py:934-968
+        const float p = a.gt[i];
+        float ae, re, se;
+        errors(p, ap, ae, re, se);
+        acc[3].add(ae);
+        acc[4].add(re);
+        acc[5].add(se);
+        errors(expf(p - lo), bw, ae, re, se);
+        acc[6].add(ae);
+        acc[7].add(re);
+        errors(expf(ln - p), iw, ae, re, se);
+        acc[8].add(ae);
+        acc[9].add(re);
       }
     }
   }
@@ -110,61 +162,44 @@ __global__ __launch_bounds__(kThreads) void k_partial(const float* __restrict__ 
       lo = nan_min(lo, __shfl_xor(lo, o, kWave));
       hi = nan_max(hi, __shfl_xor(hi, o, kWave));
     }
-    __syncthreads();
     if (lane == 0) {
-      sh_sum[wave] = s;
-      sh_cnt[wave] = c;
-      sh_lo[wave] = lo;
-      sh_hi[wave] = hi;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      Partial r{sh_sum[0], sh_cnt[0], sh_lo[0], sh_hi[0], {0.f, 0.f}};
-      for (int w = 1; w < kWaves; ++w) {
-        r.sum += sh_sum[w];
-        r.cnt += sh_cnt[w];
-        r.lo = nan_min(r.lo, sh_lo[w]);
-        r.hi = nan_max(r.hi, sh_hi[w]);
-      }
-      partial[((int64_t)g * parts + part) * kPerGroup + j] = r;
+      sh_sum[j][wave] = s;
+      sh_cnt[j][wave] = c;
+      sh_lo[j][wave] = lo;
+      sh_hi[j][wave] = hi;
     }
   }
+  __syncthreads();
+  if (threadIdx.x < kPerGroup) {
+    const int j = threadIdx.x;
+    Partial r{sh_sum[j][0], sh_cnt[j][0], sh_lo[j][0], sh_hi[j][0], {0.f, 0.f}};
+    for (int w = 1; w < kWaves; ++w) {
+      r.sum += sh_sum[j][w];
+      r.cnt += sh_cnt[j][w];
+      r.lo = nan_min(r.lo, sh_lo[j][w]);
+      r.hi = nan_max(r.hi, sh_hi[j][w]);
+    }
+    a.partial[((int64_t)g * a.parts + part) * kPerGroup + j] = r;
+    __threadfence();
+  }
+  if (!a.work) return;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();
+    last = atomicAdd(&a.work->logged, 1) == (int)gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  for (int q = wave; q < kGroups * kPerGroup; q += kWaves) fold(a, q / kPerGroup, q % kPerGroup);
+  if (threadIdx.x == 0) a.work->logged = 0;
 }
 
-// one wave per (group, quantity): lane l folds slices l, l + 64, ... in index order, then a fixed butterfly folds
-// the lanes; out[slot] = {sum, min, max, count}
-__global__ __launch_bounds__(kWave) void k_finish(const Partial* __restrict__ partial, int parts,
-                                                  float* __restrict__ out) {
-  const int g = blockIdx.x / kPerGroup, j = blockIdx.x % kPerGroup;
-  const int slot = slot_of(g, j);
-  if (slot < 0) return;
-  double sum = 0.0, cnt = 0.0;
-  float lo = __builtin_inff(), hi = -__builtin_inff();
-  for (int p = threadIdx.x; p < parts; p += kWave) {
-    const Partial v = partial[((int64_t)g * parts + p) * kPerGroup + j];
-    sum += v.sum;
-    cnt += v.cnt;
-    lo = nan_min(lo, v.lo);
-    hi = nan_max(hi, v.hi);
-  }
-  sum = wave_sum(sum);
-  cnt = wave_sum(cnt);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = nan_min(lo, __shfl_xor(lo, o, kWave));
-    hi = nan_max(hi, __shfl_xor(hi, o, kWave));
-  }
-  if (threadIdx.x == 0) {
-    float* o = out + 4 * slot;
-    o[0] = (float)sum;
-    o[1] = lo;
-    o[2] = hi;
-    o[3] = (float)cnt;
-  }
-}
+// one wave per (group, quantity)
+__global__ __launch_bounds__(kWave) void k_finish(Args a) { fold(a, blockIdx.x / kPerGroup, blockIdx.x % kPerGroup); }
 
 inline int parts_for(int64_t n) {
-  int64_t parts = (n + 2047) / 2048;   // at least 8 tokens per thread
+  int64_t parts = (n + 511) / 512;  // two tokens per thread: bound by latency (4 096 tokens: 17.6 + 3.9 us with eight and a second launch, 14.4 us so)
   if (parts > 256) parts = 256;
   return parts < 1 ? 1 : (int)parts;
 }
@@ -180,10 +215,9 @@ extern "C" int64_t aa_logging_stats_scratch_bytes(int64_t n) {
   return (int64_t)kGroups * parts_for(n) * kPerGroup * (int64_t)sizeof(Partial);
 }
 
-extern "C" int aa_logging_stats(const float* old_logp, const float* logp, const float* prox_logp_gt,
-                                const int32_t* versions, const uint8_t* mask, int64_t n, int current_version,
-                                int methods, int with_errors, float* out, void* scratch, int64_t scratch_bytes,
-                                void* stream) {
+static int logging_stats(const float* old_logp, const float* logp, const float* prox_logp_gt, const int32_t* versions,
+                         const uint8_t* mask, int64_t n, int current_version, int methods, int with_errors, float* out,
+                         int cols, void* scratch, int64_t scratch_bytes, void* work, void* stream) {
   if (n < 0 || !out || !scratch || methods < 0 || methods > 7) return AA_ERR_INVALID_ARGUMENT;
   if (n > 0 && (!old_logp || !logp || !mask)) return AA_ERR_INVALID_ARGUMENT;
   // an empty batch may come with null data pointers: nothing is dereferenced, every row comes out empty
@@ -192,9 +226,200 @@ extern "C" int aa_logging_stats(const float* old_logp, const float* logp, const 
   const int parts = parts_for(n);
   if (scratch_bytes < (int64_t)kGroups * parts * kPerGroup * (int64_t)sizeof(Partial)) return AA_ERR_INVALID_ARGUMENT;
   hipStream_t st = (hipStream_t)stream;
-  Partial* partial = (Partial*)scratch;
-  hipLaunchKernelGGL(k_partial, dim3((unsigned)(kGroups * parts)), dim3(kThreads), 0, st, old_logp, logp, prox_logp_gt,
-                     versions, mask, n, current_version, methods, with_errors ? 1 : 0, parts, partial);
-  hipLaunchKernelGGL(k_finish, dim3(kGroups * kPerGroup), dim3(kWave), 0, st, partial, parts, out);
+  const Args a{old_logp, logp, prox_logp_gt, versions, mask, n, current_version, methods, with_errors ? 1 : 0, parts,
+               (Partial*)scratch, out, cols, (StepWork*)work};
+  const int groups = 1 + __builtin_popcount((unsigned)methods);
+  hipLaunchKernelGGL(k_partial, dim3((unsigned)(groups * parts)), dim3(kThreads), 0, st, a);
+  if (!work) hipLaunchKernelGGL(k_finish, dim3(kGroups * kPerGroup), dim3(kWave), 0, st, a);
+  return launch_status();
+}
+
+extern "C" int aa_logging_stats(const float* old_logp, const float* logp, const float* prox_logp_gt,
+                                const int32_t* versions, const uint8_t* mask, int64_t n, int current_version,
+                                int methods, int with_errors, float* out, void* scratch, int64_t scratch_bytes,
+                                void* stream) {
+  return logging_stats(old_logp, logp, prox_logp_gt, versions, mask, n, current_version, methods, with_errors, out, 4,
+                       scratch, scratch_bytes, nullptr, stream);
+}
+
+extern "C" int aa_logging_stats_table(const float* old_logp, const float* logp, const float* prox_logp_gt,
+                                      const int32_t* versions, const uint8_t* mask, int64_t n, int current_version,
+                                      int methods, int with_errors, float* out, void* scratch, int64_t scratch_bytes,
+                                      void* work, void* stream) {
+  if (!work) return AA_ERR_INVALID_ARGUMENT;
+  return logging_stats(old_logp, logp, prox_logp_gt, versions, mask, n, current_version, methods, with_errors, out, 5,
+                       scratch, scratch_bytes, work, stream);
+}
+
+// ------------------------------------------------------------------------------------------------------------------
+// Masked moments of per-token tensors (areal/utils/stats_tracker.py:227-285): every tensor under a mask of its own,
+// float32 or one byte per token, all in one launch.  A tensor is cut into slices of kMomentSlice tokens (64 at most),
+// one workgroup each; the last workgroup of a tensor to finish folds its slices in index order.  Bound by latency: what
+// this replaces is a launch per mask, one workgroup per tensor (7 us at 4 096 tokens), a division per tensor and a
+// conversion of every byte tensor, some twenty launches of a loss function.
+// ------------------------------------------------------------------------------------------------------------------
+namespace aa {
+namespace logstats {
+
+constexpr int kMomentThreads = 256;
+constexpr int kMomentSlice = 2048;
+constexpr int kMomentParts = 64;
+
+struct MomentPartial {
+  double sum;
+  int32_t cnt;
+  float lo, hi, pad;
+};
+
+struct MomentArgs {
+  const void* v[kTableTensors];
+  const uint8_t* mask[kTableTensors];  // nullable: every token
+  uint32_t bytes;                      // bit k: tensor k has one byte per token
+  int64_t n;
+  int parts, cols;
+  MomentPartial* partial;  // [tensors][parts], not used with one part
+  StepWork* work;          // not used with one part
+  float* out;              // [tensors][cols]: sum, min, max, count(, mean)
+};
+
+__global__ __launch_bounds__(kMomentThreads) void k_moments(MomentArgs a) {
+  constexpr int kW = kMomentThreads / kWave;
+  __shared__ double sh_s[kW];
+  __shared__ int sh_c[kW];
+  __shared__ float sh_lo[kW], sh_hi[kW];
+  __shared__ int last;
+  const int k = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
+  const uint8_t* mask = a.mask[k];
+  const bool bytes = (a.bytes >> k) & 1;
+  const int64_t per = (a.n + a.parts - 1) / a.parts;
+  const int64_t b = (int64_t)part * per, e = b + per < a.n ? b + per : a.n;
+  double s = 0.0;
+  int c = 0;
+  float lo = __builtin_inff(), hi = -__builtin_inff();
+#pragma unroll 4
+  for (int64_t i = b + threadIdx.x; i < e; i += kMomentThreads) {
+    const bool on = mask ? mask[i] != 0 : true;
+    const float x = bytes ? (float)((const uint8_t*)a.v[k])[i] : ((const float*)a.v[k])[i];
+    if (on) {
+      s += (double)x;
+      c += 1;
+      lo = fminf(lo, x);
+      hi = fmaxf(hi, x);
+    }
+  }
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  auto fold_waves = [&](int n_waves) {
+    s = wave_sum(s);
+    c = wave_sum(c);
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+    if (n_waves > 1) {
+      if (lane == 0) {
+        sh_s[wave] = s;
+        sh_c[wave] = c;
+        sh_lo[wave] = lo;
+        sh_hi[wave] = hi;
+      }
+      __syncthreads();
+      s = sh_s[0];
+      c = sh_c[0];
+      lo = sh_lo[0];
+      hi = sh_hi[0];
+      for (int w = 1; w < n_waves; ++w) {
+        s += sh_s[w];
+        c += sh_c[w];
+        lo = fminf(lo, sh_lo[w]);
+        hi = fmaxf(hi, sh_hi[w]);
+      }
+    }
+  };
+  fold_waves(kW);
+  if (a.parts > 1) {
+    if (threadIdx.x == 0) {
+      a.partial[blockIdx.x] = MomentPartial{s, c, lo, hi, 0.f};
+      __threadfence();
+      last = atomicAdd(&a.work->moments[k], 1) == a.parts - 1;
+    }
+    __syncthreads();
+    if (!last || wave != 0) return;
+    __threadfence();
+    s = 0.0;
+    c = 0;
+    lo = __builtin_inff();
+    hi = -__builtin_inff();
+    if (lane < a.parts) {  // lane p holds slice p
+      const MomentPartial p = a.partial[k * a.parts + lane];
+      s = p.sum;
+      c = p.cnt;
+      lo = p.lo;
+      hi = p.hi;
+    }
+    fold_waves(1);
+    if (lane == 0) a.work->moments[k] = 0;
+  }
+  if (threadIdx.x == 0) {
+    float* o = a.out + (int64_t)a.cols * k;
+    o[0] = (float)s;
+    o[1] = lo;
+    o[2] = hi;
+    o[3] = (float)c;
+    if (a.cols > 4) o[4] = (float)s / (float)c;
+  }
+}
+
+static int moment_parts(int64_t n) {
+  int64_t p = (n + kMomentSlice - 1) / kMomentSlice;
+  return (int)(p < 1 ? 1 : (p > kMomentParts ? kMomentParts : p));
+}
+
+}  // namespace logstats
+}  // namespace aa
+
+extern "C" int64_t aa_moments_table_scratch_bytes(int n_tensors, int64_t n) {
+  if (n_tensors < 0 || n_tensors > kTableTensors || n < 0) return -1;
+  return (int64_t)n_tensors * moment_parts(n) * (int64_t)sizeof(MomentPartial);
+}
+
+extern "C" int aa_moments_table(const void* const* values, const uint8_t* const* masks, uint32_t byte_values,
+                                int n_tensors, int64_t n, float* out, void* scratch, int64_t scratch_bytes, void* work,
+                                void* stream) {
+  if (!values || !masks || !out || !work || n_tensors < 0 || n_tensors > kTableTensors || n < 0 || n > 0x7fffffff)
+    return AA_ERR_INVALID_ARGUMENT;
+  if (n_tensors == 0) return AA_OK;
+  MomentArgs a{};
+  a.parts = moment_parts(n);
+  if (a.parts > 1 && (!scratch || (((uintptr_t)scratch) & 7) || scratch_bytes < aa_moments_table_scratch_bytes(n_tensors, n)))
+    return AA_ERR_INVALID_ARGUMENT;
+  for (int k = 0; k < n_tensors; ++k) {
+    if (!values[k] && n > 0) return AA_ERR_INVALID_ARGUMENT;
+    a.v[k] = values[k];
+    a.mask[k] = masks[k];
+  }
+  a.bytes = byte_values;
+  a.n = n;
+  a.cols = 5;
+  a.partial = (MomentPartial*)scratch;
+  a.work = (StepWork*)work;
+  a.out = out;
+  hipLaunchKernelGGL(k_moments, dim3((unsigned)(n_tensors * a.parts)), dim3(kMomentThreads), 0, (hipStream_t)stream, a);
+  return launch_status();
+}
+
+extern "C" int aa_masked_moments(const float* const* values, int n_tensors, const uint8_t* mask, int64_t n, float* out,
+                                 void* stream) {
+  if (!values || !out || n_tensors < 0 || n_tensors > 16 || n < 0 || n > 0x7fffffff || (n > 0 && !mask))
+    return AA_ERR_INVALID_ARGUMENT;
+  if (n_tensors == 0) return AA_OK;
+  MomentArgs a{};
+  for (int k = 0; k < n_tensors; ++k) {
+    if (!values[k] && n > 0) return AA_ERR_INVALID_ARGUMENT;
+    a.v[k] = values[k];
+    a.mask[k] = mask;
+  }
+  a.n = n;
+  a.parts = 1;
+  a.cols = 4;
+  a.out = out;
+  hipLaunchKernelGGL(k_moments, dim3((unsigned)n_tensors), dim3(kMomentThreads), 0, (hipStream_t)stream, a);
   return launch_status();
 }

@@ -16,7 +16,6 @@
 namespace aa {
 
 constexpr int kSegThreads = 256;
-constexpr int kFinishBlocks = 256;  // most workgroups of a launch that finishes a step
 
 struct Segments {
   const int32_t* cu;  // [B+1] or nullptr
@@ -98,20 +97,12 @@ __global__ void k_zero_i32(int32_t* p, int n) {
 // Who takes the counts of a launch: two counters that the caller has cleared (work == nullptr), or the work buffer of a
 // step: the workgroups add up there, the last one to finish moves the sums to counts (and to host memory) and leaves the
 // buffer zero for the next launch.  One launch then does what took a clearing kernel, this one, and a copy to the host.
-struct StepWork {
-  int32_t rows[2];  // row hand-out of the fused logits kernel
-  int32_t total, hit, done;
-  int32_t finished;
-  int32_t pad[10];
-  double partial[kFinishBlocks];
-};
-static_assert(sizeof(StepWork) <= AA_STEP_WORK_BYTES, "the work buffer of a step");
-
 struct Counts {
   int32_t* counts;
   StepWork* work;
   int32_t* host;
   int32_t tag;
+  const int32_t* cu_end;  // nullable: one more number for the host, the end of the last segment
 };
 
 __device__ __forceinline__ void host_store(int32_t* p, int32_t v, int order_release) {
@@ -142,7 +133,7 @@ __device__ __forceinline__ void count_up(const Counts& c, int total, int hit) {
   if (c.host) {
     host_store(c.host + 0, total, 0);
     host_store(c.host + 1, hit, 0);
-    host_store(c.host + 2, 0, 0);
+    host_store(c.host + 2, c.cu_end ? *c.cu_end : 0, 0);
     host_store(c.host + 3, c.tag, 1);
   }
 }
@@ -420,24 +411,30 @@ __global__ __launch_bounds__(256) void k_ppo_stat_outputs(const float* __restric
 // workgroup, and k_ppo_stat_outputs were two, 9 us on the stream).  A workgroup takes a contiguous slice of the tokens
 // and leaves the fp64 sum of its masked losses; the last one to finish adds the sums in slice order: the same order in
 // every run.
-constexpr int kFinishSlice = 1024;  // tokens per workgroup, or a multiple
+// Slices are large (four tokens per thread of a large workgroup) so that ordinary micro-batches take one workgroup, or
+// few: the hand-over to the last one costs about 4 us (4 096 tokens: 10.7 us with a token at a time, 6.7 us so; two workgroups 11.5, eight 10.0 us).
+constexpr int kFinishThreads = 1024;
+constexpr int kFinishAhead = 4;
+constexpr int kFinishSlice = kFinishAhead * kFinishThreads;  // tokens per workgroup, or a multiple
 
+// (restrict: the outputs do not overlap the inputs, so that the loads of later tokens need not wait for the stores of
+// earlier ones)
 struct FinishArgs {
-  const float* logp;
-  const float* prox;
-  const float* old;
-  const float* adv;
-  const uint8_t* mask;     // the mask the loss is summed under
-  const float* behave_w;   // nullable
-  float* stat_loss;
-  float* ratio;
-  uint8_t* flags;
-  float* g_logp;
-  float* approx_kl;        // nullable: no derived entries
-  uint8_t* clip;
-  uint8_t* dual;
-  uint8_t* behave_mask;    // nullable (with behave_kl)
-  float* behave_kl;
+  const float* __restrict__ logp;
+  const float* __restrict__ prox;
+  const float* __restrict__ old;
+  const float* __restrict__ adv;
+  const uint8_t* __restrict__ mask;     // the mask the loss is summed under
+  const float* __restrict__ behave_w;   // nullable
+  float* __restrict__ stat_loss;
+  float* __restrict__ ratio;
+  uint8_t* __restrict__ flags;
+  float* __restrict__ g_logp;
+  float* __restrict__ approx_kl;        // nullable: no derived entries
+  uint8_t* __restrict__ clip;
+  uint8_t* __restrict__ dual;
+  uint8_t* __restrict__ behave_mask;    // nullable (with behave_kl)
+  float* __restrict__ behave_kl;
   const int32_t* n_valid;
   float* loss;
   StepWork* work;
@@ -448,39 +445,64 @@ struct FinishArgs {
 
 // TOKEN_LOSS: the clipped surrogate and its derivative are formed here as well (log-probs that are given, token level)
 template <bool TOKEN_LOSS>
-__global__ __launch_bounds__(256) void k_step_finish(FinishArgs a) {
-  __shared__ double smem[256 / kWave];
+__global__ __launch_bounds__(kFinishThreads) void k_step_finish(FinishArgs a) {
+  __shared__ double smem[kFinishThreads / kWave];
   __shared__ int last;
   const int nv = *a.n_valid;
   const float fn = a.P.loss_kind == AA_LOSS_NLL ? (float)nv + 1e-5f : (float)(nv < 1 ? 1 : nv);
   const int64_t b = (int64_t)blockIdx.x * a.per, e = b + a.per < a.n ? b + a.per : a.n;
   double acc = 0.0;
-  for (int64_t i = b + threadIdx.x; i < e; i += 256) {
-    const bool m = a.mask[i] != 0;
-    float l;
-    uint8_t f = 0;
-    if constexpr (TOKEN_LOSS) {
-      const float r = m ? expf(a.logp[i] - a.prox[i]) : 0.f;
-      const Surrogate s = surrogate(r, a.adv[i], a.P.has_behave_weight ? a.behave_w[i] : 1.f, a.P);
-      l = s.loss;
-      f = (uint8_t)(((s.clip && m) ? 1 : 0) | ((s.dual && m) ? 2 : 0));
-      a.stat_loss[i] = l;
-      a.ratio[i] = r;
-      a.g_logp[i] = m ? s.dloss_dr * r / fn : 0.f;
-    } else {
-      l = a.stat_loss[i];
-      if (a.approx_kl) f = a.flags[i];
+  // kFinishAhead tokens of a thread at a time, their loads issued together (a token at a time, each load waits for the
+  // one before it)
+  for (int64_t i0 = b + threadIdx.x; i0 < e; i0 += kFinishAhead * kFinishThreads) {
+    uint8_t mask[kFinishAhead], fl[kFinishAhead];
+    float lp[kFinishAhead], prox[kFinishAhead], old[kFinishAhead], adv[kFinishAhead], bw[kFinishAhead], sl[kFinishAhead];
+#pragma unroll
+    for (int q = 0; q < kFinishAhead; ++q) {
+      const int64_t i = i0 + q * kFinishThreads < e ? i0 + q * kFinishThreads : e - 1;
+      mask[q] = a.mask[i];
+      if (TOKEN_LOSS || a.approx_kl) {
+        lp[q] = a.logp[i];
+        prox[q] = a.prox[i];
+      }
+      if (a.behave_w) bw[q] = a.behave_w[i];
+      if (a.behave_mask) old[q] = a.old[i];
+      if constexpr (TOKEN_LOSS) {
+        adv[q] = a.adv[i];
+      } else {
+        sl[q] = a.stat_loss[i];
+        if (a.approx_kl) fl[q] = a.flags[i];
+      }
     }
-    if (m) acc += (double)l;
-    if (a.approx_kl) {
-      const float p = a.prox[i];
-      a.approx_kl[i] = a.logp[i] - p;
-      a.clip[i] = f & 1;
-      a.dual[i] = (f >> 1) & 1;
-      if (a.behave_mask) {
-        const bool on = a.behave_w[i] > 0.f && m;
-        a.behave_mask[i] = on ? 1 : 0;
-        a.behave_kl[i] = on ? p - a.old[i] : 0.f;
+#pragma unroll
+    for (int q = 0; q < kFinishAhead; ++q) {
+      const int64_t i = i0 + q * kFinishThreads;
+      if (i >= e) break;
+      const bool m = mask[q] != 0;
+      float l;
+      uint8_t f = 0;
+      if constexpr (TOKEN_LOSS) {
+        const float r = m ? expf(lp[q] - prox[q]) : 0.f;
+        const Surrogate s = surrogate(r, adv[q], a.P.has_behave_weight ? bw[q] : 1.f, a.P);
+        l = s.loss;
+        f = (uint8_t)(((s.clip && m) ? 1 : 0) | ((s.dual && m) ? 2 : 0));
+        a.stat_loss[i] = l;
+        a.ratio[i] = r;
+        a.g_logp[i] = m ? s.dloss_dr * r / fn : 0.f;
+      } else {
+        l = sl[q];
+        if (a.approx_kl) f = fl[q];
+      }
+      if (m) acc += (double)l;
+      if (a.approx_kl) {
+        a.approx_kl[i] = lp[q] - prox[q];
+        a.clip[i] = f & 1;
+        a.dual[i] = (f >> 1) & 1;
+        if (a.behave_mask) {
+          const bool on = bw[q] > 0.f && m;
+          a.behave_mask[i] = on ? 1 : 0;
+          a.behave_kl[i] = on ? prox[q] - old[q] : 0.f;
+        }
       }
     }
   }
@@ -702,7 +724,7 @@ extern "C" int aa_rejection_sampling(const float* prox_logp, const float* old_lo
   RsCfg c{level, action, metric, agg, has_lower, upper, lower};
   hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, counts, 3);
   if (n == 0) return launch_status();
-  const Counts cleared{counts, nullptr, nullptr, 0};
+  const Counts cleared{counts, nullptr, nullptr, 0, nullptr};
   if (level == AA_RS_LEVEL_TOKEN) {
     hipLaunchKernelGGL(k_rs_token, dim3(grid_for(n)), dim3(256), 0, st, prox_logp, old_logp, mask_in, n, c, mask_out,
                        behave_w, cleared);
@@ -753,7 +775,8 @@ int step_prepare(const aa_ppo_step& p, void* stream) {
   if (p.counts_given) return AA_OK;
   hipStream_t st = (hipStream_t)stream;
   const int64_t n = p.T_active;
-  const Counts counts{p.counts, (StepWork*)p.work, p.host_counts, p.host_tag};
+  const Counts counts{p.counts, (StepWork*)p.work, p.host_counts, p.host_tag,
+                      p.cu_seqlens ? p.cu_seqlens + p.n_segments : nullptr};
   const aa_rs_params& r = p.rs;
   if (!r.enabled || n == 0) {
     int64_t blocks = (n + 4095) / 4096;  // 16 mask bytes per thread
@@ -801,8 +824,8 @@ static int launch_finish(const aa_ppo_step& p, const float* logp, float* g_logp,
   int64_t blocks = (a.n + kFinishSlice - 1) / kFinishSlice;
   blocks = blocks < 1 ? 1 : (blocks > kFinishBlocks ? kFinishBlocks : blocks);
   a.per = (a.n + blocks - 1) / blocks;
-  if (g_logp) hipLaunchKernelGGL(k_step_finish<true>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
-  else hipLaunchKernelGGL(k_step_finish<false>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+  if (g_logp) hipLaunchKernelGGL(k_step_finish<true>, dim3((unsigned)blocks), dim3(kFinishThreads), 0, (hipStream_t)stream, a);
+  else hipLaunchKernelGGL(k_step_finish<false>, dim3((unsigned)blocks), dim3(kFinishThreads), 0, (hipStream_t)stream, a);
   return launch_status();
 }
 

@@ -6,6 +6,21 @@
 
 namespace aa {
 
+constexpr int kFinishBlocks = 256;  // most workgroups of a launch that finishes a step
+constexpr int kTableTensors = 32;   // most tensors of a moments table
+
+// The work buffer of a step: zero before the first launch that uses it, left zero by every launch.
+struct StepWork {
+  int32_t rows[2];  // row hand-out of the fused logits kernel
+  int32_t total, hit, done;
+  int32_t finished;
+  int32_t logged;
+  int32_t pad[9];
+  int32_t moments[kTableTensors];
+  double partial[kFinishBlocks];
+};
+static_assert(sizeof(StepWork) <= AA_STEP_WORK_BYTES, "the work buffer of a step");
+
 // Argument check of the parts of a step that these launches and the loss kernels use.
 int step_args_status(const aa_ppo_step& p);
 // counts (and their copy in host memory), and with rejection sampling mask_out and behave_w

@@ -15,6 +15,7 @@ import torch
 
 from .advantages import gae_advantages, kl_regularized_rewards
 from .functional import (
+    _ppo_actor_loss,
     fused_lm_head_ppo_loss,
     fused_logprobs_ppo_loss,
     gather_logprobs,
@@ -280,6 +281,23 @@ def infer_token_denominator(input_data: dict[str, Any], fallback: torch.Tensor) 
     return torch.ones_like(fallback, **common)
 
 
+def _n_tokens(input_data: dict[str, Any], fallback: torch.Tensor, step=None) -> int:
+    """``infer_token_denominator(input_data, fallback).numel()`` without the mask; ``step``: the step whose counts came to
+    the host with the end of its ``cu_seqlens``, so that nothing else is read back."""
+    attention_mask = input_data.get("attention_mask")
+    if isinstance(attention_mask, torch.Tensor):
+        return attention_mask.numel()
+    cu_seqlens = input_data.get("cu_seqlens")
+    if isinstance(cu_seqlens, torch.Tensor) and cu_seqlens.numel() > 0:
+        if step is not None and step.slot is not None and step.struct.cu_seqlens:
+            return step.slot.read()[2]
+        return int(cu_seqlens[-1].item())
+    input_ids = input_data.get("input_ids")
+    if isinstance(input_ids, torch.Tensor) and input_ids.shape == fallback.shape:
+        return input_ids.numel()
+    return fallback.numel()
+
+
 def resolve_proximal_logp(prox_logp_gt, prox_logp_method: str, old_logp, logprobs, versions, current_version):
     """``_resolve_proximal_logp`` (areal/trainer/ppo/actor.py:687-765): the recomputed proximal log-probs when
     they are there, the log-linear approximation from per-token versions when the forward pass was skipped."""
@@ -340,7 +358,7 @@ def grpo_loss_fn(
     ``"version_stats"`` what it logs in those scopes (actor.py:573-594, 982-1110; ``proximal_logging_stats``).
     """
     from .actor_ops import apply_m2po_masking, distillation_terms, proximal_logging_stats
-    from .advantages import masked_moments
+    from .advantages import moments_table
     from .functional import sapo_loss_fn
 
     old_logp = input_data["logprobs"]
@@ -351,6 +369,7 @@ def grpo_loss_fn(
                                       input_data.get("versions"), current_version)
     if m2_threshold is not None:
         loss_mask = apply_m2po_masking(old_logp, prox_logp, loss_mask, m2_threshold)
+    step = None
     if use_sapo_loss:
         if use_decoupled_loss:
             raise ValueError(
@@ -360,9 +379,9 @@ def grpo_loss_fn(
         loss, stat = sapo_loss_fn(logprobs, old_logp, advantages, sapo_tau_pos, sapo_tau_neg, loss_mask,
                                   importance_sampling_level, input_data.get("cu_seqlens"))
     else:
-        loss, stat = ppo_actor_loss_fn(logprobs, prox_logp, old_logp, advantages, eps_clip, loss_mask, eps_clip_higher,
-                                       c_clip, rejection_sampling, importance_sampling_level,
-                                       input_data.get("cu_seqlens"))
+        loss, stat, step = _ppo_actor_loss(logprobs, prox_logp, old_logp, advantages, eps_clip, loss_mask, eps_clip_higher,
+                                           c_clip, rejection_sampling, importance_sampling_level,
+                                           input_data.get("cu_seqlens"), host_counts=True)
     rkl_stat = None
     teacher_logp = input_data.get("teacher_logp")
     if teacher_logp is not None:
@@ -377,33 +396,34 @@ def grpo_loss_fn(
             loss = rl_loss_weight * loss + distill_loss_weight * mean
             rkl_stat = term
     per_valid = dict(
-        importance_weight=stat["importance_weight"], approx_kl=stat["approx_kl"], new_logp=logprobs.detach(),
-        old_logp=old_logp, entropy=entropy.float(), actor_loss=stat["loss"], clip_ratio=stat["clip_mask"].float(),
-        dual_clip_ratio=stat["dual_clip_mask"].float(),
+        importance_weight=stat["importance_weight"], approx_kl=stat["approx_kl"], new_logp=logprobs, old_logp=old_logp,
+        entropy=entropy, actor_loss=stat["loss"], clip_ratio=stat["clip_mask"], dual_clip_ratio=stat["dual_clip_mask"],
     )
     if use_sapo_loss:
         per_valid.update(sapo_soft_gate=stat["sapo_soft_gate"], sapo_scaled_gate_pos=stat["sapo_scaled_gate_pos"],
                          sapo_scaled_gate_neg=stat["sapo_scaled_gate_neg"])
     if rkl_stat is not None:
         per_valid.update(rkl_loss=rkl_stat)
-    reduced = masked_moments(per_valid, loss_mask)
+    # every logged tensor under its own mask, one launch
+    entries = [(name, t, loss_mask) for name, t in per_valid.items()]
     if not use_sapo_loss:
         clip_mask = stat["clip_mask"]
-        reduced.update(masked_moments(dict(clipped_new_logp=logprobs.detach(), clipped_old_logp=old_logp), clip_mask))
+        entries += [("clipped_new_logp", logprobs, clip_mask), ("clipped_old_logp", old_logp, clip_mask)]
     if "behave_imp_weight" in stat:
-        reduced.update(masked_moments(dict(behave_imp_weight=stat["behave_imp_weight"],
-                                           behave_approx_kl=stat["behave_approx_kl"]), stat["behave_mask"]))
-    if "filtered_fraction" in stat:
-        reduced["rs_filtered_fraction"] = stat["filtered_fraction"]
+        entries += [(k, stat[k], stat["behave_mask"]) for k in ("behave_imp_weight", "behave_approx_kl")]
     if vocab_min_logits is not None and vocab_max_logits is not None:
-        everything = torch.ones_like(loss_mask)
-        reduced.update(masked_moments(dict(vocab_min_logits=vocab_min_logits, vocab_max_logits=vocab_max_logits),
-                                      everything))
-    reduced["n_tokens"] = infer_token_denominator(input_data, loss_mask).numel()
+        entries += [("vocab_min_logits", vocab_min_logits, None), ("vocab_max_logits", vocab_max_logits, None)]
+    reduced = moments_table(entries)
     # the compute_logp and version_stats scopes (actor.py:573-594) under the mask the loss kept
     reduced.update(proximal_logging_stats(old_logp, logprobs.detach(), input_data.get("prox_logp"),
                                           input_data.get("versions"), current_version,
                                           stat.get("behave_mask", loss_mask), prox_logp_method))
+    # what the host has to wait for comes last, when everything is queued
+    reduced["n_tokens"] = _n_tokens(input_data, loss_mask, step)
+    if step is not None:
+        step.finish(stat)
+    if "filtered_fraction" in stat:
+        reduced["rs_filtered_fraction"] = stat["filtered_fraction"]
     stat = dict(stat, loss_mask=loss_mask, reduced=reduced)
     return loss, stat
 
@@ -413,7 +433,7 @@ def critic_loss_fn(value: torch.Tensor, input_data: dict[str, Any], eps_clip: fl
 
     Returns ``(loss, stat)`` with ``stat["reduced"]`` holding what the reference logs tensor by tensor (sums,
     averages, extrema under ``n_valid_tokens`` and ``clipped_tokens``) and ``n_tokens``."""
-    from .advantages import masked_moments
+    from .advantages import moments_table
     from .functional import ppo_critic_loss_fn
 
     value = value.squeeze(-1).float()
@@ -422,10 +442,11 @@ def critic_loss_fn(value: torch.Tensor, input_data: dict[str, Any], eps_clip: fl
     loss_mask = input_data["loss_mask"].bool()
     loss, stat = ppo_critic_loss_fn(value, old_value, target_value, eps_clip, loss_mask)
     clip_mask = stat["clip_mask"]
-    reduced = masked_moments(dict(new_value=value.detach(), old_value=old_value, target_value=target_value,
-                                  critic_loss=stat["loss"], clip_ratio=clip_mask.float()), loss_mask)
-    reduced.update(masked_moments(dict(clipped_new_value=value.detach(), clipped_old_value=old_value), clip_mask))
-    reduced["n_tokens"] = infer_token_denominator(input_data, value).numel()
+    reduced = moments_table(
+        [("new_value", value, loss_mask), ("old_value", old_value, loss_mask), ("target_value", target_value, loss_mask),
+         ("critic_loss", stat["loss"], loss_mask), ("clip_ratio", clip_mask, loss_mask),
+         ("clipped_new_value", value, clip_mask), ("clipped_old_value", old_value, clip_mask)])
+    reduced["n_tokens"] = _n_tokens(input_data, value)
     return loss, dict(stat, loss_mask=loss_mask, reduced=reduced)
 
 
@@ -468,16 +489,16 @@ def compute_packed_sft_loss(logprobs: torch.Tensor, entropy: torch.Tensor | None
     Returns ``(loss, stat)``; ``stat`` holds what the reference records: per token ``loss`` under ``n_valid_tokens``
     (= ``loss_mask``), per sequence ``ppl`` under ``n_seqs`` (the sequences with a selected token), and in
     ``stat["reduced"]`` the moments of ``loss`` and of the vocabulary extrema (under all tokens) when given."""
-    from .advantages import masked_moments
+    from .advantages import moments_table
     from .sft import sft_loss_fn
 
     del entropy  # SFT does not use entropy
     loss_mask = input_["loss_mask"].bool()
     loss, stat = sft_loss_fn(logprobs, loss_mask, input_["cu_seqlens"])
-    reduced = masked_moments(dict(loss=stat["loss"]), loss_mask)
+    entries = [("loss", stat["loss"], loss_mask)]
     if vocab_min_logits is not None and vocab_max_logits is not None:
-        reduced.update(masked_moments(dict(vocab_min_logits=vocab_min_logits, vocab_max_logits=vocab_max_logits),
-                                      torch.ones_like(loss_mask)))
+        entries += [("vocab_min_logits", vocab_min_logits, None), ("vocab_max_logits", vocab_max_logits, None)]
+    reduced = moments_table(entries)
     reduced["n_tokens"] = logprobs.shape[0]
     return loss, dict(stat, loss_mask=loss_mask, reduced=reduced)
 

@@ -459,8 +459,8 @@ class _HostSlot:
         self._device = device
         self._got = None
 
-    def read(self) -> tuple[int, int]:
-        """(non-zero entries of the loss mask, tokens filtered or clamped)"""
+    def read(self) -> tuple[int, int, int]:
+        """(non-zero entries of the loss mask, tokens filtered or clamped, end of the last segment if there are any)"""
         if self._got is not None:
             return self._got
         words, tag = self._words, self.tag
@@ -476,7 +476,7 @@ class _HostSlot:
                 if done.query() and words[3] != tag:
                     raise N.NativeLibraryError("the counts of a step never reached the host")
                 time.sleep(2e-5)
-        self._got = (words[0], words[1])
+        self._got = (words[0], words[1], words[2])
         memory, self._memory = self._memory, None
         _HostSlot._pool.append((memory, words))
         return self._got
@@ -590,9 +590,14 @@ class _Step:
         if rows:
             stat.update(logprobs=f[0], entropy=f[1], vocab_min_logits=f[3], vocab_max_logits=f[2])
         if self.rs is not None:
-            total, hit = self.slot.read()
-            stat.update(behave_approx_kl=f[7], behave_imp_weight=f[8], behave_mask=b[4],
-                        filtered_fraction=hit / max(total, 1))
+            stat.update(behave_approx_kl=f[7], behave_imp_weight=f[8], behave_mask=b[4])
+        return stat
+
+    def finish(self, stat: dict) -> dict:
+        """Adds what has to be waited for: with rejection sampling the share of the tokens it hit."""
+        if self.rs is not None:
+            total, hit, _ = self.slot.read()
+            stat["filtered_fraction"] = hit / max(total, 1)
         return stat
 
 
@@ -662,6 +667,17 @@ def ppo_actor_loss_fn(
     ``behave_mask``, ``filtered_fraction``.  The loss is differentiable in
     ``logprobs`` (closed-form gradient computed with the forward).
     """
+    loss, stat, step = _ppo_actor_loss(logprobs, proximal_logprobs, old_logprobs, advantages, eps_clip, loss_mask,
+                                       eps_clip_higher, c_clip, rejection_sampling, importance_sampling_level, cu_seqlens)
+    return loss, step.finish(stat)
+
+
+def _ppo_actor_loss(logprobs, proximal_logprobs, old_logprobs, advantages, eps_clip, loss_mask, eps_clip_higher=None,
+                    c_clip=None, rejection_sampling=None, importance_sampling_level="token", cu_seqlens=None,
+                    host_counts=False):
+    """``ppo_actor_loss_fn`` without its wait: the caller finishes the stat dict (``_Step.finish``) when it has queued
+    what else it has.  ``host_counts``: the counts come to the host (``step.slot``) also without rejection sampling, and
+    with them the end of the last sequence of a packed batch."""
     if importance_sampling_level not in ("token", "sequence"):
         raise ValueError(
             f"Invalid importance_sampling_level: {importance_sampling_level}. Must be 'token' or 'sequence'."
@@ -685,6 +701,8 @@ def ppo_actor_loss_fn(
             cu, B = _segments(shape, cu_seqlens,
                               "cu_seqlens is required for 1D packed tensors in sequence-level filtering.")
     dev = logprobs.device
+    if cu is None and host_counts and cu_seqlens is not None and cu_seqlens.numel() > 0 and len(shape) == 1:
+        cu, B = _segments(shape, cu_seqlens, "")
     if cu is not None:
         cu = cu.to(dev)
     lp = logprobs if logprobs.dtype is torch.float32 and logprobs.is_contiguous() else _f32(logprobs)
@@ -692,9 +710,9 @@ def ppo_actor_loss_fn(
         lp = lp.reshape(-1)
     n = lp.numel()
     step = _Step(dev, n, n, _mask_bytes(loss_mask), _f32_values(proximal_logprobs), _f32_values(old_logprobs),
-                 _f32_values(advantages), params, rs, cu, B)
+                 _f32_values(advantages), params, rs, cu, B, host_counts=host_counts)
     loss = _PpoLoss.apply(lp, step, seq_level)
-    return loss, step.stats(rows=False, shape=shape)
+    return loss, step.stats(rows=False, shape=shape), step
 
 
 # ----------------------------------------------------------------------------
@@ -860,7 +878,7 @@ def fused_logprobs_ppo_loss(
     step = _ppo_step(dev, T, T_active, loss_mask, proximal_logprobs, old_logprobs, advantages, eps_clip, eps_clip_higher,
                      c_clip, rejection_sampling, cu_seqlens, loss_scale)
     loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
-    return loss, step.stats(rows=True)
+    return loss, step.finish(step.stats(rows=True))
 
 
 # ----------------------------------------------------------------------------
@@ -1420,7 +1438,7 @@ def fused_lm_head_ppo_loss(
         kept = _device_or_read_back_counts(T, T_active, mask_eff, False)
     loss = _FusedLmHeadPpo.apply(hidden.contiguous(), weight.contiguous(), step, y, float(temperature), kept,
                                  _LMHEAD_BACKWARD[backward])
-    return loss, step.stats(rows=True)
+    return loss, step.finish(step.stats(rows=True))
 
 
 # ----------------------------------------------------------------------------

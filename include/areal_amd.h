@@ -138,7 +138,8 @@ typedef struct {
                             input, the mask is not counted                     */
   float* loss;           /* the scaled scalar loss                             */
   int32_t* host_counts;  /* NULL, or 4 words of pinned host memory: {counts[0],
-                            counts[1], 0, host_tag}, written as soon as the
+                            counts[1], cu_seqlens[n_segments] (0 without
+                            segments), host_tag}, written as soon as the
                             counts are known, the tag last                     */
   int32_t host_tag;
   void* work;            /* AA_STEP_WORK_BYTES */
@@ -624,6 +625,18 @@ int aa_logging_stats(const float* old_logp, const float* logp,
                      int64_t scratch_bytes, void* stream);
 
 /*
+ * The same in one launch, with the mean behind the count: out
+ * [AA_LOGSTAT_SLOTS, 5] float32 = {sum, min, max, count, sum / count}.
+ * work: AA_STEP_WORK_BYTES, see aa_ppo_step.
+ */
+int aa_logging_stats_table(const float* old_logp, const float* logp,
+                           const float* prox_logp_gt, const int32_t* versions,
+                           const uint8_t* mask, int64_t n, int current_version,
+                           int methods, int with_errors, float* out,
+                           void* scratch, int64_t scratch_bytes, void* work,
+                           void* stream);
+
+/*
  * compute_rw_loss (areal/trainer/rw/rw_engine.py:115-146) over a packed batch
  * of interleaved (chosen, rejected) sequences: the score of a sequence is
  * scores[cu_seqlens[s + 1] - 1]; a pair is valid when both sequences are
@@ -728,6 +741,21 @@ int aa_normalize(const float* x, const float* loss_mask, int64_t bs,
  */
 int aa_masked_moments(const float* const* values, int n_tensors,
                       const uint8_t* mask, int64_t n, float* out, void* stream);
+
+/*
+ * Masked moments of up to 32 per-token tensors, each under a mask of its own,
+ * in one launch: out[k] = {sum, min, max, count, sum / count} (NaN mean when
+ * nothing is selected).  values and masks are HOST arrays of n_tensors device
+ * pointers; a NULL mask selects every token; bit k of byte_values: tensor k has
+ * one byte per token instead of a float32.  scratch:
+ * aa_moments_table_scratch_bytes(n_tensors, n) bytes, 8-byte aligned; work:
+ * AA_STEP_WORK_BYTES, see aa_ppo_step.
+ */
+int64_t aa_moments_table_scratch_bytes(int n_tensors, int64_t n);
+int aa_moments_table(const void* const* values, const uint8_t* const* masks,
+                     uint32_t byte_values, int n_tensors, int64_t n, float* out,
+                     void* scratch, int64_t scratch_bytes, void* work,
+                     void* stream);
 
 /* ------------------------------------------------------------------ */
 /* Fused lm_head path (no counterpart in the reference: its equivalent is  */

@@ -279,3 +279,40 @@ def test_kl_estimator_matches_oracle(device, estimator, clamp):
     assert val == pytest.approx(quoted, abs=1e-4)
     with pytest.raises(ValueError, match="Invalid KL estimator"):
         areal_amd.KLEstimator("k4")
+
+
+@pytest.mark.parametrize("n", [1, 63, 2048, 2049, 131072, 300001])
+def test_moments_under_masks_of_their_own(device, n):
+    """One workgroup per tensor, several slices, and more slices than one round of them; float and byte tensors, a mask
+    each or none, an empty mask; twice on one work buffer, bit-equal; and the 16-tensor entry point of the C ABI.  Sums
+    are fp64 sums rounded once to float32: 2^-23 of the sum of magnitudes."""
+    import ctypes
+
+    from areal_amd import _native as N
+    from areal_amd.advantages import moments_table
+
+    g = torch.Generator().manual_seed(n)
+    x, y = torch.randn(n, generator=g), 3.0 + torch.randn(n, generator=g)
+    flag = torch.rand(n, generator=g) < 0.2
+    m1, m2, none = torch.rand(n, generator=g) < 0.6, torch.rand(n, generator=g) < 0.1, torch.zeros(n, dtype=torch.bool)
+    cpu = [("x", x, m1), ("y", y, m2), ("all", y, None), ("flag", flag, m1), ("flag_all", flag, None), ("empty", x, none)]
+    entries = [(k, t.to(device), None if m is None else m.to(device)) for k, t, m in cpu]
+    got, again = moments_table(entries), moments_table(entries)
+    for name, t, m in cpu:
+        v = t.double() if m is None else t.double()[m]
+        r = {k: float(c) for k, c in got[name].items()}
+        assert r["count"] == v.numel()
+        assert abs(r["sum"] - float(v.sum())) <= 2.0 ** -23 * float(v.abs().sum()) + 1e-30
+        assert r["min"] == (float(v.min()) if v.numel() else float("inf"))
+        assert r["max"] == (float(v.max()) if v.numel() else float("-inf"))
+        assert (r["avg"] != r["avg"]) if v.numel() == 0 else abs(r["avg"] - r["sum"] / r["count"]) <= 2.0 ** -23 * abs(r["avg"])
+        for k in r:
+            assert torch.equal(got[name][k], again[name][k]) or v.numel() == 0
+    lib, dev_x, dev_y, dev_m = N.load(), x.to(device), y.to(device), m1.to(device)
+    out = torch.empty(2, 4, device=device)
+    ptrs = (ctypes.c_void_p * 2)(dev_x.data_ptr(), dev_y.data_ptr())
+    N.check(lib.aa_masked_moments(ptrs, 2, dev_m.data_ptr(), n, out.data_ptr(), torch.cuda.current_stream().cuda_stream), "aa_masked_moments")
+    want = O.masked_moments([x, y], m1)
+    assert torch.equal(out[:, 1:].cpu(), want[:, 1:])
+    bound = 2.0 ** -23 * torch.stack([v.double()[m1].abs().sum() for v in (x, y)])
+    assert bool(((out[:, 0].cpu().double() - want[:, 0].double()).abs() <= bound + 1e-30).all())

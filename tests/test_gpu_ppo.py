@@ -209,10 +209,10 @@ def test_empty_batches_do_not_raise(device):
     assert adv.shape == (0, 8) and ret.shape == (0, 8)
 
 
-@pytest.mark.parametrize("n", [1, 255, 1023, 1024, 1025, 5000, 262144, 262145])
+@pytest.mark.parametrize("n", [1, 255, 1025, 4096, 4097, 8200, 262144, 1048577])
 @pytest.mark.parametrize("rs", [None, dict(level="token", upper=1.3), dict(level="sequence", upper=1.02)])
 def test_step_launches_at_the_edges_of_their_slices(device, n, rs):
-    """One workgroup, whole and ragged slices of 1024 tokens, and more tokens than the largest grid takes one slice of:
+    """One workgroup, whole and ragged slices of 4096 tokens, and more tokens than the largest grid takes one slice of:
     counts, per-token outputs and loss of the launches around the loss, twice on one work buffer (it comes back zero).
     Whole numbers exactly; the loss is an fp64 sum of fp32 terms rounded once (and the terms differ by a few ulps of
     expf): 1e-5 relative to the mean absolute term."""
