@@ -15,6 +15,11 @@ import torch
 
 from .advantages import gae_advantages, kl_regularized_rewards
 from .functional import (
+    COUNT_ON_DEVICE_BYTES,
+    _HostCounts,
+    _PerValidToken,
+    _lm_head_impl,
+    _logprobs_impl,
     _ppo_actor_loss,
     fused_lm_head_ppo_loss,
     fused_logprobs_ppo_loss,
@@ -37,6 +42,17 @@ def rolled_labels(model_inputs: dict[str, Any]) -> torch.Tensor:
     if labels.ndim == 2 and labels.shape[0] == 1:
         labels = labels.squeeze(0)
     return labels
+
+
+def _weight_is_zero(local_weight):
+    """A function that tells whether the weight of the micro-batch is zero.  A device tensor starts on its way to the host
+    now, behind what is queued already; the answer is asked for when the next long kernel has been queued as well, so that
+    the device has work while the host waits."""
+    if isinstance(local_weight, torch.Tensor) and local_weight.is_cuda:
+        pending = _HostCounts(local_weight.detach().reshape(()))
+        return lambda: pending.tolist() == 0
+    zero = bool(local_weight == 0)
+    return lambda: zero
 
 
 def compute_logprobs(logits: torch.Tensor, model_inputs: dict[str, Any], temperature: float = 1.0) -> torch.Tensor:
@@ -73,12 +89,21 @@ def compute_logprobs_and_loss(
     place of the clip, on the behaviour log-probs (actor.py:448-462: SAPO takes ``old_logp``, no proximal policy).
     """
     loss_mask = mb_input["loss_mask"].bool()
+    old_logp = mb_input["logprobs"]
+    prox_logp = mb_input.get("prox_logp")
+    if (fused and not use_sapo_loss and importance_sampling_level == "token" and prox_logp is not None
+            and not inplace_backward and torch.is_grad_enabled() and logits.requires_grad):
+        # one call that counts the tokens itself; a micro-batch without any is found out afterwards (nothing of it is used)
+        scale = _PerValidToken(total_loss_weight, loss_multiplier)
+        out = fused_logprobs_ppo_loss(
+            logits, rolled_labels(model_inputs), prox_logp, old_logp, mb_input["advantages"], eps_clip, loss_mask,
+            eps_clip_higher, c_clip, rejection_sampling, importance_sampling_level, mb_input.get("cu_seqlens"), temperature,
+            scale)
+        return out if scale.valid_tokens else (logits.mean() * 0.0, {})
     local_weight = loss_mask.count_nonzero()
     if local_weight == 0:
         return logits.mean() * 0.0, {}
     labels = rolled_labels(model_inputs)
-    old_logp = mb_input["logprobs"]
-    prox_logp = mb_input.get("prox_logp")
     if prox_logp is None and not use_sapo_loss:
         raise ValueError("prox_logp is None: only the recomputed proximal log-probs are supported here")
     scale = local_weight / total_loss_weight * loss_multiplier
@@ -169,21 +194,32 @@ def compute_lm_head_and_loss(
         local_weight: Any = int(host.sum())
         chunk = lm_head_chunk_tokens()
         kept = [int(host[i:i + chunk].sum()) for i in range(0, hidden.shape[0], chunk)]
-    else:
-        local_weight = loss_mask.count_nonzero()
-    if local_weight == 0:
-        return hidden.mean() * 0.0 + weight.mean() * 0.0, {}
     old_logp = mb_input["logprobs"]
     prox_logp = mb_input.get("prox_logp")
+    scale: Any = None
+    if host_loss_mask is None:
+        if (prox_logp is not None and importance_sampling_level == "token" and torch.is_grad_enabled()
+                and (hidden.requires_grad or weight.requires_grad)):
+            # the step counts the tokens itself; a micro-batch without any is found out afterwards
+            scale = _PerValidToken(total_loss_weight, loss_multiplier)
+        else:
+            local_weight = loss_mask.count_nonzero()
+    if scale is None and local_weight == 0:
+        return hidden.mean() * 0.0 + weight.mean() * 0.0, {}
     if prox_logp is None:
         raise ValueError("prox_logp is None: only the recomputed proximal log-probs are supported here")
-    scale = local_weight / total_loss_weight * loss_multiplier
-    return fused_lm_head_ppo_loss(
+    per_token = scale is not None
+    if not per_token:
+        scale = local_weight / total_loss_weight * loss_multiplier
+    out = fused_lm_head_ppo_loss(
         hidden, weight, rolled_labels(model_inputs), prox_logp, old_logp, mb_input["advantages"], eps_clip=eps_clip,
         loss_mask=loss_mask, eps_clip_higher=eps_clip_higher, c_clip=c_clip, rejection_sampling=rejection_sampling,
         importance_sampling_level=importance_sampling_level, cu_seqlens=mb_input.get("cu_seqlens"),
         temperature=temperature, loss_scale=scale, kept_per_chunk=kept, backward=backward,
     )
+    if per_token and not scale.valid_tokens:
+        return hidden.mean() * 0.0 + weight.mean() * 0.0, {}
+    return out
 
 
 def compute_advantages(
@@ -536,7 +572,8 @@ def compute_loss_with(logits: torch.Tensor, model_inputs: dict[str, Any], mb_inp
     loss functions of this module; the return value has the same form.  A micro-batch of weight 0 returns
     ``logits.mean() * 0``."""
     local_weight = loss_weight_fn(mb_input)
-    if local_weight == 0:
+    is_zero = _weight_is_zero(local_weight)
+    if (is_critic or trie_node is not None) and is_zero():
         return logits.mean() * 0.0
     if is_critic:
         if trie_node is not None:
@@ -555,9 +592,15 @@ def compute_loss_with(logits: torch.Tensor, model_inputs: dict[str, Any], mb_inp
             logp, entropy = gather_packed_tree_logprobs_entropy(logits, trie_node, mb_input["input_ids"],
                                                                 temperature=temperature)
         else:
-            logp, entropy, vmin, vmax = gather_logprobs_entropy_stats(logits, rolled_labels(model_inputs), temperature)
-            if pad_length > 0:
-                logp, entropy, vmin, vmax = (t[:-pad_length] for t in (logp, entropy, vmin, vmax))
+            if logits.dim() == 2:
+                logp, entropy, vmax, vmin = _logprobs_impl(logits, rolled_labels(model_inputs), temperature, None, True, True,
+                                                           T_active=logits.shape[0] - pad_length if pad_length > 0 else None)
+            else:
+                logp, entropy, vmin, vmax = gather_logprobs_entropy_stats(logits, rolled_labels(model_inputs), temperature)
+                if pad_length > 0:
+                    logp, entropy, vmin, vmax = (t[:-pad_length] for t in (logp, entropy, vmin, vmax))
+            if is_zero():  # found out while the pass over the logits runs
+                return logits.mean() * 0.0
         out = loss_fn(logp, entropy, mb_input, vocab_min_logits=vmin, vocab_max_logits=vmax)
     scale = local_weight / total_loss_weight * loss_multiplier
     if isinstance(out, tuple):
@@ -585,20 +628,22 @@ def compute_lm_head_loss_with(hidden: torch.Tensor, weight: torch.Tensor, model_
     if hidden.ndim == 3 and hidden.shape[0] == 1:
         hidden = hidden.squeeze(0)
     local_weight = loss_weight_fn(mb_input)
-    if local_weight == 0:
-        return hidden.mean() * 0.0 + weight.mean() * 0.0
+    is_zero = _weight_is_zero(local_weight)
+    n_rows = hidden.shape[0] - pad_length if pad_length > 0 else hidden.shape[0]
     if grad_token_mask is None and backward == "carry":
         grad_token_mask = mb_input.get("loss_mask")
     if grad_token_mask is not None:
-        grad_token_mask = grad_token_mask.reshape(-1).ne(0)
-        if pad_length > 0:
-            grad_token_mask = torch.nn.functional.pad(grad_token_mask, (0, hidden.shape[0] - grad_token_mask.shape[0]))
-    logp, entropy, vmin, vmax = lm_head_logprobs_entropy_stats(
-        hidden, weight, rolled_labels(model_inputs), temperature, backward=backward,
-        grad_token_mask=grad_token_mask if backward == "carry" else None,
-        kept_per_chunk=kept_per_chunk if backward == "carry" else None)
-    if pad_length > 0:
-        logp, entropy, vmin, vmax = (t[:-pad_length] for t in (logp, entropy, vmin, vmax))
+        grad_token_mask = grad_token_mask.reshape(-1)
+        if grad_token_mask.dtype is not torch.bool:
+            grad_token_mask = grad_token_mask.ne(0)
+        grad_token_mask = grad_token_mask[:n_rows]
+    carry = backward == "carry"
+    logp, entropy, vmin, vmax = _lm_head_impl(
+        hidden, weight, rolled_labels(model_inputs), temperature, None, True, backward, grad_token_mask if carry else None,
+        kept_per_chunk if carry else None, count_on_device=2 * n_rows * weight.shape[0] <= COUNT_ON_DEVICE_BYTES,
+        T_active=n_rows)
+    if is_zero():  # found out while the logits tiles run
+        return hidden.mean() * 0.0 + weight.mean() * 0.0
     out = loss_fn(logp, entropy, mb_input, vocab_min_logits=vmin, vocab_max_logits=vmax)
     scale = local_weight / total_loss_weight * loss_multiplier
     if isinstance(out, tuple):
@@ -616,6 +661,12 @@ def compute_logprobs_and_sft_loss(logits: torch.Tensor, model_inputs: dict[str, 
     from .sft import fused_logprobs_sft_loss
 
     loss_mask = mb_input["loss_mask"].bool()
+    if torch.is_grad_enabled() and logits.requires_grad:
+        # one call that counts the tokens itself; a micro-batch without any is found out afterwards (nothing of it is used)
+        per_token = _PerValidToken(total_loss_weight, loss_multiplier)
+        out = fused_logprobs_sft_loss(logits, rolled_labels(model_inputs), loss_mask, mb_input["cu_seqlens"], temperature,
+                                      loss_scale=per_token)
+        return out if per_token.valid_tokens else (logits.mean() * 0.0, {})
     local_weight = loss_mask.count_nonzero()
     if local_weight == 0:
         return logits.mean() * 0.0, {}

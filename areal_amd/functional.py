@@ -162,10 +162,13 @@ class _LogprobsEntropy(torch.autograd.Function):
     """logp, entropy, vocab max, vocab min of each row; differentiable in logits."""
 
     @staticmethod
-    def forward(ctx, logits2d, labels1d, temperature, stride, want_entropy, want_minmax, inplace=False):
+    def forward(ctx, logits2d, labels1d, temperature, stride, want_entropy, want_minmax, inplace=False, T_active=None):
+        ctx.set_materialize_grads(False)  # no zero-filled gradients for the outputs that have none
         lib = N.load()
         ctx.inplace = bool(inplace)
         T, V = logits2d.shape
+        if T_active is not None:  # the rows past it are batch padding: no outputs, a zero gradient
+            T = T_active
         dev = logits2d.device
         kw = dict(dtype=torch.float32, device=dev)
         logp = torch.empty(T, **kw)
@@ -195,12 +198,13 @@ class _LogprobsEntropy(torch.autograd.Function):
     def backward(ctx, g_logp, g_entropy, _g_vmax, _g_vmin):
         lib = N.load()
         logits2d, labels1d, row_lse, row_ez = ctx.saved_tensors
+        if g_logp is None and g_entropy is None:
+            return (None,) * 8
         T, V = logits2d.shape
         dev = logits2d.device
-        if g_logp is None:
-            g_logp = torch.zeros(T, dtype=torch.float32, device=dev)
-        g_logp = _f32(g_logp)
-        g_entropy = _f32(g_entropy) if (g_entropy is not None and row_ez is not None) else None
+        T_active = row_lse.shape[0]
+        g_logp = torch.zeros(T_active, dtype=torch.float32, device=dev) if g_logp is None else _f32_values(g_logp)
+        g_entropy = _f32_values(g_entropy) if (g_entropy is not None and row_ez is not None) else None
         if ctx.inplace:
             # the gradient takes the place of the logits (the kernel reads an element before it writes it); the version
             # bump below makes any other operation that kept the logits for its own backward fail loudly
@@ -212,13 +216,13 @@ class _LogprobsEntropy(torch.autograd.Function):
                 lib.aa_logits_bwd(
                     _ptr(logits2d), _DTYPES[logits2d.dtype], T, V, ctx.stride, _ptr(labels1d),
                     1.0 / ctx.temperature, _ptr(row_lse), _ptr(row_ez), _ptr(g_logp), _ptr(g_entropy),
-                    T, _ptr(dlogits), _stream(dev),
+                    T_active, _ptr(dlogits), _stream(dev),
                 ),
                 "aa_logits_bwd",
             )
         if ctx.inplace:
             torch.autograd.graph.increment_version(logits2d)
-        return dlogits, None, None, None, None, None, None
+        return (dlogits,) + (None,) * 7
 
 
 def _device_or_read_back_counts(T: int, T_active: int, mask_u8: torch.Tensor, on_device: bool) -> list[int]:
@@ -235,23 +239,21 @@ def _device_or_read_back_counts(T: int, T_active: int, mask_u8: torch.Tensor, on
     return _HostCounts(on.view(n_chunks, chunk).sum(1)).tolist()
 
 
-def _logprobs_impl(logits, labels, temperature, tp_group, want_entropy, want_minmax, inplace_backward=False):
+def _logprobs_impl(logits, labels, temperature, tp_group, want_entropy, want_minmax, inplace_backward=False,
+                   T_active=None):
+    """``T_active`` (2-D logits): only the first rows have outputs (of that length) and a gradient."""
     _check_tp(tp_group)
     _require_gpu(logits, "logits")
     assert logits.shape[0] > 0, "Input logits must have at least one element"
     if tuple(labels.shape) != tuple(logits.shape[:-1]):
         raise ValueError(f"labels shape {tuple(labels.shape)} != logits shape[:-1] {tuple(logits.shape[:-1])}")
     x, T, V, stride = _rows(logits)
-    y = labels.reshape(-1).to(device=x.device, dtype=torch.int64).contiguous()
-    logp, entropy, vmax, vmin = _LogprobsEntropy.apply(x, y, float(temperature), stride, want_entropy, want_minmax,
-                                                       bool(inplace_backward))
-    shp = labels.shape
-    return (
-        logp.view(shp),
-        entropy.view(shp) if entropy is not None else None,
-        vmax.view(shp) if vmax is not None else None,
-        vmin.view(shp) if vmin is not None else None,
-    )
+    y = _labels_i64(labels, x.device)
+    outs = _LogprobsEntropy.apply(x, y if y.dim() == 1 else y.reshape(-1), float(temperature), stride, want_entropy,
+                                  want_minmax, bool(inplace_backward), T_active)
+    if T_active is not None or labels.dim() == 1:
+        return outs
+    return tuple(None if t is None else t.view(labels.shape) for t in outs)
 
 
 def gather_logprobs(
@@ -490,10 +492,16 @@ class _PerValidToken:
     """Loss scale ``loss_mask.count_nonzero() / total * multiplier`` (fsdp_engine.py:1983-1985, 2045), formed inside the
     kernels from the count they have anyway.  ``total`` is a number or a tensor with one element."""
 
-    __slots__ = ("total", "multiplier")
+    __slots__ = ("total", "multiplier", "valid_tokens")
 
     def __init__(self, total, multiplier: float):
         self.total, self.multiplier = total, multiplier
+        self.valid_tokens = None  # the count, once a step that was given this scale has it on the host
+
+
+def _note_valid_tokens(scale, step) -> None:
+    if isinstance(scale, _PerValidToken):
+        scale.valid_tokens = step.slot.read()[0]
 
 
 def _scale_struct(scale, dev: torch.device):
@@ -542,7 +550,7 @@ class _Step:
         self.loss = torch.empty((), dtype=torch.float32, device=dev)
         work = _work_words(dev)
         scale_c, scale_t = _scale_struct(scale, dev)
-        self.slot = _HostSlot(dev) if (rs is not None or host_counts) else None
+        self.slot = _HostSlot(dev) if (rs is not None or host_counts or isinstance(scale, _PerValidToken)) else None
         f0, b0, row = f.data_ptr(), b.data_ptr(), pitch * 4
         c = self.struct = N.PpoStep()
         c.T, c.T_active = T, T_active
@@ -878,7 +886,9 @@ def fused_logprobs_ppo_loss(
     step = _ppo_step(dev, T, T_active, loss_mask, proximal_logprobs, old_logprobs, advantages, eps_clip, eps_clip_higher,
                      c_clip, rejection_sampling, cu_seqlens, loss_scale)
     loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
-    return loss, step.finish(step.stats(rows=True))
+    stat = step.finish(step.stats(rows=True))
+    _note_valid_tokens(loss_scale, step)
+    return loss, stat
 
 
 # ----------------------------------------------------------------------------
@@ -907,10 +917,10 @@ def _lmhead_workspace(T: int, H: int, V: int, dev, forward_only: bool = False, e
 
 class _LmHeadLogprobsEntropy(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, hidden, weight, labels, temperature, want_minmax=False):
+    def forward(ctx, hidden, weight, labels, temperature, want_minmax, T):
         ctx.set_materialize_grads(False)
         lib = N.load()
-        T, H = hidden.shape
+        H = hidden.shape[1]
         V = weight.shape[0]
         dev = hidden.device
         f32 = dict(dtype=torch.float32, device=dev)
@@ -936,22 +946,22 @@ class _LmHeadLogprobsEntropy(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_logp, g_entropy, _g_vmax=None, _g_vmin=None):
         if g_logp is None and g_entropy is None:
-            return None, None, None, None, None
+            return (None,) * 6
         hidden, weight, labels, row_lse, row_ez = ctx.saved_tensors
         d_hidden, d_weight = _lmhead_recompute_backward(hidden, weight, labels, ctx.temperature, row_lse, row_ez,
                                                         g_logp, g_entropy)
-        return d_hidden, d_weight, None, None, None
+        return (d_hidden, d_weight) + (None,) * 4
 
 
 def _lmhead_recompute_backward(hidden, weight, labels, temperature, row_lse, row_ez, g_logp, g_entropy):
     """``aa_lmhead_bwd``: the logits tiles of the tokens with a gradient are formed again."""
     lib = N.load()
-    T, H = hidden.shape
+    T, H = row_lse.shape[0], hidden.shape[1]  # the rows past T are batch padding
     V = weight.shape[0]
     dev = hidden.device
     g_logp = torch.zeros(T, dtype=torch.float32, device=dev) if g_logp is None else _f32(g_logp)
     g_entropy = None if g_entropy is None else _f32(g_entropy)
-    d_hidden = torch.empty_like(hidden)
+    d_hidden = _empty_hidden_gradient(hidden, T)
     d_weight = torch.empty_like(weight)  # bf16: rounded once, after fp32 accumulation over the chunks
     ws = _lmhead_workspace(T, H, V, dev)
     # Rows whose upstream gradients are all zero (masked tokens) are left out of the gradient GEMMs; the device counts
@@ -978,10 +988,10 @@ class _LmHeadCarry(torch.autograd.Function):
     ``aa_lmhead_bwd_carry``)."""
 
     @staticmethod
-    def forward(ctx, hidden, weight, labels, temperature, grad_mask, kept_per_chunk, want_minmax):
+    def forward(ctx, hidden, weight, labels, temperature, grad_mask, kept_per_chunk, want_minmax, T):
         ctx.set_materialize_grads(False)
         lib = N.load()
-        T, H = hidden.shape
+        H = hidden.shape[1]
         V = weight.shape[0]
         dev = hidden.device
         f32 = dict(dtype=torch.float32, device=dev)
@@ -1020,25 +1030,25 @@ class _LmHeadCarry(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_logp, g_entropy, _g_vmax=None, _g_vmin=None):
         if g_logp is None and g_entropy is None:
-            return (None,) * 7
+            return (None,) * 8
         hidden, weight, labels, logp, row_lse, row_ez, panel, grad_mask = ctx.saved_tensors
         if g_entropy is not None:  # an entropy gradient is no multiple of the stored rows: form the logits again
             d_hidden, d_weight = _lmhead_recompute_backward(hidden, weight, labels, ctx.temperature, row_lse, row_ez,
                                                             g_logp, g_entropy)
-            return (d_hidden, d_weight) + (None,) * 5
+            return (d_hidden, d_weight) + (None,) * 6
         # the backward patches the stored rows (and may overwrite a chunk of them): they serve one backward
         if getattr(ctx, "handed_out", False):
             raise RuntimeError("the stored rows of this lm_head forward were already used by a backward; run the forward "
                                "pass again instead of a second backward through a retained graph")
         ctx.handed_out = True
         lib = N.load()
-        T, H = hidden.shape
+        T, H = logp.shape[0], hidden.shape[1]
         V = weight.shape[0]
         dev = hidden.device
         g_logp = _f32(g_logp)
         kept_per_chunk = ctx.kept_per_chunk
         kept = None if kept_per_chunk is None else (C.c_int64 * len(kept_per_chunk))(*kept_per_chunk)
-        d_hidden = torch.empty_like(hidden)
+        d_hidden = _empty_hidden_gradient(hidden, T)
         d_weight = torch.empty_like(weight)
         ws = torch.empty(lib.aa_lmhead_carry_workspace_bytes(T, H, V), dtype=torch.uint8, device=dev)
         with _on(dev):
@@ -1050,7 +1060,7 @@ class _LmHeadCarry(torch.autograd.Function):
                 ),
                 "aa_lmhead_bwd_carry",
             )
-        return (d_hidden, d_weight) + (None,) * 5
+        return (d_hidden, d_weight) + (None,) * 6
 
 
 def lm_head_logprobs_entropy(
@@ -1114,21 +1124,24 @@ def lm_head_logprobs_entropy_stats(
 
 
 def _lm_head_apply(hidden, weight, y, temperature, want_minmax, backward, grad_mask, kept_per_chunk,
-                   count_on_device=False):
-    """One of the two autograd functions on a contiguous batch; ``grad_mask``: bool / uint8 ``[T]`` or None."""
+                   count_on_device=False, T_active=None):
+    """``T_active``: the rows past it are batch padding, without outputs and with a zero gradient (``grad_mask`` then has
+    an entry for each of the others)."""
     needs_grad = torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)
+    T = hidden.shape[0] if T_active is None else T_active
     if backward != "carry" or not needs_grad:
-        return _LmHeadLogprobsEntropy.apply(hidden, weight, y, float(temperature), want_minmax)
-    T = hidden.shape[0]
+        return _LmHeadLogprobsEntropy.apply(hidden, weight, y, float(temperature), want_minmax, T)
     chunk = lm_head_chunk_tokens()
     n_chunks = (T + chunk - 1) // chunk
     m8 = kept = None
     if grad_mask is not None:
-        m8 = _mask_u8(grad_mask)
+        m8 = _mask_bytes(grad_mask)
         if kept_per_chunk is not None:
             kept = [max(0, min(int(v), chunk)) for v in kept_per_chunk]
             if len(kept) != n_chunks:
-                raise ValueError(f"kept_per_chunk needs one count per chunk of {chunk} tokens")
+                if len(kept) != (hidden.shape[0] + chunk - 1) // chunk:
+                    raise ValueError(f"kept_per_chunk needs one count per chunk of {chunk} tokens")
+                kept = kept[:n_chunks]  # chunks of nothing but padding
         elif count_on_device:
             kept = [N.AA_LMHEAD_COUNT_ON_DEVICE] * n_chunks
         else:
@@ -1136,11 +1149,26 @@ def _lm_head_apply(hidden, weight, y, temperature, want_minmax, backward, grad_m
             if n_chunks * chunk != T:
                 on = torch.nn.functional.pad(on, (0, n_chunks * chunk - T))
             kept = _HostCounts(on.view(n_chunks, chunk).sum(1)).tolist()
-    return _LmHeadCarry.apply(hidden, weight, y, float(temperature), m8, kept, want_minmax)
+    return _LmHeadCarry.apply(hidden, weight, y, float(temperature), m8, kept, want_minmax, T)
+
+
+def _empty_hidden_gradient(hidden, T):
+    """An array for the gradient of ``hidden`` whose rows past ``T`` (batch padding) are zeros."""
+    d_hidden = torch.empty_like(hidden)
+    if T != hidden.shape[0]:
+        d_hidden[T:].zero_()
+    return d_hidden
+
+
+# Rows that the carried op of compute_lm_head_loss_with may keep room for without knowing how many the mask holds
+# (2 bytes x V per token).  Up to here the count stays on the device: reading it back makes the host wait for everything
+# queued before, about 60 us in which nothing is queued behind it.  Beyond, the forward alone takes milliseconds and the
+# exact size is worth more.
+COUNT_ON_DEVICE_BYTES = 2 << 30
 
 
 def _lm_head_impl(hidden, weight, labels, temperature, token_mask, want_minmax, backward="recompute",
-                  grad_token_mask=None, kept_per_chunk=None, count_on_device=False):
+                  grad_token_mask=None, kept_per_chunk=None, count_on_device=False, T_active=None):
     if backward not in _LMHEAD_BACKWARD:
         raise ValueError(f"backward must be one of {sorted(_LMHEAD_BACKWARD)}, got {backward!r}")
     _require_gpu(hidden, "hidden")
@@ -1151,7 +1179,7 @@ def _lm_head_impl(hidden, weight, labels, temperature, token_mask, want_minmax, 
     assert hidden.shape[0] > 0, "Input must have at least one token"
     if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         raise TypeError("fused lm_head expects bf16 hidden states and weights")
-    y = labels.to(device=hidden.device, dtype=torch.int64).contiguous()
+    y = _labels_i64(labels, hidden.device)
     if token_mask is not None:
         if tuple(token_mask.shape) != (hidden.shape[0],):
             raise ValueError(f"token_mask shape {tuple(token_mask.shape)} != ({hidden.shape[0]},)")
@@ -1168,11 +1196,12 @@ def _lm_head_impl(hidden, weight, labels, temperature, token_mask, want_minmax, 
             sub_mask, None, count_on_device)   # the caller's counts are per chunk of the whole batch, not of these tokens
         full = lambda v: torch.zeros(T, dtype=torch.float32, device=dev).index_copy(0, idx, v)
         return full(lp), full(ent), (full(vmin) if want_minmax else None), (full(vmax) if want_minmax else None)
-    if grad_token_mask is not None and tuple(grad_token_mask.shape) != (hidden.shape[0],):
-        raise ValueError(f"grad_token_mask shape {tuple(grad_token_mask.shape)} != ({hidden.shape[0]},)")
+    n_rows = hidden.shape[0] if T_active is None else T_active
+    if grad_token_mask is not None and tuple(grad_token_mask.shape) != (n_rows,):
+        raise ValueError(f"grad_token_mask shape {tuple(grad_token_mask.shape)} != ({n_rows},)")
     lp, ent, vmax, vmin = _lm_head_apply(hidden.contiguous(), weight.contiguous(), y, temperature, want_minmax, backward,
                                          None if grad_token_mask is None else grad_token_mask.to(hidden.device),
-                                         kept_per_chunk, count_on_device)
+                                         kept_per_chunk, count_on_device, T_active)
     return lp, ent, vmin, vmax
 
 
@@ -1438,7 +1467,9 @@ def fused_lm_head_ppo_loss(
         kept = _device_or_read_back_counts(T, T_active, mask_eff, False)
     loss = _FusedLmHeadPpo.apply(hidden.contiguous(), weight.contiguous(), step, y, float(temperature), kept,
                                  _LMHEAD_BACKWARD[backward])
-    return loss, step.finish(step.stats(rows=True))
+    stat = step.finish(step.stats(rows=True))
+    _note_valid_tokens(loss_scale, step)
+    return loss, stat
 
 
 # ----------------------------------------------------------------------------

@@ -19,6 +19,7 @@ from .functional import (
     _labels_i64,
     _mask_bytes,
     _mask_u8,
+    _note_valid_tokens,
     _on,
     _ptr,
     _require_gpu,
@@ -115,9 +116,9 @@ def sft_loss_fn(logprobs: torch.Tensor, loss_mask: torch.Tensor, cu_seqlens: tor
     return loss, _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs)
 
 
-def _nll_step(dev, T, T_active, loss_mask, loss_scale, host_counts=False):
+def _nll_step(dev, T, T_active, loss_mask, loss_scale):
     return _Step(dev, T, T_active, _mask_bytes(loss_mask.to(dev)), None, None, None, _nll_params(), scale=loss_scale,
-                 derived=False, host_counts=host_counts)
+                 derived=False)
 
 
 def _step_stat(step, cu, n_seqs, extrema):
@@ -163,7 +164,9 @@ def fused_logprobs_sft_loss(logits: torch.Tensor, labels: torch.Tensor, loss_mas
     x, T, V, stride = _rows(logits)
     step = _nll_step(dev, T, T_active, loss_mask, loss_scale)
     loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
-    return loss, _step_stat(step, cu, n_seqs, extrema=True)
+    stat = _step_stat(step, cu, n_seqs, extrema=True)
+    _note_valid_tokens(loss_scale, step)
+    return loss, stat
 
 
 def fused_lm_head_sft_loss(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, loss_mask: torch.Tensor,

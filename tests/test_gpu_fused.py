@@ -784,3 +784,30 @@ def test_register_kernel_and_twice_read_kernel_agree_on_unaligned_rows(device, V
     assert float((g0 == g1).float().mean()) > 0.999
     assert bool((g0[mask == 0] == 0).all()) and bool((g1[mask == 0] == 0).all())
 
+
+@pytest.mark.parametrize("total", ["number", "int64 tensor", "float tensor", "host tensor"])
+@pytest.mark.parametrize("masked", [False, True])
+def test_weight_of_the_micro_batch_inside_the_kernels(device, total, masked):
+    """``local_weight / total_loss_weight * multiplier`` formed by the kernels from the count they have: bit-equal to the
+    same factor given as ``loss_scale`` (the expression is the same in float32), whatever the total comes as; a
+    micro-batch without a token gives a zero that keeps the graph."""
+    g = torch.Generator().manual_seed(7)
+    T, pad, V = 130, 9, 20000
+    mask = torch.zeros(T, dtype=torch.bool) if masked else torch.rand(T, generator=g) < 0.6
+    x = torch.randn(T + pad, V, generator=g).bfloat16().to(device)
+    ids = torch.randint(0, V, (T + pad,), generator=g).to(device)
+    mb = {k: torch.randn(T, generator=g).to(device) - 2.0 for k in ("logprobs", "prox_logp", "advantages")}
+    mb.update(loss_mask=mask.to(device), cu_seqlens=torch.tensor([0, T], dtype=torch.int32, device=device))
+    weight = {"number": 977.0, "int64 tensor": torch.tensor(977, device=device),
+              "float tensor": torch.tensor([977.0], device=device), "host tensor": torch.tensor(977.0)}[total]
+    a, b = x.clone().requires_grad_(True), x.clone().requires_grad_(True)
+    loss, stat = engine_glue.compute_logprobs_and_loss(a, {"rolled_input_ids": ids}, mb, pad, weight, 0.2, loss_multiplier=3.0)
+    loss.backward()
+    if masked:
+        assert stat == {} and float(loss) == 0.0 and float(a.grad.float().abs().max()) == 0.0
+        return
+    scale = mb["loss_mask"].count_nonzero() / 977.0 * 3.0
+    want, _ = areal_amd.fused_logprobs_ppo_loss(b, ids, mb["prox_logp"], mb["logprobs"], mb["advantages"], 0.2,
+                                                mb["loss_mask"], cu_seqlens=mb["cu_seqlens"], loss_scale=scale)
+    want.backward()
+    assert torch.equal(loss, want) and torch.equal(a.grad, b.grad)
