@@ -124,6 +124,39 @@ class NormParams(C.Structure):
     ]
 
 
+class AdvantageStep(C.Structure):
+    """``aa_advantage_step``"""
+
+    _fields_ = [
+        ("bs", C.c_int64),
+        ("L", C.c_int64),
+        ("loss_mask", C.c_void_p),
+        ("loss_mask_bytes", C.c_int32),
+        ("roll_logp", C.c_int32),
+        ("logp", C.c_void_p),
+        ("ref_logp", C.c_void_p),
+        ("attention_mask", C.c_void_p),
+        ("seqlens", C.c_void_p),
+        ("reward_score", C.c_void_p),
+        ("values", C.c_void_p),
+        ("kl_ctl", C.c_float),
+        ("discount", C.c_float),
+        ("gae_lambda", C.c_float),
+        ("kl_estimator", C.c_int32),
+        ("mask_no_eos_with_zero", C.c_int32),
+        ("norm", C.POINTER(NormParams)),
+        ("mask_out", C.c_void_p),
+        ("logp_out", C.c_void_p),
+        ("kl_rewards", C.c_void_p),
+        ("rewards", C.c_void_p),
+        ("advantages", C.c_void_p),
+        ("returns", C.c_void_p),
+        ("scratch", C.c_void_p),
+        ("scratch_bytes", C.c_int64),
+        ("work", C.c_void_p),
+    ]
+
+
 _p = C.c_void_p
 _i64 = C.c_int64
 _f = C.c_float
@@ -194,6 +227,9 @@ SIGNATURES = {
     "aa_rw_pair_loss": (_i, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p]),
     "aa_m2po_workspace_bytes": (_i64, [_i64]),
     "aa_m2po_mask": (_i, [_p, _p, _p, _i64, _f, _p, _p, _p, _i64, _p]),
+    "aa_reward_scores": (_i, [_p, _i64, _f, _f, _f, C.POINTER(NormParams), _p, _p]),
+    "aa_advantages_scratch_bytes": (_i64, [_i64]),
+    "aa_advantages": (_i, [C.POINTER(AdvantageStep), _p]),
     "aa_kl_rewards": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _f, _i, _i, _p, _p, _p]),
     "aa_gae": (_i, [_p, _p, _p, _p, _i64, _i64, _f, _f, _p, _p, _p]),
     "aa_normalize_scratch_bytes": (_i64, [_i64, _i64, _i64]),

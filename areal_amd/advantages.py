@@ -41,6 +41,10 @@ class Normalization:
                 f"group_size must be a positive integer when using group normalization, got {self.group_size}"
             )
 
+    def _params(self) -> N.NormParams:
+        return N.NormParams(_LEVELS[self.mean_level], int(bool(self.mean_leave1out)), _LEVELS[self.std_level],
+                            int(bool(self.std_unbiased)), float(self.eps), int(self.group_size))
+
     @torch.no_grad()
     def __call__(self, x: torch.Tensor, loss_mask: torch.Tensor | None = None, high_precision: bool = True,
                  reduce_group=None) -> torch.Tensor:
@@ -58,8 +62,7 @@ class Normalization:
         xf = _f32(x)
         mf = None if loss_mask is None else _f32(loss_mask)
         inner = xf.numel() // bs
-        params = N.NormParams(_LEVELS[self.mean_level], int(bool(self.mean_leave1out)), _LEVELS[self.std_level],
-                              int(bool(self.std_unbiased)), float(self.eps), int(self.group_size))
+        params = self._params()
         lib = N.load()
         dev = xf.device
         grouped = params.mean_level == 2 or params.std_level == 2
@@ -107,6 +110,83 @@ def gae_advantages(rewards: torch.Tensor, values: torch.Tensor | None, loss_mask
             "aa_gae",
         )
     return adv, ret
+
+
+def _one_process(group=None) -> bool:
+    dist = torch.distributed
+    return not (dist.is_available() and dist.is_initialized() and dist.get_world_size(group) > 1)
+
+
+def _plain(t: torch.Tensor | None, shape, dev) -> bool:
+    """A float32 array that a kernel may take, and write, as it is."""
+    return t is None or (t.dtype is torch.float32 and t.is_contiguous() and t.shape == shape and t.device == dev
+                         and not t.requires_grad)
+
+
+@torch.no_grad()
+def reward_scores(rewards: torch.Tensor, bias: float, scaling: float, clip: float, norm) -> torch.Tensor | None:
+    """``norm(clip((rewards + bias) * scaling, -clip, clip))`` (actor.py:166-172) in one launch; None when the inputs ask
+    for the general way (``norm`` another callable than ``Normalization``, more rewards than one launch takes)."""
+    if norm is not None and not (type(norm) is Normalization and _one_process() and rewards.numel() <= 8192):
+        return None
+    if not _plain(rewards, rewards.shape, rewards.device) or rewards.ndim != 1 or not rewards.is_cuda or rewards.numel() == 0:
+        return None
+    out = torch.empty_like(rewards)
+    dev = rewards.device
+    with _on(dev):
+        N.check(N.load().aa_reward_scores(_ptr(rewards), rewards.numel(), float(bias), float(scaling), float(clip),
+                                          None if norm is None else norm._params(), _ptr(out), _stream(dev)),
+                "aa_reward_scores")
+    return out
+
+
+@torch.no_grad()
+def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, values, kl_ctl, kl_estimator, discount,
+                   gae_lambda, mask_no_eos_with_zero, norm):
+    """Masks, rewards, GAE and the normalisation of the advantages in one pass per row (``aa_advantages``): returns
+    ``(mask, logp, kl_rewards, rewards, advantages, returns)``, ``ref_logp`` (and, without ``roll``, ``logp``) masked in
+    place; None when the inputs ask for the general way."""
+    if loss_mask.ndim != 2 or not loss_mask.is_cuda or loss_mask.numel() == 0 or kl_estimator not in _KL_IDS:
+        return None
+    shape, dev = loss_mask.shape, loss_mask.device
+    bs, L = shape
+    if norm is not None and not (type(norm) is Normalization and _one_process()
+                                 and not (norm.mean_leave1out and _LEVELS[norm.mean_level] != 0)):
+        return None
+    if logp is None or not all(_plain(t, shape, dev) for t in (logp, ref_logp, values)):
+        return None
+    if attention_mask.shape != shape or attention_mask.device != dev or score.shape != (bs,) or not _plain(score, (bs,), dev):
+        return None
+    if loss_mask.dtype is torch.bool:
+        mask, is_bytes = (loss_mask if loss_mask.is_contiguous() else loss_mask.contiguous()), 1
+    else:
+        mask, is_bytes = _f32(loss_mask), 0
+    attention = seqlens = None
+    if attention_mask.dtype is torch.bool and attention_mask.is_contiguous():
+        attention = attention_mask
+    else:
+        seqlens = attention_mask.sum(-1).long()
+    lib = N.load()
+    new = lambda: torch.empty(shape, dtype=torch.float32, device=dev)
+    mask_out, kl_rewards, rewards, adv, returns = new(), new(), new(), new(), new()
+    logp_out = new() if roll else logp
+    a = N.AdvantageStep()
+    a.bs, a.L = bs, L
+    a.loss_mask, a.loss_mask_bytes, a.roll_logp = _ptr(mask), is_bytes, int(roll)
+    a.logp, a.ref_logp, a.values, a.reward_score = _ptr(logp), _ptr(ref_logp), _ptr(values), _ptr(score)
+    a.attention_mask, a.seqlens = _ptr(attention), _ptr(seqlens)
+    a.kl_ctl, a.discount, a.gae_lambda = float(kl_ctl), float(discount), float(gae_lambda)
+    a.kl_estimator, a.mask_no_eos_with_zero = _KL_IDS[kl_estimator], int(bool(mask_no_eos_with_zero))
+    a.mask_out, a.logp_out, a.kl_rewards, a.rewards = _ptr(mask_out), _ptr(logp_out), _ptr(kl_rewards), _ptr(rewards)
+    a.advantages, a.returns = _ptr(adv), _ptr(returns)
+    if norm is not None:
+        params = norm._params()
+        scratch = torch.empty(lib.aa_advantages_scratch_bytes(bs) // 8, dtype=torch.float64, device=dev)
+        a.norm = C.pointer(params)
+        a.scratch, a.scratch_bytes, a.work = _ptr(scratch), scratch.numel() * 8, _ptr(_work_words(dev))
+    with _on(dev):
+        N.check(lib.aa_advantages(a, _stream(dev)), "aa_advantages")
+    return mask_out, logp_out, kl_rewards, rewards, adv, returns
 
 
 _MOMENT_KEYS = ("sum", "min", "max", "count", "avg")

@@ -2,6 +2,7 @@
 // masked moments the statistics logger asks for.  Reference: areal/trainer/ppo/actor.py:209-236 (GAE, a Python
 // loop over max_seqlen), areal/utils/data.py:1378-1596 (Normalization), areal/utils/stats_tracker.py:227-285.
 #include "device_utils.h"
+#include "ppo_step.h"
 
 namespace aa {
 namespace adv {
@@ -264,59 +265,141 @@ __global__ __launch_bounds__(kWave) void k_norm_finish(const double2* __restrict
   }
 }
 
+// ------------------------------------------------------------------------------------------------------------------
+// Normalization of a few thousand values in one launch (the five launches above cost 5 us each, whatever they do): one
+// workgroup per group (plus one for the rows past the last full group, or one in all), which forms the statistics it
+// needs from the whole input: the same two passes in float64, the sums of a segment in another order.  `scores`: the
+// values are first turned from rewards into scores, clip((x + bias) * scaling) (actor.py:166-170).
+// ------------------------------------------------------------------------------------------------------------------
+constexpr int64_t kSmallNorm = 8192;  // values; a workgroup reads them all when a level is "batch"
+constexpr int kSmallThreads = 256;
+
+struct Scores {
+  int on;
+  float bias, scaling, clip;
+};
+
+__device__ __forceinline__ float score_of(const Scores& s, float x) {
+  if (!s.on) return x;
+  const float v = (x + s.bias) * s.scaling;
+  return v != v ? v : fminf(fmaxf(v, -s.clip), s.clip);
+}
+
 __device__ __forceinline__ double level_std(double Q, double F, bool unbiased) {
   if (unbiased) return F <= 1.0 ? 1.0 : sqrt(Q / (F - 1.0));
   return F == 0.0 ? 1.0 : sqrt(Q / F);
 }
 
-__global__ __launch_bounds__(256) void k_norm_apply(NormArgs a, const double4* __restrict__ stats,
-                                                    float* __restrict__ out) {
+// one element of the output (`passthrough`: nothing is active, the input comes back unchanged); stats: batch, own group
+__device__ __forceinline__ float norm_element(const NormArgs& a, const double4& batch, const double4& group, bool grouped,
+                                              bool passthrough, float xi, float mi) {
+  if (passthrough) return xi;
   const bool has_mask = a.mask != nullptr;
-  const bool passthrough = has_mask && stats[0].y == 0.0;  // nothing active: the input comes back unchanged
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x) {
-    const float xi = a.x[i];
-    if (passthrough) {
-      out[i] = xi;
-      continue;
-    }
-    const float mi = has_mask ? a.mask[i] : 1.f;
-    bool mean_f;
-    const double mean = mean_at(a, stats, i, xi, mi, mean_f);
-    // x - mean, then * mask, in the precision the reference's tensors have at that point
-    double cen;
-    if (mean_f) {
-      float c = xi - (float)mean;
-      if (has_mask) c *= mi;
-      cen = (double)c;
-    } else {
-      cen = (double)xi - mean;
-      if (has_mask) cen *= (double)mi;
-    }
-    double sd;
-    bool std_f = true;
-    float eps = a.eps;
-    if (a.std_level == 0) {
-      sd = 1.0;
-      eps = 0.f;
-    } else if (a.std_level == 1) {
-      sd = level_std(stats[0].z, stats[0].y, a.std_unbiased != 0);
-      std_f = false;
-    } else {
-      const int64_t g = i / a.seg_elems;
-      if (g >= a.n_groups) sd = 0.0;
-      else if (a.group_size == 1 && a.std_unbiased) sd = 1.0;
-      else sd = (double)(float)level_std(stats[1 + g].z, stats[1 + g].y, a.std_unbiased != 0);
-    }
-    float r;
-    if (std_f && mean_f) {
-      r = (float)cen / ((float)sd + eps);
-    } else if (std_f) {
-      r = (float)(cen / (double)((float)sd + eps));
-    } else {
-      r = (float)(cen / (sd + (double)eps));
-    }
-    out[i] = r;
+  double mean = 0.0;
+  bool mean_f = true;
+  if (a.mean_level == 1) {
+    mean_f = false;
+    mean = level_mean(batch.x, batch.y, a.mean_leave1out != 0, has_mask, xi, mi);
+  } else if (a.mean_level == 2 && grouped && !(a.group_size == 1 && a.mean_leave1out)) {
+    mean = (double)(float)level_mean(group.x, group.y, a.mean_leave1out != 0, has_mask, xi, mi);
   }
+  // x - mean, then * mask, in the precision the reference's tensors have at that point
+  double cen;
+  if (mean_f) {
+    float c = xi - (float)mean;
+    if (has_mask) c *= mi;
+    cen = (double)c;
+  } else {
+    cen = (double)xi - mean;
+    if (has_mask) cen *= (double)mi;
+  }
+  double sd = 1.0;
+  bool std_f = true;
+  float eps = a.eps;
+  if (a.std_level == 0) {
+    eps = 0.f;
+  } else if (a.std_level == 1) {
+    sd = level_std(batch.z, batch.y, a.std_unbiased != 0);
+    std_f = false;
+  } else {
+    if (!grouped) sd = 0.0;
+    else if (a.group_size == 1 && a.std_unbiased) sd = 1.0;
+    else sd = (double)(float)level_std(group.z, group.y, a.std_unbiased != 0);
+  }
+  if (std_f && mean_f) return (float)cen / ((float)sd + eps);
+  if (std_f) return (float)(cen / (double)((float)sd + eps));
+  return (float)(cen / (sd + (double)eps));
+}
+
+// out may be x itself (an element is read, then written, by the same thread)
+__global__ __launch_bounds__(256) void k_norm_apply(NormArgs a, const double4* __restrict__ stats, float* out) {
+  const bool passthrough = a.mask != nullptr && stats[0].y == 0.0;
+  const bool by_group = a.mean_level == 2 || a.std_level == 2;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t g = by_group ? i / a.seg_elems : a.n_groups;
+    const bool grouped = g < a.n_groups;
+    out[i] = norm_element(a, stats[0], stats[grouped ? 1 + g : 0], grouped, passthrough, a.x[i], a.mask ? a.mask[i] : 1.f);
+  }
+}
+
+__global__ __launch_bounds__(kSmallThreads) void k_norm_small(NormArgs a, Scores sc, float* __restrict__ out) {
+  __shared__ double smem[kSmallThreads / kWave];
+  const int64_t g = blockIdx.x;
+  const bool grouped = g < a.n_groups;
+  const int64_t gb = grouped ? g * a.seg_elems : a.n_groups * a.seg_elems;
+  const int64_t ge = grouped ? gb + a.seg_elems : a.n;
+  auto value = [&](int64_t i) { return score_of(sc, a.x[i]); };
+  auto weight = [&](int64_t i) { return a.mask ? a.mask[i] : 1.f; };
+  auto sums = [&](int64_t b, int64_t e) {
+    double s = 0.0, f = 0.0;
+    for (int64_t i = b + threadIdx.x; i < e; i += kSmallThreads) {
+      const double m = (double)weight(i);
+      s += (double)value(i) * m;
+      f += m;
+    }
+    s = block_sum<double>(s, smem);
+    f = block_sum<double>(f, smem);
+    return make_double4(s, f, 0.0, 0.0);
+  };
+  const double4 none = make_double4(0.0, 0.0, 0.0, 0.0);
+  const bool batch_level = a.mean_level == 1 || a.std_level == 1;
+  double4 batch = (batch_level || a.mask) ? sums(0, a.n) : none, group = grouped ? sums(gb, ge) : none;
+  const bool passthrough = a.mask != nullptr && batch.y == 0.0;
+  // sum of (x m - mean m)^2 about the mean of the element's own level
+  auto squares = [&](int64_t b, int64_t e) {
+    double q = 0.0;
+    for (int64_t i = b + threadIdx.x; i < e; i += kSmallThreads) {
+      const float xi = value(i), mi = weight(i);
+      double mean = 0.0;
+      if (a.mean_level == 1) {
+        mean = level_mean(batch.x, batch.y, a.mean_leave1out != 0, a.mask != nullptr, xi, mi);
+      } else if (a.mean_level == 2 && i < a.n_groups * a.seg_elems && !(a.group_size == 1 && a.mean_leave1out)) {
+        double4 own = group;
+        if (i < gb || i >= ge) {  // a batch-wide deviation about group means: the sums of that element's group
+          own = none;
+          const int64_t first = i / a.seg_elems * a.seg_elems;
+          for (int64_t j = first; j < first + a.seg_elems; ++j) {
+            own.x += (double)value(j) * (double)weight(j);
+            own.y += (double)weight(j);
+          }
+        }
+        mean = (double)(float)level_mean(own.x, own.y, a.mean_leave1out != 0, a.mask != nullptr, xi, mi);
+      }
+      const double d = (double)xi * (double)mi - mean * (double)mi;
+      q += d * d;
+    }
+    return block_sum<double>(q, smem);
+  };
+  if (a.std_level == 1) batch.z = squares(0, a.n);
+  if (a.std_level == 2 && grouped) group.z = squares(gb, ge);
+  for (int64_t i = gb + threadIdx.x; i < ge; i += kSmallThreads)
+    out[i] = norm_element(a, batch, group, grouped, passthrough, value(i), weight(i));
+}
+
+// without a normalisation: the scores themselves
+__global__ __launch_bounds__(256) void k_scores(const float* __restrict__ x, int64_t n, Scores sc, float* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = score_of(sc, x[i]);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -352,6 +435,259 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
       r += (mask_no_eos_with_zero && no_eos) ? 0.f : score[b];
     }
     rewards[i] = r;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------------
+// The advantage pipeline of a padded batch (PPOActor._compute_advantages, actor.py:172-236) in one pass per row: mask and
+// log-probs rolled and masked, KL-regularised rewards, the GAE scan, and the sums that the normalisation of the
+// advantages needs.  One workgroup per row, super-blocks of 4096 positions from the end as in k_gae: a super-block's
+// inputs are read once, what the scan needs of them stays in LDS.  Bound by memory: 26 bytes in and 24 out per token (30
+// in with values); the separate launches (rolls, products, KL, GAE, two passes of sums; thirteen of them) moved about
+// three times as much.
+// ------------------------------------------------------------------------------------------------------------------
+// Per row: sums for the normalisation.  F = sum m, S = sum x m; A = sum m^2, B = sum m^2 (x - c), C = sum m^2 (x - c)^2
+// about a centre c of the row's own (its mean in the first super-block), from which the sum of squares about any mean
+// follows without cancellation.
+struct RowSums {
+  double F, S, A, B, C, c;
+};
+
+struct RowArgs {
+  const void* mask_in;      // [bs, L] loss mask: one byte (mask_bytes) or one float per token
+  const float* logp;        // [bs, L]
+  float* ref;               // nullable; masked in place
+  const uint8_t* attention; // nullable: [bs, L], one byte per token ...
+  const int64_t* seqlens;   // ... or the lengths [bs]
+  const float* score;       // [bs]
+  const float* values;      // nullable
+  float* mask_out;
+  float* old_out;           // may be logp itself when it is not rolled
+  float* kl_rewards;
+  float* rewards;
+  float* adv;
+  float* returns;
+  RowSums* sums;            // nullable: no normalisation
+  double4* stats;           // with sums: one per segment of the normalisation (see k_norm_partial)
+  StepWork* work;           // with sums
+  int64_t bs, L;
+  float kl_ctl, gamma, lam;
+  int estimator, mask_no_eos_with_zero, mask_bytes, roll;
+  NormArgs norm;            // levels and groups of the normalisation (no leave-one-out)
+};
+
+__device__ __forceinline__ float mask_at(const RowArgs& a, int64_t i) {
+  return a.mask_bytes ? (((const uint8_t*)a.mask_in)[i] ? 1.f : 0.f) : ((const float*)a.mask_in)[i];
+}
+
+// mean that the normalisation subtracts in a row, from the sums of the row's segment
+__device__ __forceinline__ double row_mean(const NormArgs& n, const double4* stats, int64_t row) {
+  if (n.mean_level == 0) return 0.0;
+  if (n.mean_level == 1) return stats[0].y == 0.0 ? 0.0 : stats[0].x / stats[0].y;
+  const int64_t g = row / n.group_size;
+  if (g >= n.n_groups) return 0.0;
+  const double4 s = stats[1 + g];
+  return (double)(float)(s.y == 0.0 ? 0.0 : s.x / s.y);
+}
+
+__global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
+  __shared__ float sr[kGaeLds], sv[kGaeLds], sm[kGaeLds];
+  __shared__ Affine wave_tot[kGaeThreads / kWave];
+  __shared__ float carry[2];
+  __shared__ double smem[kGaeThreads / kWave];
+  __shared__ int smem_i[kGaeThreads / kWave];
+  __shared__ int last;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int64_t row = blockIdx.x, L = a.L, r0 = row * L;
+  int64_t sl;
+  if (a.attention) {
+    int n = 0;
+#pragma unroll 8
+    for (int64_t t = tid; t < L; t += kGaeThreads) n += a.attention[r0 + t];
+    sl = block_sum<int>(n, smem_i);
+  } else {
+    sl = a.seqlens[row];
+  }
+  int64_t at_last = sl - 1;
+  if (at_last < 0) at_last += L;  // Python's negative index, as the reference's fancy indexing does
+  int64_t put = sl - 2;
+  if (put < 0) put = 0;
+  const bool no_eos = sl == L;
+  const float score = (a.mask_no_eos_with_zero && no_eos) ? 0.f : a.score[row];
+  const float gl = a.gamma * a.lam;
+  const float v_end = a.values ? a.values[r0 + L - 1] : 0.f;
+  // one position: everything that does not depend on its neighbours; returns mask, reward and value for the scan
+  auto position = [&](int64_t t, float& m, float& r, float& v) {
+    const int64_t next = t + 1 < L ? t + 1 : 0;  // torch.roll(x, -1)
+    m = mask_at(a, r0 + next);
+    const float lo = a.logp[r0 + (a.roll ? next : t)] * m;
+    float lr = 0.f;
+    if (a.ref) {
+      lr = a.ref[r0 + t] * m;
+      a.ref[r0 + t] = lr;
+    }
+    v = a.values ? a.values[r0 + t] : 0.f;
+    a.mask_out[r0 + t] = m;
+    a.old_out[r0 + t] = lo;
+    float d = lo * m - lr * m;
+    if (a.estimator == 1) d = d * d / 2.0f;
+    else if (a.estimator == 2) { d = -d; d = expf(d) - 1.f - d; }
+    d = (d != d) ? d : fminf(fmaxf(d, -10.f), 10.f);  // torch.clamp keeps NaN
+    const float kr = -a.kl_ctl * d;
+    a.kl_rewards[r0 + t] = kr;
+    r = (t == at_last) ? 0.f : kr;
+    if (t == put) r += score;
+    a.rewards[r0 + t] = r;
+  };
+  float m_end = 0.f;
+  if (tid == 0) {
+    float r, v;
+    position(L - 1, m_end, r, v);
+    a.adv[r0 + L - 1] = 0.f;
+    a.returns[r0 + L - 1] = v_end;
+    carry[0] = no_eos ? v_end : 0.f;
+    carry[1] = 0.f;
+  }
+  // thread 0 carries position L - 1 (advantage 0) in its sums
+  double F = tid == 0 ? (double)m_end : 0.0, S = 0.0, A = F * F, B = 0.0, C = 0.0, c = 0.0;
+  const Affine ident{1.f, 0.f, 1.f, 0.f, 0.f};
+  bool first = true;
+  for (int64_t end = L - 1; end > 0; end -= kGaeBlock) {
+    const int64_t base = end > kGaeBlock ? end - kGaeBlock : 0;
+    const int cnt = (int)(end - base);
+    __syncthreads();  // the previous super-block has been written out; carry is visible
+#pragma unroll 4
+    for (int i = tid; i < cnt; i += kGaeThreads) {
+      float m, r, v;
+      position(base + i, m, r, v);
+      const int slot = gae_slot(i);
+      sr[slot] = r;
+      sv[slot] = v;
+      sm[slot] = m;
+    }
+    __syncthreads();
+    const int hi = cnt - 1 - tid * kGaeChunk;
+    const int lo = hi - kGaeChunk + 1 > 0 ? hi - kGaeChunk + 1 : 0;
+    Affine x = ident;
+    for (int i = hi; i >= lo; --i) {
+      const int slot = gae_slot(i);
+      const float mt = sm[slot], vt = sv[slot], rt = sr[slot];
+      Affine e;
+      e.a = 1.f - mt;
+      e.e = mt * vt;
+      e.c = mt * a.gamma;
+      e.d = (1.f - mt) + mt * gl;
+      e.f = mt * (rt - vt);
+      x = compose(x, e);
+    }
+    Affine inc = x;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const Affine prev = shfl_up(inc, o);
+      if (lane >= o) inc = compose(prev, inc);
+    }
+    if (lane == kWave - 1) wave_tot[wave] = inc;
+    const float nv0 = carry[0], lg0 = carry[1];
+    __syncthreads();
+    Affine before = ident;  // everything processed in this super-block before this thread's chunk
+    for (int w = 0; w < wave; ++w) before = compose(before, wave_tot[w]);
+    Affine excl = shfl_up(inc, 1);
+    if (lane == 0) excl = ident;
+    before = compose(before, excl);
+    float nv = fmaf(before.a, nv0, before.e);
+    float lg = fmaf(before.c, nv0, fmaf(before.d, lg0, before.f));
+    double f_here = 0.0, s_here = 0.0;
+    for (int i = hi; i >= lo; --i) {
+      const int slot = gae_slot(i);
+      const float mt = sm[slot], vt = sv[slot], rt = sr[slot];
+      const float delta = rt + a.gamma * nv - vt;
+      const float newlg = delta + gl * lg;
+      nv = nv * (1.f - mt) + vt * mt;
+      lg = lg * (1.f - mt) + newlg * mt;
+      sr[slot] = lg;        // advantages
+      sv[slot] = lg + vt;   // returns
+      f_here += (double)mt;
+      s_here += (double)lg * (double)mt;
+    }
+    if (tid == kGaeThreads - 1) {  // the last thread ends at the front of the super-block: its state carries on
+      carry[0] = nv;
+      carry[1] = lg;
+    }
+    F += f_here;
+    S += s_here;
+    if (a.sums && first) {  // the centre of the row's squares: its mean so far
+      const double f = block_sum<double>(F, smem), s = block_sum<double>(S, smem);
+      c = f != 0.0 ? s / f : 0.0;
+      first = false;
+      if (tid == 0) {  // position L - 1
+        const double mm = (double)m_end * (double)m_end;
+        B = -mm * c;
+        C = mm * c * c;
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < cnt; i += kGaeThreads) {
+      const int slot = gae_slot(i);
+      const float ad = sr[slot];
+      a.adv[r0 + base + i] = ad;
+      a.returns[r0 + base + i] = sv[slot];
+      if (a.sums) {
+        const double mm = (double)sm[slot] * (double)sm[slot], d = (double)ad - c;
+        A += mm;
+        B += mm * d;
+        C += mm * d * d;
+      }
+    }
+  }
+  if (!a.sums) return;
+  F = block_sum<double>(F, smem);
+  S = block_sum<double>(S, smem);
+  A = block_sum<double>(A, smem);
+  B = block_sum<double>(B, smem);
+  C = block_sum<double>(C, smem);
+  if (tid == 0) {
+    a.sums[row] = RowSums{F, S, A, B, C, c};
+    __threadfence();
+    last = atomicAdd(&a.work->finished, 1) == (int)gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  // the last workgroup: the segments of the normalisation from the sums of their rows, in row order
+  __threadfence();
+  const NormArgs& n = a.norm;
+  for (int64_t g = tid; g < n.n_groups; g += kGaeThreads) {
+    double4 st = make_double4(0.0, 0.0, 0.0, 0.0);
+    for (int64_t r = g * n.group_size; r < (g + 1) * n.group_size; ++r) {
+      st.x += a.sums[r].S;
+      st.y += a.sums[r].F;
+    }
+    a.stats[1 + g] = st;
+  }
+  double bs = 0.0, bf = 0.0;
+  for (int64_t r = tid; r < a.bs; r += kGaeThreads) {
+    bs += a.sums[r].S;
+    bf += a.sums[r].F;
+  }
+  bs = block_sum<double>(bs, smem);
+  bf = block_sum<double>(bf, smem);
+  if (tid == 0) a.stats[0] = make_double4(bs, bf, 0.0, 0.0);
+  __syncthreads();  // the segment sums are visible to the whole workgroup
+  auto squares = [&](int64_t r) {
+    const RowSums q = a.sums[r];
+    const double d = row_mean(n, a.stats, r) - q.c;
+    return q.C - 2.0 * d * q.B + d * d * q.A;
+  };
+  for (int64_t g = tid; g < n.n_groups; g += kGaeThreads) {
+    double z = 0.0;
+    for (int64_t r = g * n.group_size; r < (g + 1) * n.group_size; ++r) z += squares(r);
+    a.stats[1 + g].z = z > 0.0 ? z : 0.0;
+  }
+  double z = 0.0;
+  for (int64_t r = tid; r < a.bs; r += kGaeThreads) z += squares(r);
+  z = block_sum<double>(z, smem);
+  if (tid == 0) {
+    a.stats[0].z = z > 0.0 ? z : 0.0;
+    a.work->finished = 0;
   }
 }
 
@@ -497,6 +833,11 @@ static int norm_parts(int64_t n) {
   return (int)(p < 1 ? 1 : (p > 256 ? 256 : p));
 }
 
+static void launch_norm_small(const NormArgs& a, const Scores& sc, float* out, hipStream_t st) {
+  const unsigned grid = (unsigned)(a.n_groups + (a.n_groups * a.seg_elems < a.n ? 1 : 0));
+  hipLaunchKernelGGL(k_norm_small, dim3(grid), dim3(kSmallThreads), 0, st, a, sc, out);
+}
+
 extern "C" int64_t aa_normalize_scratch_bytes(int64_t bs, int64_t inner, int64_t group_size) {
   if (bs < 0 || inner < 1 || group_size < 1) return -1;
   const int64_t segs = 1 + bs / group_size;
@@ -522,6 +863,10 @@ extern "C" int aa_normalize(const float* x, const float* loss_mask, int64_t bs, 
   NormArgs a{x, loss_mask, bs * inner, gs * inner, n_groups, gs, p.mean_level, p.mean_leave1out, p.std_level,
              p.std_unbiased, p.eps};
   hipStream_t st = (hipStream_t)stream;
+  if (a.n <= kSmallNorm && out != x) {
+    launch_norm_small(a, Scores{0, 0.f, 1.f, 0.f}, out, st);
+    return launch_status();
+  }
   double4* stats = (double4*)scratch;
   double2* partial = (double2*)(stats + segs);
   const unsigned fin = (unsigned)segs;
@@ -535,6 +880,90 @@ extern "C" int aa_normalize(const float* x, const float* loss_mask, int64_t bs, 
   int64_t blocks = (a.n + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   hipLaunchKernelGGL(k_norm_apply, dim3((unsigned)blocks), dim3(256), 0, st, a, stats, out);
+  return launch_status();
+}
+
+extern "C" int aa_reward_scores(const float* rewards, int64_t bs, float bias, float scaling, float clip,
+                                const aa_norm_params* norm, float* out, void* stream) {
+  if (bs < 0 || (bs > 0 && (!rewards || !out || rewards == out))) return AA_ERR_INVALID_ARGUMENT;
+  if (bs == 0) return AA_OK;
+  hipStream_t st = (hipStream_t)stream;
+  const Scores sc{1, bias, scaling, clip};
+  if (!norm) {
+    hipLaunchKernelGGL(k_scores, dim3((unsigned)((bs + 255) / 256)), dim3(256), 0, st, rewards, bs, sc, out);
+    return launch_status();
+  }
+  const aa_norm_params& p = *norm;
+  if (p.mean_level < 0 || p.mean_level > 2 || p.std_level < 0 || p.std_level > 2) return AA_ERR_INVALID_ARGUMENT;
+  const bool grouped = p.mean_level == 2 || p.std_level == 2;
+  if (grouped && p.group_size < 1) return AA_ERR_INVALID_ARGUMENT;
+  if (bs > kSmallNorm) return AA_ERR_UNSUPPORTED;
+  const int64_t gs = grouped ? p.group_size : bs;
+  const NormArgs a{rewards, nullptr, bs, gs, grouped ? bs / gs : 0, gs, p.mean_level, p.mean_leave1out, p.std_level,
+                   p.std_unbiased, p.eps};
+  launch_norm_small(a, sc, out, st);
+  return launch_status();
+}
+
+extern "C" int64_t aa_advantages_scratch_bytes(int64_t bs) {
+  if (bs < 0) return -1;
+  return (1 + bs) * (int64_t)sizeof(double4) + bs * (int64_t)sizeof(RowSums);
+}
+
+extern "C" int aa_advantages(const aa_advantage_step* step, void* stream) {
+  if (!step) return AA_ERR_INVALID_ARGUMENT;
+  const aa_advantage_step& p = *step;
+  if (p.bs < 0 || p.L < 1 || p.bs > 0x7fffffff || p.kl_estimator < 0 || p.kl_estimator > 2) return AA_ERR_INVALID_ARGUMENT;
+  if (p.bs == 0) return AA_OK;
+  if (!p.loss_mask || !p.logp || !p.reward_score || (!p.attention_mask && !p.seqlens) || !p.mask_out || !p.logp_out ||
+      !p.kl_rewards || !p.rewards || !p.advantages || !p.returns)
+    return AA_ERR_INVALID_ARGUMENT;
+  if (p.roll_logp && p.logp_out == p.logp) return AA_ERR_INVALID_ARGUMENT;
+  RowArgs a{};
+  a.mask_in = p.loss_mask;
+  a.logp = p.logp;
+  a.ref = p.ref_logp;
+  a.attention = p.attention_mask;
+  a.seqlens = p.seqlens;
+  a.score = p.reward_score;
+  a.values = p.values;
+  a.mask_out = p.mask_out;
+  a.old_out = p.logp_out;
+  a.kl_rewards = p.kl_rewards;
+  a.rewards = p.rewards;
+  a.adv = p.advantages;
+  a.returns = p.returns;
+  a.bs = p.bs;
+  a.L = p.L;
+  a.kl_ctl = p.kl_ctl;
+  a.gamma = p.discount;
+  a.lam = p.gae_lambda;
+  a.estimator = p.kl_estimator;
+  a.mask_no_eos_with_zero = p.mask_no_eos_with_zero;
+  a.mask_bytes = p.loss_mask_bytes;
+  a.roll = p.roll_logp;
+  if (p.norm) {
+    const aa_norm_params& q = *p.norm;
+    if (q.mean_level < 0 || q.mean_level > 2 || q.std_level < 0 || q.std_level > 2) return AA_ERR_INVALID_ARGUMENT;
+    if (q.mean_leave1out && q.mean_level != 0) return AA_ERR_UNSUPPORTED;
+    const bool grouped = q.mean_level == 2 || q.std_level == 2;
+    if (grouped && q.group_size < 1) return AA_ERR_INVALID_ARGUMENT;
+    if (!p.scratch || (((uintptr_t)p.scratch) & 31) || p.scratch_bytes < aa_advantages_scratch_bytes(p.bs) || !p.work)
+      return AA_ERR_INVALID_ARGUMENT;
+    const int64_t gs = grouped ? q.group_size : p.bs;
+    a.norm = NormArgs{p.advantages, p.mask_out, p.bs * p.L, gs * p.L, grouped ? p.bs / gs : 0, gs, q.mean_level, 0,
+                      q.std_level, q.std_unbiased, q.eps};
+    a.stats = (double4*)p.scratch;
+    a.sums = (RowSums*)(a.stats + 1 + p.bs);
+    a.work = (StepWork*)p.work;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL(k_advantage_rows, dim3((unsigned)p.bs), dim3(kGaeThreads), 0, st, a);
+  if (p.norm) {
+    int64_t blocks = (a.norm.n + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    hipLaunchKernelGGL(k_norm_apply, dim3((unsigned)blocks), dim3(256), 0, st, a.norm, a.stats, p.advantages);
+  }
   return launch_status();
 }
 

@@ -1052,6 +1052,61 @@ int aa_lmhead_ppo_step(const aa_ppo_step* step, const void* hidden,
                        void* d_hidden, void* d_weight, int d_weight_dtype,
                        void* workspace, int64_t workspace_bytes, void* stream);
 
+/*
+ * out[b] = clip((rewards[b] + bias) * scaling, -clip, clip) (actor.py:166-170),
+ * normalised as aa_normalize does without a mask when norm is given (then at
+ * most 8192 rewards; AA_ERR_UNSUPPORTED otherwise).  One launch; out is not
+ * rewards.
+ */
+int aa_reward_scores(const float* rewards, int64_t bs, float bias,
+                     float scaling, float clip, const aa_norm_params* norm,
+                     float* out, void* stream);
+
+/*
+ * PPOActor._compute_advantages (areal/trainer/ppo/actor.py:172-236) behind the
+ * reward scores, for padded [bs, L] arrays, in one pass per row (and one more
+ * over the advantages when they are normalised):
+ *   mask_out   = roll(loss_mask, -1) as float32
+ *   logp_out   = (roll_logp ? roll(logp, -1) : logp) * mask_out  (without the
+ *                roll logp_out may be logp itself)
+ *   ref_logp  *= mask_out, in place (nullable)
+ *   kl_rewards, rewards: as aa_kl_rewards with sequence lengths = row sums of
+ *                attention_mask (one byte per token), or seqlens when that is
+ *                NULL
+ *   advantages, returns: as aa_gae, seq_no_eos = (length == L)
+ *   norm       nullable: advantages are normalised under mask_out as
+ *                aa_normalize does (no leave-one-out: AA_ERR_UNSUPPORTED)
+ * scratch: aa_advantages_scratch_bytes(bs) bytes, 32-byte aligned, and work:
+ * AA_STEP_WORK_BYTES (see aa_ppo_step), both only with norm.
+ */
+typedef struct {
+  int64_t bs, L;
+  const void* loss_mask;    /* float32, or one byte per token (loss_mask_bytes) */
+  int32_t loss_mask_bytes;
+  int32_t roll_logp;
+  const float* logp;
+  float* ref_logp;
+  const uint8_t* attention_mask;
+  const int64_t* seqlens;
+  const float* reward_score;
+  const float* values;      /* nullable */
+  float kl_ctl, discount, gae_lambda;
+  int32_t kl_estimator;     /* 0 k1, 1 k2, 2 k3 */
+  int32_t mask_no_eos_with_zero;
+  const aa_norm_params* norm;
+  float* mask_out;
+  float* logp_out;
+  float* kl_rewards;
+  float* rewards;
+  float* advantages;
+  float* returns;
+  void* scratch;
+  int64_t scratch_bytes;
+  void* work;
+} aa_advantage_step;
+int64_t aa_advantages_scratch_bytes(int64_t bs);
+int aa_advantages(const aa_advantage_step* step, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

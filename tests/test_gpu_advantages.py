@@ -316,3 +316,51 @@ def test_moments_under_masks_of_their_own(device, n):
     assert torch.equal(out[:, 1:].cpu(), want[:, 1:])
     bound = 2.0 ** -23 * torch.stack([v.double()[m1].abs().sum() for v in (x, y)])
     assert bool(((out[:, 0].cpu().double() - want[:, 0].double()).abs() <= bound + 1e-30).all())
+
+
+@pytest.mark.parametrize("bs,L", [(1, 1), (3, 2), (7, 17), (4, 4096), (5, 4097), (4, 4098), (6, 9000), (300, 33)])
+@pytest.mark.parametrize("variant", ["batch", "group", "group mean, batch deviation", "no normalisation", "recomputed"])
+def test_advantage_rows_agree_with_the_separate_kernels(device, bs, L, variant):
+    """The one-pass kernel (one super-block of 4096 positions, edges, several; rows past the last full group) against the
+    separate rolls, products, KL, GAE and two-pass normalisation, which an adv_norm that is no ``Normalization`` takes.
+    What moves and multiplies is bit-equal; so are advantages and returns (the same scan); normalised advantages differ
+    by the rounding of float64 sums in another order, then once to float32: 4 ulps of the largest."""
+    from areal_amd import engine_glue
+
+    g = torch.Generator().manual_seed(bs * 10007 + L)
+    lens = torch.randint(1, L + 1, (bs, 1), generator=g)
+    at = torch.arange(L)[None]
+    attention = at < lens
+    mask = attention & (torch.rand(bs, L, generator=g) < 0.7)
+    logp = -2.0 * torch.rand(bs, L, generator=g)
+    base = dict(attention_mask=attention, loss_mask=mask if L % 2 else mask.float(), logprobs=logp,
+                rewards=torch.randn(bs, generator=g), prox_logp=logp + 0.05 * torch.randn(bs, L, generator=g))
+    if variant != "no normalisation":
+        base["ref_logp"] = logp + 0.05 * torch.randn(bs, L, generator=g)
+    if variant in ("batch", "recomputed"):
+        base["values"] = torch.randn(bs, L, generator=g) + 3.0
+    cfg = {"group": dict(mean_level="group", std_level="group", group_size=4),
+           "group mean, batch deviation": dict(mean_level="group", std_level="batch", group_size=4),
+           "no normalisation": None}.get(variant, dict(mean_level="batch", std_level="batch"))
+    norm = None if cfg is None else Normalization(NormConfig(**cfg))
+    reward = Normalization(NormConfig(mean_level="group", mean_leave1out=True, std_level="batch", group_size=4))
+    kw = dict(kl_ctl=0.1, kl_estimator="k3", discount=0.99, gae_lambda=0.95, reward_bias=0.1, reward_scaling=2.0,
+              use_decoupled_loss=variant != "recomputed", recompute_logprob=variant == "recomputed")
+
+    def run(adv_norm, reward_norm):
+        data = {k: v.clone().to(device) for k, v in base.items()}
+        return engine_glue.compute_advantages(data, adv_norm=adv_norm, reward_norm=reward_norm, **kw)
+
+    got, again = run(norm, reward), run(norm, reward)
+    want = run(lambda x, m: x.clone() if norm is None else norm(x, m), lambda x: reward(x))
+    for k in ("loss_mask", "logprobs", "prox_logp", "ref_logp", "kl_rewards", "tot_rewards", "returns", "advantages"):
+        if k not in want:
+            continue
+        a, b = got[k], want[k]
+        assert torch.equal(got[k], again[k]) and a.dtype == b.dtype and a.shape == b.shape, k
+        if k == "advantages" and norm is not None:
+            assert float((a - b).abs().max()) <= 4 * 2.0 ** -23 * max(float(b.abs().max()), 1.0), k
+        elif k in ("tot_rewards", "returns", "advantages"):  # the reward scores go through float64 sums of another order
+            assert float((a - b).abs().max()) <= 4 * 2.0 ** -23 * max(float(b.abs().max()), 1.0), k
+        else:
+            assert torch.equal(a, b), k
