@@ -334,7 +334,7 @@ __device__ __forceinline__ float norm_element(const NormArgs& a, const double4& 
 // out may be x itself (an element is read, then written, by the same thread).
 // BATCH (batch-wide mean and deviation, no leave-one-out, the usual normalisation of advantages): the same expression
 // for every element, its mean and the reciprocal of its deviation formed once; the general form divides and takes a root
-// in float64 per element (512 x 4096: 9.8 us, against APPLY_US).
+// in float64 per element (512 x 4096: 9.8 us, against 7.7 us so).
 template <bool BATCH>
 __global__ __launch_bounds__(256) void k_norm_apply(NormArgs a, const double4* __restrict__ stats, float* out) {
   const bool passthrough = a.mask != nullptr && stats[0].y == 0.0;
