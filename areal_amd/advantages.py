@@ -123,6 +123,12 @@ def _plain(t: torch.Tensor | None, shape, dev) -> bool:
                          and not t.requires_grad)
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two contiguous arrays share memory."""
+    pa, pb = a.data_ptr(), b.data_ptr()
+    return pa < pb + b.numel() * b.element_size() and pb < pa + a.numel() * a.element_size()
+
+
 @torch.no_grad()
 def reward_scores(rewards: torch.Tensor, bias: float, scaling: float, clip: float, norm) -> torch.Tensor | None:
     """``norm(clip((rewards + bias) * scaling, -clip, clip))`` (actor.py:166-172) in one launch; None when the inputs ask
@@ -155,6 +161,11 @@ def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, value
         return None
     if logp is None or not all(_plain(t, shape, dev) for t in (logp, ref_logp, values)):
         return None
+    # what is masked in place is an array of its own: the kernel reads a neighbour's log-prob after that has been masked
+    if ref_logp is not None and any(t is not None and _overlap(ref_logp, t) for t in (logp if roll else None, values)):
+        return None
+    if not roll and values is not None and _overlap(logp, values):
+        return None
     if attention_mask.shape != shape or attention_mask.device != dev or score.shape != (bs,) or not _plain(score, (bs,), dev):
         return None
     if loss_mask.dtype is torch.bool:
@@ -186,6 +197,9 @@ def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, value
         a.scratch, a.scratch_bytes, a.work = _ptr(scratch), scratch.numel() * 8, _ptr(_work_words(dev))
     with _on(dev):
         N.check(lib.aa_advantages(a, _stream(dev)), "aa_advantages")
+    for t in (ref_logp, None if roll else logp):  # written through a raw pointer: autograd is told
+        if t is not None:
+            torch.autograd.graph.increment_version(t)
     return mask_out, logp_out, kl_rewards, rewards, adv, returns
 
 
