@@ -134,7 +134,10 @@ _WORK: dict = {}
 
 def _work_words(dev: torch.device) -> torch.Tensor:
     """The work buffer of the steps on the current stream of ``dev`` (AA_STEP_WORK_BYTES, zero between launches; its
-    first two words are the row hand-out of the fused kernel): one per (device, stream), kept."""
+    first two words are the row hand-out of the fused kernel): one per (device, stream), kept.  A graph that is being
+    captured gets one of its own, cleared by the graph: it may be replayed on any stream, beside eager steps."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.zeros(N.STEP_WORK_BYTES // 4, dtype=torch.int32, device=dev)
     key = (dev.index, _stream(dev))
     buf = _WORK.get(key)
     if buf is None:

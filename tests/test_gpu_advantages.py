@@ -410,3 +410,30 @@ def test_advantages_of_arrays_that_share_memory(device, shared):
     assert torch.equal(got["advantages"], adv) and torch.equal(got["returns"], ret)
     want = -0.1 * (old - arrays["ref_logp"])  # one product and one difference of float32: 2 ulps
     assert float((got["kl_rewards"].cpu() - want).abs().max()) <= 2 * 2.0 ** -23 * float(want.abs().max())
+
+
+def test_moments_in_a_graph_beside_eager_ones(device):
+    """The counters that the workgroups of a launch share are the graph's own: nothing that was captured stays in the
+    buffer kept for eager calls, and replays give the eager result."""
+    from areal_amd import functional
+    from areal_amd.advantages import moments_table
+
+    n = 300001
+    x, m = torch.zeros(n, device=device), torch.zeros(n, dtype=torch.bool, device=device)
+    N = functional.N
+    N.load()
+    kept = dict(functional._WORK)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = moments_table([("x", x, m), ("all", x, None)])
+    assert functional._WORK.keys() == kept.keys()
+    for seed in (1, 2, 3):
+        g = torch.Generator().manual_seed(seed)
+        x.copy_(torch.randn(n, generator=g))
+        m.copy_(torch.rand(n, generator=g) < 0.4)
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = moments_table([("x", x, m), ("all", x, None)])
+        for name in eager:
+            for k in eager[name]:
+                assert torch.equal(eager[name][k], captured[name][k]), (seed, name, k)
