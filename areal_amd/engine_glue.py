@@ -330,17 +330,23 @@ def infer_token_denominator(input_data: dict[str, Any], fallback: torch.Tensor) 
     return torch.ones_like(fallback, **common)
 
 
+def _ends_in_cu_seqlens(input_data: dict[str, Any]) -> bool:
+    """Whether the number of logical tokens is the end of the last packed sequence (a number on the device)."""
+    cu_seqlens = input_data.get("cu_seqlens")
+    return (not isinstance(input_data.get("attention_mask"), torch.Tensor) and isinstance(cu_seqlens, torch.Tensor)
+            and cu_seqlens.numel() > 0)
+
+
 def _n_tokens(input_data: dict[str, Any], fallback: torch.Tensor, step=None) -> int:
     """``infer_token_denominator(input_data, fallback).numel()`` without the mask; ``step``: the step whose counts came to
     the host with the end of its ``cu_seqlens``, so that nothing else is read back."""
     attention_mask = input_data.get("attention_mask")
     if isinstance(attention_mask, torch.Tensor):
         return attention_mask.numel()
-    cu_seqlens = input_data.get("cu_seqlens")
-    if isinstance(cu_seqlens, torch.Tensor) and cu_seqlens.numel() > 0:
+    if _ends_in_cu_seqlens(input_data):
         if step is not None and step.slot is not None and step.struct.cu_seqlens:
             return step.slot.read()[2]
-        return int(cu_seqlens[-1].item())
+        return int(input_data["cu_seqlens"][-1].item())
     input_ids = input_data.get("input_ids")
     if isinstance(input_ids, torch.Tensor) and input_ids.shape == fallback.shape:
         return input_ids.numel()
@@ -430,7 +436,8 @@ def grpo_loss_fn(
     else:
         loss, stat, step = _ppo_actor_loss(logprobs, prox_logp, old_logp, advantages, eps_clip, loss_mask, eps_clip_higher,
                                            c_clip, rejection_sampling, importance_sampling_level,
-                                           input_data.get("cu_seqlens"), host_counts=True)
+                                           input_data.get("cu_seqlens"),
+                                           host_counts=_ends_in_cu_seqlens(input_data))
     rkl_stat = None
     teacher_logp = input_data.get("teacher_logp")
     if teacher_logp is not None:

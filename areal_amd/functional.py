@@ -444,15 +444,17 @@ class _HostSlot:
     Reading them (``filtered_fraction`` is a Python float, as in the reference, and a micro-batch without a token is
     found out on the host) waits for that kernel only, not for the long ones queued after it, and needs no copy and no
     event of its own.  Slots are taken from and given back to a bounded pool (any thread, any stream): the tag tells a
-    use from the ones before it.  A slot that nobody read is not given back."""
+    use from the ones before it.  The memory of a slot that nobody read waits until its kernel has written to it."""
 
     __slots__ = ("_memory", "_words", "address", "tag", "_device", "_got")
     _pool: deque = deque(maxlen=64)
     _tags = itertools.count(1)
-    _unread: list = []  # memory that a kernel may still write to
+    _unread: deque = deque()  # memory that a kernel may still write to, with the tag that says that it has
     _SPINS = 20000  # about a millisecond, then short sleeps: other threads run
 
     def __init__(self, device: torch.device):
+        if _HostSlot._unread:
+            _HostSlot._take_back()
         try:
             self._memory, self._words = _HostSlot._pool.pop()
         except IndexError:
@@ -486,9 +488,31 @@ class _HostSlot:
         _HostSlot._pool.append((memory, words))
         return self._got
 
+    @staticmethod
+    def _take_back() -> None:
+        """Unread memory that has been written to goes back to the pool.  What a failed launch left behind is never
+        written to: past a bound the device is waited for, after which nothing writes to any of it."""
+        unread = _HostSlot._unread
+        if len(unread) > _HostSlot._pool.maxlen and not torch.cuda.is_current_stream_capturing():
+            old = [unread.popleft() for _ in range(len(unread))]
+            for index in {device.index for *_, device in old}:
+                torch.cuda.synchronize(index)
+            _HostSlot._pool.extend((memory, words) for memory, words, _, _ in old)
+            return
+        for _ in range(len(unread)):
+            try:
+                entry = unread.popleft()
+            except IndexError:  # another thread was faster
+                return
+            memory, words, tag, _ = entry
+            if words[3] == tag:
+                _HostSlot._pool.append((memory, words))
+            else:
+                unread.append(entry)
+
     def __del__(self):
         if getattr(self, "_memory", None) is not None:
-            _HostSlot._unread.append(self._memory)
+            _HostSlot._unread.append((self._memory, self._words, self.tag, self._device))
 
 
 class _PerValidToken:

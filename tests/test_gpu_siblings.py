@@ -373,6 +373,34 @@ def test_grpo_loss_fn_reports_the_logging_scopes(device):
     assert list(st["reduced"]["compute_logp"]) == ["prox_logp_gt"] and st["reduced"]["version_stats"] == {}
 
 
+def test_counts_on_the_host_are_asked_for_only_where_they_are_read(device):
+    """With an attention mask nothing of the loss waits for the device; what an abandoned step leaves in host memory goes
+    back to the pool when its kernel has written there."""
+    from areal_amd import engine_glue as G
+    from areal_amd import functional as F
+
+    n = 512
+    lp, old, adv, mask = _tok(n, 6)
+    data = dict(logprobs=old.to(device), advantages=adv.to(device), loss_mask=mask.to(device), prox_logp=old.to(device),
+                cu_seqlens=torch.tensor([0, 200, n], dtype=torch.int32, device=device))
+    kw = dict(eps_clip=0.2, eps_clip_higher=None, c_clip=None, use_decoupled_loss=True)
+    run = lambda **more: G.grpo_loss_fn(lp.to(device), torch.rand(n, device=device), dict(data, **more), **kw)[1]
+    assert run()["reduced"]["n_tokens"] == n
+    taken = next(F._HostSlot._tags)
+    unread = len(F._HostSlot._unread)
+    attention = torch.ones(2, 400, dtype=torch.bool, device=device)
+    for _ in range(3):
+        assert run(attention_mask=attention)["reduced"]["n_tokens"] == 800
+    assert len(F._HostSlot._unread) == unread and next(F._HostSlot._tags) == taken + 1
+    args = (lp.to(device), data["prox_logp"], data["logprobs"], data["advantages"], 0.2, data["loss_mask"])
+    for _ in range(3):
+        F._ppo_actor_loss(*args, host_counts=True)
+    torch.cuda.synchronize()
+    assert len(F._HostSlot._unread) >= 1
+    run()
+    assert len(F._HostSlot._unread) == unread
+
+
 # ---------------------------------------------------------------------------------------------------------------
 # SAPO fused with the log-prob op (one pass over the logits) and with the lm_head (no logits in memory)
 # ---------------------------------------------------------------------------------------------------------------
