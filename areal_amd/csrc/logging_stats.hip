@@ -74,11 +74,11 @@ __device__ __forceinline__ void fold(const Args& a, int g, int j) {
   float lo = __builtin_inff(), hi = -__builtin_inff();
   if (active(a, g)) {
     for (int p = lane; p < a.parts; p += kWave) {
-      const Partial v = a.partial[((int64_t)g * a.parts + p) * kPerGroup + j];
-      sum += v.sum;
-      cnt += v.cnt;
-      lo = nan_min(lo, v.lo);
-      hi = nan_max(hi, v.hi);
+      const Partial* v = a.partial + ((int64_t)g * a.parts + p) * kPerGroup + j;
+      sum += published(&v->sum);
+      cnt += published(&v->cnt);
+      lo = nan_min(lo, published(&v->lo));
+      hi = nan_max(hi, published(&v->hi));
     }
     sum = wave_sum(sum);
     cnt = wave_sum(cnt);
@@ -179,18 +179,16 @@ __global__ __launch_bounds__(kThreads) void k_partial(Args a) {
       r.lo = nan_min(r.lo, sh_lo[j][w]);
       r.hi = nan_max(r.hi, sh_hi[j][w]);
     }
-    a.partial[((int64_t)g * a.parts + part) * kPerGroup + j] = r;
-    __threadfence();
+    Partial* o = a.partial + ((int64_t)g * a.parts + part) * kPerGroup + j;
+    publish(&o->sum, r.sum);
+    publish(&o->cnt, r.cnt);
+    publish(&o->lo, r.lo);
+    publish(&o->hi, r.hi);
   }
   if (!a.work) return;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();
-    last = atomicAdd(&a.work->logged, 1) == (int)gridDim.x - 1;
-  }
+  if (threadIdx.x == 0) last = last_to_finish(&a.work->logged, (int)gridDim.x);  // the first wave published
   __syncthreads();
   if (!last) return;
-  __threadfence();
   for (int q = wave; q < kGroups * kPerGroup; q += kWaves) fold(a, q / kPerGroup, q % kPerGroup);
   if (threadIdx.x == 0) a.work->logged = 0;
 }
@@ -336,23 +334,25 @@ __global__ __launch_bounds__(kMomentThreads) void k_moments(MomentArgs a) {
   fold_waves(kW);
   if (a.parts > 1) {
     if (threadIdx.x == 0) {
-      a.partial[blockIdx.x] = MomentPartial{s, c, lo, hi, 0.f};
-      __threadfence();
-      last = atomicAdd(&a.work->moments[k], 1) == a.parts - 1;
+      MomentPartial* o = a.partial + blockIdx.x;
+      publish(&o->sum, s);
+      publish(&o->cnt, c);
+      publish(&o->lo, lo);
+      publish(&o->hi, hi);
+      last = last_to_finish(&a.work->moments[k], a.parts);
     }
     __syncthreads();
     if (!last || wave != 0) return;
-    __threadfence();
     s = 0.0;
     c = 0;
     lo = __builtin_inff();
     hi = -__builtin_inff();
     if (lane < a.parts) {  // lane p holds slice p
-      const MomentPartial p = a.partial[k * a.parts + lane];
-      s = p.sum;
-      c = p.cnt;
-      lo = p.lo;
-      hi = p.hi;
+      const MomentPartial* p = a.partial + k * a.parts + lane;
+      s = published(&p->sum);
+      c = published(&p->cnt);
+      lo = published(&p->lo);
+      hi = published(&p->hi);
     }
     fold_waves(1);
     if (lane == 0) a.work->moments[k] = 0;

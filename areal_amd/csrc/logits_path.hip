@@ -861,11 +861,10 @@ __global__ __launch_bounds__(1024) void k_fused_f32_hold(const float* logits, in
     for (int j = 0; j < Plan::issued_at(0); ++j) issue(rsrc, j);
   }
   if (work && tid == 0) {  // the last workgroup to finish leaves both words at zero for the next launch
-    __threadfence();
-    if (atomicAdd(&work[1], 1) == (int)gridDim.x - 1) {
+    // every row number this workgroup asked work[0] for has come back
+    if (last_to_finish(&work[1], (int)gridDim.x)) {
       work[0] = 0;
       work[1] = 0;
-      __threadfence();
     }
   }
 }
@@ -1412,11 +1411,10 @@ void k_fused_regs(typename InPtr<ALIAS, uint4>::type logits, int V, int64_t stri
     t = tn; y = y_n; y_ok = y_ok_n; xy_raw = xy_raw_n; tin = tin_n;
   }
   if (work && tid == 0) {
-    __threadfence();
-    if (atomicAdd(&work[1], 1) == (int)gridDim.x - 1) {
+    // every row number this workgroup asked work[0] for has come back
+    if (last_to_finish(&work[1], (int)gridDim.x)) {
       work[0] = 0;
       work[1] = 0;
-      __threadfence();
     }
   }
 }

@@ -120,9 +120,7 @@ __device__ __forceinline__ void count_up(const Counts& c, int total, int hit) {
   if (gridDim.x > 1) {
     if (total) atomicAdd(&c.work->total, total);
     if (hit) atomicAdd(&c.work->hit, hit);
-    __threadfence();
-    if (atomicAdd(&c.work->done, 1) != (int)gridDim.x - 1) return;
-    __threadfence();
+    if (!last_to_finish(&c.work->done, (int)gridDim.x)) return;
     total = atomicExch(&c.work->total, 0);
     hit = atomicExch(&c.work->hit, 0);
     atomicExch(&c.work->done, 0);
@@ -510,18 +508,15 @@ __global__ __launch_bounds__(kFinishThreads) void k_step_finish(FinishArgs a) {
   if (threadIdx.x == 0) {
     last = 1;
     if (gridDim.x > 1) {
-      a.work->partial[blockIdx.x] = acc;
-      __threadfence();
-      last = atomicAdd(&a.work->finished, 1) == (int)gridDim.x - 1;
+      publish(&a.work->partial[blockIdx.x], acc);
+      last = last_to_finish(&a.work->finished, (int)gridDim.x);
     }
   }
   __syncthreads();
   if (!last) return;
   if (gridDim.x > 1) {
-    __threadfence();
     double part = 0.0;
-    if (threadIdx.x < gridDim.x)
-      part = __hip_atomic_load(&a.work->partial[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < gridDim.x) part = published(&a.work->partial[threadIdx.x]);
     acc = block_sum<double>(part, smem);
   }
   if (threadIdx.x == 0) {
