@@ -471,6 +471,10 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // inputs are read once, what the scan needs of them stays in LDS.  Bound by memory: 26 bytes in and 24 out per token (30
 // in with values); the separate launches (rolls, products, KL, GAE, two passes of sums; thirteen of them) moved about
 // three times as much.
+// The sums of a row are published past the caches for the last workgroup to fold: with a __threadfence() in every
+// workgroup (a write-back of its XCD's L2, full of the outputs' lines) 512 x 4096 took 40.2 us, so 35.7.
+// Also measured, slower, at 512 x 4096 per pass (46 us so): 512 threads with chunks of 8 57 us; a chunk held in registers
+// for both walks 66 us (128 registers a lane are not enough for it).
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int kRowsAhead = 8;  // positions of a thread whose inputs are on their way together
 
@@ -692,14 +696,26 @@ __global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
   B = block_sum<double>(B, smem);
   C = block_sum<double>(C, smem);
   if (tid == 0) {
-    a.sums[row] = RowSums{F, S, A, B, C, c};
-    __threadfence();
-    last = atomicAdd(&a.work->finished, 1) == (int)gridDim.x - 1;
+    RowSums* o = a.sums + row;
+    publish(&o->F, F);
+    publish(&o->S, S);
+    publish(&o->A, A);
+    publish(&o->B, B);
+    publish(&o->C, C);
+    publish(&o->c, c);
+    last = last_to_finish(&a.work->finished, (int)gridDim.x);
   }
   __syncthreads();
   if (!last) return;
-  // the last workgroup: the segments of the normalisation from the sums of their rows, in row order
-  __threadfence();
+  // the last workgroup: the segments of the normalisation from the sums of their rows, in row order.  The sums of all
+  // rows are fetched at once and stored again as this workgroup's own, so that the loops below, which walk the rows of
+  // a segment one after the other, find them in its caches.
+  for (int64_t r = tid; r < a.bs; r += kGaeThreads) {
+    const RowSums* q = a.sums + r;
+    const RowSums own{published(&q->F), published(&q->S), published(&q->A), published(&q->B), published(&q->C), published(&q->c)};
+    a.sums[r] = own;
+  }
+  __syncthreads();
   const NormArgs& n = a.norm;
   for (int64_t g = tid; g < n.n_groups; g += kGaeThreads) {
     double4 st = make_double4(0.0, 0.0, 0.0, 0.0);
