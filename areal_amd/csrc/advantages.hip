@@ -668,6 +668,7 @@ __global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
     if (a.sums && first) {  // the centre of the row's squares: its mean so far
       const double f = block_sum<double>(F, smem), s = block_sum<double>(S, smem);
       c = f != 0.0 ? s / f : 0.0;
+      if (!isfinite(c)) c = 0.0;  // an infinity among the advantages: its square is infinite about any finite centre
       first = false;
       if (tid == 0) {  // position L - 1
         const double mm = (double)m_end * (double)m_end;
@@ -737,18 +738,19 @@ __global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
   auto squares = [&](int64_t r) {
     const RowSums q = a.sums[r];
     const double d = row_mean(n, a.stats, r) - q.c;
+    if (isinf(q.C) && isfinite(d)) return q.C;  // (the terms below are infinities of both signs)
     return q.C - 2.0 * d * q.B + d * d * q.A;
   };
   for (int64_t g = tid; g < n.n_groups; g += kGaeThreads) {
     double z = 0.0;
     for (int64_t r = g * n.group_size; r < (g + 1) * n.group_size; ++r) z += squares(r);
-    a.stats[1 + g].z = z > 0.0 ? z : 0.0;
+    a.stats[1 + g].z = z < 0.0 ? 0.0 : z;  // a rounding below zero; NaN stays
   }
   double z = 0.0;
   for (int64_t r = tid; r < a.bs; r += kGaeThreads) z += squares(r);
   z = block_sum<double>(z, smem);
   if (tid == 0) {
-    a.stats[0].z = z > 0.0 ? z : 0.0;
+    a.stats[0].z = z < 0.0 ? 0.0 : z;
     a.work->finished = 0;
   }
 }

@@ -437,3 +437,36 @@ def test_moments_in_a_graph_beside_eager_ones(device):
         for name in eager:
             for k in eager[name]:
                 assert torch.equal(eager[name][k], captured[name][k]), (seed, name, k)
+
+
+@pytest.mark.parametrize("levels", [("group", "batch"), (None, "batch"), (None, "group"), ("batch", "batch"),
+                                    ("batch", "group"), ("group", "group")])
+@pytest.mark.parametrize("L", [60, 5000])
+@pytest.mark.parametrize("what", ["nan", "inf", "-inf"])
+def test_advantages_that_are_not_finite_reach_the_deviation(device, levels, L, what):
+    """A NaN or an infinity in one row (at its first position, the last one of the scan, so that it does not spread along
+    the row by itself) does to every other row what it does in the separate kernels: in a mean or deviation that it enters
+    it stays, the rest of the batch agrees to the rounding of sums in another order."""
+    from areal_amd import engine_glue
+
+    bs = 12
+    g = torch.Generator().manual_seed(L)
+    values = torch.randn(bs, L, generator=g)
+    big = {"nan": float("nan"), "inf": -3e38, "-inf": 3e38}[what]
+    values[5, 0], values[5, 1] = big, (0.0 if what == "nan" else -big)
+    mask = torch.rand(bs, L, generator=g) < 0.7
+    mask[5, 1:3] = True  # after the roll: positions 0 and 1 count
+    logp = -torch.rand(bs, L, generator=g)
+    data = dict(attention_mask=torch.ones(bs, L, dtype=torch.bool), loss_mask=mask, logprobs=logp, values=values,
+                rewards=torch.randn(bs, generator=g))
+    norm = Normalization(NormConfig(mean_level=levels[0], std_level=levels[1], group_size=4))
+    kw = dict(kl_ctl=0.1, discount=0.99, gae_lambda=0.0, use_decoupled_loss=True)
+
+    def run(adv_norm):
+        return engine_glue.compute_advantages({k: v.clone().to(device) for k, v in data.items()}, adv_norm=adv_norm, **kw)
+
+    plain = run(None)["advantages"]
+    hit = plain[5, 0].isnan() if what == "nan" else plain[5, 0] == float(what)
+    assert bool(hit) and int((~plain.isfinite()).sum()) == 1
+    got, want = run(norm)["advantages"], run(lambda x, m: norm(x, m))["advantages"]
+    assert torch.allclose(got, want, rtol=1e-6, atol=1e-6, equal_nan=True)
