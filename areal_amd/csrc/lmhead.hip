@@ -457,7 +457,7 @@ __global__ __launch_bounds__(1024) void k_token_loss(const float* __restrict__ p
     } else {
       fn = (float)(n < 1 ? 1 : n);
     }
-    const float gscale = scale_of(a.scale, n);
+    const float gscale = scale_of(a.scale, a.n_valid);
     const bool on = a.mask_eff[t] != 0;
     if (a.P.loss_kind == AA_LOSS_NLL) {
       a.stat_loss[t] = on ? -lp : 0.f;

@@ -460,7 +460,7 @@ __device__ __forceinline__ uint32_t load_u16_uniform(const void* __restrict__ ro
 // d(surrogate)/d(logp) and d(scaled loss)/d(logp).
 __device__ __forceinline__ void load_loss_scale(const FusedTokenArgs& a, float& fn, float& gscale) {
   int n = *a.n_valid;
-  gscale = scale_of(a.scale, n);
+  gscale = scale_of(a.scale, a.n_valid);
   if (a.P.loss_kind == AA_LOSS_NLL) {
     fn = (float)n + 1e-5f;  // the supervised loss divides by 1e-5 + count (areal/trainer/sft/lm_engine.py:96)
   } else {

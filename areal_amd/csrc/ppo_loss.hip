@@ -94,7 +94,7 @@ __global__ void k_zero_i32(int32_t* p, int n) {
   if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
 }
 
-// Who takes the counts of a launch: two counters that the caller has cleared (work == nullptr), or the work buffer of a
+// Who takes the counts of a launch: three counters that the caller has cleared (work == nullptr), or the work buffer of a
 // step: the workgroups add up there, the last one to finish moves the sums to counts (and to host memory) and leaves the
 // buffer zero for the next launch.  One launch then does what took a clearing kernel, this one, and a copy to the host.
 struct Counts {
@@ -110,24 +110,27 @@ __device__ __forceinline__ void host_store(int32_t* p, int32_t v, int order_rele
   else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// one thread per workgroup
-__device__ __forceinline__ void count_up(const Counts& c, int total, int hit) {
+// one thread per workgroup; outside: tokens of the mask that no sequence covers
+__device__ __forceinline__ void count_up(const Counts& c, int total, int hit, int outside = 0) {
   if (!c.work) {
     if (total) atomicAdd(&c.counts[0], total);
     if (hit) atomicAdd(&c.counts[1], hit);
+    if (outside) atomicAdd(&c.counts[2], outside);
     return;
   }
   if (gridDim.x > 1) {
     if (total) atomicAdd(&c.work->total, total);
     if (hit) atomicAdd(&c.work->hit, hit);
+    if (outside) atomicAdd(&c.work->outside, outside);
     if (!last_to_finish(&c.work->done, (int)gridDim.x)) return;
     total = atomicExch(&c.work->total, 0);
     hit = atomicExch(&c.work->hit, 0);
+    outside = atomicExch(&c.work->outside, 0);
     atomicExch(&c.work->done, 0);
   }
   c.counts[0] = total;
   c.counts[1] = hit;
-  c.counts[2] = 0;
+  c.counts[2] = outside;
   if (c.host) {
     host_store(c.host + 0, total, 0);
     host_store(c.host + 1, hit, 0);
@@ -180,8 +183,14 @@ __global__ __launch_bounds__(kSegThreads) void k_rs_sequence(const float* __rest
   int64_t beg, end;
   seg.range(b, beg, end);
   if (b == seg.B) {  // tokens no sequence covers
-    for (int64_t i = beg + threadIdx.x; i < end; i += kSegThreads) { mask_out[i] = 0; w_out[i] = 0.f; }
-    if (threadIdx.x == 0) count_up(counts, 0, 0);
+    int outside = 0;
+    for (int64_t i = beg + threadIdx.x; i < end; i += kSegThreads) {
+      outside += mask[i] != 0 ? 1 : 0;
+      mask_out[i] = 0;
+      w_out[i] = 0.f;
+    }
+    outside = block_sum<int>(outside, smem_i);
+    if (threadIdx.x == 0) count_up(counts, 0, 0, outside);
     return;
   }
   const bool log_agg = c.metric == AA_RS_RATIO;
@@ -521,7 +530,7 @@ __global__ __launch_bounds__(kFinishThreads) void k_step_finish(FinishArgs a) {
   }
   if (threadIdx.x == 0) {
     a.work->finished = 0;
-    a.loss[0] = (float)acc / fn * scale_of(a.scale, nv);
+    a.loss[0] = (float)acc / fn * scale_of(a.scale, a.n_valid);
   }
 }
 

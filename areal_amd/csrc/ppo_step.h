@@ -15,7 +15,8 @@ struct StepWork {
   int32_t total, hit, done;
   int32_t finished;
   int32_t logged;
-  int32_t pad[9];
+  int32_t outside;
+  int32_t pad[8];
   int32_t moments[kTableTensors];
   double partial[kFinishBlocks];
 };

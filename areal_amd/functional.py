@@ -528,7 +528,8 @@ class _PerValidToken:
 
 def _note_valid_tokens(scale, step) -> None:
     if isinstance(scale, _PerValidToken):
-        scale.valid_tokens = step.slot.read()[0]
+        # the count on the host is that of the tokens inside the sequences; without any, the mask itself is asked
+        scale.valid_tokens = step.slot.read()[0] or int(step.mask.count_nonzero())
 
 
 def _scale_struct(scale, dev: torch.device):
@@ -1449,7 +1450,7 @@ def fused_lm_head_ppo_loss(
             if rs.action != "mask":
                 mask_eff = m8
         else:
-            n_valid = _count_nonzero(m8)
+            n_valid = torch.nn.functional.pad(_count_nonzero(m8), (0, 2))  # the three counts of a step
         # only the tokens with a mask go through the lm_head: gather them (autograd scatters d(hidden) back), run the
         # step on the closed-up batch with an all-true mask, and put the per-token results back at their tokens
         idx = mask_eff.nonzero().squeeze(-1)

@@ -85,8 +85,8 @@ typedef struct {
 
 /* The factor a loss and its gradient are multiplied by:
  *   value, times *factor when factor is given, and, with per_valid_token != 0,
- *   times (number of non-zero entries of the loss mask) / (*total or, when
- *   total is NULL, total_value): the engine's local_weight /
+ *   times (number of non-zero entries of the loss mask, counts[0] + counts[2]
+ *   of the step) / (*total or, when total is NULL, total_value): the engine's local_weight /
  *   total_loss_weight * multiplier (fsdp_engine.py:2045) without a launch or a
  *   copy of its own. */
 typedef struct {
@@ -317,8 +317,11 @@ int aa_logits_pairs_scatter(void* dlogits, int dtype, int64_t T, int64_t V,
  *   mask_in  uint8 [n]  (non-zero = valid)
  *   mask_out uint8 [n]  updated mask (action mask) or a copy (action clamp)
  *   behave_w float [n]  importance weight, zero where mask_out is zero
- *   counts   int32 [3]  {non-zero entries of mask_in, filtered-or-clamped
- *                        valid tokens, unused}; written, not accumulated
+ *   counts   int32 [3]  {non-zero entries of mask_in (at level sequence:
+ *                        inside the segments), filtered-or-clamped valid
+ *                        tokens, non-zero entries of mask_in behind the last
+ *                        segment (0 at level token)}; written, not
+ *                        accumulated
  * lower is ignored unless has_lower != 0.
  */
 int aa_rejection_sampling(const float* prox_logp, const float* old_logp,

@@ -811,3 +811,36 @@ def test_weight_of_the_micro_batch_inside_the_kernels(device, total, masked):
                                                 mb["loss_mask"], cu_seqlens=mb["cu_seqlens"], loss_scale=scale)
     want.backward()
     assert torch.equal(loss, want) and torch.equal(a.grad, b.grad)
+
+
+@pytest.mark.parametrize("entry", ["logits", "lm_head"])
+@pytest.mark.parametrize("inside", ["some", "none"])
+def test_weight_counts_the_tokens_outside_every_sequence(device, entry, inside):
+    """``cu_seqlens`` that end before the tokens do: the weight of the micro-batch is the count of its whole loss mask,
+    while sequence-level rejection sampling leaves what lies outside the sequences without a loss."""
+    g = torch.Generator().manual_seed(11)
+    T, covered, V, H = 130, 100, 640, 64
+    mask = torch.rand(T, generator=g) < 0.6
+    if inside == "none":
+        mask[:covered] = False
+    mask[-1] = True
+    rs = RejectionSamplingConfig(level="sequence", action="mask", metric="ratio", agg="mean", upper=100.0)
+    ids = torch.randint(0, V, (T,), generator=g).to(device)
+    mb = {k: torch.randn(T, generator=g).to(device) - 2.0 for k in ("logprobs", "prox_logp", "advantages")}
+    mb.update(loss_mask=mask.to(device), cu_seqlens=torch.tensor([0, 40, covered], dtype=torch.int32, device=device))
+    if entry == "logits":
+        ins = [torch.randn(T, V, generator=g).bfloat16().to(device)]
+        step, glue = areal_amd.fused_logprobs_ppo_loss, engine_glue.compute_logprobs_and_loss
+    else:
+        ins = [torch.randn(T, H, generator=g).bfloat16().to(device), (0.1 * torch.randn(V, H, generator=g)).bfloat16().to(device)]
+        step, glue = areal_amd.fused_lm_head_ppo_loss, engine_glue.compute_lm_head_and_loss
+    a, b = ([t.clone().requires_grad_(True) for t in ins] for _ in range(2))
+    loss, stat = glue(*a, {"rolled_input_ids": ids}, mb, 0, 977.0, 0.2, rejection_sampling=rs, loss_multiplier=3.0)
+    loss.backward()
+    scale = mb["loss_mask"].count_nonzero() / 977.0 * 3.0
+    want, want_stat = step(*b, ids, mb["prox_logp"], mb["logprobs"], mb["advantages"], 0.2, mb["loss_mask"],
+                           rejection_sampling=rs, cu_seqlens=mb["cu_seqlens"], loss_scale=scale)
+    want.backward()
+    assert torch.equal(loss, want) and stat.keys() == want_stat.keys()
+    for x, y in zip(a, b):
+        assert torch.equal(x.grad, y.grad)
