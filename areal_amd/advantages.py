@@ -161,8 +161,9 @@ def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, value
         return None
     if logp is None or not all(_plain(t, shape, dev) for t in (logp, ref_logp, values)):
         return None
-    # what is masked in place is an array of its own: the kernel reads a neighbour's log-prob after that has been masked
-    if ref_logp is not None and any(t is not None and _overlap(ref_logp, t) for t in (logp if roll else None, values)):
+    # what is masked in place is an array of its own: the kernel reads a neighbour's log-prob after that has been masked,
+    # and one array as both policies is masked twice
+    if ref_logp is not None and any(t is not None and _overlap(ref_logp, t) for t in (logp, values)):
         return None
     if not roll and values is not None and _overlap(logp, values):
         return None

@@ -470,3 +470,19 @@ def test_advantages_that_are_not_finite_reach_the_deviation(device, levels, L, w
     assert bool(hit) and int((~plain.isfinite()).sum()) == 1
     got, want = run(norm)["advantages"], run(lambda x, m: norm(x, m))["advantages"]
     assert torch.allclose(got, want, rtol=1e-6, atol=1e-6, equal_nan=True)
+
+
+def test_advantages_of_one_array_as_both_policies(device):
+    """Recomputed log-probs that are also the reference policy's are masked twice, as in the reference: with a mask of
+    fractions that shows."""
+    from areal_amd import engine_glue
+
+    bs, L = 4, 33
+    g = torch.Generator().manual_seed(8)
+    mask, one = torch.rand(bs, L, generator=g), -torch.rand(bs, L, generator=g)
+    shared = one.clone().to(device)
+    data = dict(attention_mask=torch.ones(bs, L, dtype=torch.bool, device=device), loss_mask=mask.to(device),
+                logprobs=one.to(device), prox_logp=shared, ref_logp=shared, rewards=torch.zeros(bs, device=device))
+    engine_glue.compute_advantages(data, use_decoupled_loss=False, recompute_logprob=True)
+    m = torch.roll(mask, -1, -1)
+    assert torch.equal(shared.cpu(), one * m * m)
