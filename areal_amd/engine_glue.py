@@ -55,6 +55,12 @@ def _weight_is_zero(local_weight):
     return lambda: zero
 
 
+def _float32_total(total_loss_weight) -> bool:
+    """Whether ``local_weight / total_loss_weight * multiplier`` is a float32 expression, which the kernels can form
+    themselves (a float64 total makes torch form it in float64)."""
+    return not (isinstance(total_loss_weight, torch.Tensor) and total_loss_weight.dtype is torch.float64)
+
+
 def compute_logprobs(logits: torch.Tensor, model_inputs: dict[str, Any], temperature: float = 1.0) -> torch.Tensor:
     """Forward-only log-probs of a micro-batch (fsdp_engine.py:1938-1964)."""
     return gather_logprobs(logits, rolled_labels(model_inputs), temperature=temperature)
@@ -92,7 +98,8 @@ def compute_logprobs_and_loss(
     old_logp = mb_input["logprobs"]
     prox_logp = mb_input.get("prox_logp")
     if (fused and not use_sapo_loss and importance_sampling_level == "token" and prox_logp is not None
-            and not inplace_backward and torch.is_grad_enabled() and logits.requires_grad):
+            and not inplace_backward and torch.is_grad_enabled() and logits.requires_grad
+            and _float32_total(total_loss_weight)):
         # one call that counts the tokens itself; a micro-batch without any is found out afterwards (nothing of it is used)
         scale = _PerValidToken(total_loss_weight, loss_multiplier)
         out = fused_logprobs_ppo_loss(
@@ -199,7 +206,7 @@ def compute_lm_head_and_loss(
     scale: Any = None
     if host_loss_mask is None:
         if (prox_logp is not None and importance_sampling_level == "token" and torch.is_grad_enabled()
-                and (hidden.requires_grad or weight.requires_grad)):
+                and (hidden.requires_grad or weight.requires_grad) and _float32_total(total_loss_weight)):
             # the step counts the tokens itself; a micro-batch without any is found out afterwards
             scale = _PerValidToken(total_loss_weight, loss_multiplier)
         else:
@@ -681,7 +688,7 @@ def compute_logprobs_and_sft_loss(logits: torch.Tensor, model_inputs: dict[str, 
     from .sft import fused_logprobs_sft_loss
 
     loss_mask = mb_input["loss_mask"].bool()
-    if torch.is_grad_enabled() and logits.requires_grad:
+    if torch.is_grad_enabled() and logits.requires_grad and _float32_total(total_loss_weight):
         # one call that counts the tokens itself; a micro-batch without any is found out afterwards (nothing of it is used)
         per_token = _PerValidToken(total_loss_weight, loss_multiplier)
         out = fused_logprobs_sft_loss(logits, rolled_labels(model_inputs), loss_mask, mb_input["cu_seqlens"], temperature,

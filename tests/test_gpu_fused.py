@@ -844,3 +844,35 @@ def test_weight_counts_the_tokens_outside_every_sequence(device, entry, inside):
     assert torch.equal(loss, want) and stat.keys() == want_stat.keys()
     for x, y in zip(a, b):
         assert torch.equal(x.grad, y.grad)
+
+
+@pytest.mark.parametrize("entry", ["ppo", "sft", "lm_head"])
+def test_weight_against_a_total_in_float64(device, entry):
+    """torch forms ``local_weight / total * multiplier`` in float64 when the total is float64, and rounds once: bit-equal
+    to that factor given as ``loss_scale``, for counts at which three float32 roundings come out differently."""
+    from areal_amd.sft import fused_logprobs_sft_loss
+
+    g = torch.Generator().manual_seed(7)
+    T, V, H = 40, 640, 64
+    ins = [torch.randn(T, V, generator=g).bfloat16().to(device)]
+    if entry == "lm_head":
+        ins = [torch.randn(T, H, generator=g).bfloat16().to(device), (0.1 * torch.randn(V, H, generator=g)).bfloat16().to(device)]
+    ids = torch.randint(0, V, (T,), generator=g).to(device)
+    mb = {k: torch.randn(T, generator=g).to(device) - 2.0 for k in ("logprobs", "prox_logp", "advantages")}
+    mb["cu_seqlens"] = torch.tensor([0, T], dtype=torch.int32, device=device)
+    total = torch.tensor(977.1, dtype=torch.float64, device=device)
+    for n in range(1, T, 3):
+        mask = mb["loss_mask"] = torch.arange(T, device=device) < n
+        a, b = ([t.clone().requires_grad_(True) for t in ins] for _ in range(2))
+        scale = mask.count_nonzero() / total * 3.0
+        ppo = (mb["prox_logp"], mb["logprobs"], mb["advantages"], 0.2, mask)
+        if entry == "sft":
+            loss, _ = engine_glue.compute_logprobs_and_sft_loss(*a, {"rolled_input_ids": ids}, mb, total, loss_multiplier=3.0)
+            want, _ = fused_logprobs_sft_loss(*b, ids, mask, mb["cu_seqlens"], loss_scale=scale)
+        elif entry == "ppo":
+            loss, _ = engine_glue.compute_logprobs_and_loss(*a, {"rolled_input_ids": ids}, mb, 0, total, 0.2, loss_multiplier=3.0)
+            want, _ = areal_amd.fused_logprobs_ppo_loss(*b, ids, *ppo, loss_scale=scale)
+        else:
+            loss, _ = engine_glue.compute_lm_head_and_loss(*a, {"rolled_input_ids": ids}, mb, 0, total, 0.2, loss_multiplier=3.0)
+            want, _ = areal_amd.fused_lm_head_ppo_loss(*b, ids, *ppo, loss_scale=scale)
+        assert torch.equal(loss, want), n
