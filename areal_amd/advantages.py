@@ -236,6 +236,7 @@ def moments_table(entries: list[tuple[str, torch.Tensor, torch.Tensor | None]]) 
         values[i] = v.data_ptr()
         keep.append(v)
         if mask is not None:
+            _require_gpu(mask, f"the mask of {name}")
             m = _mask_bytes(mask)
             masks[i] = m.data_ptr()
             keep.append(m)

@@ -137,3 +137,21 @@ def test_gradient_array_is_laid_out_like_the_logits(V, stride, lead):
     out.fill_(1.0)
     assert float(flat.abs().sum()) == 0.0
     assert float(out.float().sum()) == T * V
+
+
+def test_moments_of_a_mask_in_host_memory_are_refused(monkeypatch):
+    """Every mask is asked for its device before its address goes to a kernel: the supervised loss function takes a mask
+    from anywhere, and its statistics used to refuse one in host memory."""
+    from areal_amd import advantages as A
+
+    def stands_for_a_device(t, name):
+        if "mask" in name:
+            raise areal_amd.NativeLibraryError(f"{name}: no CPU fallback")
+
+    def launched():
+        raise AssertionError("the address of the mask went to the library")
+
+    monkeypatch.setattr(A, "_require_gpu", stands_for_a_device)
+    monkeypatch.setattr(A.N, "load", launched)
+    with pytest.raises(areal_amd.NativeLibraryError, match="the mask of x"):
+        A.moments_table([("x", torch.zeros(4), torch.ones(4, dtype=torch.bool))])
