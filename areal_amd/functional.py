@@ -494,10 +494,19 @@ class _HostSlot:
         written to: past a bound the device is waited for, after which nothing writes to any of it."""
         unread = _HostSlot._unread
         if len(unread) > _HostSlot._pool.maxlen and not torch.cuda.is_current_stream_capturing():
-            old = [unread.popleft() for _ in range(len(unread))]
-            for index in {device.index for *_, device in old}:
-                torch.cuda.synchronize(index)
-            _HostSlot._pool.extend((memory, words) for memory, words, _, _ in old)
+            old = []
+            try:
+                while len(old) <= 2 * _HostSlot._pool.maxlen:
+                    old.append(unread.popleft())
+            except IndexError:  # that was all, or another thread takes the rest
+                pass
+            try:
+                for index in {device.index for *_, device in old}:
+                    torch.cuda.synchronize(index)
+            except RuntimeError:  # (not while another thread captures a graph): kernels may still write to any of it
+                unread.extend(old)
+            else:
+                _HostSlot._pool.extend((memory, words) for memory, words, _, _ in old)
             return
         for _ in range(len(unread)):
             try:

@@ -155,3 +155,35 @@ def test_moments_of_a_mask_in_host_memory_are_refused(monkeypatch):
     monkeypatch.setattr(A.N, "load", launched)
     with pytest.raises(areal_amd.NativeLibraryError, match="the mask of x"):
         A.moments_table([("x", torch.zeros(4), torch.ones(4, dtype=torch.bool))])
+
+
+@pytest.mark.parametrize("waiting_fails", [False, True])
+def test_host_memory_of_abandoned_steps_under_threads(monkeypatch, waiting_fails):
+    """Past the bound the memory that nobody read goes back once the device has been waited for.  Another thread may take
+    entries after their number was read, and the wait may fail: nothing is raised into the caller's step, and memory that
+    a kernel may still write to is not let go."""
+    from collections import deque
+
+    from areal_amd.functional import _HostSlot
+
+    class AnotherThreadTakesSome(deque):
+        def __len__(self):
+            return super().__len__() + 3
+
+    def wait(index):
+        waited.append(index)
+        if waiting_fails:
+            raise RuntimeError("operation not permitted when stream is capturing")
+
+    entries = [([tag], [0, 0, 0, -1], tag, torch.device("cuda:0")) for tag in range(1, 71)]
+    unread, pool, waited = AnotherThreadTakesSome(entries), deque(maxlen=64), []
+    monkeypatch.setattr(_HostSlot, "_unread", unread)
+    monkeypatch.setattr(_HostSlot, "_pool", pool)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "synchronize", wait)
+    _HostSlot._take_back()
+    assert waited == [0]
+    if waiting_fails:
+        assert list(unread) == entries and not pool
+    else:
+        assert not list(unread) and [m for m, _ in pool] == [[tag] for tag in range(7, 71)]
