@@ -462,7 +462,7 @@ class _HostSlot:
             self._words = (C.c_int32 * 4).from_address(self._memory.data_ptr())
             self._words[3] = 0
         self.address = self._memory.data_ptr()
-        self.tag = next(_HostSlot._tags) & 0x7FFFFFFF or next(_HostSlot._tags)
+        self.tag = next(_HostSlot._tags) % 0x7FFFFFFF + 1  # 31 bits, never 0
         self._device = device
         self._got = None
 

@@ -187,3 +187,19 @@ def test_host_memory_of_abandoned_steps_under_threads(monkeypatch, waiting_fails
         assert list(unread) == entries and not pool
     else:
         assert not list(unread) and [m for m, _ in pool] == [[tag] for tag in range(7, 71)]
+
+
+def test_tags_of_steps_fit_the_word_they_come_back_in(monkeypatch):
+    """A tag is compared with an int32 in host memory, also after 2^31 steps."""
+    import ctypes
+    import itertools
+    from collections import deque
+
+    from areal_amd.functional import _HostSlot
+
+    for first in (1, 0x7FFFFFFE, 0x80000000, 0xFFFFFFFF, 2 ** 40):
+        monkeypatch.setattr(_HostSlot, "_tags", itertools.count(first))
+        monkeypatch.setattr(_HostSlot, "_unread", deque())
+        monkeypatch.setattr(_HostSlot, "_pool", deque((torch.empty(4), None) for _ in range(3)))
+        tags = [_HostSlot(torch.device("cuda:0")).tag for _ in range(3)]
+        assert all(t > 0 and ctypes.c_int32(t).value == t for t in tags) and len(set(tags)) == 3
