@@ -201,5 +201,8 @@ def test_tags_of_steps_fit_the_word_they_come_back_in(monkeypatch):
         monkeypatch.setattr(_HostSlot, "_tags", itertools.count(first))
         monkeypatch.setattr(_HostSlot, "_unread", deque())
         monkeypatch.setattr(_HostSlot, "_pool", deque((torch.empty(4), None) for _ in range(3)))
-        tags = [_HostSlot(torch.device("cuda:0")).tag for _ in range(3)]
+        slots = [_HostSlot(torch.device("cuda:0")) for _ in range(3)]
+        tags = [slot.tag for slot in slots]
+        for slot in slots:
+            slot._memory = None  # nothing is given back
         assert all(t > 0 and ctypes.c_int32(t).value == t for t in tags) and len(set(tags)) == 3
