@@ -45,14 +45,48 @@ def rolled_labels(model_inputs: dict[str, Any]) -> torch.Tensor:
 
 
 def _weight_is_zero(local_weight):
-    """A function that tells whether the weight of the micro-batch is zero.  A device tensor starts on its way to the host
-    now, behind what is queued already; the answer is asked for when the next long kernel has been queued as well, so that
-    the device has work while the host waits."""
+    """(a function that tells whether the weight of the micro-batch is zero, whether it has to wait for the device).  A
+    device tensor starts on its way to the host now, behind what is queued already."""
     if isinstance(local_weight, torch.Tensor) and local_weight.is_cuda:
         pending = _HostCounts(local_weight.detach().reshape(()))
-        return lambda: pending.tolist() == 0
+        return lambda: pending.tolist() == 0, True
     zero = bool(local_weight == 0)
-    return lambda: zero
+    return lambda: zero, False
+
+
+def _no_tokens(scale: _PerValidToken, loss_mask: torch.Tensor):
+    """The same for a step that counts the mask itself."""
+    def is_zero():
+        if scale.valid_tokens is None:
+            scale.valid_tokens = int(loss_mask.count_nonzero())
+        return scale.valid_tokens == 0
+
+    return is_zero, loss_mask.numel() > 0
+
+
+# A forward of at most this much work is queued before the host knows the weight of the micro-batch, so that the device
+# has work while the host waits; what it computed is dropped when the weight is zero.  About 1 ms of forward at 6.4 TB/s
+# and 1.2 PFLOP/s: asking first costs 15 to 80 us of a pass (4 096 x 151 936 bf16 logits 672 against 650 us, PPO step
+# 511 / 437; from hidden states 1 900 x 1 024 1 751 / 1 738, PPO step 1 608 / 1 532), 1 to 3 % of the passes past this
+# line (2 048 x 2 048 2 965 / 2 918, PPO 2 760 / 2 690; 4 096 x 4 096 9 980 / 9 890), and a micro-batch without a token
+# never pays more than this for a result that nobody reads.
+RUN_AHEAD_BYTES = 6_400_000_000
+RUN_AHEAD_FLOPS = 1_200_000_000_000
+
+
+def _unless_weightless(forward, weight, run_ahead: bool):
+    """``forward()``, or None for a micro-batch of weight zero, whatever else it holds (an incomplete one may make
+    ``forward`` raise).  ``weight``: what ``_weight_is_zero`` returned."""
+    is_zero, waits = weight
+    if not (run_ahead and waits) and is_zero():
+        return None
+    try:
+        out = forward()
+    except Exception:
+        if is_zero():
+            return None
+        raise
+    return None if is_zero() else out
 
 
 def _float32_total(total_loss_weight) -> bool:
@@ -100,13 +134,15 @@ def compute_logprobs_and_loss(
     if (fused and not use_sapo_loss and importance_sampling_level == "token" and prox_logp is not None
             and not inplace_backward and torch.is_grad_enabled() and logits.requires_grad
             and _float32_total(total_loss_weight)):
-        # one call that counts the tokens itself; a micro-batch without any is found out afterwards (nothing of it is used)
+        # one call that counts the tokens itself
         scale = _PerValidToken(total_loss_weight, loss_multiplier)
-        out = fused_logprobs_ppo_loss(
-            logits, rolled_labels(model_inputs), prox_logp, old_logp, mb_input["advantages"], eps_clip, loss_mask,
-            eps_clip_higher, c_clip, rejection_sampling, importance_sampling_level, mb_input.get("cu_seqlens"), temperature,
-            scale)
-        return out if scale.valid_tokens else (logits.mean() * 0.0, {})
+        out = _unless_weightless(
+            lambda: fused_logprobs_ppo_loss(
+                logits, rolled_labels(model_inputs), prox_logp, old_logp, mb_input["advantages"], eps_clip, loss_mask,
+                eps_clip_higher, c_clip, rejection_sampling, importance_sampling_level, mb_input.get("cu_seqlens"),
+                temperature, scale),
+            _no_tokens(scale, loss_mask), 2 * logits.numel() * logits.element_size() <= RUN_AHEAD_BYTES)
+        return (logits.mean() * 0.0, {}) if out is None else out
     local_weight = loss_mask.count_nonzero()
     if local_weight == 0:
         return logits.mean() * 0.0, {}
@@ -207,7 +243,7 @@ def compute_lm_head_and_loss(
     if host_loss_mask is None:
         if (prox_logp is not None and importance_sampling_level == "token" and torch.is_grad_enabled()
                 and (hidden.requires_grad or weight.requires_grad) and _float32_total(total_loss_weight)):
-            # the step counts the tokens itself; a micro-batch without any is found out afterwards
+            # the step counts the tokens itself
             scale = _PerValidToken(total_loss_weight, loss_multiplier)
         else:
             local_weight = loss_mask.count_nonzero()
@@ -215,18 +251,20 @@ def compute_lm_head_and_loss(
         return hidden.mean() * 0.0 + weight.mean() * 0.0, {}
     if prox_logp is None:
         raise ValueError("prox_logp is None: only the recomputed proximal log-probs are supported here")
-    per_token = scale is not None
-    if not per_token:
-        scale = local_weight / total_loss_weight * loss_multiplier
-    out = fused_lm_head_ppo_loss(
-        hidden, weight, rolled_labels(model_inputs), prox_logp, old_logp, mb_input["advantages"], eps_clip=eps_clip,
-        loss_mask=loss_mask, eps_clip_higher=eps_clip_higher, c_clip=c_clip, rejection_sampling=rejection_sampling,
-        importance_sampling_level=importance_sampling_level, cu_seqlens=mb_input.get("cu_seqlens"),
-        temperature=temperature, loss_scale=scale, kept_per_chunk=kept, backward=backward,
-    )
-    if per_token and not scale.valid_tokens:
-        return hidden.mean() * 0.0 + weight.mean() * 0.0, {}
-    return out
+
+    def step(loss_scale):
+        return fused_lm_head_ppo_loss(
+            hidden, weight, rolled_labels(model_inputs), prox_logp, old_logp, mb_input["advantages"], eps_clip=eps_clip,
+            loss_mask=loss_mask, eps_clip_higher=eps_clip_higher, c_clip=c_clip, rejection_sampling=rejection_sampling,
+            importance_sampling_level=importance_sampling_level, cu_seqlens=mb_input.get("cu_seqlens"),
+            temperature=temperature, loss_scale=loss_scale, kept_per_chunk=kept, backward=backward,
+        )
+
+    if scale is None:
+        return step(local_weight / total_loss_weight * loss_multiplier)
+    out = _unless_weightless(lambda: step(scale), _no_tokens(scale, loss_mask),
+                             2 * hidden.numel() * weight.shape[0] <= RUN_AHEAD_FLOPS)
+    return (hidden.mean() * 0.0 + weight.mean() * 0.0, {}) if out is None else out
 
 
 def compute_advantages(
@@ -599,8 +637,8 @@ def compute_loss_with(logits: torch.Tensor, model_inputs: dict[str, Any], mb_inp
     loss functions of this module; the return value has the same form.  A micro-batch of weight 0 returns
     ``logits.mean() * 0``."""
     local_weight = loss_weight_fn(mb_input)
-    is_zero = _weight_is_zero(local_weight)
-    if (is_critic or trie_node is not None) and is_zero():
+    zero_weight = _weight_is_zero(local_weight)
+    if (is_critic or trie_node is not None) and zero_weight[0]():
         return logits.mean() * 0.0
     if is_critic:
         if trie_node is not None:
@@ -619,15 +657,19 @@ def compute_loss_with(logits: torch.Tensor, model_inputs: dict[str, Any], mb_inp
             logp, entropy = gather_packed_tree_logprobs_entropy(logits, trie_node, mb_input["input_ids"],
                                                                 temperature=temperature)
         else:
-            if logits.dim() == 2:
-                logp, entropy, vmax, vmin = _logprobs_impl(logits, rolled_labels(model_inputs), temperature, None, True, True,
-                                                           T_active=logits.shape[0] - pad_length if pad_length > 0 else None)
-            else:
-                logp, entropy, vmin, vmax = gather_logprobs_entropy_stats(logits, rolled_labels(model_inputs), temperature)
-                if pad_length > 0:
-                    logp, entropy, vmin, vmax = (t[:-pad_length] for t in (logp, entropy, vmin, vmax))
-            if is_zero():  # found out while the pass over the logits runs
+            def forward():
+                labels = rolled_labels(model_inputs)
+                if logits.dim() == 2 and logits.shape[0] > pad_length:
+                    lp, ent, hi, lo = _logprobs_impl(logits, labels, temperature, None, True, True,
+                                                     T_active=logits.shape[0] - pad_length if pad_length > 0 else None)
+                    return lp, ent, lo, hi
+                rows = gather_logprobs_entropy_stats(logits, labels, temperature)
+                return tuple(t[:-pad_length] for t in rows) if pad_length > 0 else rows
+
+            rows = _unless_weightless(forward, zero_weight, logits.numel() * logits.element_size() <= RUN_AHEAD_BYTES)
+            if rows is None:
                 return logits.mean() * 0.0
+            logp, entropy, vmin, vmax = rows
         out = loss_fn(logp, entropy, mb_input, vocab_min_logits=vmin, vocab_max_logits=vmax)
     scale = local_weight / total_loss_weight * loss_multiplier
     if isinstance(out, tuple):
@@ -655,22 +697,31 @@ def compute_lm_head_loss_with(hidden: torch.Tensor, weight: torch.Tensor, model_
     if hidden.ndim == 3 and hidden.shape[0] == 1:
         hidden = hidden.squeeze(0)
     local_weight = loss_weight_fn(mb_input)
-    is_zero = _weight_is_zero(local_weight)
-    n_rows = hidden.shape[0] - pad_length if pad_length > 0 else hidden.shape[0]
-    if grad_token_mask is None and backward == "carry":
-        grad_token_mask = mb_input.get("loss_mask")
-    if grad_token_mask is not None:
-        grad_token_mask = grad_token_mask.reshape(-1)
-        if grad_token_mask.dtype is not torch.bool:
-            grad_token_mask = grad_token_mask.ne(0)
-        grad_token_mask = grad_token_mask[:n_rows]
-    carry = backward == "carry"
-    logp, entropy, vmin, vmax = _lm_head_impl(
-        hidden, weight, rolled_labels(model_inputs), temperature, None, True, backward, grad_token_mask if carry else None,
-        kept_per_chunk if carry else None, count_on_device=2 * n_rows * weight.shape[0] <= COUNT_ON_DEVICE_BYTES,
-        T_active=n_rows)
-    if is_zero():  # found out while the logits tiles run
+
+    def forward():
+        # (a micro-batch of nothing but padding goes through the op with its padding rows, which are then cut off)
+        trim = 0 < hidden.shape[0] <= pad_length
+        n_rows = hidden.shape[0] - (pad_length if pad_length > 0 and not trim else 0)
+        carry = backward == "carry"
+        mask = grad_token_mask
+        if mask is None and carry:
+            mask = mb_input.get("loss_mask")
+        if mask is not None:
+            mask = mask.reshape(-1)
+            if mask.dtype is not torch.bool:
+                mask = mask.ne(0)
+            mask = torch.nn.functional.pad(mask, (0, n_rows - mask.shape[0])) if trim else mask[:n_rows]
+        rows = _lm_head_impl(
+            hidden, weight, rolled_labels(model_inputs), temperature, None, True, backward, mask if carry else None,
+            kept_per_chunk if carry else None, count_on_device=2 * n_rows * weight.shape[0] <= COUNT_ON_DEVICE_BYTES,
+            T_active=n_rows)
+        return tuple(t[:-pad_length] for t in rows) if trim else rows
+
+    rows = _unless_weightless(forward, _weight_is_zero(local_weight),
+                              2 * hidden.numel() * weight.shape[0] <= RUN_AHEAD_FLOPS)
+    if rows is None:
         return hidden.mean() * 0.0 + weight.mean() * 0.0
+    logp, entropy, vmin, vmax = rows
     out = loss_fn(logp, entropy, mb_input, vocab_min_logits=vmin, vocab_max_logits=vmax)
     scale = local_weight / total_loss_weight * loss_multiplier
     if isinstance(out, tuple):
@@ -689,11 +740,13 @@ def compute_logprobs_and_sft_loss(logits: torch.Tensor, model_inputs: dict[str, 
 
     loss_mask = mb_input["loss_mask"].bool()
     if torch.is_grad_enabled() and logits.requires_grad and _float32_total(total_loss_weight):
-        # one call that counts the tokens itself; a micro-batch without any is found out afterwards (nothing of it is used)
+        # one call that counts the tokens itself
         per_token = _PerValidToken(total_loss_weight, loss_multiplier)
-        out = fused_logprobs_sft_loss(logits, rolled_labels(model_inputs), loss_mask, mb_input["cu_seqlens"], temperature,
-                                      loss_scale=per_token)
-        return out if per_token.valid_tokens else (logits.mean() * 0.0, {})
+        out = _unless_weightless(
+            lambda: fused_logprobs_sft_loss(logits, rolled_labels(model_inputs), loss_mask, mb_input["cu_seqlens"],
+                                            temperature, loss_scale=per_token),
+            _no_tokens(per_token, loss_mask), 2 * logits.numel() * logits.element_size() <= RUN_AHEAD_BYTES)
+        return (logits.mean() * 0.0, {}) if out is None else out
     local_weight = loss_mask.count_nonzero()
     if local_weight == 0:
         return logits.mean() * 0.0, {}

@@ -876,3 +876,89 @@ def test_weight_against_a_total_in_float64(device, entry):
             loss, _ = engine_glue.compute_lm_head_and_loss(*a, {"rolled_input_ids": ids}, mb, 0, total, 0.2, loss_multiplier=3.0)
             want, _ = areal_amd.fused_lm_head_ppo_loss(*b, ids, *ppo, loss_scale=scale)
         assert torch.equal(loss, want), n
+
+
+def _glue_inputs(device, T=130, pad=9, V=640, H=64):
+    g = torch.Generator().manual_seed(7)
+    hidden = torch.randn(T + pad, H, generator=g).bfloat16().to(device)
+    weight = (0.1 * torch.randn(V, H, generator=g)).bfloat16().to(device)
+    logits = torch.randn(T + pad, V, generator=g).bfloat16().to(device)
+    ids = torch.randint(0, V, (T + pad,), generator=g).to(device)
+    mb = {k: torch.randn(T, generator=g).to(device) - 2.0 for k in ("logprobs", "prox_logp", "advantages")}
+    mb.update(loss_mask=torch.zeros(T, dtype=torch.bool, device=device),
+              cu_seqlens=torch.tensor([0, T], dtype=torch.int32, device=device))
+    return hidden.requires_grad_(), weight.requires_grad_(), logits.requires_grad_(), ids, mb
+
+
+def _zero_weight_calls():
+    loss_fn = lambda logp, entropy, mb, **kw: logp.sum()
+    count = lambda mb: mb["loss_mask"].count_nonzero()
+    return {
+        "ppo": lambda h, w, x, ids, mb, pad: engine_glue.compute_logprobs_and_loss(x, ids, mb, pad, 977.0, 0.2)[0],
+        "sft": lambda h, w, x, ids, mb, pad: engine_glue.compute_logprobs_and_sft_loss(x, ids, mb, 977.0)[0],
+        "lm_head ppo": lambda h, w, x, ids, mb, pad: engine_glue.compute_lm_head_and_loss(h, w, ids, mb, pad, 977.0, 0.2)[0],
+        "any": lambda h, w, x, ids, mb, pad: engine_glue.compute_loss_with(x, ids, mb, pad, loss_fn, count, 977.0),
+        "lm_head any": lambda h, w, x, ids, mb, pad: engine_glue.compute_lm_head_loss_with(h, w, ids, mb, pad, loss_fn, count, 977.0),
+    }
+
+
+@pytest.mark.parametrize("call", ["ppo", "sft", "lm_head ppo", "any", "lm_head any"])
+@pytest.mark.parametrize("odd", ["nothing", "no labels", "labels of another length", "no advantages", "padding only"])
+def test_micro_batch_of_weight_zero_is_a_zero_whatever_else_it_holds(device, call, odd):
+    hidden, weight, logits, ids, mb = _glue_inputs(device)
+    pad, inputs = 9, {"rolled_input_ids": ids}
+    if odd == "no labels":
+        inputs = {}
+    elif odd == "labels of another length":
+        inputs = {"rolled_input_ids": ids[:-3]}
+    elif odd == "no advantages":
+        mb = dict(loss_mask=mb["loss_mask"], logprobs=mb["logprobs"], prox_logp=mb["prox_logp"])
+    elif odd == "padding only":
+        pad, mb = 139, {k: v[:0] for k, v in mb.items()}
+        mb["cu_seqlens"] = torch.zeros(1, dtype=torch.int32, device=device)
+    loss = _zero_weight_calls()[call](hidden, weight, logits, inputs, mb, pad)
+    assert float(loss.detach()) == 0.0
+    loss.backward()
+    grads = [hidden.grad, weight.grad] if call.startswith("lm_head") else [logits.grad]
+    for grad in grads:
+        assert float(grad.float().abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("lm_head", [False, True])
+def test_padding_only_with_a_weight_of_its_own(device, lm_head):
+    """No token at all, but a weight function that does not count tokens: the loss function gets empty tensors."""
+    hidden, weight, logits, ids, mb = _glue_inputs(device)
+    seen = []
+    loss_fn = lambda logp, entropy, mb, vocab_min_logits, vocab_max_logits: seen.append(
+        [t.shape for t in (logp, entropy, vocab_min_logits, vocab_max_logits)]) or logp.sum()
+    kw = dict(loss_fn=loss_fn, loss_weight_fn=lambda mb: 1.0, total_loss_weight=2.0, pad_length=139)
+    mb = dict(loss_mask=mb["loss_mask"][:0])
+    if lm_head:
+        loss = engine_glue.compute_lm_head_loss_with(hidden, weight, {"rolled_input_ids": ids}, mb, **kw)
+    else:
+        loss = engine_glue.compute_loss_with(logits, {"rolled_input_ids": ids}, mb, **kw)
+    assert seen == [[torch.Size([0])] * 4] and float(loss.detach()) == 0.0
+    loss.backward()
+    for grad in ([hidden.grad, weight.grad] if lm_head else [logits.grad]):
+        assert float(grad.float().abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("call", ["ppo", "sft", "lm_head ppo", "any", "lm_head any"])
+def test_long_forward_of_a_micro_batch_of_weight_zero_is_not_queued(device, monkeypatch, call):
+    """Past the bound on what is queued ahead the weight is asked for first; up to it the forward runs at most once."""
+    from areal_amd import sft
+
+    hidden, weight, logits, ids, mb = _glue_inputs(device)
+    ran = []
+    for module, name in ((engine_glue, "fused_logprobs_ppo_loss"), (sft, "fused_logprobs_sft_loss"), (engine_glue, "_logprobs_impl"),
+                         (engine_glue, "fused_lm_head_ppo_loss"), (engine_glue, "_lm_head_impl")):
+        plain = getattr(module, name)
+        monkeypatch.setattr(module, name, lambda *a, plain=plain, **kw: ran.append(name) or plain(*a, **kw))
+    args = (hidden, weight, logits, {"rolled_input_ids": ids}, mb, 9)
+    assert float(_zero_weight_calls()[call](*args).detach()) == 0.0 and len(ran) <= 1
+    ran.clear()
+    monkeypatch.setattr(engine_glue, "RUN_AHEAD_BYTES", 0)
+    monkeypatch.setattr(engine_glue, "RUN_AHEAD_FLOPS", 0)
+    assert float(_zero_weight_calls()[call](*args).detach()) == 0.0 and not ran
+    mb["loss_mask"][5] = True
+    assert float(_zero_weight_calls()[call](*args).detach()) != 0.0 and len(ran) == 1

@@ -206,3 +206,16 @@ def test_tags_of_steps_fit_the_word_they_come_back_in(monkeypatch):
         for slot in slots:
             slot._memory = None  # nothing is given back
         assert all(t > 0 and ctypes.c_int32(t).value == t for t in tags) and len(set(tags)) == 3
+
+
+def test_weight_zero_that_the_host_knows_runs_no_forward(monkeypatch):
+    from areal_amd import engine_glue as G
+
+    ran = []
+    monkeypatch.setattr(G, "_logprobs_impl", lambda *a, **kw: ran.append("logits"))
+    monkeypatch.setattr(G, "_lm_head_impl", lambda *a, **kw: ran.append("lm_head"))
+    x = torch.ones(4, 8, requires_grad=True)
+    for zero in (0, 0.0, torch.tensor(0)):
+        assert float(G.compute_loss_with(x, {}, {}, 0, None, lambda mb: zero, 1.0).detach()) == 0.0
+        assert float(G.compute_lm_head_loss_with(x, x, {}, {}, 0, None, lambda mb: zero, 1.0).detach()) == 0.0
+    assert not ran
