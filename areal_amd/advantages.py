@@ -8,6 +8,7 @@ are refused.
 from __future__ import annotations
 
 import ctypes as C
+from numbers import Real
 from typing import Any, Mapping
 
 import torch
@@ -132,7 +133,10 @@ def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
 @torch.no_grad()
 def reward_scores(rewards: torch.Tensor, bias: float, scaling: float, clip: float, norm) -> torch.Tensor | None:
     """``norm(clip((rewards + bias) * scaling, -clip, clip))`` (actor.py:166-172) in one launch; None when the inputs ask
-    for the general way (``norm`` another callable than ``Normalization``, more rewards than one launch takes)."""
+    for the general way (``norm`` another callable than ``Normalization``, more rewards than one launch takes, tensors for
+    numbers)."""
+    if not all(isinstance(v, Real) for v in (bias, scaling, clip)):
+        return None
     if norm is not None and not (type(norm) is Normalization and _one_process() and rewards.numel() <= 8192):
         return None
     if not _plain(rewards, rewards.shape, rewards.device) or rewards.ndim != 1 or not rewards.is_cuda or rewards.numel() == 0:

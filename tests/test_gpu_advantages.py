@@ -486,3 +486,22 @@ def test_advantages_of_one_array_as_both_policies(device):
     engine_glue.compute_advantages(data, use_decoupled_loss=False, recompute_logprob=True)
     m = torch.roll(mask, -1, -1)
     assert torch.equal(shared.cpu(), one * m * m)
+
+
+def test_reward_scores_with_a_bias_per_sequence(device):
+    """Bias, scaling and clip may be tensors, as in the torch expressions of the reference."""
+    from areal_amd import engine_glue
+
+    bs, L = 6, 12
+    g = torch.Generator().manual_seed(5)
+    bias, scaling = torch.randn(bs, generator=g), torch.rand(bs, generator=g)
+    data = dict(attention_mask=torch.ones(bs, L, dtype=torch.bool), loss_mask=torch.ones(bs, L, dtype=torch.bool),
+                logprobs=torch.zeros(bs, L), rewards=torch.randn(bs, generator=g))
+    norm = Normalization(NormConfig(mean_level="group", std_level="group", group_size=3))
+    for reward_norm in (None, norm):
+        out = engine_glue.compute_advantages({k: v.clone().to(device) for k, v in data.items()}, reward_bias=bias.to(device),
+                                             reward_scaling=scaling.to(device), reward_norm=reward_norm)
+        want = (data["rewards"] + bias) * scaling
+        if reward_norm is not None:
+            want = O.normalization(want, None, mean_level="group", std_level="group", group_size=3, eps=1e-5)
+        assert torch.allclose(out["tot_rewards"][:, L - 2].cpu(), want, rtol=1e-5, atol=1e-6)
