@@ -710,7 +710,8 @@ def compute_lm_head_loss_with(hidden: torch.Tensor, weight: torch.Tensor, model_
             mask = mask.reshape(-1)
             if mask.dtype is not torch.bool:
                 mask = mask.ne(0)
-            mask = torch.nn.functional.pad(mask, (0, n_rows - mask.shape[0])) if trim else mask[:n_rows]
+            if pad_length > 0:  # without padding the op refuses a mask of another length
+                mask = torch.nn.functional.pad(mask, (0, n_rows - mask.shape[0])) if mask.shape[0] < n_rows else mask[:n_rows]
         rows = _lm_head_impl(
             hidden, weight, rolled_labels(model_inputs), temperature, None, True, backward, mask if carry else None,
             kept_per_chunk if carry else None, count_on_device=2 * n_rows * weight.shape[0] <= COUNT_ON_DEVICE_BYTES,

@@ -219,3 +219,25 @@ def test_weight_zero_that_the_host_knows_runs_no_forward(monkeypatch):
         assert float(G.compute_loss_with(x, {}, {}, 0, None, lambda mb: zero, 1.0).detach()) == 0.0
         assert float(G.compute_lm_head_loss_with(x, x, {}, {}, 0, None, lambda mb: zero, 1.0).detach()) == 0.0
     assert not ran
+
+
+@pytest.mark.parametrize("length,pad,want", [(10, 0, [1] * 10), (12, 0, [1] * 12), (8, 0, [1] * 8), (7, 3, [1] * 7),
+                                             (10, 3, [1] * 7), (5, 3, [1] * 5 + [0] * 2), (0, 10, [0] * 10)])
+def test_gradient_mask_of_a_padded_micro_batch(monkeypatch, length, pad, want):
+    """Ten rows: with batch padding the mask is cut or continued with zeros to the rows without padding, without any it
+    goes to the op as it is (which refuses other lengths)."""
+    from areal_amd import engine_glue as G
+
+    class Reached(Exception):
+        pass
+
+    def op(hidden, weight, labels, temperature, token_mask, want_minmax, backward, grad_token_mask, kept_per_chunk, **kw):
+        seen.append(grad_token_mask.tolist())
+        raise Reached
+
+    seen = []
+    monkeypatch.setattr(G, "_lm_head_impl", op)
+    with pytest.raises(Reached):
+        G.compute_lm_head_loss_with(torch.zeros(10, 8), torch.zeros(16, 8), dict(rolled_input_ids=torch.zeros(10)), {}, pad,
+                                    None, lambda mb: 1.0, 1.0, grad_token_mask=torch.ones(length, dtype=torch.bool))
+    assert seen == [[bool(v) for v in want]]
