@@ -268,10 +268,11 @@ __global__ __launch_bounds__(kWave) void k_norm_finish(const double2* __restrict
 // ------------------------------------------------------------------------------------------------------------------
 // Normalization of a few thousand values in one launch (the five launches above cost 5 us each, whatever they do): one
 // workgroup per group (plus one for the rows past the last full group, or one in all), which forms the statistics it
-// needs from the whole input: the same two passes in float64, the sums of a segment in another order.  `scores`: the
+// needs from the whole input: the same two passes in float64, the sums of a segment in another order.  Bound by the latency
+// of its loads, a few dependent ones per 256 values and pass.  `scores`: the
 // values are first turned from rewards into scores, clip((x + bias) * scaling) (actor.py:166-170).
 // ------------------------------------------------------------------------------------------------------------------
-constexpr int64_t kSmallNorm = 8192;  // values; a workgroup reads them all when a level is "batch"
+constexpr int64_t kSmallNorm = 8192;  // values
 constexpr int kSmallThreads = 256;
 
 struct Scores {
@@ -397,29 +398,64 @@ __global__ __launch_bounds__(kSmallThreads) void k_norm_small(NormArgs a, Scores
     for (int64_t i = b + threadIdx.x; i < e; i += kSmallThreads) {
       const float xi = value(i), mi = weight(i);
       double mean = 0.0;
-      if (a.mean_level == 1) {
+      if (a.mean_level == 1)
         mean = level_mean(batch.x, batch.y, a.mean_leave1out != 0, a.mask != nullptr, xi, mi);
-      } else if (a.mean_level == 2 && i < a.n_groups * a.seg_elems && !(a.group_size == 1 && a.mean_leave1out)) {
-        double4 own = group;
-        if (i < gb || i >= ge) {  // a batch-wide deviation about group means: the sums of that element's group
-          own = none;
-          const int64_t first = i / a.seg_elems * a.seg_elems;
-          for (int64_t j = first; j < first + a.seg_elems; ++j) {
-            own.x += (double)value(j) * (double)weight(j);
-            own.y += (double)weight(j);
-          }
-        }
-        mean = (double)(float)level_mean(own.x, own.y, a.mean_leave1out != 0, a.mask != nullptr, xi, mi);
-      }
+      else if (a.mean_level == 2 && b < a.n_groups * a.seg_elems && !(a.group_size == 1 && a.mean_leave1out))
+        mean = (double)(float)level_mean(group.x, group.y, a.mean_leave1out != 0, a.mask != nullptr, xi, mi);
       const double d = (double)xi * (double)mi - mean * (double)mi;
       q += d * d;
     }
     return block_sum<double>(q, smem);
   };
-  if (a.std_level == 1) batch.z = squares(0, a.n);
+  // A batch-wide deviation about group means: `lanes` threads (one, or a wave, which then adds up its lanes) take a group
+  // at a time, its sums first and then its squares, so that every value is read twice whatever the groups are.
+  auto squares_by_group = [&](int lanes) {
+    double q = 0.0;
+    const int lane = threadIdx.x % lanes;
+    for (int64_t h = threadIdx.x / lanes; h < a.n_groups; h += kSmallThreads / lanes) {
+      const int64_t b = h * a.seg_elems, e = b + a.seg_elems;
+      double s = 0.0, f = 0.0;
+      for (int64_t i = b + lane; i < e; i += lanes) {
+        const double m = (double)weight(i);
+        s += (double)value(i) * m;
+        f += m;
+      }
+      if (lanes > 1) {
+        s = wave_sum(s);
+        f = wave_sum(f);
+      }
+      for (int64_t i = b + lane; i < e; i += lanes) {
+        const float xi = value(i), mi = weight(i);
+        double mean = 0.0;
+        if (!(a.group_size == 1 && a.mean_leave1out))
+          mean = (double)(float)level_mean(s, f, a.mean_leave1out != 0, a.mask != nullptr, xi, mi);
+        const double d = (double)xi * (double)mi - mean * (double)mi;
+        q += d * d;
+      }
+    }
+    return block_sum<double>(q, smem) + squares(a.n_groups * a.seg_elems, a.n);  // rows past the groups: about zero
+  };
+  if (a.std_level == 1)
+    batch.z = a.mean_level == 2 ? squares_by_group(a.seg_elems < kWave ? 1 : kWave) : squares(0, a.n);
   if (a.std_level == 2 && grouped) group.z = squares(gb, ge);
   for (int64_t i = gb + threadIdx.x; i < ge; i += kSmallThreads)
     out[i] = norm_element(a, batch, group, grouped, passthrough, value(i), weight(i));
+}
+
+// Whether one launch is the faster one: its time goes with the values that a workgroup reads, with less of a slope where
+// no mask is read with them (one launch / several, us).  Under a mask: batch-wide, 2 048 values 9 / 17, 4 096 14 / 17,
+// 6 144 20 / 18, 8 192 25 / 19; groups of 1 024 of 8 192 14 / 21, of 2 048 16 / 21, of 4 096 22 / 21; group means with a
+// batch-wide deviation, which read all values twice more at less of a rate, 2 048 in groups of 8 12 / 19, 3 072 20 / 20,
+// 4 096 23 / 22.  Without: groups of 4 096 12 / 19, of 6 144 17 / 20, of 8 192 20 / 21, and the last kind 4 096 in groups
+// of 8 16 / 22, 6 144 26 / 25.
+static bool one_launch(const NormArgs& a) {
+  if (a.n > kSmallNorm) return false;
+  const bool grouped = a.n_groups > 0 || a.mean_level == 2 || a.std_level == 2;
+  int64_t reads = grouped ? 2 * a.seg_elems : a.n;  // its own values for the output, and for the sums of its group
+  if (a.mean_level == 1 || a.std_level == 1 || a.mask) reads += a.n;
+  if (a.std_level == 1) reads += a.mean_level == 2 ? 3 * a.n : a.n;
+  if (a.std_level == 2) reads += a.seg_elems;
+  return reads <= (a.mask ? 15360 : 18432);
 }
 
 // without a normalisation: the scores themselves
@@ -927,7 +963,7 @@ extern "C" int aa_normalize(const float* x, const float* loss_mask, int64_t bs, 
   NormArgs a{x, loss_mask, bs * inner, gs * inner, n_groups, gs, p.mean_level, p.mean_leave1out, p.std_level,
              p.std_unbiased, p.eps};
   hipStream_t st = (hipStream_t)stream;
-  if (a.n <= kSmallNorm && out != x) {
+  if (out != x && one_launch(a)) {
     launch_norm_small(a, Scores{0, 0.f, 1.f, 0.f}, out, st);
     return launch_status();
   }

@@ -505,3 +505,44 @@ def test_reward_scores_with_a_bias_per_sequence(device):
         if reward_norm is not None:
             want = O.normalization(want, None, mean_level="group", std_level="group", group_size=3, eps=1e-5)
         assert torch.allclose(out["tot_rewards"][:, L - 2].cpu(), want, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("bs,inner,gs", [(512, 1, 16), (2049, 1, 8), (3000, 1, 63), (3000, 1, 64), (3001, 1, 65), (8, 1024, 4),
+                                         (8, 1023, 3), (4097, 1, 1), (8192, 1, 4096), (8192, 1, 2), (1, 5120, 1)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_normalization_of_a_few_thousand_values(device, bs, inner, gs, masked):
+    """Either side of the line between one launch and several, groups of less than, as many as and more than a wave, rows
+    past the last group; a group mean with a batch-wide deviation, where long groups used to be summed once per value
+    ([8, 1024] in groups of 4: 10.6 ms).  The float32 output has one rounding; 2e-6 of the largest, as above."""
+    from areal_amd import engine_glue
+
+    g = torch.Generator().manual_seed(bs + inner)
+    x = torch.randn(bs, inner, generator=g) * 2.0 + 0.5
+    mask = (torch.rand(bs, inner, generator=g) < 0.6).float() if masked else None
+    for mean, std, loo in (("group", "batch", False), ("group", "batch", True), ("batch", "batch", False), ("group", "group", False),
+                           (None, "batch", False), ("batch", "group", True)):
+        cfg = dict(mean_level=mean, std_level=std, mean_leave1out=loo, eps=1e-5, group_size=gs)
+        want = O.normalization(x, mask, **cfg)
+        norm = Normalization(NormConfig(**cfg))
+        got = norm(x.to(device), None if mask is None else mask.to(device)).cpu()
+        assert float((got - want).abs().max()) <= 2e-6 * (float(want.abs().max()) + 1.0), cfg
+        if inner == 1 and not masked:  # the same as reward scores: two positions, the scores land on the first
+            data = dict(attention_mask=torch.ones(bs, 2, dtype=torch.bool), loss_mask=torch.ones(bs, 2, dtype=torch.bool),
+                        logprobs=torch.zeros(bs, 2), rewards=x[:, 0].clone())
+            out = engine_glue.compute_advantages({k: v.to(device) for k, v in data.items()}, reward_norm=norm)
+            got = out["tot_rewards"][:, 0].cpu()
+            assert float((got - want[:, 0]).abs().max()) <= 2e-6 * (float(want.abs().max()) + 1.0), cfg
+
+
+def test_group_means_with_a_batch_deviation_are_linear_in_the_values(device):
+    """[8, 1024] in groups of 4 rows: some 20 us a call; summing a value's whole group per value took 10 ms."""
+    x, m = torch.randn(8, 1024, device=device), torch.ones(8, 1024, device=device)
+    norm = Normalization(NormConfig(mean_level="group", std_level="batch", group_size=4))
+    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    norm(x, m)
+    begin.record()
+    for _ in range(20):
+        norm(x, m)
+    end.record()
+    end.synchronize()
+    assert begin.elapsed_time(end) < 20 * 2.0
