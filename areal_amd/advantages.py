@@ -266,6 +266,7 @@ def masked_moments(values: Mapping[str, torch.Tensor], mask: torch.Tensor) -> di
         raise ValueError("at most 16 tensors per call")
     if values:
         _require_gpu(mask, "mask")
+        mask = (mask if mask.dtype is torch.bool else mask != 0).contiguous()  # once, not once per tensor
     return moments_table([(name, t, mask) for name, t in values.items()])
 
 

@@ -546,3 +546,21 @@ def test_group_means_with_a_batch_deviation_are_linear_in_the_values(device):
     end.record()
     end.synchronize()
     assert begin.elapsed_time(end) < 20 * 2.0
+
+
+def test_masked_moments_read_their_mask_once(device, monkeypatch):
+    """A mask that is not bool is converted once, not once per tensor."""
+    from areal_amd import advantages as A
+    from areal_amd import functional as F
+
+    n, calls = 777, []
+    g = torch.Generator().manual_seed(2)
+    mask = (torch.rand(n, generator=g) < 0.5).long()
+    values = {f"v{i}": torch.randn(n, generator=g) for i in range(5)}
+    plain = F._mask_u8
+    monkeypatch.setattr(F, "_mask_u8", lambda m: calls.append(m.dtype) or plain(m))
+    got = A.masked_moments({k: v.to(device) for k, v in values.items()}, mask.to(device))
+    assert len([c for c in calls if c is not torch.bool]) <= 1
+    for k, v in values.items():
+        assert float(got[k]["sum"]) == pytest.approx(float(v.double()[mask.bool()].sum()), abs=1e-4)
+        assert int(got[k]["count"]) == int(mask.sum())
