@@ -260,6 +260,9 @@ namespace aa {
 namespace logstats {
 
 constexpr int kMomentThreads = 256;
+// Of a tensor that one workgroup reduces by itself (aa_masked_moments, which has no scratch), when it is longer than
+// kMomentSlice: 16 tensors, 256 / 1 024 threads: 32 768 tokens 33 / 13 us, 262 144 244 / 71 us.
+constexpr int kMomentThreadsAlone = 1024;
 constexpr int kMomentSlice = 2048;
 constexpr int kMomentParts = 64;
 
@@ -280,8 +283,9 @@ struct MomentArgs {
   float* out;              // [tensors][cols]: sum, min, max, count(, mean)
 };
 
-__global__ __launch_bounds__(kMomentThreads) void k_moments(MomentArgs a) {
-  constexpr int kW = kMomentThreads / kWave;
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_moments(MomentArgs a) {
+  constexpr int kW = THREADS / kWave;
   __shared__ double sh_s[kW];
   __shared__ int sh_c[kW];
   __shared__ float sh_lo[kW], sh_hi[kW];
@@ -295,7 +299,7 @@ __global__ __launch_bounds__(kMomentThreads) void k_moments(MomentArgs a) {
   int c = 0;
   float lo = __builtin_inff(), hi = -__builtin_inff();
 #pragma unroll 4
-  for (int64_t i = b + threadIdx.x; i < e; i += kMomentThreads) {
+  for (int64_t i = b + threadIdx.x; i < e; i += THREADS) {
     const bool on = mask ? mask[i] != 0 : true;
     const float x = bytes ? (float)((const uint8_t*)a.v[k])[i] : ((const float*)a.v[k])[i];
     if (on) {
@@ -401,7 +405,8 @@ extern "C" int aa_moments_table(const void* const* values, const uint8_t* const*
   a.partial = (MomentPartial*)scratch;
   a.work = (StepWork*)work;
   a.out = out;
-  hipLaunchKernelGGL(k_moments, dim3((unsigned)(n_tensors * a.parts)), dim3(kMomentThreads), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(k_moments<kMomentThreads>, dim3((unsigned)(n_tensors * a.parts)), dim3(kMomentThreads), 0,
+                     (hipStream_t)stream, a);
   return launch_status();
 }
 
@@ -420,6 +425,10 @@ extern "C" int aa_masked_moments(const float* const* values, int n_tensors, cons
   a.parts = 1;
   a.cols = 4;
   a.out = out;
-  hipLaunchKernelGGL(k_moments, dim3((unsigned)n_tensors), dim3(kMomentThreads), 0, (hipStream_t)stream, a);
+  if (n > kMomentSlice)
+    hipLaunchKernelGGL(k_moments<kMomentThreadsAlone>, dim3((unsigned)n_tensors), dim3(kMomentThreadsAlone), 0,
+                       (hipStream_t)stream, a);
+  else
+    hipLaunchKernelGGL(k_moments<kMomentThreads>, dim3((unsigned)n_tensors), dim3(kMomentThreads), 0, (hipStream_t)stream, a);
   return launch_status();
 }
