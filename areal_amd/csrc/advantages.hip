@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 constexpr int kRowsAhead = 8;  // positions of a thread whose inputs are on their way together
 
 // Per row: sums for the normalisation.  F = sum m, S = sum x m; A = sum m^2, B = sum m^2 (x - c), C = sum m^2 (x - c)^2
-// about a centre c of the row's own (its mean in the first super-block), from which the sum of squares about any mean
+// about a centre c of the row's own (its mean in the first super-block with a token that counts), from which the sum of squares about any mean
 // follows without cancellation.
 struct RowSums {
   double F, S, A, B, C, c;
@@ -701,15 +701,19 @@ __global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
     }
     F += f_here;
     S += s_here;
-    if (a.sums && first) {  // the centre of the row's squares: its mean so far
+    if (a.sums && first) {
+      // the centre of the row's squares: its mean so far, as soon as a token counts (a masked super-block adds nothing to
+      // A, B and C, whatever the centre)
       const double f = block_sum<double>(F, smem), s = block_sum<double>(S, smem);
-      c = f != 0.0 ? s / f : 0.0;
-      if (!isfinite(c)) c = 0.0;  // an infinity among the advantages: its square is infinite about any finite centre
-      first = false;
-      if (tid == 0) {  // position L - 1
-        const double mm = (double)m_end * (double)m_end;
-        B = -mm * c;
-        C = mm * c * c;
+      if (f != 0.0) {
+        c = s / f;
+        if (!isfinite(c)) c = 0.0;  // an infinity among the advantages: its square is infinite about any finite centre
+        first = false;
+        if (tid == 0) {  // position L - 1
+          const double mm = (double)m_end * (double)m_end;
+          B -= mm * c;
+          C += mm * c * c;
+        }
       }
     }
     __syncthreads();

@@ -564,3 +564,27 @@ def test_masked_moments_read_their_mask_once(device, monkeypatch):
     for k, v in values.items():
         assert float(got[k]["sum"]) == pytest.approx(float(v.double()[mask.bool()].sum()), abs=1e-4)
         assert int(got[k]["count"]) == int(mask.sum())
+
+
+def test_advantages_of_rows_with_a_long_masked_tail(device):
+    """Rows whose last super-block (4096 positions) has no token with a loss: the squares of such a row are taken about
+    the mean of the tokens that count all the same, so a mean a million times the spread costs no digits."""
+    from areal_amd import engine_glue
+
+    bs, L = 6, 9000
+    g = torch.Generator().manual_seed(4)
+    mask = torch.zeros(bs, L, dtype=torch.bool)
+    mask[:, 1:3001] = True
+    data = dict(attention_mask=torch.ones(bs, L, dtype=torch.bool), loss_mask=mask, logprobs=torch.zeros(bs, L),
+                values=-4096.0 - 2.0 ** -8 * torch.rand(bs, L, generator=g), rewards=torch.zeros(bs))
+    for levels in (("batch", "batch"), ("group", "group")):
+        norm = Normalization(NormConfig(mean_level=levels[0], std_level=levels[1], group_size=3, eps=0.0))
+
+        def run(adv_norm):
+            d = {k: v.clone().to(device) for k, v in data.items()}
+            return engine_glue.compute_advantages(d, adv_norm=adv_norm, discount=0.0, gae_lambda=0.0, use_decoupled_loss=True)
+
+        got, want = run(norm)["advantages"], run(lambda x, m: norm(x, m))["advantages"]
+        # the float64 rounding of a shifted sum of squares would be 2^-53 (mean / spread)^2, some 1e-4; what remains is
+        # that of the sums, then one rounding to float32
+        assert float((got - want).abs().max()) <= 4 * 2.0 ** -23 * float(want.abs().max())
