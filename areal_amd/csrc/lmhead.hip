@@ -973,9 +973,11 @@ static Workspace plan(int64_t T, int64_t H, int64_t V, bool external_panel = fal
   w.off_panel = off;   off += external_panel ? 0 : up(w.chunk * w.panel_ld * 2);
   w.off_hc = off;      off += up(w.chunk * H * 2);
   w.off_dw = off;      off += T > w.chunk ? up(V * H * 4) : 0;
-  // kFewSplits parts over all rows of a chunk, or more parts of a product whose parts all run in one round
-  const int64_t few = kFewSplits * w.chunk * H, one_round = (int64_t)compute_units() * BM * BN;
-  w.off_dhp = off;     off += up((few > one_round ? few : one_round) * 4);
+  // kFewSplits parts over all rows of a chunk, or up to kMaxSplits parts of a product whose parts all run in one round
+  const int64_t few = kFewSplits * w.chunk * H, most = kMaxSplits * w.chunk * H;
+  int64_t planes = (int64_t)compute_units() * BM * BN;  // one round
+  planes = planes < few ? few : (planes > most ? most : planes);
+  w.off_dhp = off;     off += up(planes * 4);
   w.bytes = off;
   return w;
 }

@@ -972,3 +972,12 @@ def test_any_loss_function_on_the_hidden_states(device, variant, backward):
     z = engine_glue.compute_lm_head_loss_with(h, w, model_inputs, mb_d, pad, loss_fn, weight_fn, total_w)
     z.backward()
     assert float(z.detach()) == 0.0 and float(h.grad.float().abs().max()) == 0.0
+
+
+def test_workspace_of_a_small_step_follows_its_size(device):
+    """The fp32 planes of d(hidden) take up to 32 parts of the rows of a chunk, not one round of tiles of the whole chip
+    (64 MB) whatever the size: 256 tokens x 64 hidden entries, 2 MB."""
+    lib = _native.load()
+    chunk, H, V = 256, 64, 1024
+    partials, panel, rows, vectors = 4 * 2 * (V // 256) * chunk * 4, chunk * V * 2, chunk * H * 2, 1 << 16
+    assert lib.aa_lmhead_workspace_bytes(chunk, H, V) <= partials + panel + rows + vectors + 32 * chunk * H * 4
