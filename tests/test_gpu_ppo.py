@@ -238,3 +238,94 @@ def test_step_launches_at_the_edges_of_their_slices(device, n, rs):
             assert stat["filtered_fraction"] == want["filtered_fraction"]
         kept = mask if not rs else want["behave_mask"]
         assert float(x.grad[~kept.to(device)].abs().sum()) == 0.0
+
+
+@pytest.mark.parametrize("n,covered", [(1, 1), (300, 300), (5000, 4321)])
+@pytest.mark.parametrize("rs", [None, dict(level="token", upper=1.3), dict(level="sequence", upper=1.02)])
+@pytest.mark.parametrize("level", ["token", "sequence"])
+def test_separate_entry_points_of_the_c_abi_agree_with_the_step(device, n, covered, rs, level):
+    """aa_rejection_sampling / aa_count_nonzero_u8, aa_ppo_loss, aa_ppo_stat_outputs and aa_masked_sum against the one call
+    that does the same, and its first launch alone (counts_only).  The same expressions: whole numbers and masks exactly,
+    floats to 4 ulps (a product or quotient taken in another order); the loss is one fp64 sum in two orders."""
+    import ctypes
+
+    from areal_amd import _native as N
+    from areal_amd import functional as F
+
+    lib = N.load()
+    g = torch.Generator().manual_seed(n)
+    prox = -2 + 0.5 * torch.randn(n, generator=g)
+    old, lp, adv = prox + 0.3 * torch.randn(n, generator=g), prox + 0.3 * torch.randn(n, generator=g), torch.randn(n, generator=g)
+    mask = torch.rand(n, generator=g) < 0.7
+    mask[-1] = True
+    cu = torch.tensor([0] + sorted({covered // 3, covered // 2, covered} - {0}), dtype=torch.int32)
+    lp, prox, old, adv, mask, cu = _to(device, lp, prox, old, adv, mask, cu)
+    B, seq = cu.numel() - 1, level == "sequence"
+    cfg = None if rs is None else RejectionSamplingConfig(action="mask", metric="ratio", **rs)
+    params = F._ppo_params(0.2, 0.28, 3.0, cfg is not None)
+    P, st = (lambda t: None if t is None else t.data_ptr()), torch.cuda.current_stream().cuda_stream
+
+    def new_step():
+        return F._Step(device, n, n, mask, prox, old, adv, params, cfg, cu, B)
+
+    step, g_step = new_step(), torch.empty_like(lp)
+    N.check(lib.aa_ppo_loss_step(step.struct, P(lp), int(seq), 0, P(g_step), st), "aa_ppo_loss_step")
+    counted = new_step()
+    N.check(lib.aa_ppo_loss_step(counted.struct, None, 0, 1, None, st), "aa_ppo_loss_step")
+    three = lambda s: s.floats.view(torch.int32)[9, :3].tolist()
+
+    floats = lambda k: [torch.empty(n, device=device) for _ in range(k)]
+    m8, w, mask_eff, counts = mask.view(torch.uint8), None, mask.view(torch.uint8), torch.empty(3, dtype=torch.int32, device=device)
+    if cfg is None:
+        N.check(lib.aa_count_nonzero_u8(P(m8), n, P(counts), st), "aa_count_nonzero_u8")
+        assert three(step)[0] == three(counted)[0] == int(counts[0])
+    else:
+        mask_eff, w = torch.empty_like(m8), torch.empty(n, device=device)
+        N.check(lib.aa_rejection_sampling(P(prox), P(old), P(m8), n, P(cu), B, N.RS_LEVEL[cfg.level], N.RS_ACTION[cfg.action],
+                                          N.RS_METRIC[cfg.metric], N.RS_AGG[cfg.agg], float(cfg.upper), 0.0, 0, P(mask_eff),
+                                          P(w), P(counts), st), "aa_rejection_sampling")
+        assert three(step) == three(counted) == counts.tolist()
+        outside = int(mask[covered:].sum()) if cfg.level == "sequence" else 0
+        assert counts.tolist()[0] + outside == int(mask.sum()) and counts.tolist()[2] == outside
+        for s in (step, counted):
+            assert torch.equal(s.bools[1, :n], mask_eff.bool()) and torch.equal(s.floats[8, :n], w)
+    stat_loss, ratio, g_logp, approx_kl, behave_kl = floats(5)
+    flags, clip, dual, behave = (torch.empty(n, dtype=torch.uint8, device=device) for _ in range(4))
+    N.check(lib.aa_ppo_loss(P(lp), P(prox), P(adv), P(mask_eff), P(w), n, P(cu), B, int(seq), ctypes.byref(params), P(counts),
+                            P(stat_loss), P(ratio), P(flags), P(g_logp), st), "aa_ppo_loss")
+    N.check(lib.aa_ppo_stat_outputs(P(lp), P(prox), P(old), P(flags), P(w), P(mask_eff), n, P(approx_kl), P(clip), P(dual),
+                                    P(behave) if cfg else None, P(behave_kl) if cfg else None, st), "aa_ppo_stat_outputs")
+    loss = torch.empty((), device=device)
+    N.check(lib.aa_masked_sum(P(stat_loss), P(mask_eff), n, P(counts), None, P(loss), st), "aa_masked_sum")
+    stat = step.stats(rows=False)
+    for got, want in ((clip, stat["clip_mask"]), (dual, stat["dual_clip_mask"])) + (((behave, stat["behave_mask"]),) if cfg else ()):
+        assert torch.equal(got.bool(), want)
+    ulps = 4 * 2.0 ** -23
+    for got, want in ((stat_loss, stat["loss"]), (ratio, stat["importance_weight"]), (g_logp, g_step), (approx_kl, stat["approx_kl"]),
+                      *(((behave_kl, stat["behave_approx_kl"]),) if cfg else ())):
+        assert torch.allclose(got, want, rtol=ulps, atol=0.0)
+    assert abs(float(loss) - float(step.loss)) <= ulps * float((stat_loss.abs() * mask_eff).sum()) / max(int(counts[0]), 1) + 1e-30
+
+
+@pytest.mark.parametrize("n", [1, 512, 513, 140001])
+@pytest.mark.parametrize("methods,with_errors", [(0, 0), (1, 0), (7, 1)])
+def test_logging_stats_with_and_without_the_mean(device, n, methods, with_errors):
+    """aa_logging_stats (a launch to fold the slices) against aa_logging_stats_table (the last workgroup folds them): the
+    same slices in the same order, so the same bits; the mean is the quotient."""
+    from areal_amd import _native as N
+    from areal_amd import functional as F
+
+    lib = N.load()
+    g = torch.Generator().manual_seed(n)
+    old, lp, gt = (-torch.rand(n, generator=g) for _ in range(3))
+    versions, mask = torch.randint(-1, 6, (n,), generator=g, dtype=torch.int32), torch.rand(n, generator=g) < 0.7
+    old, lp, gt, versions, mask = _to(device, old, lp, gt, versions, mask)
+    args = [t.data_ptr() for t in (old, lp, gt, versions, mask)] + [n, 6, methods, with_errors]
+    scratch, st = torch.empty(lib.aa_logging_stats_scratch_bytes(n), dtype=torch.uint8, device=device), torch.cuda.current_stream().cuda_stream
+    four, five = torch.empty(36, 4, device=device), torch.empty(36, 5, device=device)
+    N.check(lib.aa_logging_stats(*args, four.data_ptr(), scratch.data_ptr(), scratch.numel(), st), "aa_logging_stats")
+    N.check(lib.aa_logging_stats_table(*args, five.data_ptr(), scratch.data_ptr(), scratch.numel(), F._work_words(device).data_ptr(), st),
+            "aa_logging_stats_table")
+    assert torch.equal(four, five[:, :4])
+    assert torch.allclose(five[:, 4], four[:, 0] / four[:, 3], rtol=2.0 ** -23, atol=0.0, equal_nan=True)
+    assert int(four[0, 3]) == int(mask.sum())
