@@ -197,17 +197,12 @@ __device__ __forceinline__ double level_mean(double S, double F, bool loo, bool 
   return F == 0.0 ? 0.0 : S / F;
 }
 
-// The mean the reference subtracts from element i.  `as_float`: the reference keeps group-level (and absent) means
-// in a tensor of the dtype of x, batch-level means in float64.
-__device__ __forceinline__ double mean_at(const NormArgs& a, const double4* stats, int64_t i, float xi, float mi,
-                                          bool& as_float) {
-  as_float = true;
+// The mean the reference subtracts from element i (group-level means are kept in a tensor of the dtype of x, batch-level
+// means in float64).
+__device__ __forceinline__ double mean_at(const NormArgs& a, const double4* stats, int64_t i, float xi, float mi) {
   if (a.mean_level == 0) return 0.0;
   const bool has_mask = a.mask != nullptr;
-  if (a.mean_level == 1) {
-    as_float = false;
-    return level_mean(stats[0].x, stats[0].y, a.mean_leave1out != 0, has_mask, xi, mi);
-  }
+  if (a.mean_level == 1) return level_mean(stats[0].x, stats[0].y, a.mean_leave1out != 0, has_mask, xi, mi);
   const int64_t g = i / a.seg_elems;
   if (g >= a.n_groups) return 0.0;
   if (a.group_size == 1 && a.mean_leave1out) return 0.0;
@@ -235,8 +230,7 @@ __global__ __launch_bounds__(kThreads) void k_norm_partial(NormArgs a, const dou
       s += (double)xi * (double)mi;
       f += (double)mi;
     } else {
-      bool as_float;
-      const double mean = mean_at(a, stats, i, xi, mi, as_float);
+      const double mean = mean_at(a, stats, i, xi, mi);
       const double d = (double)xi * (double)mi - mean * (double)mi;  // x_masked - mean * mask
       s += d * d;
     }

@@ -666,12 +666,6 @@ class _PpoLoss(torch.autograd.Function):
         return g_logp * g_loss, None, None
 
 
-def _flag_bits(flags: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    """(clip_mask, dual_clip_mask) as bool tensors from the kernels' flag bytes (bit 0, bit 1): one launch each, the
-    0 / 1 bytes reinterpreted as bool."""
-    return torch.bitwise_and(flags, 1).view(torch.bool), torch.bitwise_right_shift(flags, 1).view(torch.bool)
-
-
 def _count_nonzero(mask_u8: torch.Tensor) -> torch.Tensor:
     lib = N.load()
     dev = mask_u8.device

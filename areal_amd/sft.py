@@ -5,7 +5,6 @@ with the log-prob op (one pass over the logits that also writes their gradient) 
 """
 from __future__ import annotations
 
-
 import torch
 
 from . import _native as N
