@@ -498,9 +498,11 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // The advantage pipeline of a padded batch (PPOActor._compute_advantages, actor.py:172-236) in one pass per row: mask and
 // log-probs rolled and masked, KL-regularised rewards, the GAE scan, and the sums that the normalisation of the
 // advantages needs.  One workgroup per row, super-blocks of 4096 positions from the end as in k_gae: a super-block's
-// inputs are read once, what the scan needs of them stays in LDS.  Bound by memory: 26 bytes in and 24 out per token (30
-// in with values); the separate launches (rolls, products, KL, GAE, two passes of sums; thirteen of them) moved about
-// three times as much.
+// inputs are read once, what the scan needs of them stays in LDS.  With byte masks and a reference policy 10 bytes in per
+// token (14 with values) and 28 out (24 without a reference policy): 88 MB at 512 x 4096 with values, 14 us at the rate of
+// an even mix of reads and writes.  It takes 36 us, bound by the chain of a row (count of the attention bytes, loads, scan,
+// sums) on one-element memory instructions, some ten a token.  The separate launches (rolls, products, KL, GAE, two passes
+// of sums; thirteen of them) moved about three times as much.
 // The sums of a row are published past the caches for the last workgroup to fold: with a __threadfence() in every
 // workgroup (a write-back of its XCD's L2, full of the outputs' lines) 512 x 4096 took 40.2 us, so 35.7.
 // Also measured, slower, at 512 x 4096 per pass (46 us so): 512 threads with chunks of 8 57 us; a chunk held in registers

@@ -210,6 +210,16 @@ __device__ __forceinline__ int wave_sum(int v) {
 // workgroup.  That bounded the end of the fused logits kernel, whose L2 is full of gradient lines while 256 or 512
 // workgroups finish: us a launch with the fence / so: 6048 x 50257 f16: 253/225, 8320 x 32768 bf16: 212/186; per pass
 // 4718 x 151936: 523/505.  k_step_finish behind it: 10.3/6.8 us.
+//
+// All accesses are relaxed: the order is that of the instructions, which on gfx950 is enough (agent-scope accesses of
+// global memory bypass the L1 and the L2s of the XCDs, and vmcnt counts stores and atomics as well as loads), and not
+// that of the memory model.  It is part of the contract, so a caller
+//   - writes what it leaves with publish() only (or with atomics), and reads it with published() only: a plain load may
+//     find a line that its caches hold from before;
+//   - calls last_to_finish() from the wave that published, or, when several waves did, from behind a barrier that each of
+//     them reached after a wait_published() of its own;
+//   - puts a __syncthreads() between the call and the first published() of any other thread.  It hands over the answer and
+//     keeps those loads behind the counter; the calling thread's own loads wait for the answer that they depend on.
 template <typename T>
 __device__ __forceinline__ void publish(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -693,7 +693,9 @@ def compute_lm_head_loss_with(hidden: torch.Tensor, weight: torch.Tensor, model_
     ``backward="carry"`` (default): the op keeps the bf16 probability ratios of the tokens named by ``grad_token_mask``
     (default: ``mb_input["loss_mask"]``; tokens outside it get no gradient) from its forward to its backward, which is
     then two GEMMs instead of three; ``kept_per_chunk``: their number per chunk of ``lm_head_chunk_tokens()`` tokens,
-    if the host knows it (else it is read back).  ``"recompute"`` keeps nothing and forms the logits again."""
+    if the host knows it.  Otherwise the device counts them, and the op keeps room for every token, up to
+    ``COUNT_ON_DEVICE_BYTES`` (2 GiB) of rows; past that the counts are read back and the rows sized by them.
+    ``"recompute"`` keeps nothing and forms the logits again."""
     if hidden.ndim == 3 and hidden.shape[0] == 1:
         hidden = hidden.squeeze(0)
     local_weight = loss_weight_fn(mb_input)
