@@ -457,7 +457,7 @@ __global__ __launch_bounds__(1024) void k_token_loss(const float* __restrict__ p
     } else {
       fn = (float)(n < 1 ? 1 : n);
     }
-    const float gscale = scale_of(a.scale, a.n_valid);
+    const float gscale = scale_of(a.scale, n);
     const bool on = a.mask_eff[t] != 0;
     if (a.P.loss_kind == AA_LOSS_NLL) {
       a.stat_loss[t] = on ? -lp : 0.f;
@@ -1682,7 +1682,7 @@ extern "C" int aa_lmhead_ppo_step(const aa_ppo_step* step, const void* hidden, c
   if (st != AA_OK) return st;
   const aa_ppo_params params = step_params(p);
   st = lmhead_ppo(hidden, weight, p.T, H, V, labels, inv_temperature, p.T_active, p.prox_logp, p.adv, step_mask(p),
-                  params.has_behave_weight ? p.behave_w : nullptr, &params, p.counts, p.scale, kept_per_chunk, backward_mode, p.logp,
+                  params.has_behave_weight ? p.behave_w : nullptr, &params, p.counts, step_scale(p), kept_per_chunk, backward_mode, p.logp,
                   p.entropy, p.stat_loss, p.ratio, p.flags, p.vmax, p.vmin, d_hidden, d_weight, d_weight_dtype, workspace,
                   workspace_bytes, stream);
   return st == AA_OK ? step_finish(p, stream) : st;

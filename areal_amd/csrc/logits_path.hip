@@ -460,7 +460,7 @@ __device__ __forceinline__ uint32_t load_u16_uniform(const void* __restrict__ ro
 // d(surrogate)/d(logp) and d(scaled loss)/d(logp).
 __device__ __forceinline__ void load_loss_scale(const FusedTokenArgs& a, float& fn, float& gscale) {
   int n = *a.n_valid;
-  gscale = scale_of(a.scale, a.n_valid);
+  gscale = scale_of(a.scale, n);
   if (a.P.loss_kind == AA_LOSS_NLL) {
     fn = (float)n + 1e-5f;  // the supervised loss divides by 1e-5 + count (areal/trainer/sft/lm_engine.py:96)
   } else {
@@ -1842,7 +1842,7 @@ extern "C" int aa_logits_ppo_step(const aa_ppo_step* step, const void* logits, i
   if (st != AA_OK) return st;
   const aa_ppo_params params = step_params(p);
   st = launch_fused(logits, dtype, p.T, V, row_stride, labels, inv_temperature, p.T_active, p.prox_logp, p.adv,
-                    step_mask(p), params.has_behave_weight ? p.behave_w : nullptr, &params, p.counts, p.scale, p.logp, p.entropy,
+                    step_mask(p), params.has_behave_weight ? p.behave_w : nullptr, &params, p.counts, step_scale(p), p.logp, p.entropy,
                     p.vmax, p.vmin, p.stat_loss, p.ratio, p.flags, dlogits, (int32_t*)p.work, stream);
   return st == AA_OK ? step_finish(p, stream) : st;
 }

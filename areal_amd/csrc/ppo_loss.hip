@@ -103,6 +103,8 @@ struct Counts {
   int32_t* host;
   int32_t tag;
   const int32_t* cu_end;  // nullable: one more number for the host, the end of the last segment
+  aa_loss_scale scale;    // see step_scale
+  float* factor;          // nullable
 };
 
 __device__ __forceinline__ void host_store(int32_t* p, int32_t v, int order_release) {
@@ -131,6 +133,7 @@ __device__ __forceinline__ void count_up(const Counts& c, int total, int hit, in
   c.counts[0] = total;
   c.counts[1] = hit;
   c.counts[2] = outside;
+  if (c.factor) *c.factor = scale_of(c.scale, total + outside);
   if (c.host) {
     host_store(c.host + 0, total, 0);
     host_store(c.host + 1, hit, 0);
@@ -530,7 +533,7 @@ __global__ __launch_bounds__(kFinishThreads) void k_step_finish(FinishArgs a) {
   }
   if (threadIdx.x == 0) {
     a.work->finished = 0;
-    a.loss[0] = (float)acc / fn * scale_of(a.scale, a.n_valid);
+    a.loss[0] = (float)acc / fn * scale_of(a.scale, nv);
   }
 }
 
@@ -728,7 +731,7 @@ extern "C" int aa_rejection_sampling(const float* prox_logp, const float* old_lo
   RsCfg c{level, action, metric, agg, has_lower, upper, lower};
   hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, counts, 3);
   if (n == 0) return launch_status();
-  const Counts cleared{counts, nullptr, nullptr, 0, nullptr};
+  const Counts cleared{counts, nullptr, nullptr, 0, nullptr, {}, nullptr};
   if (level == AA_RS_LEVEL_TOKEN) {
     hipLaunchKernelGGL(k_rs_token, dim3(grid_for(n)), dim3(256), 0, st, prox_logp, old_logp, mask_in, n, c, mask_out,
                        behave_w, cleared);
@@ -780,7 +783,8 @@ int step_prepare(const aa_ppo_step& p, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   const int64_t n = p.T_active;
   const Counts counts{p.counts, (StepWork*)p.work, p.host_counts, p.host_tag,
-                      p.cu_seqlens ? p.cu_seqlens + p.n_segments : nullptr};
+                      p.cu_seqlens ? p.cu_seqlens + p.n_segments : nullptr, p.scale,
+                      scale_ahead(p) ? &((StepWork*)p.work)->factor : nullptr};
   const aa_rs_params& r = p.rs;
   if (!r.enabled || n == 0) {
     int64_t blocks = (n + 4095) / 4096;  // 16 mask bytes per thread
@@ -823,7 +827,7 @@ static int launch_finish(const aa_ppo_step& p, const float* logp, float* g_logp,
   a.n_valid = p.counts;
   a.loss = p.loss;
   a.work = (StepWork*)p.work;
-  a.scale = p.scale;
+  a.scale = step_scale(p);
   a.n = p.T_active;
   int64_t blocks = (a.n + kFinishSlice - 1) / kFinishSlice;
   blocks = blocks < 1 ? 1 : (blocks > kFinishBlocks ? kFinishBlocks : blocks);

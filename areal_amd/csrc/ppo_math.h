@@ -17,12 +17,11 @@ struct Surrogate {
   bool dual;       // pg_loss3 < max(pg_loss1, pg_loss2)
 };
 
-// The factor of a loss and its gradient; counts: those of the step, counts[0] alone without per_valid_token (float32
-// throughout, in the order of the tensor expression local_weight / total_loss_weight * multiplier).  The weight is the
-// count of the whole loss mask, with the tokens that no sequence covers.
-__device__ __forceinline__ float scale_of(const aa_loss_scale& s, const int32_t* counts) {
+// The factor of a loss and its gradient; n_valid: the non-zero entries of the loss mask (float32 throughout, in the order
+// of the tensor expression local_weight / total_loss_weight * multiplier).
+__device__ __forceinline__ float scale_of(const aa_loss_scale& s, int n_valid) {
   float f = s.value;
-  if (s.per_valid_token) f = (float)(counts[0] + counts[2]) / (s.total ? *s.total : s.total_value) * f;
+  if (s.per_valid_token) f = (float)n_valid / (s.total ? *s.total : s.total_value) * f;
   if (s.factor) f *= *s.factor;
   return f;
 }

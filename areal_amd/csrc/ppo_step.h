@@ -16,7 +16,8 @@ struct StepWork {
   int32_t finished;
   int32_t logged;
   int32_t outside;
-  int32_t pad[8];
+  float factor;  // see step_scale (written before it is read, not left zero)
+  int32_t pad[7];
   int32_t moments[kTableTensors];
   double partial[kFinishBlocks];
 };
@@ -34,6 +35,16 @@ inline aa_ppo_params step_params(const aa_ppo_step& p) {
   aa_ppo_params q = p.params;
   if (p.rs.enabled) q.has_behave_weight = 1;
   return q;
+}
+
+// The scale as the loss kernels take it.  The weight of a micro-batch is the count of its whole loss mask; with
+// sequence-level rejection sampling counts[0] is that of the tokens inside the sequences, and the launch that counts them
+// forms the factor from all of them.
+inline bool scale_ahead(const aa_ppo_step& p) {
+  return p.scale.per_valid_token && p.rs.enabled && p.rs.level == AA_RS_LEVEL_SEQUENCE && p.T_active > 0;
+}
+inline aa_loss_scale step_scale(const aa_ppo_step& p) {
+  return scale_ahead(p) ? aa_loss_scale{&((StepWork*)p.work)->factor, nullptr, 1.f, 1.f, 0} : p.scale;
 }
 
 // the mask the loss is summed under

@@ -1453,7 +1453,7 @@ def fused_lm_head_ppo_loss(
             if rs.action != "mask":
                 mask_eff = m8
         else:
-            n_valid = torch.nn.functional.pad(_count_nonzero(m8), (0, 2))  # the three counts of a step
+            n_valid = _count_nonzero(m8)
         # only the tokens with a mask go through the lm_head: gather them (autograd scatters d(hidden) back), run the
         # step on the closed-up batch with an all-true mask, and put the per-token results back at their tokens
         idx = mask_eff.nonzero().squeeze(-1)

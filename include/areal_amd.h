@@ -86,7 +86,8 @@ typedef struct {
 /* The factor a loss and its gradient are multiplied by:
  *   value, times *factor when factor is given, and, with per_valid_token != 0,
  *   times (number of non-zero entries of the loss mask, counts[0] + counts[2]
- *   of the step) / (*total or, when total is NULL, total_value): the engine's local_weight /
+ *   of the step; counts[0] when the counts are given) / (*total or, when total
+ *   is NULL, total_value): the engine's local_weight /
  *   total_loss_weight * multiplier (fsdp_engine.py:2045) without a launch or a
  *   copy of its own. */
 typedef struct {
@@ -98,7 +99,8 @@ typedef struct {
 } aa_loss_scale;
 
 /* Bytes of the work buffer of a step: zero before the first launch that uses
- * it, left zero by every launch; one per stream. */
+ * it, left ready for the next one (zero but for a word that is written before
+ * it is read) by every launch; one per stream. */
 #define AA_STEP_WORK_BYTES 4096
 
 /* The per-token side of one micro-batch's loss, for the aa_*_step entry
