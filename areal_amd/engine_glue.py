@@ -66,10 +66,11 @@ def _no_tokens(scale: _PerValidToken, loss_mask: torch.Tensor):
 
 # A forward of at most this much work is queued before the host knows the weight of the micro-batch, so that the device
 # has work while the host waits; what it computed is dropped when the weight is zero.  About 1 ms of forward at 6.4 TB/s
-# and 1.2 PFLOP/s: asking first costs 15 to 80 us of a pass (4 096 x 151 936 bf16 logits 672 against 650 us, PPO step
-# 511 / 437; from hidden states 1 900 x 1 024 1 751 / 1 738, PPO step 1 608 / 1 532), 1 to 3 % of the passes past this
-# line (2 048 x 2 048 2 965 / 2 918, PPO 2 760 / 2 690; 4 096 x 4 096 9 980 / 9 890), and a micro-batch without a token
-# never pays more than this for a result that nobody reads.
+# and 1.2 PFLOP/s: asking first costs 10 to 50 us of a pass (us, forward and backward, first / ahead: 256 x 151 936 bf16
+# logits PPO 158 / 131, 4 096 any loss 680 / 650, PPO 486 / 437, supervised 511 / 462; from hidden states of 1 024 entries
+# 1 900 tokens any loss 1 700 / 1 660, PPO 1 550 / 1 498), 1 to 2 % of the passes past this line (16 384 x 151 936 PPO
+# 1 672 / 1 625, 2 048 x 2 048 2 705 / 2 660, 4 096 x 4 096 9 520 / 9 480), and a micro-batch without a token never pays
+# more than this for a result that nobody reads.
 RUN_AHEAD_BYTES = 6_400_000_000
 RUN_AHEAD_FLOPS = 1_200_000_000_000
 
@@ -127,6 +128,7 @@ def compute_logprobs_and_loss(
     ``logits.mean() * 0`` like the reference (fsdp_engine.py:1988-1989).  ``inplace_backward``: the gradient is
     written over the logits, see ``fused_logprobs_ppo_loss``.  ``use_sapo_loss`` (token level, fused): the SAPO gate in
     place of the clip, on the behaviour log-probs (actor.py:448-462: SAPO takes ``old_logp``, no proximal policy).
+    The tensors of the stat dict share memory: one that is kept for longer keeps all of them, 45 bytes a token.
     """
     loss_mask = mb_input["loss_mask"].bool()
     old_logp = mb_input["logprobs"]

@@ -572,7 +572,8 @@ def _rs_struct(cfg) -> N.RsParams:
 class _Step:
     """One micro-batch's per-token arrays and the ``aa_ppo_step`` that describes them to the library.
 
-    The outputs are rows of two arrays (float32 and bytes), so that a step allocates three times and not sixteen."""
+    The outputs are rows of two arrays (float32 and bytes), so that a step allocates three times and not sixteen; an entry
+    of the stat dict that is kept keeps all of them (45 bytes a token, a clone its own four)."""
 
     # floats: logp, entropy, vmax, vmin, stat_loss, ratio, approx_kl, behave_kl, behave_w, (counts)
     # bools: (flags), mask_out, clip_mask, dual_clip_mask, behave_mask
