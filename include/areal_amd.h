@@ -773,8 +773,9 @@ int aa_moments_table(const void* const* values, const uint8_t* const* masks,
  * C (softmax partials and smallest logit per 128 vocabulary rows and token), 2 * C * H (the hidden rows of the tokens with a
  * gradient, closed up), 16 * C * H (four fp32 planes of d_hidden rows: the
  * product that forms them has few tiles and is cut along the vocabulary into
- * up to four parts when that fills the chip better), plus 4 * H * V (an fp32
- * accumulator for a bf16 d_weight) when there is more than one chunk.  No
+ * parts when that fills the chip better; up to 32 planes, 128 * C * H, while
+ * they stay below one round of tiles of the chip, 64 MB), plus 4 * H * V (an
+ * fp32 accumulator for a bf16 d_weight) when there is more than one chunk.  No
  * transposed copy of anything is made.  Returns -1 for sizes the path does
  * not take. */
 int64_t aa_lmhead_workspace_bytes(int64_t T, int64_t H, int64_t V);
