@@ -784,7 +784,7 @@ int step_prepare(const aa_ppo_step& p, void* stream) {
   const int64_t n = p.T_active;
   const Counts counts{p.counts, (StepWork*)p.work, p.host_counts, p.host_tag,
                       p.cu_seqlens ? p.cu_seqlens + p.n_segments : nullptr, p.scale,
-                      scale_ahead(p) ? &((StepWork*)p.work)->factor : nullptr};
+                      scale_ahead(p) ? p.loss : nullptr};
   const aa_rs_params& r = p.rs;
   if (!r.enabled || n == 0) {
     int64_t blocks = (n + 4095) / 4096;  // 16 mask bytes per thread

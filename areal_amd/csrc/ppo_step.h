@@ -9,15 +9,15 @@ namespace aa {
 constexpr int kFinishBlocks = 256;  // most workgroups of a launch that finishes a step
 constexpr int kTableTensors = 32;   // most tensors of a moments table
 
-// The work buffer of a step: zero before the first launch that uses it, left zero by every launch.
+// The work buffer of a step: its counters are zero before the first launch that uses it and left zero by every launch.
+// Nothing in it outlives a launch: several threads may launch steps on one stream, and theirs come in any order.
 struct StepWork {
   int32_t rows[2];  // row hand-out of the fused logits kernel
   int32_t total, hit, done;
   int32_t finished;
   int32_t logged;
   int32_t outside;
-  float factor;  // see step_scale (written before it is read, not left zero)
-  int32_t pad[7];
+  int32_t pad[8];
   int32_t moments[kTableTensors];
   double partial[kFinishBlocks];
 };
@@ -39,12 +39,13 @@ inline aa_ppo_params step_params(const aa_ppo_step& p) {
 
 // The scale as the loss kernels take it.  The weight of a micro-batch is the count of its whole loss mask; with
 // sequence-level rejection sampling counts[0] is that of the tokens inside the sequences, and the launch that counts them
-// forms the factor from all of them.
+// forms the factor from all of them.  It waits in the step's own output, p.loss, which the last kernel overwrites when it
+// has read it.
 inline bool scale_ahead(const aa_ppo_step& p) {
   return p.scale.per_valid_token && p.rs.enabled && p.rs.level == AA_RS_LEVEL_SEQUENCE && p.T_active > 0;
 }
 inline aa_loss_scale step_scale(const aa_ppo_step& p) {
-  return scale_ahead(p) ? aa_loss_scale{&((StepWork*)p.work)->factor, nullptr, 1.f, 1.f, 0} : p.scale;
+  return scale_ahead(p) ? aa_loss_scale{p.loss, nullptr, 1.f, 1.f, 0} : p.scale;
 }
 
 // the mask the loss is summed under

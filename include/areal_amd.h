@@ -99,8 +99,7 @@ typedef struct {
 } aa_loss_scale;
 
 /* Bytes of the work buffer of a step: zero before the first launch that uses
- * it, left ready for the next one (zero but for a word that is written before
- * it is read) by every launch; one per stream. */
+ * it, left ready for the next one by every launch; one per stream. */
 #define AA_STEP_WORK_BYTES 4096
 
 /* The per-token side of one micro-batch's loss, for the aa_*_step entry

@@ -962,3 +962,22 @@ def test_long_forward_of_a_micro_batch_of_weight_zero_is_not_queued(device, monk
     assert float(_zero_weight_calls()[call](*args).detach()) == 0.0 and not ran
     mb["loss_mask"][5] = True
     assert float(_zero_weight_calls()[call](*args).detach()) != 0.0 and len(ran) == 1
+
+
+def test_work_buffer_keeps_nothing_between_the_launches_of_a_step(device):
+    """Several threads may launch steps on one stream, whose launches then come in any order: what one launch of a step
+    leaves for the next is in the step's own arrays, and the counters of the work buffer are zero behind every launch."""
+    from areal_amd import functional as F
+
+    T, V = 600, 640
+    g = torch.Generator().manual_seed(3)
+    ids = torch.randint(0, V, (T,), generator=g).to(device)
+    mb = {k: torch.randn(T, generator=g).to(device) - 2.0 for k in ("logprobs", "prox_logp", "advantages")}
+    mb.update(loss_mask=(torch.rand(T, generator=g) < 0.6).to(device),
+              cu_seqlens=torch.tensor([0, 100, 350, 500], dtype=torch.int32, device=device))
+    for level in ("token", "sequence"):
+        rs = RejectionSamplingConfig(level=level, action="mask", metric="ratio", upper=100.0)
+        x = torch.randn(T, V, generator=g).bfloat16().to(device).requires_grad_()
+        loss, _ = engine_glue.compute_logprobs_and_loss(x, {"rolled_input_ids": ids}, mb, 0, 977.0, 0.2, rejection_sampling=rs)
+        assert float(loss.detach()) != 0.0
+        assert not F._work_words(device)[:48].any()  # 16 words of counters, 32 of the moments table
