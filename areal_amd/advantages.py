@@ -121,7 +121,7 @@ def _one_process(group=None) -> bool:
 def _plain(t: torch.Tensor | None, shape, dev) -> bool:
     """A float32 array that a kernel may take, and write, as it is."""
     return t is None or (t.dtype is torch.float32 and t.is_contiguous() and t.shape == shape and t.device == dev
-                         and not t.requires_grad)
+                         and not t.requires_grad and (not t.is_inference() or torch.is_inference_mode_enabled()))
 
 
 def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:

@@ -241,3 +241,17 @@ def test_gradient_mask_of_a_padded_micro_batch(monkeypatch, length, pad, want):
         G.compute_lm_head_loss_with(torch.zeros(10, 8), torch.zeros(16, 8), dict(rolled_input_ids=torch.zeros(10)), {}, pad,
                                     None, lambda mb: 1.0, 1.0, grad_token_mask=torch.ones(length, dtype=torch.bool))
     assert seen == [[bool(v) for v in want]]
+
+
+def test_arrays_that_the_advantage_kernel_may_write():
+    """A tensor made in inference mode may not be written outside it: torch refuses the in-place product, and so the
+    one-pass kernel, which masks in place through an address, does not take it."""
+    from areal_amd.advantages import _plain
+
+    cpu, made = torch.device("cpu"), torch.zeros(2, 3)
+    with torch.inference_mode():
+        made_there = torch.zeros(2, 3)
+        assert _plain(made_there, (2, 3), cpu) and _plain(made, (2, 3), cpu)
+    assert _plain(made, (2, 3), cpu) and not _plain(made_there, (2, 3), cpu)
+    assert not _plain(made.double(), (2, 3), cpu) and not _plain(torch.zeros(3, 2).t(), (2, 3), cpu)
+    assert not _plain(torch.zeros(2, 3, requires_grad=True), (2, 3), cpu) and _plain(None, (2, 3), cpu)
