@@ -353,6 +353,11 @@ __device__ __forceinline__ Side16 make_side16(const Operand& X, int x0, int wq, 
   return s;
 }
 
+// Says that the accumulators are in the accumulation half of the register file here.  Ahead of the loop and behind it, so
+// that what the caller does with them, and keeps alive across the loop, leaves the loop's allocation alone: without, the
+// compiler moves some of them back and forth in every slice (48 moves and 9 waits of 356 instructions, 7 % of the time).
+__device__ __forceinline__ void pin_accumulators(f32x4acc_t& v) { asm volatile("" : "+a"(v)); }
+
 // A slice is two 32-wide k steps of 64 MFMAs (A sub-tile mt x B sub-tile nt, 8 x 8); the fragments of both steps live
 // in registers (2 x 16 fragments).  A step is issued as two halves of 32 MFMAs: the first half multiplies A0-3 with
 // B0-3, then with B4-7; the second half A4-7 with B0-7.  So a step can start once A0-3 and B0-3 are there, B4-7 are
@@ -394,13 +399,6 @@ __device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, i
   auto g_load1 = [&](const Unit& c, const Side16& s, int j) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rs, (lds_ptr_t)(uintptr_t)(c.dst + j * 4096), 16, s.voffj[j], 0, 0, 0);
   };
-
-#pragma unroll
-  for (int mt = 0; mt < kAcc16Tiles; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < kAcc16Tiles; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc.v[mt][nt][i] = 0.f;
 
   bf16x8_t fa[2][8], fb[2][8];
   // fragment read r (0..7) of a half: group = 0 reads B0-3 then A0-3, group = 1 reads B4-7 then A4-7, of k step kk of
@@ -447,6 +445,17 @@ __device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, i
   open_unit(cx, sb_, 1, 3);
 #pragma unroll
   for (int j = 0; j < 4; ++j) g_load1(cx, sb_, j);
+  // cleared while the first loads are on their way
+#pragma unroll
+  for (int mt = 0; mt < kAcc16Tiles; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < kAcc16Tiles; ++nt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc.v[mt][nt][i] = 0.f;
+#pragma unroll
+  for (int mt = 0; mt < kAcc16Tiles; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < kAcc16Tiles; ++nt) pin_accumulators(acc.v[mt][nt]);
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(12, 15));  // this wave's parts of units 0 and 1 have landed
   __builtin_amdgcn_s_barrier();
 #pragma unroll
@@ -469,6 +478,10 @@ __device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, i
     half(1, 1, 0, sa1, sb1, 0, 0, cx, sb_, 0);
     sa = sa1;
   }
+#pragma unroll
+  for (int mt = 0; mt < kAcc16Tiles; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < kAcc16Tiles; ++nt) pin_accumulators(acc.v[mt][nt]);
   // the empty loads of the last slices may still deposit zeros: let them finish before the caller reuses LDS
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
   __builtin_amdgcn_s_barrier();

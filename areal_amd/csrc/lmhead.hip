@@ -39,6 +39,10 @@ constexpr int kChunkTokens = 16384;
 constexpr int kPanelPitch = BM + 8;        // pitch (elements) of the tile staged in LDS as [token][vocab]
 constexpr int kStageBytes = 256 * kPanelPitch * 2;  // 135168 B, inside the 160 KiB the main loop uses
 static_assert(kStageBytes + 256 * 4 <= kLdsBytes, "the staged tile and its 256 row numbers must fit the main loop's LDS");
+constexpr int kStripTokens = 16;           // tokens of a wave's strip of panel values staged in LDS
+constexpr int kStripPitch = 128 + 8;       // pitch (elements) of such a strip, [token][vocab]
+constexpr int kWaveStageBytes = kStripTokens * kStripPitch * 2 + 128 * 4;  // one strip and the panel rows of 128 tokens
+static_assert(kWaveStageBytes % 16 == 0 && 4 * kWaveStageBytes <= kLdsBytes, "the strips of four waves share the main loop's LDS");
 
 __host__ __device__ __forceinline__ int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
@@ -93,14 +97,66 @@ constexpr float kCarryMinLogp = -80.f;
 // entry has to stay a normal number (above 2^-126) for entries down to 2^-26 of magnitude, or the chunk is redone
 constexpr float kCarryMinFactor = 0x1p-100f;
 
+// How a wave's 128 x 128 block of panel values leaves: in strips of 16 tokens (one column of accumulator tiles) through a
+// piece of LDS that is the wave's own, so that its waves do not wait for each other and the stores of a strip are issued
+// behind the arithmetic of the next one.  A store instruction covers four panel rows of 256 bytes each.  The row numbers
+// are looked up before the main loop and shared through LDS, four to a read.  (With the whole tile staged, a barrier and a
+// loop that looked up the row of every piece, those lookups and the label logits asked for column by column were a serial
+// chain of some 40 waits on memory per tile.  The tiles that also write the panel, 4 096 x 1 536 x 151 936: 1 890 us so,
+// 1 800 now; H = 1 024: 1 515 and 1 420; H = 4 096: 3 930 and 3 840.  The `nt` policy leaves the softmax partials in the
+// caches: the merge behind these tiles takes 27 us instead of 30.)  Bound by the stores: every compute unit has its
+// 128 KB at about the same time.
+struct PanelOut {
+  char* stage;      // kWaveStageBytes of the wave
+  uint16_t* out;    // panel, at this lane's piece of eight vocabulary entries
+  int64_t ld;
+  bool live;        // the piece starts inside the vocabulary (it ends inside the row's pitch)
+  int lane;
+  u32x4_t piece[4];
+  int row[4];
+
+  __device__ __forceinline__ uint16_t* strip() { return (uint16_t*)stage; }
+  __device__ __forceinline__ int32_t* rows() { return (int32_t*)(stage + kStripTokens * kStripPitch * 2); }
+  // ra, rb: panel rows of the wave's tokens `lane` and 64 + `lane` (negative: none)
+  __device__ __forceinline__ void open(char* lds, int wave, int lane_, uint16_t* panel, int64_t ld_, int m, int V, int ra, int rb) {
+    lane = lane_;
+    stage = lds + wave * kWaveStageBytes;
+    m += 8 * (lane & 15);
+    out = panel + m;
+    ld = ld_;
+    live = m < V;
+    rows()[lane] = ra;
+    rows()[64 + lane] = rb;
+  }
+  // four consecutive vocabulary entries of the strip's token lane % 16: rows 16 mt + 4 (lane / 16) ... of the block
+  __device__ __forceinline__ void put(int mt, uint2 v) {
+    *(uint2*)(strip() + (lane & 15) * kStripPitch + acc16_row(mt, 0, lane)) = v;
+  }
+  // LDS serves a wave's accesses in order, so what the other lanes put is there without a wait; the compiler must not
+  // move the accesses across each other
+  __device__ __forceinline__ void take(int nt) {
+    asm volatile("" ::: "memory");
+    const int t0 = 4 * (lane >> 4);
+    const int4 r = *(const int4*)(rows() + nt * kStripTokens + t0);
+    row[0] = r.x; row[1] = r.y; row[2] = r.z; row[3] = r.w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) piece[j] = *(const u32x4_t*)(strip() + (t0 + j) * kStripPitch + 8 * (lane & 15));
+    asm volatile("" ::: "memory");
+  }
+  __device__ __forceinline__ void store() {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (live && row[j] >= 0) __builtin_nontemporal_store(piece[j], (u32x4_t*)(out + (int64_t)row[j] * ld));
+  }
+};
+
 // Statistics (and, with CARRY, the staged probability ratios) of one wave's 128 x 128 block, accumulators in the
 // 16 x 16 tile layout: a lane holds, for each of 8 tokens (nt), 8 runs (mt) of 4 consecutive vocabulary rows, and the
 // lanes l ^ 16, l ^ 32 hold the other rows of the same tokens.  RAGGED: the block may reach past the vocabulary (last
 // tile row only), rows at or past V are left out.
 template <bool CARRY, bool RAGGED>
 __device__ __forceinline__ void block_stats(const Acc16& acc, const TileArgs& a, int tm, int wm, int wn, int n0, int N,
-                                            int V, int mbase, int lane, uint16_t* Z) {
-  constexpr int PZ = kPanelPitch;
+                                            int V, int mbase, int lane, float kref_a, float kref_b, PanelOut& po) {
 #pragma unroll
   for (int nt = 0; nt < kAcc16Tiles; ++nt) {
     const int nloc = wn * 128 + acc16_col(nt, lane);
@@ -139,7 +195,7 @@ __device__ __forceinline__ void block_stats(const Acc16& acc, const TileArgs& a,
     const float k = fmaxf(mx * a.c, kNegBig);   // kNegBig: no valid row in this block
     float to_ref = 1.f;                         // 2^(k - kref): block-relative -> label-relative exponentials
     if constexpr (CARRY) {
-      const float kref = n < N ? a.xy[n] * a.c : 0.f;
+      const float kref = __shfl(nt < 4 ? kref_a : kref_b, 16 * (nt & 3) + (lane & 15), kWave);
       // a label outside the vocabulary has no logit (NaN): keep the block-relative values, the row's factor is NaN or 0
       to_ref = fabsf(kref) < 1e30f ? fast_exp2(fminf(k - kref, kCarryMaxShift)) : 1.f;
     }
@@ -159,8 +215,12 @@ __device__ __forceinline__ void block_stats(const Acc16& acc, const TileArgs& a,
         uint2 pk;
         pk.x = Elem<AA_BF16>::pack(e[0] * to_ref, e[1] * to_ref);
         pk.y = Elem<AA_BF16>::pack(e[2] * to_ref, e[3] * to_ref);
-        *(uint2*)(Z + nloc * PZ + wm * 128 + acc16_row(mt, 0, lane)) = pk;
+        po.put(mt, pk);
       }
+    }
+    if constexpr (CARRY) {
+      if (nt > 0) po.store();
+      po.take(nt);
     }
     s += __shfl_xor(s, 16, kWave);
     s += __shfl_xor(s, 32, kWave);
@@ -173,6 +233,7 @@ __device__ __forceinline__ void block_stats(const Acc16& acc, const TileArgs& a,
       a.pu[at] = u;
     }
   }
+  if constexpr (CARRY) po.store();
 }
 
 // One 256 x 256 tile: rows m = vocabulary (operand A = weight), columns n = tokens (operand B = hidden states), so
@@ -197,21 +258,33 @@ __global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd
   int tm, tn;
   tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
-  Acc16 acc;
-  mainloop16(W, Hd, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
-
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int V = W.rows, N = Hd.rows;
   const int mbase = m0 + wm * 128;  // first vocabulary row of this wave's block
-  uint16_t* Z = (uint16_t*)lds;     // [256 tokens][kPanelPitch] bf16
-  constexpr int PZ = kPanelPitch;
+  // what the epilogue needs of the wave's tokens `lane` and 64 + `lane`, asked for ahead of the main loop
+  const int na = n0 + wn * 128 + lane, nb = na + 64;
+  float kref_a = 0.f, kref_b = 0.f;
+  int row_a = -1, row_b = -1;
+  if constexpr (MODE == kModeStatsCarry) {
+    if (na < N) kref_a = a.xy[na] * a.c;
+    if (nb < N) kref_b = a.xy[nb] * a.c;
+  }
+  if constexpr (MODE != kModeStats) {
+    if (na < N) row_a = a.out_rows ? a.out_rows[na] : na;
+    if (nb < N) row_b = a.out_rows ? a.out_rows[nb] : nb;
+  }
+  Acc16 acc;
+  mainloop16(W, Hd, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
+
+  PanelOut po;
+  if constexpr (MODE != kModeStats) po.open(lds, wave, lane, a.panel, a.panel_ld, mbase, V, row_a, row_b);
 
   if constexpr (MODE != kModeRecompute) {
     if (m0 + BM > V)  // rows past the vocabulary: last tile row only
-      block_stats<MODE == kModeStatsCarry, true>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, Z);
+      block_stats<MODE == kModeStatsCarry, true>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
     else
-      block_stats<MODE == kModeStatsCarry, false>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, Z);
+      block_stats<MODE == kModeStatsCarry, false>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
   } else {
     const bool ragged_rows = m0 + BM > V;
 #pragma unroll
@@ -253,30 +326,12 @@ __global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd
         uint2 pk;
         pk.x = Elem<AA_BF16>::pack(o[0], o[1]);
         pk.y = Elem<AA_BF16>::pack(o[2], o[3]);
-        *(uint2*)(Z + nloc * PZ + wm * 128 + r0) = pk;
+        po.put(mt, pk);
       }
+      if (nt > 0) po.store();
+      po.take(nt);
     }
-  }
-  if constexpr (MODE != kModeStats) {
-    // panel row of each of the tile's 256 tokens (-1: none), looked up once and shared through LDS behind the staged
-    // tile, so that the store loop below has no dependent global load in it
-    int32_t* rows_lds = (int32_t*)(lds + 256 * PZ * 2);
-    {
-      const int n = n0 + tid;
-      rows_lds[tid] = n < N ? (a.out_rows ? a.out_rows[n] : n) : -1;
-    }
-    __syncthreads();
-    // panel rows: 16-byte pieces along the vocabulary (the pitch is a multiple of 8: the piece that straddles V ends in
-    // the row's own padding, whose entries were formed as zeros)
-    const int mc = (tid & 31) * 8, m = m0 + mc;
-    if (m < V) {
-#pragma unroll 8
-      for (int i = 0; i < 32; ++i) {
-        const int nloc = (tid >> 5) + 8 * i;
-        const int r = rows_lds[nloc];
-        if (r >= 0) *(u32x4_t*)(a.panel + (int64_t)r * a.panel_ld + m) = *(const u32x4_t*)(Z + nloc * PZ + mc);
-      }
-    }
+    po.store();
   }
 }
 
