@@ -1,7 +1,7 @@
 // bf16 tile GEMM on gfx950 matrix cores:  D[m][n] = sum_k A[m][k] * B[n][k], fp32 accumulation.
 //
 // One workgroup of 4 waves computes a 256 x 256 tile of D with v_mfma_f32_32x32x16_bf16, each wave a 128 x 128 block
-// (256 accumulator registers).  Either operand may be stored K-contiguous (row x of the array holds A[x][0..K), the
+// (256 accumulator registers); in the last row or column of tiles, 128 of either side where no more is in use.  Either operand may be stored K-contiguous (row x of the array holds A[x][0..K), the
 // usual "row-major [M, K]") or K-major (row k of the array holds A[0..M)[k], i.e. the array is [K, M]): the second
 // form lets a product contract over the rows of two row-major arrays without a transposed copy of either.
 //
@@ -40,10 +40,20 @@ constexpr int kUnits = 5;
 constexpr int kLdsBytes = kUnits * kUnitBytes;  // 160 KiB
 constexpr int kThreads = 256;
 
-// Accumulators of one wave: v[mt][nt] is the 32 x 32 tile at rows mt * 32, columns nt * 32 of its 128 x 128 block.
+// Accumulators of one wave: v[mt][nt] is the 32 x 32 tile at rows mt * 32, columns nt * 32 of its block.  MT and NT are
+// 4, or 2 for the last row or column of tiles when at most 128 of its rows or columns are in use: the workgroup tile is
+// 64 MT x 64 NT.
+template <int MT, int NT>
 struct Acc {
-  f32x16_t v[4][4];
+  f32x16_t v[MT][NT];
 };
+
+// Says that the accumulators are in the accumulation half of the register file here.  Ahead of a main loop and behind it,
+// so that what the caller does with them, and keeps alive across the loop, leaves the loop's allocation alone: without, the
+// compiler moves some of them back and forth in every slice (mainloop16: 48 moves and 9 waits of 356 instructions, 7 % of
+// the time).
+template <typename V>
+__device__ __forceinline__ void pin_accumulators(V& v) { asm volatile("" : "+a"(v)); }
 
 // row (m) and column (n) inside the wave's block of accumulator element (mt, nt, i) of lane `lane`
 __device__ __forceinline__ int acc_row(int mt, int i, int lane) { return mt * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3); }
@@ -138,11 +148,14 @@ struct Side {
   int frag[4];             // fragment read: per-lane byte offsets inside a unit (K-contiguous: per kk; K-major: per x)
 };
 
-template <bool KMAJOR>
+//
+// NX: sub-tiles of 32 per wave, 4 or 2.  With 2 a K-contiguous unit holds 128 rows (loads 0..3); a K-major one keeps its
+// layout, and its loads fetch nothing for the upper half of a k-row.
+template <bool KMAJOR, int NX>
 __device__ __forceinline__ Side make_side(const Operand& X, int x0, int wq, int wave, int lane) {
   Side s;
   s.ld = X.ld;
-  const int valid = (X.rows - x0) < 256 ? (X.rows - x0) : 256;
+  const int valid = (X.rows - x0) < 64 * NX ? (X.rows - x0) : 64 * NX;
   if constexpr (!KMAJOR) {
     const int ld_row = 8 * wave + (lane >> 3);
     s.chunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
@@ -151,7 +164,7 @@ __device__ __forceinline__ Side make_side(const Operand& X, int x0, int wq, int 
     s.jstep = (int)(32 * X.ld * 2);
     s.bytes = (int)((int64_t)valid * X.ld * 2);
     const int half = lane >> 5, r7 = (lane >> 1) & 7;
-    const int fr = (wq * 128 + (lane & 31)) * 128;
+    const int fr = (wq * (32 * NX) + (lane & 31)) * 128;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) s.frag[kk] = fr + (((2 * kk + half) ^ r7) << 4);
   } else {
@@ -163,9 +176,9 @@ __device__ __forceinline__ Side make_side(const Operand& X, int x0, int wq, int 
     s.jstep = (int)(8 * X.ld * 2);
     s.bytes = 0;  // per slice: the valid k-rows times ld
     const int sl = lane & 15, half = lane >> 5, mb = (lane >> 4) & 1;
-    const int lanebase = (8 * half + (sl >> 2)) * 512 + 16 * (16 * wq + 2 * mb + ((sl >> 1) & 1)) + 8 * (sl & 1);
+    const int lanebase = (8 * half + (sl >> 2)) * 512 + 16 * (2 * mb + ((sl >> 1) & 1)) + 8 * (sl & 1);
 #pragma unroll
-    for (int x = 0; x < 4; ++x) s.frag[x] = lanebase + 64 * (x ^ (sl >> 2));
+    for (int x = 0; x < NX; ++x) s.frag[x] = lanebase + 64 * ((NX * wq + x) ^ (sl >> 2));
   }
   return s;
 }
@@ -173,24 +186,25 @@ __device__ __forceinline__ Side make_side(const Operand& X, int x0, int wq, int 
 // Main loop.  Leaves the result in `acc`; `lds` is kLdsBytes of dynamic shared memory.  K % 8 == 0.
 // AKM / BKM: the operand is K-major.
 //
-// Per slice (four 16-wide k steps, fragments double buffered in registers; every step issues its 16 MFMAs with the 8
-// fragment reads of the next step behind MFMAs 0-7 and 4 global loads behind MFMAs 8, 10, 12, 14 (a load blocks the
-// wave's issue for about as long as one MFMA runs: next to a fragment read it costs idle cycles), in exactly the order
-// written here):
+// Per slice (four 16-wide k steps, fragments double buffered in registers; every step issues its MT x NT MFMAs with the
+// fragment reads of the next step behind the first ones and its global loads (4, or 2 where the operand's unit holds 128
+// rows) behind later ones, MFMAs 8, 10, 12, 14 of 16 (a load blocks the wave's issue for about as long as one MFMA runs:
+// next to a fragment read it costs idle cycles), in exactly the order written here):
 //   steps 0, 1, 2; wait: own fragment reads done, own loads through B(k+1) landed (A(k+2) may be in flight); barrier;
 //   step 3 (reads the first fragments of slice k + 1)
 // Slices at or past K get an empty descriptor (no memory traffic, zeros in LDS) so that the count of loads per slice,
 // and with it the vmcnt arithmetic, is the same from the first slice to the last.
-template <bool AKM, bool BKM>
-__device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int K, int m0, int n0, Acc& acc, char* lds) {
-  constexpr int MN = 16, NR = 8;
+template <bool AKM, bool BKM, int MT, int NT>
+__device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int K, int m0, int n0, Acc<MT, NT>& acc, char* lds) {
+  constexpr int MN = MT * NT, NR = MT + NT;
+  constexpr int LA = AKM ? 8 : 2 * MT, LB = BKM ? 8 : 2 * NT;  // loads of a unit
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS block addresses stay in scalar registers
   const int wm = wave >> 1, wn = wave & 1;
   const uint32_t lds32 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
-  const Side sa_ = make_side<AKM>(A, m0, wm, wave, lane);
-  const Side sb_ = make_side<BKM>(B, n0, wn, wave, lane);
+  const Side sa_ = make_side<AKM, MT>(A, m0, wm, wave, lane);
+  const Side sb_ = make_side<BKM, NT>(B, n0, wn, wave, lane);
 
   // unit u = 2 slice + operand lives in slot u % 5
   auto open_unit = [&](Cursor& c, const Side& s, bool kmajor, int slice, int slot) {
@@ -216,14 +230,7 @@ __device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int
     __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rs, (lds_ptr_t)(uintptr_t)(c.dst + j * 4096), 16, c.voff + j * jstep, 0, 0, 0);
   };
 
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc.v[mt][nt][i] = 0.f;
-
-  bf16x8_t fa[2][4], fb[2][4];
+  bf16x8_t fa[2][MT], fb[2][NT];
   // fragment of sub-tile x at k step kk from the unit in `slot`
   auto frag = [&](const Side& s, bool kmajor, int slot, int kk, int x) -> bf16x8_t {
     if (!kmajor) return __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(lds + slot * kUnitBytes + s.frag[kk] + x * 4096));
@@ -232,25 +239,35 @@ __device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int
     const s16x4_t hi = lds_read_tr(at, kk * 8192 + 2048);
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  // fragment r of a step: r < 4 is A sub-tile r, otherwise B sub-tile r - 4; slot_a / slot_b are the units' slots
+  // fragment r of a step: r < MT is A sub-tile r, otherwise B sub-tile r - MT; slot_a / slot_b are the units' slots
   auto f_load1 = [&](int buf, int slot_a, int slot_b, int kk, int r) {
-    if (r < 4)
+    if (r < MT)
       fa[buf][r] = frag(sa_, AKM, slot_a, kk, r);
     else
-      fb[buf][r - 4] = frag(sb_, BKM, slot_b, kk, r - 4);
+      fb[buf][r - MT] = frag(sb_, BKM, slot_b, kk, r - MT);
   };
   auto mfma1 = [&](int buf, int i) {
-    const int mt = i >> 2, nt = i & 3;
+    const int mt = i / NT, nt = i % NT;
     acc.v[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[buf][mt], fb[buf][nt], acc.v[mt][nt], 0, 0, 0);
   };
-  // one 16-wide k step: 16 MFMAs from fragment buffer `buf`; in their shadow the 8 fragment reads of the next step
-  // (k step nkk of the units in slots na, nb) and 4 global loads (blocks j0 .. j0 + 3 of the unit behind `c`)
-  auto step = [&](int buf, int na, int nb, int nkk, const Cursor& c, int jstep, int j0) {
+  // one 16-wide k step: the MFMAs from fragment buffer `buf`; in their shadow the fragment reads of the next step
+  // (k step nkk of the units in slots na, nb; two to an MFMA where there are few) and `loads` global loads (blocks
+  // j0 ... of the unit behind `c`)
+  auto step = [&](int buf, int na, int nb, int nkk, const Cursor& c, int jstep, int j0, int loads) {
+    constexpr int RP = MN >= 16 ? 1 : 2;      // reads behind an MFMA
+    constexpr int L0 = MN >= 16 ? 8 : MN / 2;  // first MFMA with a load behind it
+    const int every = MN >= 16 ? 2 : 1, most = MN >= 16 ? 1 : (loads + MN - L0 - 1) / (MN - L0);
 #pragma unroll
     for (int i = 0; i < MN; ++i) {
       mfma1(buf, i);
-      if (i < NR) f_load1(buf ^ 1, na, nb, nkk, i);
-      if (i >= 8 && !(i & 1)) g_load1(c, jstep, j0 + ((i - 8) >> 1));  // behind MFMAs 8, 10, 12, 14
+#pragma unroll
+      for (int r = RP * i; r < RP * i + RP; ++r)
+        if (r < NR) f_load1(buf ^ 1, na, nb, nkk, r);
+      if (i >= L0 && (i - L0) % every == 0) {
+#pragma unroll
+        for (int l = (i - L0) / every * most; l < (i - L0) / every * most + most; ++l)
+          if (l < loads) g_load1(c, jstep, j0 + l);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     // the transposing reads are invisible to the compiler's own wait insertion: they were issued in the first half
@@ -267,17 +284,26 @@ __device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int
   // units 0, 1, 2 (A0, B0, A1) and the first half of unit 3 (B1)
   open_a(cy, 0, 0);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) g_load1(cy, sa_.jstep, j);
+  for (int j = 0; j < LA; ++j) g_load1(cy, sa_.jstep, j);
   open_b(cx, 0, 1);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) g_load1(cx, sb_.jstep, j);
+  for (int j = 0; j < LB; ++j) g_load1(cx, sb_.jstep, j);
   open_a(cy, 1, 2);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) g_load1(cy, sa_.jstep, j);
+  for (int j = 0; j < LA; ++j) g_load1(cy, sa_.jstep, j);
   open_b(cx, 1, 3);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) g_load1(cx, sb_.jstep, j);
-  __builtin_amdgcn_s_waitcnt(waitcnt_imm(12, 15));  // this wave's parts of units 0 and 1 have landed
+  for (int j = 0; j < LB / 2; ++j) g_load1(cx, sb_.jstep, j);
+  // cleared while the first loads are on their way
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc.v[mt][nt][i] = 0.f;
+      pin_accumulators(acc.v[mt][nt]);
+    }
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(LA + LB / 2, 15));  // this wave's parts of units 0 and 1 have landed
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int r = 0; r < NR; ++r) f_load1(0, 0, 1, 0, r);
@@ -287,19 +313,23 @@ __device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int
     const int sb = next_slot(sa, 1), sa1 = next_slot(sa, 2), sb1 = next_slot(sa, 3), s4 = next_slot(sa, 4);
     // cx is unit 2 k + 3 = B(k + 1) in slot sb1, opened when its first half was issued
     __builtin_amdgcn_sched_barrier(0);
-    step(0, sa, sb, 1, cx, sb_.jstep, 4);
+    step(0, sa, sb, 1, cx, sb_.jstep, LB / 2, LB / 2);
     open_a(cy, k + 2, s4);  // unit 2 k + 4 = A(k + 2)
     __builtin_amdgcn_sched_barrier(0);
-    step(1, sa, sb, 2, cy, sa_.jstep, 0);
-    step(0, sa, sb, 3, cy, sa_.jstep, 4);
+    step(1, sa, sb, 2, cy, sa_.jstep, 0, LA / 2);
+    step(0, sa, sb, 3, cy, sa_.jstep, LA / 2, LA / 2);
     // own reads of slice k done; own loads through unit 2 k + 3 landed (unit 2 k + 4 may be in flight)
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(8, 0));
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(LA, 0));
     __builtin_amdgcn_s_barrier();
     open_b(cx, k + 2, sa);  // unit 2 k + 5 = B(k + 2) takes the slot of A(k)
     __builtin_amdgcn_sched_barrier(0);
-    step(1, sa1, sb1, 0, cx, sb_.jstep, 0);
+    step(1, sa1, sb1, 0, cx, sb_.jstep, 0, LB / 2);
     sa = sa1;
   }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) pin_accumulators(acc.v[mt][nt]);
   // the empty loads of the last slices may still deposit zeros: let them finish before the caller reuses LDS
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
   __builtin_amdgcn_s_barrier();
@@ -320,9 +350,11 @@ __device__ __forceinline__ void mainloop(const Operand& A, const Operand& B, int
 //   D, lane l, register i: n = l % 16, m = 4 (l / 16) + i
 // i.e. a lane owns one column n of D and 4 consecutive rows m; the lanes l ^ 16, l ^ 32 own the other rows of that n.
 typedef float f32x4acc_t __attribute__((ext_vector_type(4)));
-constexpr int kAcc16Tiles = 8;  // per direction: a wave's 128 x 128 block is 8 x 8 tiles of 16 x 16
+constexpr int kAcc16Tiles = 8;  // down the rows m: a wave's block of 128 rows is 8 tiles of 16 x 16
+constexpr int kWide = 8, kNarrow = 4;  // NT, the tiles along n: a workgroup tile of 256 or of 128 columns
+template <int NT>
 struct Acc16 {
-  f32x4acc_t v[kAcc16Tiles][kAcc16Tiles];
+  f32x4acc_t v[kAcc16Tiles][NT];
 };
 __device__ __forceinline__ int acc16_row(int mt, int i, int lane) { return mt * 16 + 4 * (lane >> 4) + i; }
 __device__ __forceinline__ int acc16_col(int nt, int lane) { return nt * 16 + (lane & 15); }
@@ -337,9 +369,17 @@ struct Side16 {
   int frag[2];           // fragment read: per-lane byte offset inside a unit, per k step
 };
 
+// what a wave needs to bring its blocks of one unit of this loop
+struct Unit {
+  __amdgpu_buffer_rsrc_t rs;
+  uint32_t dst;
+};
+
+// ROWS: 256, or 128 for the operand of a narrow tile (its unit then holds 128 rows, loads 0..3)
+template <int ROWS>
 __device__ __forceinline__ Side16 make_side16(const Operand& X, int x0, int wq, int wave, int lane) {
   Side16 s;
-  const int valid = (X.rows - x0) < 256 ? (X.rows - x0) : 256;
+  const int valid = (X.rows - x0) < ROWS ? (X.rows - x0) : ROWS;
   const int ld_row = 8 * wave + (lane >> 3);
   s.chunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
   s.base = X.ptr + (int64_t)x0 * X.ld;
@@ -347,16 +387,11 @@ __device__ __forceinline__ Side16 make_side16(const Operand& X, int x0, int wq, 
   for (int j = 0; j < 8; ++j) s.voffj[j] = (int)((((int64_t)ld_row + 32 * j) * X.ld + s.chunk * 8) * 2);
   s.bytes = (int)((int64_t)valid * X.ld * 2);
   const int kgrp = lane >> 4, r7 = (lane >> 1) & 7;  // row 16 x + lane % 16: (row >> 1) & 7 = (lane >> 1) & 7
-  const int fr = (wq * 128 + (lane & 15)) * 128;
+  const int fr = (wq * (ROWS / 2) + (lane & 15)) * 128;
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) s.frag[kk] = fr + (((4 * kk + kgrp) ^ r7) << 4);
   return s;
 }
-
-// Says that the accumulators are in the accumulation half of the register file here.  Ahead of the loop and behind it, so
-// that what the caller does with them, and keeps alive across the loop, leaves the loop's allocation alone: without, the
-// compiler moves some of them back and forth in every slice (48 moves and 9 waits of 356 instructions, 7 % of the time).
-__device__ __forceinline__ void pin_accumulators(f32x4acc_t& v) { asm volatile("" : "+a"(v)); }
 
 // A slice is two 32-wide k steps of 64 MFMAs (A sub-tile mt x B sub-tile nt, 8 x 8); the fragments of both steps live
 // in registers (2 x 16 fragments).  A step is issued as two halves of 32 MFMAs: the first half multiplies A0-3 with
@@ -370,18 +405,22 @@ __device__ __forceinline__ void pin_accumulators(f32x4acc_t& v) { asm volatile("
 //   wait: own fragment reads done, own loads through B(k+1) landed (A(k+2) may be in flight); barrier
 //   half 3 (step 1, second)   reads B0-3, A0-3 of slice k+1 step 0  loads the first half of B(k+2) into A(k)'s slot
 // The ring of units, the counted waits and the empty descriptors past K are those of mainloop().
-__device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, int K, int m0, int n0, Acc16& acc, char* lds) {
+//
+// NT = kNarrow: a tile of 256 x 128 for a last column of tiles with at most 128 columns of D in use.  B units hold 128
+// rows (two loads in half 0, two in half 3), a half is 16 MFMAs; A units, ring, waits and order are the same.  It needs
+// 48 B/clk of loads at full MFMA rate, near what a compute unit sustains, and takes about 0.7 of a wide tile's time (a 17th
+// column of 594 tiles at K = 1 536: 65 us narrow, 90 us wide).
+template <int NT>
+__device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, int K, int m0, int n0, Acc16<NT>& acc, char* lds) {
+  static_assert(NT == kWide || NT == kNarrow, "a wave's block is 128 or 64 columns wide");
+  constexpr int NB = NT;  // loads of a B unit (32 rows each, so one per 16 columns of a wave's block)
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const uint32_t lds32 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
-  Side16 sa_ = make_side16(A, m0, wm, wave, lane);
-  Side16 sb_ = make_side16(B, n0, wn, wave, lane);
-  struct Unit {
-    __amdgpu_buffer_rsrc_t rs;
-    uint32_t dst;
-  };
+  Side16 sa_ = make_side16<256>(A, m0, wm, wave, lane);
+  Side16 sb_ = make_side16<32 * NB>(B, n0, wn, wave, lane);
   auto open_unit = [&](Unit& c, Side16& s, int slice, int slot) {
     const int k0 = slice * BK;
     const bool live = k0 < K;
@@ -400,31 +439,33 @@ __device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, i
     __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rs, (lds_ptr_t)(uintptr_t)(c.dst + j * 4096), 16, s.voffj[j], 0, 0, 0);
   };
 
-  bf16x8_t fa[2][8], fb[2][8];
-  // fragment read r (0..7) of a half: group = 0 reads B0-3 then A0-3, group = 1 reads B4-7 then A4-7, of k step kk of
-  // the units in slot_a / slot_b, into fragment buffer buf
+  bf16x8_t fa[2][8], fb[2][NT];
+  // fragment read r (0..7) of a half: group = 0 reads B0-3 then A0-3, group = 1 reads B4-7 (of a wide tile) then A4-7, of
+  // k step kk of the units in slot_a / slot_b, into fragment buffer buf
   auto f_load1 = [&](int buf, int slot_a, int slot_b, int kk, int group, int r) {
     const int x = 4 * group + (r & 3);
-    if (r < 4)
-      fb[buf][x] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(lds + slot_b * kUnitBytes + sb_.frag[kk] + x * 2048));
-    else
+    if (r < 4) {
+      if (x < NT) fb[buf][x < NT ? x : 0] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(lds + slot_b * kUnitBytes + sb_.frag[kk] + x * 2048));
+    } else {
       fa[buf][x] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(lds + slot_a * kUnitBytes + sa_.frag[kk] + x * 2048));
+    }
   };
   auto mfma1 = [&](int buf, int mt, int nt) {
     acc.v[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[buf][mt], fb[buf][nt], acc.v[mt][nt], 0, 0, 0);
   };
-  // one half of a 32-wide k step: 32 MFMAs from fragment buffer `buf` (second = 0: A0-3 x B0-3, then A0-3 x B4-7;
+  // one half of a 32-wide k step: 32 (or 16) MFMAs from fragment buffer `buf` (second = 0: A0-3 x B0-3, then A0-3 x B4-7;
   // second = 1: A4-7 x B0-7); in their shadow 8 fragment reads (group rgroup of k step rkk of the units in slots ra, rb,
-  // into buffer rbuf) and 4 global loads (blocks j0 .. j0 + 3 of the unit `c` of operand side `cs`)
-  auto half = [&](int buf, int second, int rbuf, int ra, int rb, int rkk, int rgroup, const Unit& c, const Side16& cs, int j0) {
+  // into buffer rbuf) and `loads` global loads (blocks j0 ... of the unit `c` of operand side `cs`)
+  auto half = [&](int buf, int second, int rbuf, int ra, int rb, int rkk, int rgroup, const Unit& c, const Side16& cs, int j0, int loads) {
+    constexpr int MN = 4 * NT;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < MN; ++i) {
       if (second)
-        mfma1(buf, 4 + (i >> 3), i & 7);
+        mfma1(buf, 4 + i / NT, i % NT);
       else
         mfma1(buf, (i >> 2) & 3, (i & 3) + 4 * (i >> 4));
       if (i < 8) f_load1(rbuf, ra, rb, rkk, rgroup, i);
-      if ((i & 7) == 7) g_load1(c, cs, j0 + (i >> 3));
+      if (i % (MN / loads) == MN / loads - 1) g_load1(c, cs, j0 + i / (MN / loads));
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -438,25 +479,25 @@ __device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, i
   for (int j = 0; j < 8; ++j) g_load1(cy, sa_, j);
   open_unit(cx, sb_, 0, 1);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) g_load1(cx, sb_, j);
+  for (int j = 0; j < NB; ++j) g_load1(cx, sb_, j);
   open_unit(cy, sa_, 1, 2);
 #pragma unroll
   for (int j = 0; j < 8; ++j) g_load1(cy, sa_, j);
   open_unit(cx, sb_, 1, 3);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) g_load1(cx, sb_, j);
+  for (int j = 0; j < NB / 2; ++j) g_load1(cx, sb_, j);
   // cleared while the first loads are on their way
 #pragma unroll
   for (int mt = 0; mt < kAcc16Tiles; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < kAcc16Tiles; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc.v[mt][nt][i] = 0.f;
 #pragma unroll
   for (int mt = 0; mt < kAcc16Tiles; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < kAcc16Tiles; ++nt) pin_accumulators(acc.v[mt][nt]);
-  __builtin_amdgcn_s_waitcnt(waitcnt_imm(12, 15));  // this wave's parts of units 0 and 1 have landed
+    for (int nt = 0; nt < NT; ++nt) pin_accumulators(acc.v[mt][nt]);
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(8 + NB / 2, 15));  // this wave's parts of units 0 and 1 have landed
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int r = 0; r < 8; ++r) f_load1(0, 0, 1, 0, 0, r);
@@ -465,23 +506,23 @@ __device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, i
     const int sb = next_slot(sa, 1), sa1 = next_slot(sa, 2), sb1 = next_slot(sa, 3), s4 = next_slot(sa, 4);
     // cx is unit 2 k + 3 = B(k + 1) in slot sb1, opened when its first half was issued
     __builtin_amdgcn_sched_barrier(0);
-    half(0, 0, 0, sa, sb, 0, 1, cx, sb_, 4);
+    half(0, 0, 0, sa, sb, 0, 1, cx, sb_, NB / 2, NB / 2);
     open_unit(cy, sa_, k + 2, s4);  // unit 2 k + 4 = A(k + 2)
     __builtin_amdgcn_sched_barrier(0);
-    half(0, 1, 1, sa, sb, 1, 0, cy, sa_, 0);
-    half(1, 0, 1, sa, sb, 1, 1, cy, sa_, 4);
+    half(0, 1, 1, sa, sb, 1, 0, cy, sa_, 0, 4);
+    half(1, 0, 1, sa, sb, 1, 1, cy, sa_, 4, 4);
     // own reads of slice k done; own loads through unit 2 k + 3 landed (unit 2 k + 4 may be in flight)
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(8, 0));
     __builtin_amdgcn_s_barrier();
     open_unit(cx, sb_, k + 2, sa);  // unit 2 k + 5 = B(k + 2) takes the slot of A(k)
     __builtin_amdgcn_sched_barrier(0);
-    half(1, 1, 0, sa1, sb1, 0, 0, cx, sb_, 0);
+    half(1, 1, 0, sa1, sb1, 0, 0, cx, sb_, 0, NB / 2);
     sa = sa1;
   }
 #pragma unroll
   for (int mt = 0; mt < kAcc16Tiles; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < kAcc16Tiles; ++nt) pin_accumulators(acc.v[mt][nt]);
+    for (int nt = 0; nt < NT; ++nt) pin_accumulators(acc.v[mt][nt]);
   // the empty loads of the last slices may still deposit zeros: let them finish before the caller reuses LDS
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
   __builtin_amdgcn_s_barrier();

@@ -150,17 +150,16 @@ struct PanelOut {
   }
 };
 
-// Statistics (and, with CARRY, the staged probability ratios) of one wave's 128 x 128 block, accumulators in the
-// 16 x 16 tile layout: a lane holds, for each of 8 tokens (nt), 8 runs (mt) of 4 consecutive vocabulary rows, and the
+// Statistics (and, with CARRY, the staged probability ratios) of one wave's 128 x 16 NT block, accumulators in the
+// 16 x 16 tile layout: a lane holds, for each of NT tokens (nt), 8 runs (mt) of 4 consecutive vocabulary rows, and the
 // lanes l ^ 16, l ^ 32 hold the other rows of the same tokens.  RAGGED: the block may reach past the vocabulary (last
 // tile row only), rows at or past V are left out.
-template <bool CARRY, bool RAGGED>
-__device__ __forceinline__ void block_stats(const Acc16& acc, const TileArgs& a, int tm, int wm, int wn, int n0, int N,
+template <bool CARRY, bool RAGGED, int NT>
+__device__ __forceinline__ void block_stats(const Acc16<NT>& acc, const TileArgs& a, int tm, int wm, int wn, int n0, int N,
                                             int V, int mbase, int lane, float kref_a, float kref_b, PanelOut& po) {
 #pragma unroll
-  for (int nt = 0; nt < kAcc16Tiles; ++nt) {
-    const int nloc = wn * 128 + acc16_col(nt, lane);
-    const int n = n0 + nloc;
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = n0 + wn * (16 * NT) + acc16_col(nt, lane);
     float mx = -FLT_MAX;
     if constexpr (!RAGGED) {
 #pragma unroll
@@ -236,34 +235,18 @@ __device__ __forceinline__ void block_stats(const Acc16& acc, const TileArgs& a,
   if constexpr (CARRY) po.store();
 }
 
-// One 256 x 256 tile: rows m = vocabulary (operand A = weight), columns n = tokens (operand B = hidden states), so
+// One tile of 256 x 32 NT: rows m = vocabulary (operand A = weight), columns n = tokens (operand B = hidden states), so
 // that everything a token needs from the tile sits in one lane and its partner lanes ^ 16, ^ 32.  Both operands are
 // K-contiguous: the 16 x 16 x 32 main loop.
-template <int MODE>
-__global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd, int K, int tiles_m, int tiles_n,
-                                                                 TileArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  if constexpr (MODE == kModeRecompute) {
-    if (a.run_if && *a.run_if == 0) return;  // uniform over the grid
-  }
-  if constexpr (MODE == kModeRecompute) {
-    // token columns in use, known to the device alone: the tiles that cover them are numbered as if the host had
-    // launched exactly those (the same walk over the XCDs), the workgroups beyond them return
-    if (a.n_bound) {
-      const int live = a.n_bound[kRowsLive];
-      tiles_n = live < tiles_n ? live : tiles_n;
-      if ((int)blockIdx.x >= tiles_m * tiles_n) return;  // the same decision in every thread of the workgroup
-    }
-  }
-  int tm, tn;
-  tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+template <int MODE, int NT>
+__device__ __forceinline__ void lmhead_tile(const Operand& W, const Operand& Hd, int K, int tm, int n0, const TileArgs& a, char* lds) {
+  const int m0 = tm * BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int V = W.rows, N = Hd.rows;
   const int mbase = m0 + wm * 128;  // first vocabulary row of this wave's block
-  // what the epilogue needs of the wave's tokens `lane` and 64 + `lane`, asked for ahead of the main loop
-  const int na = n0 + wn * 128 + lane, nb = na + 64;
+  // what the epilogue needs of the wave's tokens `lane` and, in a wide tile, 64 + `lane`, asked for ahead of the main loop
+  const int na = n0 + wn * (16 * NT) + lane, nb = NT == kWide ? na + 64 : N;
   float kref_a = 0.f, kref_b = 0.f;
   int row_a = -1, row_b = -1;
   if constexpr (MODE == kModeStatsCarry) {
@@ -274,23 +257,22 @@ __global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd
     if (na < N) row_a = a.out_rows ? a.out_rows[na] : na;
     if (nb < N) row_b = a.out_rows ? a.out_rows[nb] : nb;
   }
-  Acc16 acc;
-  mainloop16(W, Hd, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
+  Acc16<NT> acc;
+  mainloop16<NT>(W, Hd, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
 
   PanelOut po;
   if constexpr (MODE != kModeStats) po.open(lds, wave, lane, a.panel, a.panel_ld, mbase, V, row_a, row_b);
 
   if constexpr (MODE != kModeRecompute) {
     if (m0 + BM > V)  // rows past the vocabulary: last tile row only
-      block_stats<MODE == kModeStatsCarry, true>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
+      block_stats<MODE == kModeStatsCarry, true, NT>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
     else
-      block_stats<MODE == kModeStatsCarry, false>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
+      block_stats<MODE == kModeStatsCarry, false, NT>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
   } else {
     const bool ragged_rows = m0 + BM > V;
 #pragma unroll
-    for (int nt = 0; nt < kAcc16Tiles; ++nt) {
-      const int nloc = wn * 128 + acc16_col(nt, lane);
-      const int n = n0 + nloc;
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = n0 + wn * (16 * NT) + acc16_col(nt, lane);
       float A = 0.f, B = 0.f, lab_add = 0.f, lse2 = 0.f;
       int64_t y = -1;
       const int t = n < N ? (a.col_tokens ? a.col_tokens[n] : n) : -1;
@@ -333,6 +315,37 @@ __global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd
     }
     po.store();
   }
+}
+
+// A last column of tiles with at most 128 tokens is one of narrow tiles: that is as many as they hold, and up to there they
+// are the shorter ones.  Forward, us wide / narrow: 4 160 x 1 536 x 151 936: 1 650 / 1 600, 8 000 x 2 048: 3 943 / 3 899,
+// 1 900 x 1 024 x 50 257: 220 / 209, 100 x 2 048 x 151 936: 190 / 163.
+template <int MODE>
+__global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd, int K, int tiles_m, int tiles_n,
+                                                                 TileArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  if constexpr (MODE == kModeRecompute) {
+    if (a.run_if && *a.run_if == 0) return;  // uniform over the grid
+  }
+  int columns = Hd.rows;
+  if constexpr (MODE == kModeRecompute) {
+    // token columns in use, known to the device alone: the tiles that cover them are numbered as if the host had
+    // launched exactly those (the same walk over the XCDs), the workgroups beyond them return
+    if (a.n_bound) {
+      const int live = a.n_bound[kRowsLive];
+      tiles_n = live < tiles_n ? live : tiles_n;
+      if ((int)blockIdx.x >= tiles_m * tiles_n) return;  // the same decision in every thread of the workgroup
+      const int total = a.n_bound[kRowsTotal];
+      columns = total < columns ? total : columns;
+    }
+  }
+  int tm, tn;
+  tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int n0 = tn * BN;
+  if (columns - n0 > BN / 2)  // uniform
+    lmhead_tile<MODE, kWide>(W, Hd, K, tm, n0, a, lds);
+  else
+    lmhead_tile<MODE, kNarrow>(W, Hd, K, tm, n0, a, lds);
 }
 
 // Raw label logit of every token: xy[t] = hidden[t] . weight[label[t]] in fp32 (NaN for a label outside [0, V)).  One
@@ -644,6 +657,70 @@ __device__ __forceinline__ int choose_splits_wave(int tiles, int slices, int uni
 // return at once), and the whole grid returns when the product over those rows is one that k_gemm_splitk, queued
 // beside it, cuts along K.  kBoundK: the contraction stops at the count rounded up to a whole K slice (the rows up to
 // there are zero).  kBoundNone is the kernel without any of this.
+template <bool AKM, bool BKM, typename OutT, bool ACCUM, int MT, int NT>
+__device__ __forceinline__ void gemm_store_tile(const Operand& A, const Operand& B, int K, int m0, int n0, OutT* __restrict__ C,
+                                                int64_t ldc, const int32_t* __restrict__ c_rows,
+                                                const float* __restrict__ n_scale, char* lds) {
+  Acc<MT, NT> acc;
+  mainloop<AKM, BKM, MT, NT>(A, B, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int M = A.rows, N = B.rows;
+  if constexpr (sizeof(OutT) == 2) {
+    uint16_t* Z = (uint16_t*)lds;  // [256 n][kPanelPitch] bf16
+    constexpr int PZ = kPanelPitch;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int nloc = wn * (32 * NT) + acc_col(nt, lane);
+      // optional factor per row of C (a lane owns one n): applied to the fp32 sums, before the one rounding to bf16.  A
+      // factor of zero gives a zero row whatever the sums hold (a row without gradient may have summed to infinity)
+      const float f = (n_scale && n0 + nloc < N) ? n_scale[n0 + nloc] : 1.f;
+      const bool dead = f == 0.f;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          uint2 pk;
+          pk.x = dead ? 0u : Elem<AA_BF16>::pack(acc.v[mt][nt][g4 * 4] * f, acc.v[mt][nt][g4 * 4 + 1] * f);
+          pk.y = dead ? 0u : Elem<AA_BF16>::pack(acc.v[mt][nt][g4 * 4 + 2] * f, acc.v[mt][nt][g4 * 4 + 3] * f);
+          *(uint2*)(Z + nloc * PZ + wm * (32 * MT) + mt * 32 + 8 * g4 + 4 * (lane >> 5)) = pk;
+        }
+    }
+    int32_t* rows_lds = (int32_t*)(lds + 256 * PZ * 2);  // row of C of each of the tile's n (-1: past the end)
+    {
+      const int n = n0 + tid;
+      rows_lds[tid] = n < N ? (c_rows ? c_rows[n] : n) : -1;
+    }
+    __syncthreads();
+    const int mc = (tid & 31) * 8, m = m0 + mc;  // M % 8 == 0 (M is a hidden size): a piece never straddles the end
+    if (m < M) {
+#pragma unroll 8
+      for (int i = 0; i < 8 * NT; ++i) {
+        const int nloc = (tid >> 5) + 8 * i;
+        const int r = rows_lds[nloc];
+        if (r >= 0) *(u32x4_t*)(C + (int64_t)r * ldc + m) = *(const u32x4_t*)(Z + nloc * PZ + mc);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = n0 + wn * (32 * NT) + acc_col(nt, lane);
+      if (n >= N) continue;
+      float* row = (float*)C + (c_rows ? c_rows[n] : n) * ldc;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const int m = m0 + wm * (32 * MT) + mt * 32 + 8 * g4 + 4 * (lane >> 5);  // M % 4 == 0
+          if (m >= M) continue;
+          f32x4_t v = {acc.v[mt][nt][g4 * 4], acc.v[mt][nt][g4 * 4 + 1], acc.v[mt][nt][g4 * 4 + 2], acc.v[mt][nt][g4 * 4 + 3]};
+          if (ACCUM) v += *(const f32x4_t*)(row + m);
+          *(f32x4_t*)(row + m) = v;
+        }
+    }
+  }
+}
+
 template <bool AKM, bool BKM, typename OutT, bool ACCUM, int BOUND>
 __global__ __launch_bounds__(kThreads) void k_gemm_store(Operand A, Operand B, int K, int tiles_m, int tiles_n,
                                                          OutT* __restrict__ C, int64_t ldc,
@@ -664,64 +741,25 @@ __global__ __launch_bounds__(kThreads) void k_gemm_store(Operand A, Operand B, i
     const int kb = bounds[kRowsSliced];
     K = kb < K ? kb : K;
   }
-  Acc acc;
-  mainloop<AKM, BKM>(A, B, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int M = A.rows, N = B.rows;
-  if constexpr (sizeof(OutT) == 2) {
-    uint16_t* Z = (uint16_t*)lds;  // [256 n][kPanelPitch] bf16
-    constexpr int PZ = kPanelPitch;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int nloc = wn * 128 + acc_col(nt, lane);
-      // optional factor per row of C (a lane owns one n): applied to the fp32 sums, before the one rounding to bf16.  A
-      // factor of zero gives a zero row whatever the sums hold (a row without gradient may have summed to infinity)
-      const float f = (n_scale && n0 + nloc < N) ? n_scale[n0 + nloc] : 1.f;
-      const bool dead = f == 0.f;
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          uint2 pk;
-          pk.x = dead ? 0u : Elem<AA_BF16>::pack(acc.v[mt][nt][g4 * 4] * f, acc.v[mt][nt][g4 * 4 + 1] * f);
-          pk.y = dead ? 0u : Elem<AA_BF16>::pack(acc.v[mt][nt][g4 * 4 + 2] * f, acc.v[mt][nt][g4 * 4 + 3] * f);
-          *(uint2*)(Z + nloc * PZ + wm * 128 + mt * 32 + 8 * g4 + 4 * (lane >> 5)) = pk;
-        }
-    }
-    int32_t* rows_lds = (int32_t*)(lds + 256 * PZ * 2);  // row of C of each of the tile's 256 n (-1: past the end)
-    {
-      const int n = n0 + tid;
-      rows_lds[tid] = n < N ? (c_rows ? c_rows[n] : n) : -1;
-    }
-    __syncthreads();
-    const int mc = (tid & 31) * 8, m = m0 + mc;  // M % 8 == 0 (M is a hidden size): a piece never straddles the end
-    if (m < M) {
-#pragma unroll 8
-      for (int i = 0; i < 32; ++i) {
-        const int nloc = (tid >> 5) + 8 * i;
-        const int r = rows_lds[nloc];
-        if (r >= 0) *(u32x4_t*)(C + (int64_t)r * ldc + m) = *(const u32x4_t*)(Z + nloc * PZ + mc);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int n = n0 + wn * 128 + acc_col(nt, lane);
-      if (n >= N) continue;
-      float* row = (float*)C + (c_rows ? c_rows[n] : n) * ldc;
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int m = m0 + wm * 128 + mt * 32 + 8 * g4 + 4 * (lane >> 5);  // M % 4 == 0
-          if (m >= M) continue;
-          f32x4_t v = {acc.v[mt][nt][g4 * 4], acc.v[mt][nt][g4 * 4 + 1], acc.v[mt][nt][g4 * 4 + 2], acc.v[mt][nt][g4 * 4 + 3]};
-          if (ACCUM) v += *(const f32x4_t*)(row + m);
-          *(f32x4_t*)(row + m) = v;
-        }
+  // A last row or column of tiles with at most 128 in use is one of narrow tiles, as in the forward.  Both gradients
+  // together with a hidden size that ends in such a row of tiles, whole steps, us wide / narrow: 2 000 x 600 x 64 000:
+  // 583 / 536, 700 x 3 584 x 100 000 (490 rows with a gradient): 1 390 / 1 311, 1 000 x 2 696 x 90 000: 1 377 / 1 335.
+  const bool narrow_m = A.rows - m0 <= BM / 2;
+  int columns = B.rows;
+  if constexpr (BOUND == kBoundN) columns = bounds[kRowsTotal] < columns ? bounds[kRowsTotal] : columns;
+  if constexpr (!BKM) {  // a K-major B is the panel as d_weight reads it: its columns are the vocabulary
+    if (columns - n0 <= BN / 2) {
+      if (narrow_m)
+        gemm_store_tile<AKM, BKM, OutT, ACCUM, 2, 2>(A, B, K, m0, n0, C, ldc, c_rows, n_scale, lds);
+      else
+        gemm_store_tile<AKM, BKM, OutT, ACCUM, 4, 2>(A, B, K, m0, n0, C, ldc, c_rows, n_scale, lds);
+      return;
     }
   }
+  if (narrow_m)
+    gemm_store_tile<AKM, BKM, OutT, ACCUM, 2, 4>(A, B, K, m0, n0, C, ldc, c_rows, n_scale, lds);
+  else
+    gemm_store_tile<AKM, BKM, OutT, ACCUM, 4, 4>(A, B, K, m0, n0, C, ldc, c_rows, n_scale, lds);
 }
 
 // ---- the same product cut along K ------------------------------------------------------------------------------
@@ -735,6 +773,31 @@ __global__ __launch_bounds__(kThreads) void k_gemm_store(Operand A, Operand B, i
 // BOUNDED (the rows of B in use are known to the device alone; `bounds`: the row-count words of the chunk): the tiles
 // over those rows are numbered as a grid of just those, cut into the number of parts that the host would have chosen
 // with that count; the workgroups beyond tiles x parts return at once, all of them when the product is not cut.
+template <bool AKM, bool BKM, int MT, int NT>
+__device__ __forceinline__ void gemm_plane_tile(const Operand& A, const Operand& B, int K, int m0, int n0, float* __restrict__ C,
+                                                int64_t ldc, char* lds) {
+  Acc<MT, NT> acc;
+  mainloop<AKM, BKM, MT, NT>(A, B, K, m0, n0, acc, lds);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int M = A.rows, N = B.rows;
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = n0 + wn * (32 * NT) + acc_col(nt, lane);
+    if (n >= N) continue;
+    float* row = C + n * ldc;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int m = m0 + wm * (32 * MT) + mt * 32 + 8 * g4 + 4 * (lane >> 5);  // M % 4 == 0
+        if (m >= M) continue;
+        const f32x4_t v = {acc.v[mt][nt][g4 * 4], acc.v[mt][nt][g4 * 4 + 1], acc.v[mt][nt][g4 * 4 + 2], acc.v[mt][nt][g4 * 4 + 3]};
+        *(f32x4_t*)(row + m) = v;
+      }
+  }
+}
+
 template <bool AKM, bool BKM, bool BOUNDED>
 __global__ __launch_bounds__(kThreads) void k_gemm_splitk(Operand A, Operand B, int K, int tiles_m, int tiles_n, int splits,
                                                           float* __restrict__ part, int64_t ldc, int64_t plane,
@@ -760,26 +823,19 @@ __global__ __launch_bounds__(kThreads) void k_gemm_splitk(Operand A, Operand B, 
   const int64_t shift = k_len > 0 ? k_begin : 0;
   A.ptr += AKM ? shift * A.ld : shift;
   B.ptr += BKM ? shift * B.ld : shift;
-  Acc acc;
-  mainloop<AKM, BKM>(A, B, k_len, m0, n0, acc, lds);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int M = A.rows, N = B.rows;
   float* C = part + (int64_t)split * plane;
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int n = n0 + wn * 128 + acc_col(nt, lane);
-    if (n >= N) continue;
-    float* row = C + n * ldc;
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int m = m0 + wm * 128 + mt * 32 + 8 * g4 + 4 * (lane >> 5);  // M % 4 == 0
-        if (m >= M) continue;
-        const f32x4_t v = {acc.v[mt][nt][g4 * 4], acc.v[mt][nt][g4 * 4 + 1], acc.v[mt][nt][g4 * 4 + 2], acc.v[mt][nt][g4 * 4 + 3]};
-        *(f32x4_t*)(row + m) = v;
-      }
+  const bool narrow_m = A.rows - m0 <= BM / 2;
+  int columns = B.rows;
+  if constexpr (BOUNDED) columns = bounds[kRowsTotal] < columns ? bounds[kRowsTotal] : columns;
+  if (columns - n0 <= BN / 2) {
+    if (narrow_m)
+      gemm_plane_tile<AKM, BKM, 2, 2>(A, B, k_len, m0, n0, C, ldc, lds);
+    else
+      gemm_plane_tile<AKM, BKM, 4, 2>(A, B, k_len, m0, n0, C, ldc, lds);
+  } else if (narrow_m) {
+    gemm_plane_tile<AKM, BKM, 2, 4>(A, B, k_len, m0, n0, C, ldc, lds);
+  } else {
+    gemm_plane_tile<AKM, BKM, 4, 4>(A, B, k_len, m0, n0, C, ldc, lds);
   }
 }
 

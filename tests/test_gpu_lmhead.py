@@ -102,6 +102,33 @@ def test_backward_matches_autograd_of_oracle(device, T, H, V, temperature, with_
     assert_same_magnitude(w_d.grad, w_o.grad, what="d(W)")
 
 
+@pytest.mark.parametrize("backward", ["carry", "recompute"])
+@pytest.mark.parametrize("T,H,V", [
+    (1, 8, 1088), (128, 128, 1088), (129, 136, 1097),     # one tile: narrow both ways, wide both ways
+    (384, 384, 1088), (385, 392, 1001),                    # the last of two: 128 in use, 129 in use
+    (300, 640, 16640), (70, 264, 16643), (200, 320, 16640),  # the same with d(hidden) cut along the vocabulary
+])
+def test_last_row_and_column_of_tiles(device, backward, T, H, V):
+    """Tiles with at most 128 of their 256 tokens, or hidden entries, in use run as narrow ones."""
+    hidden, weight, labels = _case(T, H, V, seed=T + H + V, w_std=0.3 / math.sqrt(H / 64))
+    g = torch.randn(T, generator=torch.Generator().manual_seed(T))
+    h_d, w_d = hidden.to(device).requires_grad_(True), weight.to(device).requires_grad_(True)
+    lp, ent, vmin, vmax = areal_amd.lm_head_logprobs_entropy_stats(h_d, w_d, labels.to(device), backward=backward)
+    (lp * g.to(device)).sum().backward()
+    h_o, w_o = hidden.float().requires_grad_(True), weight.float().requires_grad_(True)
+    logits = oracle.lmhead_logits(h_o, w_o)
+    r_lp, r_ent = oracle.logprobs_entropy_f64(logits.detach(), labels, 1.0)
+    # fp32 sums of at most 640 products and of 16 643 exponentials: 2e-5 of values around 10
+    assert float((lp.detach().cpu().double() - r_lp).abs().max()) < 1e-4
+    assert float((ent.detach().cpu().double() - r_ent).abs().max()) < 1e-4
+    assert_within(vmax, logits.detach().max(-1).values, 1e-4, "largest logit")
+    assert_within(vmin, logits.detach().min(-1).values, 1e-4, "smallest logit")
+    (oracle.logprobs_entropy(logits, labels, 1.0)[0] * g).sum().backward()
+    assert cosine(h_d.grad.cpu(), h_o.grad) > 0.9999 and cosine(w_d.grad.cpu(), w_o.grad) > 0.9999
+    assert_same_magnitude(h_d.grad, h_o.grad, what="d(hidden)")
+    assert_same_magnitude(w_d.grad, w_o.grad, what="d(W)")
+
+
 def test_lm_head_into_ppo_loss_end_to_end(device):
     """hidden -> fused lm_head -> PPO loss -> backward, against the oracle pipeline on materialised logits."""
     T, H, V = 384, 128, 1600
