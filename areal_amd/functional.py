@@ -1283,11 +1283,19 @@ class _FusedLmHeadPpo(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, step, labels, temperature, kept_per_chunk, backward_mode):
         lib = N.load()
-        kept = None if kept_per_chunk is None else (C.c_int64 * len(kept_per_chunk))(*kept_per_chunk)
         T, H = hidden.shape
         V = weight.shape[0]
         dev = step.device
-        d_hidden = torch.empty_like(hidden)
+        # Batch padding has no outputs and a zero gradient: it stays out of the tiles where that makes them fewer (tiles
+        # end at multiples of 128 tokens).  4 096 + 56 tokens x 1 536 x 151 936: 4 112 us a step with, 3 973 without the
+        # padding; elsewhere clearing its gradient rows in a launch of their own would only cost, about 4 us.
+        if 0 < step.T_active and (step.T_active + 127) // 128 < (T + 127) // 128:
+            T = step.struct.T = step.T_active
+            if kept_per_chunk is not None:
+                chunk = lm_head_chunk_tokens()
+                kept_per_chunk = kept_per_chunk[: (T + chunk - 1) // chunk]
+        kept = None if kept_per_chunk is None else (C.c_int64 * len(kept_per_chunk))(*kept_per_chunk)
+        d_hidden = _empty_hidden_gradient(hidden, T)
         d_weight = torch.empty_like(weight)  # bf16: rounded once, after fp32 accumulation over the chunks
         ws = _lmhead_workspace(T, H, V, dev)
         with _on(dev):

@@ -439,6 +439,33 @@ def test_padding_only_chunk_and_no_active_token(device):
     assert float(loss.detach()) == 0.0 and float(x.grad.float().abs().sum()) == 0.0
 
 
+@pytest.mark.parametrize("counts", ["device", "host", "dense"])
+@pytest.mark.parametrize("T_pad,T", [(520, 256), (300, 260), (CHUNK + 130, CHUNK), (257, 1)])
+def test_batch_padding_stays_out_of_the_tiles(device, T_pad, T, counts):
+    """The step on a padded micro-batch is the step on its tokens, bit for bit, with zero gradient rows behind them,
+    whatever the padding holds."""
+    hidden, weight, labels, prox, old, adv, mask = (t.to(device) for t in _inputs(T_pad, T, 64, 1097, seed=T))
+    hidden[T:] = float("nan")
+    if T == 1:
+        mask[:] = True
+    out = []
+    for rows in (T, T_pad):
+        h, w = hidden[:rows].clone().requires_grad_(True), weight.clone().requires_grad_(True)
+        kw = dict(skip_masked_tokens=False) if counts == "dense" else {}
+        if counts == "host":
+            kw["kept_per_chunk"] = [int(mask[c:c + CHUNK].sum()) for c in range(0, rows, CHUNK)]
+        loss, stat = areal_amd.fused_lm_head_ppo_loss(h, w, labels[:rows], prox, old, adv, 0.2, mask, c_clip=3.0, **kw)
+        loss.backward()
+        out.append((loss.detach(), stat, h.grad, w.grad))
+    (l0, s0, h0, w0), (l1, s1, h1, w1) = out
+    trimmed = (T + 127) // 128 < (T_pad + 127) // 128
+    assert torch.equal(l0, l1) and torch.equal(h0, h1[:T]) and float(h1[T:].abs().sum()) == 0.0
+    for k in s0:
+        assert torch.equal(s0[k], s1[k]), k
+    if trimmed or counts != "dense":  # a dense backward multiplies the padding's hidden rows through, by zeros
+        assert torch.equal(w0, w1)
+
+
 @pytest.mark.parametrize("pattern", ["random", "second_chunk_masked", "first_chunk_masked", "all_masked", "one_token",
                                      "random_long_rows"])
 def test_skipping_masked_tokens_equals_the_dense_backward(device, pattern):
