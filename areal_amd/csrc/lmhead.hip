@@ -21,6 +21,8 @@
 //               GEMM and no pass over the panel.  A chunk that holds a token whose label is too unlikely for that
 //               range (log-prob below -80) is redone by the recompute tiles, decided on the device.
 // Tokens whose loss mask is zero have a zero gradient row: they are left out of the panel and of both GEMMs.
+#include <type_traits>
+
 #include "device_utils.h"
 #include "gemm_tn.h"
 #include "ppo_math.h"
@@ -150,65 +152,104 @@ struct PanelOut {
   }
 };
 
+// Softmax partial of some of a token's logits: k = max x c, s = sum 2^(x c - k), u = sum (x c - k) 2^(x c - k), and the
+// smallest raw logit
+struct Partial {
+  float k, s, u, mn;
+};
+
+// The partials of two tokens, each spread over two halves of the wave (ROWS16: over neighbouring rows of 16 lanes), brought
+// together: the lower half (even rows) is left with the first token, the upper half (odd rows) with the second.
+template <bool ROWS16, bool MIN>
+__device__ __forceinline__ Partial merge_lanes(const Partial& a, const Partial& b) {
+  auto swap = [](float x, float y, float& p, float& q) {
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    u32x2_t r;
+    if constexpr (ROWS16)
+      r = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false));
+    else
+      r = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false));
+    p = __uint_as_float(r[0]);
+    q = __uint_as_float(r[1]);
+  };
+  Partial x, y, m;
+  swap(a.k, b.k, x.k, y.k);
+  swap(a.s, b.s, x.s, y.s);
+  swap(a.u, b.u, x.u, y.u);
+  m.k = fmaxf(x.k, y.k);
+  const float dx = x.k - m.k, dy = y.k - m.k;
+  const float fx = fast_exp2(dx), fy = fast_exp2(dy);
+  m.u = fx * fmaf(dx, x.s, x.u) + fy * fmaf(dy, y.s, y.u);
+  m.s = x.s * fx + y.s * fy;
+  m.mn = FLT_MAX;
+  if constexpr (MIN) {
+    swap(a.mn, b.mn, x.mn, y.mn);
+    m.mn = fminf(x.mn, y.mn);
+  }
+  return m;
+}
+
 // Statistics (and, with CARRY, the staged probability ratios) of one wave's 128 x 16 NT block, accumulators in the
 // 16 x 16 tile layout: a lane holds, for each of NT tokens (nt), 8 runs (mt) of 4 consecutive vocabulary rows, and the
 // lanes l ^ 16, l ^ 32 hold the other rows of the same tokens.  RAGGED: the block may reach past the vocabulary (last
 // tile row only), rows at or past V are left out.
-template <bool CARRY, bool RAGGED, int NT>
-__device__ __forceinline__ void block_stats(const Acc16<NT>& acc, const TileArgs& a, int tm, int wm, int wn, int n0, int N,
+// A lane reduces its 32 values of a token relative to their own maximum, so that no lane waits for another between the
+// tokens; the four lanes of a token are brought together at the end, four tokens to a merge, which leaves token `lane` of
+// 64 in every lane.  MIN: the caller wants the smallest logit of every token as well.
+// Bound by its vector instructions (an exponential at a quarter of the rate and nine others per logit: 9 k cycles a tile).
+// With the maximum of all four lanes first, six shuffles through LDS and a store per 16 tokens, one after the other, it took
+// 5 k more.  us, so / now: forward 4 096 x 1 536 x 151 936: 1 575 / 1 470, 16 384 x 4 096: 14 406 / 14 055, 1 900 x 1 024 x
+// 50 257: 205 / 195; steps 4 080 / 3 989, 36 138 / 35 841, 587 / 574.  Error against 64 bits as before (log-prob 5-7e-7,
+// entropy 6-7e-7 root mean square, H = 512 to 5 376).
+template <bool CARRY, bool RAGGED, bool MIN, int NT>
+__device__ __forceinline__ void block_stats(Acc16<NT>& acc, const TileArgs& a, int tm, int wm, int wn, int n0, int N,
                                             int V, int mbase, int lane, float kref_a, float kref_b, PanelOut& po) {
+  Partial part[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
-    const int n = n0 + wn * (16 * NT) + acc16_col(nt, lane);
-    float mx = -FLT_MAX;
-    if constexpr (!RAGGED) {
+    float mx = -FLT_MAX, mn = FLT_MAX;
+    // not read from the accumulation registers before their turn: there is no room for all of them in the other half
 #pragma unroll
-      for (int mt = 0; mt < kAcc16Tiles; ++mt)
+    for (int mt = 0; mt < kAcc16Tiles; ++mt) pin_accumulators(acc.v[mt][nt]);
 #pragma unroll
-        for (int i = 0; i < 4; i += 2) mx = fmaxf(fmaxf(mx, acc.v[mt][nt][i]), acc.v[mt][nt][i + 1]);  // one v_max3 per pair
-    } else {
+    for (int mt = 0; mt < kAcc16Tiles; ++mt)
 #pragma unroll
-      for (int mt = 0; mt < kAcc16Tiles; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) mx = (mbase + acc16_row(mt, i, lane) < V) ? fmaxf(mx, acc.v[mt][nt][i]) : mx;
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));  // four lanes hold the same token
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-    if (a.pn) {  // uniform: the caller wants the smallest logit of every token as well
-      float mn = FLT_MAX;
-      if constexpr (!RAGGED) {
-#pragma unroll
-        for (int mt = 0; mt < kAcc16Tiles; ++mt)
-#pragma unroll
-          for (int i = 0; i < 4; i += 2) mn = fminf(fminf(mn, acc.v[mt][nt][i]), acc.v[mt][nt][i + 1]);
-      } else {
-#pragma unroll
-        for (int mt = 0; mt < kAcc16Tiles; ++mt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) mn = (mbase + acc16_row(mt, i, lane) < V) ? fminf(mn, acc.v[mt][nt][i]) : mn;
+      for (int i = 0; i < 4; i += 2) {
+        const float x0 = acc.v[mt][nt][i], x1 = acc.v[mt][nt][i + 1];
+        if constexpr (!RAGGED) {
+          mx = fmaxf(fmaxf(mx, x0), x1);  // one v_max3 per pair
+          if constexpr (MIN) mn = fminf(fminf(mn, x0), x1);
+        } else {
+          const bool in0 = mbase + acc16_row(mt, i, lane) < V, in1 = mbase + acc16_row(mt, i + 1, lane) < V;
+          mx = in0 ? fmaxf(mx, x0) : mx;
+          mx = in1 ? fmaxf(mx, x1) : mx;
+          if constexpr (MIN) {
+            mn = in0 ? fminf(mn, x0) : mn;
+            mn = in1 ? fminf(mn, x1) : mn;
+          }
+        }
       }
-      mn = fminf(mn, __shfl_xor(mn, 16, kWave));
-      mn = fminf(mn, __shfl_xor(mn, 32, kWave));
-      if (lane < 16 && n < N) a.pn[(int64_t)(tm * 2 + wm) * a.pitch_t + n] = mn;  // FLT_MAX: no valid row in this block
-    }
-    const float k = fmaxf(mx * a.c, kNegBig);   // kNegBig: no valid row in this block
-    float to_ref = 1.f;                         // 2^(k - kref): block-relative -> label-relative exponentials
+    const float k = fmaxf(mx * a.c, kNegBig);  // kNegBig: no valid row in this lane
+    float to_ref = 1.f;                        // 2^(k - kref): lane-relative -> label-relative exponentials
     if constexpr (CARRY) {
       const float kref = __shfl(nt < 4 ? kref_a : kref_b, 16 * (nt & 3) + (lane & 15), kWave);
-      // a label outside the vocabulary has no logit (NaN): keep the block-relative values, the row's factor is NaN or 0
+      // a label outside the vocabulary has no logit (NaN): whatever is kept, the row's factor is NaN or 0
       to_ref = fabsf(kref) < 1e30f ? fast_exp2(fminf(k - kref, kCarryMaxShift)) : 1.f;
     }
     float s = 0.f, u = 0.f;
 #pragma unroll
     for (int mt = 0; mt < kAcc16Tiles; ++mt) {
-      float e[4];
+      float e[4], t[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float t = fmaf(acc.v[mt][nt][q], a.c, -k);
-        e[q] = fast_exp2(t);
+        t[q] = fmaf(acc.v[mt][nt][q], a.c, -k);
+        e[q] = fast_exp2(t[q]);
         if constexpr (RAGGED) e[q] = (mbase + acc16_row(mt, q, lane) < V) ? e[q] : 0.f;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
         s += e[q];
-        u = fmaf(t, e[q], u);
+        u = fmaf(t[q], e[q], u);
       }
       if constexpr (CARRY) {
         uint2 pk;
@@ -221,24 +262,31 @@ __device__ __forceinline__ void block_stats(const Acc16<NT>& acc, const TileArgs
       if (nt > 0) po.store();
       po.take(nt);
     }
-    s += __shfl_xor(s, 16, kWave);
-    s += __shfl_xor(s, 32, kWave);
-    u += __shfl_xor(u, 16, kWave);
-    u += __shfl_xor(u, 32, kWave);
-    if (lane < 16 && n < N) {
-      const int64_t at = (int64_t)(tm * 2 + wm) * a.pitch_t + n;
-      a.pk[at] = k;
-      a.ps[at] = s;
-      a.pu[at] = u;
-    }
+    // formed here: the compiler would otherwise put the sums off to where they are merged, and keep every term until then
+    asm volatile("" : "+v"(s), "+v"(u), "+v"(mn));
+    part[nt] = {k, s, u, mn};
   }
   if constexpr (CARRY) po.store();
+#pragma unroll
+  for (int h = 0; h < NT / 4; ++h) {
+    const Partial p02 = merge_lanes<false, MIN>(part[4 * h], part[4 * h + 2]);
+    const Partial p13 = merge_lanes<false, MIN>(part[4 * h + 1], part[4 * h + 3]);
+    const Partial m = merge_lanes<true, MIN>(p02, p13);
+    const int n = n0 + wn * (16 * NT) + 64 * h + lane;
+    if (n < N) {
+      const int64_t at = (int64_t)(tm * 2 + wm) * a.pitch_t + n;
+      a.pk[at] = m.k;
+      a.ps[at] = m.s;
+      a.pu[at] = m.u;
+      if constexpr (MIN) a.pn[at] = m.mn;  // FLT_MAX: no valid row in this block
+    }
+  }
 }
 
 // One tile of 256 x 32 NT: rows m = vocabulary (operand A = weight), columns n = tokens (operand B = hidden states), so
 // that everything a token needs from the tile sits in one lane and its partner lanes ^ 16, ^ 32.  Both operands are
 // K-contiguous: the 16 x 16 x 32 main loop.
-template <int MODE, int NT>
+template <int MODE, bool MIN, int NT>
 __device__ __forceinline__ void lmhead_tile(const Operand& W, const Operand& Hd, int K, int tm, int n0, const TileArgs& a, char* lds) {
   const int m0 = tm * BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -265,9 +313,9 @@ __device__ __forceinline__ void lmhead_tile(const Operand& W, const Operand& Hd,
 
   if constexpr (MODE != kModeRecompute) {
     if (m0 + BM > V)  // rows past the vocabulary: last tile row only
-      block_stats<MODE == kModeStatsCarry, true, NT>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
+      block_stats<MODE == kModeStatsCarry, true, MIN, NT>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
     else
-      block_stats<MODE == kModeStatsCarry, false, NT>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
+      block_stats<MODE == kModeStatsCarry, false, MIN, NT>(acc, a, tm, wm, wn, n0, N, V, mbase, lane, kref_a, kref_b, po);
   } else {
     const bool ragged_rows = m0 + BM > V;
 #pragma unroll
@@ -320,7 +368,7 @@ __device__ __forceinline__ void lmhead_tile(const Operand& W, const Operand& Hd,
 // A last column of tiles with at most 128 tokens is one of narrow tiles: that is as many as they hold, and up to there they
 // are the shorter ones.  Forward, us wide / narrow: 4 160 x 1 536 x 151 936: 1 650 / 1 600, 8 000 x 2 048: 3 943 / 3 899,
 // 1 900 x 1 024 x 50 257: 220 / 209, 100 x 2 048 x 151 936: 190 / 163.
-template <int MODE>
+template <int MODE, bool MIN>
 __global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd, int K, int tiles_m, int tiles_n,
                                                                  TileArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -343,9 +391,9 @@ __global__ __launch_bounds__(kThreads) void k_lmhead_tiles(Operand W, Operand Hd
   tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int n0 = tn * BN;
   if (columns - n0 > BN / 2)  // uniform
-    lmhead_tile<MODE, kWide>(W, Hd, K, tm, n0, a, lds);
+    lmhead_tile<MODE, MIN, kWide>(W, Hd, K, tm, n0, a, lds);
   else
-    lmhead_tile<MODE, kNarrow>(W, Hd, K, tm, n0, a, lds);
+    lmhead_tile<MODE, MIN, kNarrow>(W, Hd, K, tm, n0, a, lds);
 }
 
 // Raw label logit of every token: xy[t] = hidden[t] . weight[label[t]] in fp32 (NaN for a label outside [0, V)).  One
@@ -1110,8 +1158,10 @@ static bool prepare_kernels() {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
   if (done[dev]) return true;
-  const bool ok = allow_big_lds(k_lmhead_tiles<kModeStats>) && allow_big_lds(k_lmhead_tiles<kModeStatsCarry>) &&
-                  allow_big_lds(k_lmhead_tiles<kModeRecompute>) &&
+  const bool ok = allow_big_lds(k_lmhead_tiles<kModeStats, false>) && allow_big_lds(k_lmhead_tiles<kModeStats, true>) &&
+                  allow_big_lds(k_lmhead_tiles<kModeStatsCarry, false>) &&
+                  allow_big_lds(k_lmhead_tiles<kModeStatsCarry, true>) &&
+                  allow_big_lds(k_lmhead_tiles<kModeRecompute, false>) &&
                   allow_big_lds(k_gemm_store<true, false, uint16_t, false, kBoundNone>) &&
                   allow_big_lds(k_gemm_store<true, false, uint16_t, false, kBoundN>) &&
                   allow_big_lds(k_gemm_store<true, true, uint16_t, false, kBoundNone>) &&
@@ -1145,8 +1195,14 @@ static void launch_tiles(hipStream_t st, const void* weight, const uint16_t* hid
   const int tiles_m = (int)((V + BM - 1) / BM), tiles_n = (int)((n_tok + BN - 1) / BN);
   Operand W{(const uint16_t*)weight, H, (int)V};
   Operand Hd{hid, H, (int)n_tok};
-  hipLaunchKernelGGL(k_lmhead_tiles<MODE>, dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads), kLdsBytes, st,
-                     W, Hd, (int)H, tiles_m, tiles_n, a);
+  const dim3 grid((unsigned)(tiles_m * tiles_n)), group(kThreads);
+  if constexpr (MODE != kModeRecompute) {
+    if (a.pn) {
+      hipLaunchKernelGGL((k_lmhead_tiles<MODE, true>), grid, group, kLdsBytes, st, W, Hd, (int)H, tiles_m, tiles_n, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_lmhead_tiles<MODE, false>), grid, group, kLdsBytes, st, W, Hd, (int)H, tiles_m, tiles_n, a);
 }
 
 // C [N, M] = B . A^T over K (rows of C through c_rows when given); lda / ldb: leading dimensions of the arrays as stored.
