@@ -38,13 +38,10 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // token chunk of the panel.  Measured: with 32768 the forward tiles run 2.4 % slower at H = 4096 (the hidden rows of
 // a chunk, 2 * chunk * H bytes, no longer fit the 256 MB memory-side cache that every band of tiles re-reads them from)
 constexpr int kChunkTokens = 16384;
-constexpr int kPanelPitch = BM + 8;        // pitch (elements) of the tile staged in LDS as [token][vocab]
-constexpr int kStageBytes = 256 * kPanelPitch * 2;  // 135168 B, inside the 160 KiB the main loop uses
-static_assert(kStageBytes + 256 * 4 <= kLdsBytes, "the staged tile and its 256 row numbers must fit the main loop's LDS");
-constexpr int kStripTokens = 16;           // tokens of a wave's strip of panel values staged in LDS
-constexpr int kStripPitch = 128 + 8;       // pitch (elements) of such a strip, [token][vocab]
-constexpr int kWaveStageBytes = kStripTokens * kStripPitch * 2 + 128 * 4;  // one strip and the panel rows of 128 tokens
-static_assert(kWaveStageBytes % 16 == 0 && 4 * kWaveStageBytes <= kLdsBytes, "the strips of four waves share the main loop's LDS");
+constexpr int kStripPitch = 128 + 8;  // pitch (elements) of a wave's strip of values staged in LDS, [token][column]
+// LDS of one wave: a strip of `rows` tokens and the row numbers of its 128 tokens
+constexpr int strip_bytes(int rows) { return rows * kStripPitch * 2 + 128 * 4; }
+static_assert(strip_bytes(32) % 16 == 0 && 4 * strip_bytes(32) <= kLdsBytes, "the strips of four waves share the main loop's LDS");
 
 __host__ __device__ __forceinline__ int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
@@ -99,55 +96,66 @@ constexpr float kCarryMinLogp = -80.f;
 // entry has to stay a normal number (above 2^-126) for entries down to 2^-26 of magnitude, or the chunk is redone
 constexpr float kCarryMinFactor = 0x1p-100f;
 
-// How a wave's 128 x 128 block of panel values leaves: in strips of 16 tokens (one column of accumulator tiles) through a
+// How a wave's block of bf16 values leaves: in strips of ROWS tokens (one column of accumulator tiles, 16 or 32) through a
 // piece of LDS that is the wave's own, so that its waves do not wait for each other and the stores of a strip are issued
-// behind the arithmetic of the next one.  A store instruction covers four panel rows of 256 bytes each.  The row numbers
-// are looked up before the main loop and shared through LDS, four to a read.  (With the whole tile staged, a barrier and a
+// behind the arithmetic of the next one.  A store instruction covers four rows of 256 bytes each.  The row numbers of
+// the panel are looked up before the main loop and shared through LDS, four to a read.  (With the whole tile staged, a barrier and a
 // loop that looked up the row of every piece, those lookups and the label logits asked for column by column were a serial
 // chain of some 40 waits on memory per tile.  The tiles that also write the panel, 4 096 x 1 536 x 151 936: 1 890 us so,
 // 1 800 now; H = 1 024: 1 515 and 1 420; H = 4 096: 3 930 and 3 840.  The `nt` policy leaves the softmax partials in the
 // caches: the merge behind these tiles takes 27 us instead of 30.)  Bound by the stores: every compute unit has its
 // 128 KB at about the same time.
-struct PanelOut {
-  char* stage;      // kWaveStageBytes of the wave
-  uint16_t* out;    // panel, at this lane's piece of eight vocabulary entries
+// The gradient products leave the same way, in strips of 32.  What they gain is the end of the launch: with plain stores
+// the L2s are full of lines to write back when the last tiles are through.  Steps, us, whole tile staged / strips with plain
+// stores / strips: 1 900 x 1 024 x 50 257: 566 / 573 / 518, 700 x 3 584 x 100 000: 1 288 / 1 293 / 1 151, 2 000 x 600 x
+// 64 000: 493 / 507 / 467, 4 096 x 1 536 x 151 936: 3 782 / 3 856 / 3 760, 16 384 x 4 096: 35 310 / 36 627 / 35 241 (two
+// runs).  The fp32 planes of a cut product and the softmax partials, which the next launch reads, are better off with plain
+// stores (518 / 548 and 587).
+template <int ROWS>
+struct StripOut {
+  static constexpr int kBytes = strip_bytes(ROWS);
+  char* stage;      // kBytes of the wave
+  uint16_t* out;    // the array, at this lane's piece of eight columns
   int64_t ld;
-  bool live;        // the piece starts inside the vocabulary (it ends inside the row's pitch)
+  bool live;        // the piece starts inside the array's columns (it ends inside the row's pitch)
   int lane;
-  u32x4_t piece[4];
-  int row[4];
+  u32x4_t piece[ROWS / 4];
+  int row[ROWS / 4];
 
   __device__ __forceinline__ uint16_t* strip() { return (uint16_t*)stage; }
-  __device__ __forceinline__ int32_t* rows() { return (int32_t*)(stage + kStripTokens * kStripPitch * 2); }
-  // ra, rb: panel rows of the wave's tokens `lane` and 64 + `lane` (negative: none)
-  __device__ __forceinline__ void open(char* lds, int wave, int lane_, uint16_t* panel, int64_t ld_, int m, int V, int ra, int rb) {
+  __device__ __forceinline__ int32_t* rows() { return (int32_t*)(stage + ROWS * kStripPitch * 2); }
+  // columns m ... of the array, `width` of them the wave's, M of them the array's; ra, rb: rows of the wave's tokens `lane`
+  // and 64 + `lane` (negative: none)
+  __device__ __forceinline__ void open(char* lds, int wave, int lane_, uint16_t* array, int64_t ld_, int m, int width, int M,
+                                       int ra, int rb) {
     lane = lane_;
-    stage = lds + wave * kWaveStageBytes;
-    m += 8 * (lane & 15);
-    out = panel + m;
+    stage = lds + wave * kBytes;
+    const int at = 8 * (lane & 15);
+    out = array + m + at;
     ld = ld_;
-    live = m < V;
+    live = at < width && m + at < M;
     rows()[lane] = ra;
     rows()[64 + lane] = rb;
   }
-  // four consecutive vocabulary entries of the strip's token lane % 16: rows 16 mt + 4 (lane / 16) ... of the block
-  __device__ __forceinline__ void put(int mt, uint2 v) {
-    *(uint2*)(strip() + (lane & 15) * kStripPitch + acc16_row(mt, 0, lane)) = v;
-  }
+  // four consecutive columns, from m of the wave's block, of token t of the strip
+  __device__ __forceinline__ void put(int t, int m, uint2 v) { *(uint2*)(strip() + t * kStripPitch + m) = v; }
   // LDS serves a wave's accesses in order, so what the other lanes put is there without a wait; the compiler must not
   // move the accesses across each other
   __device__ __forceinline__ void take(int nt) {
     asm volatile("" ::: "memory");
-    const int t0 = 4 * (lane >> 4);
-    const int4 r = *(const int4*)(rows() + nt * kStripTokens + t0);
-    row[0] = r.x; row[1] = r.y; row[2] = r.z; row[3] = r.w;
+    const int t0 = ROWS / 4 * (lane >> 4);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) piece[j] = *(const u32x4_t*)(strip() + (t0 + j) * kStripPitch + 8 * (lane & 15));
+    for (int j = 0; j < ROWS / 4; j += 4) {
+      const int4 r = *(const int4*)(rows() + nt * ROWS + t0 + j);
+      row[j] = r.x; row[j + 1] = r.y; row[j + 2] = r.z; row[j + 3] = r.w;
+    }
+#pragma unroll
+    for (int j = 0; j < ROWS / 4; ++j) piece[j] = *(const u32x4_t*)(strip() + (t0 + j) * kStripPitch + 8 * (lane & 15));
     asm volatile("" ::: "memory");
   }
   __device__ __forceinline__ void store() {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < ROWS / 4; ++j)
       if (live && row[j] >= 0) __builtin_nontemporal_store(piece[j], (u32x4_t*)(out + (int64_t)row[j] * ld));
   }
 };
@@ -203,7 +211,7 @@ __device__ __forceinline__ Partial merge_lanes(const Partial& a, const Partial& 
 // entropy 6-7e-7 root mean square, H = 512 to 5 376).
 template <bool CARRY, bool RAGGED, bool MIN, int NT>
 __device__ __forceinline__ void block_stats(Acc16<NT>& acc, const TileArgs& a, int tm, int wm, int wn, int n0, int N,
-                                            int V, int mbase, int lane, float kref_a, float kref_b, PanelOut& po) {
+                                            int V, int mbase, int lane, float kref_a, float kref_b, StripOut<16>& po) {
   Partial part[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -255,7 +263,7 @@ __device__ __forceinline__ void block_stats(Acc16<NT>& acc, const TileArgs& a, i
         uint2 pk;
         pk.x = Elem<AA_BF16>::pack(e[0] * to_ref, e[1] * to_ref);
         pk.y = Elem<AA_BF16>::pack(e[2] * to_ref, e[3] * to_ref);
-        po.put(mt, pk);
+        po.put(lane & 15, acc16_row(mt, 0, lane), pk);
       }
     }
     if constexpr (CARRY) {
@@ -308,8 +316,8 @@ __device__ __forceinline__ void lmhead_tile(const Operand& W, const Operand& Hd,
   Acc16<NT> acc;
   mainloop16<NT>(W, Hd, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
 
-  PanelOut po;
-  if constexpr (MODE != kModeStats) po.open(lds, wave, lane, a.panel, a.panel_ld, mbase, V, row_a, row_b);
+  StripOut<16> po;
+  if constexpr (MODE != kModeStats) po.open(lds, wave, lane, a.panel, a.panel_ld, mbase, 128, V, row_a, row_b);
 
   if constexpr (MODE != kModeRecompute) {
     if (m0 + BM > V)  // rows past the vocabulary: last tile row only
@@ -356,7 +364,7 @@ __device__ __forceinline__ void lmhead_tile(const Operand& W, const Operand& Hd,
         uint2 pk;
         pk.x = Elem<AA_BF16>::pack(o[0], o[1]);
         pk.y = Elem<AA_BF16>::pack(o[2], o[3]);
-        po.put(mt, pk);
+        po.put(lane & 15, acc16_row(mt, 0, lane), pk);
       }
       if (nt > 0) po.store();
       po.take(nt);
@@ -709,20 +717,26 @@ template <bool AKM, bool BKM, typename OutT, bool ACCUM, int MT, int NT>
 __device__ __forceinline__ void gemm_store_tile(const Operand& A, const Operand& B, int K, int m0, int n0, OutT* __restrict__ C,
                                                 int64_t ldc, const int32_t* __restrict__ c_rows,
                                                 const float* __restrict__ n_scale, char* lds) {
-  Acc<MT, NT> acc;
-  mainloop<AKM, BKM, MT, NT>(A, B, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int M = A.rows, N = B.rows;
+  const int mbase = m0 + wm * (32 * MT), nbase = n0 + wn * (32 * NT);  // the wave's block
+  Acc<MT, NT> acc;
+  mainloop<AKM, BKM, MT, NT>(A, B, K, m0, n0, acc, lds);  // ends with a barrier: LDS is free
   if constexpr (sizeof(OutT) == 2) {
-    uint16_t* Z = (uint16_t*)lds;  // [256 n][kPanelPitch] bf16
-    constexpr int PZ = kPanelPitch;
+    // row of C, and the optional factor per row, of the wave's n `lane` and (wide) 64 + `lane`
+    const int na = nbase + lane, nb = NT == 4 ? na + 64 : N;
+    const int row_a = na < N ? (c_rows ? c_rows[na] : na) : -1, row_b = nb < N ? (c_rows ? c_rows[nb] : nb) : -1;
+    const float f_a = n_scale && na < N ? n_scale[na] : 1.f, f_b = n_scale && nb < N ? n_scale[nb] : 1.f;
+    StripOut<32> out;
+    out.open(lds, wave, lane, (uint16_t*)C, ldc, mbase, 32 * MT, M, row_a, row_b);  // M % 8 == 0: a piece ends inside a row
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const int nloc = wn * (32 * NT) + acc_col(nt, lane);
-      // optional factor per row of C (a lane owns one n): applied to the fp32 sums, before the one rounding to bf16.  A
-      // factor of zero gives a zero row whatever the sums hold (a row without gradient may have summed to infinity)
-      const float f = (n_scale && n0 + nloc < N) ? n_scale[n0 + nloc] : 1.f;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) pin_accumulators(acc.v[mt][nt]);  // not read before their turn
+      // the factor (a lane owns one n) is applied to the fp32 sums, before the one rounding to bf16.  A factor of zero
+      // gives a zero row whatever the sums hold (a row without gradient may have summed to infinity)
+      const float f = __shfl(nt < 2 ? f_a : f_b, 32 * (nt & 1) + (lane & 31), kWave);
       const bool dead = f == 0.f;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
@@ -731,24 +745,12 @@ __device__ __forceinline__ void gemm_store_tile(const Operand& A, const Operand&
           uint2 pk;
           pk.x = dead ? 0u : Elem<AA_BF16>::pack(acc.v[mt][nt][g4 * 4] * f, acc.v[mt][nt][g4 * 4 + 1] * f);
           pk.y = dead ? 0u : Elem<AA_BF16>::pack(acc.v[mt][nt][g4 * 4 + 2] * f, acc.v[mt][nt][g4 * 4 + 3] * f);
-          *(uint2*)(Z + nloc * PZ + wm * (32 * MT) + mt * 32 + 8 * g4 + 4 * (lane >> 5)) = pk;
+          out.put(acc_col(0, lane), acc_row(mt, 4 * g4, lane), pk);
         }
+      if (nt > 0) out.store();
+      out.take(nt);
     }
-    int32_t* rows_lds = (int32_t*)(lds + 256 * PZ * 2);  // row of C of each of the tile's n (-1: past the end)
-    {
-      const int n = n0 + tid;
-      rows_lds[tid] = n < N ? (c_rows ? c_rows[n] : n) : -1;
-    }
-    __syncthreads();
-    const int mc = (tid & 31) * 8, m = m0 + mc;  // M % 8 == 0 (M is a hidden size): a piece never straddles the end
-    if (m < M) {
-#pragma unroll 8
-      for (int i = 0; i < 8 * NT; ++i) {
-        const int nloc = (tid >> 5) + 8 * i;
-        const int r = rows_lds[nloc];
-        if (r >= 0) *(u32x4_t*)(C + (int64_t)r * ldc + m) = *(const u32x4_t*)(Z + nloc * PZ + mc);
-      }
-    }
+    out.store();
   } else {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
