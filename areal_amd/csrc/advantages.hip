@@ -27,132 +27,196 @@ __device__ __forceinline__ T block_sum(T v, T* smem) {
 //     nv <- nv (1 - m_t) + v_t m_t;    lg <- lg (1 - m_t) + new m_t;    adv_t = lg
 // which is the affine map  nv' = a nv + e,  lg' = c nv + d lg + f  with
 //     a = 1 - m, e = m v, c = m gamma, d = 1 - m + m gamma lambda, f = m (r - v).
-// Affine maps compose, so a row can be cut into chunks whose composite maps are scanned in parallel.
+// Affine maps compose, so a row can be cut into pieces whose composite maps are scanned in parallel.  The numbers that
+// decay or add up along a row are composed in 64 bits: a rounding of gamma * lambda to the n-th is the same one in every
+// piece, and 2 500 positions of gamma lambda = 0.989 would be off by 1e-6 of the result where the recurrence itself is off
+// by 3e-7.  The recurrence is then walked in 32 bits as written, four positions from the state that enters them.
 // ------------------------------------------------------------------------------------------------------------------
 struct Affine {
-  float a, c, d, e, f;
+  float a, e;
+  double c, d, f;
 };
+
+__device__ __forceinline__ Affine identity() { return {1.f, 0.f, 0.0, 1.0, 0.0}; }
+
+__device__ __forceinline__ Affine position(float m, float r, float v, float gamma, float gl) {
+  return {1.f - m, m * v, (double)(m * gamma), (double)((1.f - m) + m * gl), (double)m * ((double)r - (double)v)};
+}
 
 // `first` is applied before `second`
 __device__ __forceinline__ Affine compose(const Affine& first, const Affine& second) {
   Affine r;
   r.a = second.a * first.a;
-  r.c = fmaf(second.c, first.a, second.d * first.c);
-  r.d = second.d * first.d;
   r.e = fmaf(second.a, first.e, second.e);
-  r.f = fmaf(second.c, first.e, fmaf(second.d, first.f, second.f));
+  r.c = fma(second.c, (double)first.a, second.d * first.c);
+  r.d = second.d * first.d;
+  r.f = fma(second.c, (double)first.e, fma(second.d, first.f, second.f));
   return r;
 }
 
-__device__ __forceinline__ Affine shfl_up(const Affine& x, int delta) {
-  Affine r;
-  r.a = __shfl_up(x.a, delta, kWave);
-  r.c = __shfl_up(x.c, delta, kWave);
-  r.d = __shfl_up(x.d, delta, kWave);
-  r.e = __shfl_up(x.e, delta, kWave);
-  r.f = __shfl_up(x.f, delta, kWave);
-  return r;
+// ---- lanes of a wave without LDS ---------------------------------------------------------------------------------
+// DPP controls: row_shr:n moves a value n lanes up inside its row of 16, row_bcast15 / 31 hand the last lane of a row / of
+// the lower half on to the rows named by the mask.  Lanes that are sent nothing get `old`.
+constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp(float old, float x) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp((int)__float_as_uint(old), (int)__float_as_uint(x), CTRL, ROWS, 0xf, false));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp(double old, double x) {
+  const uint2 b = __builtin_bit_cast(uint2, x), o = __builtin_bit_cast(uint2, old);
+  uint2 r;
+  r.x = (uint32_t)__builtin_amdgcn_update_dpp((int)o.x, (int)b.x, CTRL, ROWS, 0xf, false);
+  r.y = (uint32_t)__builtin_amdgcn_update_dpp((int)o.y, (int)b.y, CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(double, r);
+}
+// the sum over the wave, in its last lane
+__device__ __forceinline__ double last_lane_sum(double v) {
+  v += dpp<kRowShr + 1, 0xf>(0.0, v);
+  v += dpp<kRowShr + 2, 0xf>(0.0, v);
+  v += dpp<kRowShr + 4, 0xf>(0.0, v);
+  v += dpp<kRowShr + 8, 0xf>(0.0, v);
+  v += dpp<kRowBcast15, 0xa>(0.0, v);
+  v += dpp<kRowBcast31, 0xc>(0.0, v);
+  return v;
+}
+// one step of an inclusive scan: the maps of the lanes below are applied first; lanes that are sent nothing keep theirs
+template <int CTRL, int ROWS>
+__device__ __forceinline__ Affine scan_step(const Affine& x) {
+  Affine p;
+  p.a = dpp<CTRL, ROWS>(1.f, x.a);
+  p.e = dpp<CTRL, ROWS>(0.f, x.e);
+  p.c = dpp<CTRL, ROWS>(0.0, x.c);
+  p.d = dpp<CTRL, ROWS>(1.0, x.d);
+  p.f = dpp<CTRL, ROWS>(0.0, x.f);
+  return compose(p, x);
+}
+__device__ __forceinline__ Affine scan_row(Affine x) {  // over each row of 16 lanes
+  x = scan_step<kRowShr + 1, 0xf>(x);
+  x = scan_step<kRowShr + 2, 0xf>(x);
+  x = scan_step<kRowShr + 4, 0xf>(x);
+  return scan_step<kRowShr + 8, 0xf>(x);
+}
+__device__ __forceinline__ Affine shfl(const Affine& x, int from) {
+  return {__shfl(x.a, from, kWave), __shfl(x.e, from, kWave), __shfl(x.c, from, kWave), __shfl(x.d, from, kWave),
+          __shfl(x.f, from, kWave)};
 }
 
-// One workgroup per row, walking the row from its end in super-blocks of 256 x 16 positions.  A super-block is
-// copied into LDS with coalesced loads; thread k then owns the k-th chunk of 16 consecutive positions counted from
-// the end of the super-block (thread order = processing order), composes the maps of its chunk, an exclusive scan
-// over the 256 threads (wave scan + wave totals through LDS) gives the state entering the chunk, the thread walks
-// its chunk with the recurrence as written, and the results leave through LDS with coalesced stores.  Chunks are
-// padded by one word in LDS so that the 64 lanes of a wave, 16 positions apart, hit different banks.
-constexpr int kGaeThreads = 256;
-constexpr int kGaeChunk = 16;
-constexpr int kGaeBlock = kGaeThreads * kGaeChunk;                 // positions per super-block
-constexpr int kGaeLds = kGaeBlock + kGaeThreads;                   // + one pad word per chunk
+// The state (nv, lg) that enters a thread's positions: (nv0, lg0) through the maps of the threads before it.  One barrier;
+// `wave_tot` (LDS, one per wave) may be written again behind another one.
+template <int WAVES>
+__device__ __forceinline__ void enter(const Affine& mine, Affine* wave_tot, float nv0, float lg0, float& nv, float& lg) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  Affine inc = scan_row(mine);
+  inc = scan_step<kRowBcast15, 0xa>(inc);
+  inc = scan_step<kRowBcast31, 0xc>(inc);
+  if (lane == kWave - 1) wave_tot[wave] = inc;
+  __syncthreads();
+  // the maps of the waves before this one: every wave scans the totals in its first lanes
+  const Affine tot = scan_row(lane < WAVES ? wave_tot[lane] : identity());
+  Affine before = wave > 0 ? shfl(tot, wave - 1) : identity();
+  const Affine up = shfl(inc, lane > 0 ? lane - 1 : 0);
+  before = compose(before, lane > 0 ? up : identity());
+  nv = fmaf(before.a, nv0, before.e);
+  lg = (float)fma(before.c, (double)nv0, fma(before.d, (double)lg0, before.f));
+}
 
-__device__ __forceinline__ int gae_slot(int i) { return i + i / kGaeChunk; }
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(kGaeThreads) void k_gae(const float* __restrict__ rewards, const float* __restrict__ values,
-                                                     const float* __restrict__ mask, const uint8_t* __restrict__ no_eos,
-                                                     int64_t bs, int64_t L, float gamma, float lam,
-                                                     float* __restrict__ adv, float* __restrict__ returns) {
-  __shared__ float sr[kGaeLds], sv[kGaeLds], sm[kGaeLds];
-  __shared__ Affine wave_tot[kGaeThreads / kWave];
-  __shared__ float carry[2];
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  const int64_t row = blockIdx.x;
-  const float* r = rewards + row * L;
-  const float* v = values ? values + row * L : nullptr;
-  const float* m = mask + row * L;
-  float* out_a = adv + row * L;
-  float* out_r = returns ? returns + row * L : nullptr;
-  const float v_last = v ? v[L - 1] : 0.f;
-  if (tid == 0) {
-    out_a[L - 1] = 0.f;
-    if (out_r) out_r[L - 1] = v_last;
-    carry[0] = (no_eos && no_eos[row]) ? v_last : 0.f;   // nextvalues = values[:, L-1] * seq_no_eos_mask
-    carry[1] = 0.f;                                       // lastgaelam
+// A row in pieces of four positions that share 16 bytes of every array, blocks of one piece a thread from the end of the
+// row: the front of a block lies up to three positions before the row where that is what it takes, and inside it positions
+// are counted from there.  Thread 0 has the end of the block.
+constexpr int kOwn = 4;
+template <int THREADS>
+struct Block {
+  static constexpr int kPositions = THREADS * kOwn;
+  int own;          // place of the thread's first position
+  int lo_in, hi_in; // the row's part of the block
+  bool whole;       // the thread's piece is inside the row, and the arrays start on 16 bytes
+  int64_t at;       // position of the row at the block's front
+
+  __device__ __forceinline__ static int64_t first(int64_t r0, int64_t L) { return ((r0 + L + 3) & ~(int64_t)3) - r0 - kPositions; }
+  __device__ __forceinline__ Block(int64_t at_, int64_t L, bool aligned) {
+    at = at_;
+    own = (THREADS - 1 - (int)threadIdx.x) * kOwn;
+    lo_in = at < 0 ? (int)-at : 0;
+    hi_in = L - at < kPositions ? (int)(L - at) : kPositions;
+    whole = aligned && own >= lo_in && own + kOwn <= hi_in;
   }
-  const float gl = gamma * lam;
-  const Affine ident{1.f, 0.f, 1.f, 0.f, 0.f};
-  // positions 0 .. L-2, super-blocks aligned to the end: [base, base + cnt)
-  for (int64_t end = L - 1; end > 0; end -= kGaeBlock) {
-    const int64_t base = end > kGaeBlock ? end - kGaeBlock : 0;
-    const int cnt = (int)(end - base);
-    __syncthreads();  // the previous super-block has been written out; carry is visible
-    for (int i = tid; i < cnt; i += kGaeThreads) {
-      const int sl = gae_slot(i);
-      sr[sl] = r[base + i];
-      sv[sl] = v ? v[base + i] : 0.f;
-      sm[sl] = m[base + i];
-    }
-    __syncthreads();
-    // local index i = position - base; thread k owns [hi - 15, hi] with hi = cnt - 1 - 16 k (clipped at 0)
-    const int hi = cnt - 1 - tid * kGaeChunk;
-    const int lo = hi - kGaeChunk + 1 > 0 ? hi - kGaeChunk + 1 : 0;
-    Affine x = ident;
-    for (int i = hi; i >= lo; --i) {
-      const int sl = gae_slot(i);
-      const float mt = sm[sl], vt = sv[sl], rt = sr[sl];
-      Affine e;
-      e.a = 1.f - mt;
-      e.e = mt * vt;
-      e.c = mt * gamma;
-      e.d = (1.f - mt) + mt * gl;
-      e.f = mt * (rt - vt);
-      x = compose(x, e);
-    }
-    Affine inc = x;
+  __device__ __forceinline__ bool in(int o) const { return o >= lo_in && o < hi_in; }
+  __device__ __forceinline__ int place(int64_t t) const { return t >= at && t < at + kPositions ? (int)(t - at) : -1; }
+  // front: the array at the block's front; what lies outside the row comes as zeros and is not written
+  __device__ __forceinline__ void load(const float* front, float* x) const {
+    if (whole) {
+      const f32x4_t w = *(const f32x4_t*)(front + own);
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const Affine prev = shfl_up(inc, o);
-      if (lane >= o) inc = compose(prev, inc);
+      for (int q = 0; q < kOwn; ++q) x[q] = w[q];
+    } else {
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q) x[q] = in(own + q) ? front[own + q] : 0.f;
     }
-    if (lane == kWave - 1) wave_tot[wave] = inc;
-    const float nv0 = carry[0], lg0 = carry[1];
-    __syncthreads();
-    Affine before = ident;  // everything processed in this super-block before this thread's chunk
-    for (int w = 0; w < wave; ++w) before = compose(before, wave_tot[w]);
-    Affine excl = shfl_up(inc, 1);
-    if (lane == 0) excl = ident;
-    before = compose(before, excl);
-    float nv = fmaf(before.a, nv0, before.e);
-    float lg = fmaf(before.c, nv0, fmaf(before.d, lg0, before.f));
-    for (int i = hi; i >= lo; --i) {
-      const int sl = gae_slot(i);
-      const float mt = sm[sl], vt = sv[sl], rt = sr[sl];
-      const float delta = rt + gamma * nv - vt;
+  }
+  __device__ __forceinline__ void store(float* front, const float* x) const {
+    if (whole) {
+      const f32x4_t w = {x[0], x[1], x[2], x[3]};
+      *(f32x4_t*)(front + own) = w;
+    } else {
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q)
+        if (in(own + q)) front[own + q] = x[q];
+    }
+  }
+};
+
+constexpr int kShortRow = Block<256>::kPositions - 3;  // a block of 256 threads holds the row, whatever its place in a piece
+
+// One workgroup per row: a block's inputs are read once and held in registers until its results are written.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_gae(const float* __restrict__ rewards, const float* __restrict__ values,
+                                                 const float* __restrict__ mask, const uint8_t* __restrict__ no_eos,
+                                                 int64_t L, float gamma, float lam, int aligned, float* adv, float* returns) {
+  constexpr int kWaves = THREADS / kWave;
+  __shared__ Affine wave_tot[kWaves];
+  __shared__ float carry[2];
+  const int64_t row = blockIdx.x, r0 = row * L;
+  const float v_end = values ? values[r0 + L - 1] : 0.f;
+  const float gl = gamma * lam;
+  float nv0 = (no_eos && no_eos[row]) ? v_end : 0.f, lg0 = 0.f;  // nextvalues = values[:, L-1] * seq_no_eos_mask
+  for (int64_t at = Block<THREADS>::first(r0, L);; at -= Block<THREADS>::kPositions) {
+    const Block<THREADS> b(at, L, aligned != 0);
+    const int64_t front = r0 + at;
+    const int p_end = b.place(L - 1);
+    float m[kOwn], r[kOwn], v[kOwn] = {0.f, 0.f, 0.f, 0.f}, out[kOwn], ret[kOwn];
+    b.load(rewards + front, r);
+    b.load(mask + front, m);
+    if (values) b.load(values + front, v);
+    Affine mine = identity();
+#pragma unroll
+    for (int q = kOwn - 1; q >= 0; --q) {
+      if (b.own + q == p_end) m[q] = r[q] = v[q] = 0.f;  // the last position is the identity, as what lies outside the row
+      mine = compose(mine, position(m[q], r[q], v[q], gamma, gl));
+    }
+    float nv, lg;
+    enter<kWaves>(mine, wave_tot, nv0, lg0, nv, lg);
+#pragma unroll
+    for (int q = kOwn - 1; q >= 0; --q) {
+      const float delta = r[q] + gamma * nv - v[q];
       const float newlg = delta + gl * lg;
-      nv = nv * (1.f - mt) + vt * mt;
-      lg = lg * (1.f - mt) + newlg * mt;
-      sr[sl] = lg;        // advantages
-      sv[sl] = lg + vt;   // returns
+      nv = nv * (1.f - m[q]) + v[q] * m[q];
+      lg = lg * (1.f - m[q]) + newlg * m[q];
+      out[q] = b.own + q == p_end ? 0.f : lg;
+      ret[q] = b.own + q == p_end ? v_end : lg + v[q];
     }
-    if (tid == kGaeThreads - 1) {  // the last thread ends at the front of the super-block: its state carries on
+    b.store(adv + front, out);
+    if (returns) b.store(returns + front, ret);
+    if (at <= 0) return;
+    if (threadIdx.x == THREADS - 1) {  // the thread at the front of the block hands its state on
       carry[0] = nv;
       carry[1] = lg;
     }
     __syncthreads();
-    for (int i = tid; i < cnt; i += kGaeThreads) {
-      const int sl = gae_slot(i);
-      out_a[base + i] = sr[sl];
-      if (out_r) out_r[base + i] = sv[sl];
-    }
+    nv0 = carry[0];
+    lg0 = carry[1];
   }
 }
 
@@ -497,18 +561,22 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // ------------------------------------------------------------------------------------------------------------------
 // The advantage pipeline of a padded batch (PPOActor._compute_advantages, actor.py:172-236) in one pass per row: mask and
 // log-probs rolled and masked, KL-regularised rewards, the GAE scan, and the sums that the normalisation of the
-// advantages needs.  One workgroup per row, super-blocks of 4096 positions from the end as in k_gae: a super-block's
-// inputs are read once, what the scan needs of them stays in LDS.  With byte masks and a reference policy 10 bytes in per
-// token (14 with values) and 28 out (24 without a reference policy): 88 MB at 512 x 4096 with values, 14 us at the rate of
-// an even mix of reads and writes.  It takes 36 us, bound by the chain of a row (count of the attention bytes, loads, scan,
-// sums) on one-element memory instructions, some ten a token.  The separate launches (rolls, products, KL, GAE, two passes
-// of sums; thirteen of them) moved about three times as much.
+// advantages needs.  One workgroup per row, a thread per four positions that share 16 bytes of every array, so that each
+// array is read and written in 16-byte pieces whatever the length of the rows (the pieces at the two ends of a row are
+// taken one element at a time).  A block of 4 THREADS positions is held in registers, from its one read to its one write;
+// longer rows go block by block from the end.  The first block's loads are queued ahead of the count of the attention
+// bytes.  The maps of the recurrence are composed per thread, scanned over the wave in the lanes themselves (DPP) and over
+// the waves by every wave alike.  256 threads where a block of theirs holds a row, 512 otherwise (1 024 have half the
+// registers and spill: 512 x 4096 takes 37 us; two pieces a thread spill too: 38).
+// With byte masks and a reference policy 10 bytes in per token (14 with values) and 28 out (24 without a reference policy):
+// 88 MB at 512 x 4096 with values, 14 us at the rate of an even mix of reads and writes.  us, with one-element memory
+// instructions and the row in LDS / so: 512 x 4096: 35.8 / 27.8, 1024 x 4096: 63.5 / 47.7, 1024 x 1001: 47.8 / 27.6,
+// 1024 x 300: 42.3 / 25.2 (maps composed in 32 bits: 24.7, 41.3, 26.2, 24.2, at two to seven times the error: 512 x 4096
+// against 64 bits, gamma lambda = 0.95: 1.7e-7 then and before, 6.8e-8 so).  A quarter to a half of it is the sums of a
+// normalisation: 64-bit arithmetic, and three trips past the caches at the end of the launch (sums out, counter, sums in).
 // The sums of a row are published past the caches for the last workgroup to fold: with a __threadfence() in every
-// workgroup (a write-back of its XCD's L2, full of the outputs' lines) 512 x 4096 took 40.2 us, so 35.7.
-// Also measured, slower, at 512 x 4096 per pass (46 us so): 512 threads with chunks of 8 57 us; a chunk held in registers
-// for both walks 66 us (128 registers a lane are not enough for it).
+// workgroup (a write-back of its XCD's L2, full of the outputs' lines) 512 x 4096 took 4 us more.
 // ------------------------------------------------------------------------------------------------------------------
-constexpr int kRowsAhead = 8;  // positions of a thread whose inputs are on their way together
 
 // Per row: sums for the normalisation.  F = sum m, S = sum x m; A = sum m^2, B = sum m^2 (x - c), C = sum m^2 (x - c)^2
 // about a centre c of the row's own (its mean in the first super-block with a token that counts), from which the sum of squares about any mean
@@ -537,6 +605,8 @@ struct RowArgs {
   int64_t bs, L;
   float kl_ctl, gamma, lam;
   int estimator, mask_no_eos_with_zero, mask_bytes, roll;
+  int whole_pieces;         // the arrays start on 16 bytes (byte masks on four)
+  int attention_words;      // the attention bytes start on four
   NormArgs norm;            // levels and groups of the normalisation (no leave-one-out)
 };
 
@@ -554,21 +624,100 @@ __device__ __forceinline__ double row_mean(const NormArgs& n, const double4* sta
   return (double)(float)(s.y == 0.0 ? 0.0 : s.x / s.y);
 }
 
-__global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
-  __shared__ float sr[kGaeLds], sv[kGaeLds], sm[kGaeLds];
-  __shared__ Affine wave_tot[kGaeThreads / kWave];
+// Sums of N doubles over the workgroup, the same in every thread; smem [waves][N].  Fixed order.
+template <int N, int WAVES>
+__device__ __forceinline__ void block_sums(double (&v)[N], double* smem) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+#pragma unroll
+  for (int q = 0; q < N; ++q) v[q] = last_lane_sum(v[q]);
+  __syncthreads();
+  if (lane == kWave - 1)
+#pragma unroll
+    for (int q = 0; q < N; ++q) smem[wave * N + q] = v[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    v[q] = smem[q];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) v[q] += smem[w * N + q];
+  }
+}
+
+template <int THREADS>
+__global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
+  constexpr int kWaves = THREADS / kWave, kBlock = Block<THREADS>::kPositions;
+  __shared__ Affine wave_tot[kWaves];
   __shared__ float carry[2];
-  __shared__ double smem[kGaeThreads / kWave];
-  __shared__ int smem_i[kGaeThreads / kWave];
+  __shared__ double smem[kWaves * 5];
+  __shared__ int smem_i[kWaves];
   __shared__ int last;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int tid = threadIdx.x;
   const int64_t row = blockIdx.x, L = a.L, r0 = row * L;
+  const float gl = a.gamma * a.lam;
+  int64_t at = Block<THREADS>::first(r0, L);
+  struct Inputs {
+    float m[kOwn + 1], lo[kOwn + 1], lr[kOwn], v[kOwn];  // mask and log-prob: one more (torch.roll(x, -1))
+  };
+  // what lies outside the row comes as zeros; position L, behind the last, is position 0
+  auto fetch = [&](int64_t at, Inputs& x) {
+    const Block<THREADS> b(at, L, a.whole_pieces != 0);
+    const int64_t front = r0 + at;  // (the arrays are addressed from the front of the block, by 32-bit places)
+    const uint8_t* mask_b = (const uint8_t*)a.mask_in + front;
+    const float *mask_f = (const float*)a.mask_in + front, *logp = a.logp + front;
+    auto mask_of = [&](int o) { return a.mask_bytes ? (mask_b[o] ? 1.f : 0.f) : mask_f[o]; };
+    if (b.whole && a.mask_bytes) {
+      const uint32_t w = *(const uint32_t*)(mask_b + b.own);
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q) x.m[q] = (w >> (8 * q)) & 0xffu ? 1.f : 0.f;
+    } else if (!a.mask_bytes) {
+      b.load(mask_f, x.m);
+    } else {
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q) x.m[q] = b.in(b.own + q) && mask_b[b.own + q] ? 1.f : 0.f;
+    }
+    b.load(logp, x.lo);
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) x.lr[q] = x.v[q] = 0.f;
+    if (a.ref) b.load(a.ref + front, x.lr);
+    if (a.values) b.load(a.values + front, x.v);
+    // the position behind the thread's own (of thread 0 in the block before this one), and position L as one of them
+    const int o = b.own + kOwn, wrap = L - at <= kBlock ? (int)(L - at) : -1;
+    const bool in = o >= b.lo_in && at + o < L;
+    x.m[kOwn] = in ? mask_of(o) : 0.f;
+    x.lo[kOwn] = in && a.roll ? logp[o] : 0.f;
+    if (wrap > b.own && wrap <= o) {
+      const float m0 = mask_at(a, r0), lo0 = a.roll ? a.logp[r0] : 0.f;
+#pragma unroll
+      for (int q = 1; q <= kOwn; ++q) {
+        x.m[q] = b.own + q == wrap ? m0 : x.m[q];
+        x.lo[q] = b.own + q == wrap ? lo0 : x.lo[q];
+      }
+    }
+  };
+  Inputs x;
+  fetch(at, x);
+  const float v_end = a.values ? a.values[r0 + L - 1] : 0.f;
   int64_t sl;
   if (a.attention) {
-    int n = 0;
+    uint32_t n = 0;
+    if (a.attention_words) {
+      const int lead = (int)(r0 & 3);
+      const int64_t words = (lead + L + 3) >> 2;
+#pragma unroll 2
+      for (int64_t j = tid; j < words; j += THREADS) {
+        const int64_t t0 = 4 * j - lead;
+        if (t0 >= 0 && t0 + 4 <= L) {
+          n = __builtin_amdgcn_sad_u8(*(const uint32_t*)(a.attention + r0 + t0), 0u, n);
+        } else {
+          for (int q = 0; q < 4; ++q)
+            if (t0 + q >= 0 && t0 + q < L) n += a.attention[r0 + t0 + q];
+        }
+      }
+    } else {
 #pragma unroll 8
-    for (int64_t t = tid; t < L; t += kGaeThreads) n += a.attention[r0 + t];
-    sl = block_sum<int>(n, smem_i);
+      for (int64_t t = tid; t < L; t += THREADS) n += a.attention[r0 + t];
+    }
+    sl = block_sum<int>((int)n, smem_i);
   } else {
     sl = a.seqlens[row];
   }
@@ -578,183 +727,164 @@ __global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
   if (put < 0) put = 0;
   const bool no_eos = sl == L;
   const float score = (a.mask_no_eos_with_zero && no_eos) ? 0.f : a.score[row];
-  const float gl = a.gamma * a.lam;
-  const float v_end = a.values ? a.values[r0 + L - 1] : 0.f;
-  // One position: its inputs, then everything that does not depend on its neighbours (the mask, reward and value that the
-  // scan takes come back).  In two halves so that the inputs of several positions are on their way together: the stores
-  // of a position may alias later loads for all the compiler knows (ref and logp are written in place, element by
-  // element), and one position at a time, each load waits for the stores before it.
-  struct Inputs {
-    float m, lo, lr, v;
-  };
-  auto fetch = [&](int64_t t) {
-    const int64_t next = t + 1 < L ? t + 1 : 0;  // torch.roll(x, -1)
-    Inputs x;
-    x.m = mask_at(a, r0 + next);
-    x.lo = a.logp[r0 + (a.roll ? next : t)];
-    x.lr = a.ref ? a.ref[r0 + t] : 0.f;
-    x.v = a.values ? a.values[r0 + t] : 0.f;
-    return x;
-  };
-  auto place = [&](int64_t t, const Inputs& x) {
-    const float m = x.m, lo = x.lo * m, lr = x.lr * m;
-    if (a.ref) a.ref[r0 + t] = lr;
-    a.mask_out[r0 + t] = m;
-    a.old_out[r0 + t] = lo;
-    float d = lo * m - lr * m;
-    if (a.estimator == 1) d = d * d / 2.0f;
-    else if (a.estimator == 2) { d = -d; d = expf(d) - 1.f - d; }
-    d = (d != d) ? d : fminf(fmaxf(d, -10.f), 10.f);  // torch.clamp keeps NaN
-    const float kr = -a.kl_ctl * d;
-    a.kl_rewards[r0 + t] = kr;
-    float r = (t == at_last) ? 0.f : kr;
-    if (t == put) r += score;
-    a.rewards[r0 + t] = r;
-    return r;
-  };
-  float m_end = 0.f;
-  if (tid == 0) {
-    const Inputs x = fetch(L - 1);
-    m_end = x.m;
-    place(L - 1, x);
-    a.adv[r0 + L - 1] = 0.f;
-    a.returns[r0 + L - 1] = v_end;
-    carry[0] = no_eos ? v_end : 0.f;
-    carry[1] = 0.f;
-  }
-  // thread 0 carries position L - 1 (advantage 0) in its sums
-  double F = tid == 0 ? (double)m_end : 0.0, S = 0.0, A = F * F, B = 0.0, C = 0.0, c = 0.0;
-  const Affine ident{1.f, 0.f, 1.f, 0.f, 0.f};
+  double F = 0.0, S = 0.0, A = 0.0, B = 0.0, C = 0.0, c = 0.0;
   bool first = true;
-  for (int64_t end = L - 1; end > 0; end -= kGaeBlock) {
-    const int64_t base = end > kGaeBlock ? end - kGaeBlock : 0;
-    const int cnt = (int)(end - base);
-    __syncthreads();  // the previous super-block has been written out; carry is visible
-    for (int i0 = tid; i0 < cnt; i0 += kRowsAhead * kGaeThreads) {
-      Inputs x[kRowsAhead];
+  float nv0 = no_eos ? v_end : 0.f, lg0 = 0.f;  // the state that enters the block
+  for (;; at -= kBlock) {
+    const Block<THREADS> b(at, L, a.whole_pieces != 0);
+    const int64_t front = r0 + at;
+    const int p_last = b.place(at_last), p_put = b.place(put), p_end = b.place(L - 1);
+    float m[kOwn], r[kOwn], v[kOwn];
+    {
+      float lo[kOwn], lr[kOwn], kr[kOwn];
 #pragma unroll
-      for (int q = 0; q < kRowsAhead; ++q) {
-        const int i = i0 + q * kGaeThreads;
-        x[q] = fetch(base + (i < cnt ? i : cnt - 1));
+      for (int q = 0; q < kOwn; ++q) {
+        m[q] = x.m[q + 1];
+        lo[q] = (a.roll ? x.lo[q + 1] : x.lo[q]) * m[q];
+        lr[q] = x.lr[q] * m[q];
+        v[q] = x.v[q];
+        float d = lo[q] * m[q] - lr[q] * m[q];
+        if (a.estimator == 1) d = d * d / 2.0f;
+        else if (a.estimator == 2) { d = -d; d = expf(d) - 1.f - d; }
+        d = (d != d) ? d : fminf(fmaxf(d, -10.f), 10.f);  // torch.clamp keeps NaN
+        kr[q] = -a.kl_ctl * d;
+        r[q] = (b.own + q == p_last) ? 0.f : kr[q];
+        r[q] = (b.own + q == p_put) ? r[q] + score : r[q];
       }
+      if (a.ref) b.store(a.ref + front, lr);
+      b.store(a.mask_out + front, m);
+      b.store(a.old_out + front, lo);
+      b.store(a.kl_rewards + front, kr);
+      b.store(a.rewards + front, r);
+    }
+    const bool more = at > 0;
+    // The composite map of the thread's positions, from the last to the first.  With m, r and v zero a position is the
+    // identity: so are the last one of the row, whose advantage is 0, and what lies outside the row.
+    float m_end = 0.f;
+    Affine mine = identity();
 #pragma unroll
-      for (int q = 0; q < kRowsAhead; ++q) {
-        const int i = i0 + q * kGaeThreads;
-        if (i >= cnt) break;
-        const int slot = gae_slot(i);
-        sr[slot] = place(base + i, x[q]);
-        sv[slot] = x[q].v;
-        sm[slot] = x[q].m;
-      }
+    for (int q = kOwn - 1; q >= 0; --q) {
+      m_end = b.own + q == p_end ? m[q] : m_end;
+      if (!b.in(b.own + q) || b.own + q == p_end) m[q] = r[q] = v[q] = 0.f;
+      mine = compose(mine, position(m[q], r[q], v[q], a.gamma, gl));
     }
-    __syncthreads();
-    const int hi = cnt - 1 - tid * kGaeChunk;
-    const int lo = hi - kGaeChunk + 1 > 0 ? hi - kGaeChunk + 1 : 0;
-    Affine x = ident;
-    for (int i = hi; i >= lo; --i) {
-      const int slot = gae_slot(i);
-      const float mt = sm[slot], vt = sv[slot], rt = sr[slot];
-      Affine e;
-      e.a = 1.f - mt;
-      e.e = mt * vt;
-      e.c = mt * a.gamma;
-      e.d = (1.f - mt) + mt * gl;
-      e.f = mt * (rt - vt);
-      x = compose(x, e);
-    }
-    Affine inc = x;
+    float nv, lg;
+    enter<kWaves>(mine, wave_tot, nv0, lg0, nv, lg);
+    float out[kOwn], ret[kOwn];
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const Affine prev = shfl_up(inc, o);
-      if (lane >= o) inc = compose(prev, inc);
-    }
-    if (lane == kWave - 1) wave_tot[wave] = inc;
-    const float nv0 = carry[0], lg0 = carry[1];
-    __syncthreads();
-    Affine before = ident;  // everything processed in this super-block before this thread's chunk
-    for (int w = 0; w < wave; ++w) before = compose(before, wave_tot[w]);
-    Affine excl = shfl_up(inc, 1);
-    if (lane == 0) excl = ident;
-    before = compose(before, excl);
-    float nv = fmaf(before.a, nv0, before.e);
-    float lg = fmaf(before.c, nv0, fmaf(before.d, lg0, before.f));
-    double f_here = 0.0, s_here = 0.0;
-    for (int i = hi; i >= lo; --i) {
-      const int slot = gae_slot(i);
-      const float mt = sm[slot], vt = sv[slot], rt = sr[slot];
-      const float delta = rt + a.gamma * nv - vt;
+    for (int q = kOwn - 1; q >= 0; --q) {
+      const float delta = r[q] + a.gamma * nv - v[q];
       const float newlg = delta + gl * lg;
-      nv = nv * (1.f - mt) + vt * mt;
-      lg = lg * (1.f - mt) + newlg * mt;
-      sr[slot] = lg;        // advantages
-      sv[slot] = lg + vt;   // returns
-      f_here += (double)mt;
-      s_here += (double)lg * (double)mt;
+      nv = nv * (1.f - m[q]) + v[q] * m[q];
+      lg = lg * (1.f - m[q]) + newlg * m[q];
+      const bool scanned = b.in(b.own + q) && b.own + q != p_end;
+      out[q] = scanned ? lg : 0.f;
+      ret[q] = scanned ? lg + v[q] : v_end;  // (outside the row it is not stored)
+      F += (double)m[q];
+      S += (double)out[q] * (double)m[q];
     }
-    if (tid == kGaeThreads - 1) {  // the last thread ends at the front of the super-block: its state carries on
+    F += (double)m_end;
+    b.store(a.adv + front, out);
+    b.store(a.returns + front, ret);
+    if (more && tid == THREADS - 1) {  // the thread at the front of the block hands its state on
       carry[0] = nv;
       carry[1] = lg;
     }
-    F += f_here;
-    S += s_here;
-    if (a.sums && first) {
-      // the centre of the row's squares: its mean so far, as soon as a token counts (a masked super-block adds nothing to
-      // A, B and C, whatever the centre)
-      const double f = block_sum<double>(F, smem), s = block_sum<double>(S, smem);
-      if (f != 0.0) {
-        c = s / f;
-        if (!isfinite(c)) c = 0.0;  // an infinity among the advantages: its square is infinite about any finite centre
-        first = false;
-        if (tid == 0) {  // position L - 1
-          const double mm = (double)m_end * (double)m_end;
-          B -= mm * c;
-          C += mm * c * c;
+    if (a.sums) {
+      if (first) {
+        // the centre of the row's squares: its mean so far, as soon as a token counts (a masked block adds nothing to A, B
+        // and C, whatever the centre)
+        double fs[2] = {F, S};
+        block_sums<2, kWaves>(fs, smem);
+        if (fs[0] != 0.0) {
+          c = fs[1] / fs[0];
+          if (!isfinite(c)) c = 0.0;  // an infinity among the advantages: its square is infinite about any finite centre
+          first = false;
         }
       }
-    }
-    __syncthreads();
-    for (int i = tid; i < cnt; i += kGaeThreads) {
-      const int slot = gae_slot(i);
-      const float ad = sr[slot];
-      a.adv[r0 + base + i] = ad;
-      a.returns[r0 + base + i] = sv[slot];
-      if (a.sums) {
-        const double mm = (double)sm[slot] * (double)sm[slot], d = (double)ad - c;
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q) {
+        const double mm = (double)m[q] * (double)m[q], d = (double)out[q] - c;
         A += mm;
         B += mm * d;
         C += mm * d * d;
       }
+      const double mm = (double)m_end * (double)m_end;  // the row's last position
+      A += mm;
+      B -= mm * c;
+      C += mm * c * c;
     }
+    if (!more) break;
+    fetch(at - kBlock, x);
+    __syncthreads();
+    nv0 = carry[0];
+    lg0 = carry[1];
   }
   if (!a.sums) return;
-  F = block_sum<double>(F, smem);
-  S = block_sum<double>(S, smem);
-  A = block_sum<double>(A, smem);
-  B = block_sum<double>(B, smem);
-  C = block_sum<double>(C, smem);
-  if (tid == 0) {
-    RowSums* o = a.sums + row;
-    publish(&o->F, F);
-    publish(&o->S, S);
-    publish(&o->A, A);
-    publish(&o->B, B);
-    publish(&o->C, C);
-    publish(&o->c, c);
-    last = last_to_finish(&a.work->finished, (int)gridDim.x);
+  {
+    double v[5] = {F, S, A, B, C};
+    block_sums<5, kWaves>(v, smem);
+    if (tid == 0) {
+      RowSums* o = a.sums + row;
+      publish(&o->F, v[0]);
+      publish(&o->S, v[1]);
+      publish(&o->A, v[2]);
+      publish(&o->B, v[3]);
+      publish(&o->C, v[4]);
+      publish(&o->c, c);
+      last = last_to_finish(&a.work->finished, (int)gridDim.x);
+    }
   }
   __syncthreads();
   if (!last) return;
-  // the last workgroup: the segments of the normalisation from the sums of their rows, in row order.  The sums of all
-  // rows are fetched at once and stored again as this workgroup's own, so that the loops below, which walk the rows of
-  // a segment one after the other, find them in its caches.
-  for (int64_t r = tid; r < a.bs; r += kGaeThreads) {
+  // The last workgroup: the segments of the normalisation from the sums of their rows.
+  const NormArgs& n = a.norm;
+  auto squares_about = [&](const RowSums& q, double mean) {
+    const double d = mean - q.c;
+    if (isinf(q.C) && isfinite(d)) return q.C;  // (the terms below are infinities of both signs)
+    return q.C - 2.0 * d * q.B + d * d * q.A;
+  };
+  constexpr int kRowsHeld = 4;
+  if (n.n_groups == 0 && a.bs <= kRowsHeld * THREADS) {
+    // The whole batch is one segment: a thread's rows are fetched at once and stay in its registers (the loads go past the
+    // caches: one after the other they were half of this tail)
+    RowSums held[kRowsHeld];
+    double bf[2] = {0.0, 0.0}, z[1] = {0.0};
+#pragma unroll
+    for (int k = 0; k < kRowsHeld; ++k) {
+      const int64_t r = tid + k * THREADS;
+      held[k] = RowSums{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      if (r < a.bs) {
+        const RowSums* q = a.sums + r;
+        held[k] = RowSums{published(&q->F), published(&q->S), published(&q->A), published(&q->B), published(&q->C), published(&q->c)};
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kRowsHeld; ++k) {
+      bf[0] += held[k].S;
+      bf[1] += held[k].F;
+    }
+    block_sums<2, kWaves>(bf, smem);
+    const double mean = n.mean_level == 0 || bf[1] == 0.0 ? 0.0 : bf[0] / bf[1];
+#pragma unroll
+    for (int k = 0; k < kRowsHeld; ++k)
+      if (tid + k * THREADS < a.bs) z[0] += squares_about(held[k], mean);
+    block_sums<1, kWaves>(z, smem);
+    if (tid == 0) {
+      a.stats[0] = make_double4(bf[0], bf[1], z[0] < 0.0 ? 0.0 : z[0], 0.0);
+      a.work->finished = 0;
+    }
+    return;
+  }
+  // In row order, one thread a segment: the sums of all rows are fetched at once and stored again as this workgroup's own,
+  // so that the loops below, which walk the rows of a segment one after the other, find them in its caches.
+  for (int64_t r = tid; r < a.bs; r += THREADS) {
     const RowSums* q = a.sums + r;
     const RowSums own{published(&q->F), published(&q->S), published(&q->A), published(&q->B), published(&q->C), published(&q->c)};
     a.sums[r] = own;
   }
   __syncthreads();
-  const NormArgs& n = a.norm;
-  for (int64_t g = tid; g < n.n_groups; g += kGaeThreads) {
+  for (int64_t g = tid; g < n.n_groups; g += THREADS) {
     double4 st = make_double4(0.0, 0.0, 0.0, 0.0);
     for (int64_t r = g * n.group_size; r < (g + 1) * n.group_size; ++r) {
       st.x += a.sums[r].S;
@@ -763,7 +893,7 @@ __global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
     a.stats[1 + g] = st;
   }
   double bs = 0.0, bf = 0.0;
-  for (int64_t r = tid; r < a.bs; r += kGaeThreads) {
+  for (int64_t r = tid; r < a.bs; r += THREADS) {
     bs += a.sums[r].S;
     bf += a.sums[r].F;
   }
@@ -771,19 +901,14 @@ __global__ __launch_bounds__(kGaeThreads) void k_advantage_rows(RowArgs a) {
   bf = block_sum<double>(bf, smem);
   if (tid == 0) a.stats[0] = make_double4(bs, bf, 0.0, 0.0);
   __syncthreads();  // the segment sums are visible to the whole workgroup
-  auto squares = [&](int64_t r) {
-    const RowSums q = a.sums[r];
-    const double d = row_mean(n, a.stats, r) - q.c;
-    if (isinf(q.C) && isfinite(d)) return q.C;  // (the terms below are infinities of both signs)
-    return q.C - 2.0 * d * q.B + d * d * q.A;
-  };
-  for (int64_t g = tid; g < n.n_groups; g += kGaeThreads) {
+  auto squares = [&](int64_t r) { return squares_about(a.sums[r], row_mean(n, a.stats, r)); };
+  for (int64_t g = tid; g < n.n_groups; g += THREADS) {
     double z = 0.0;
     for (int64_t r = g * n.group_size; r < (g + 1) * n.group_size; ++r) z += squares(r);
     a.stats[1 + g].z = z < 0.0 ? 0.0 : z;  // a rounding below zero; NaN stays
   }
   double z = 0.0;
-  for (int64_t r = tid; r < a.bs; r += kGaeThreads) z += squares(r);
+  for (int64_t r = tid; r < a.bs; r += THREADS) z += squares(r);
   z = block_sum<double>(z, smem);
   if (tid == 0) {
     a.stats[0].z = z < 0.0 ? 0.0 : z;
@@ -923,8 +1048,14 @@ extern "C" int aa_gae(const float* rewards, const float* values, const float* lo
   if (bs < 0 || L < 1) return AA_ERR_INVALID_ARGUMENT;
   if (bs == 0) return AA_OK;
   if (!rewards || !loss_mask || !advantages) return AA_ERR_INVALID_ARGUMENT;
-  hipLaunchKernelGGL(k_gae, dim3((unsigned)bs), dim3(kGaeThreads), 0, (hipStream_t)stream, rewards, values, loss_mask,
-                     seq_no_eos, bs, L, discount, gae_lambda, advantages, returns);
+  const uintptr_t arrays = (uintptr_t)rewards | (uintptr_t)values | (uintptr_t)loss_mask | (uintptr_t)advantages | (uintptr_t)returns;
+  const int aligned = (arrays & 15) == 0;
+  if (L <= kShortRow)  // as in aa_advantages: the two are one scan
+    hipLaunchKernelGGL(k_gae<256>, dim3((unsigned)bs), dim3(256), 0, (hipStream_t)stream, rewards, values, loss_mask,
+                       seq_no_eos, L, discount, gae_lambda, aligned, advantages, returns);
+  else
+    hipLaunchKernelGGL(k_gae<512>, dim3((unsigned)bs), dim3(512), 0, (hipStream_t)stream, rewards, values, loss_mask,
+                       seq_no_eos, L, discount, gae_lambda, aligned, advantages, returns);
   return launch_status();
 }
 
@@ -1056,7 +1187,16 @@ extern "C" int aa_advantages(const aa_advantage_step* step, void* stream) {
     a.work = (StepWork*)p.work;
   }
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_advantage_rows, dim3((unsigned)p.bs), dim3(kGaeThreads), 0, st, a);
+  const uintptr_t arrays = (uintptr_t)a.logp | (uintptr_t)a.ref | (uintptr_t)a.values | (uintptr_t)a.mask_out |
+                           (uintptr_t)a.old_out | (uintptr_t)a.kl_rewards | (uintptr_t)a.rewards | (uintptr_t)a.adv |
+                           (uintptr_t)a.returns | (uintptr_t)(a.mask_bytes ? nullptr : a.mask_in);
+  a.whole_pieces = (arrays & 15) == 0 && (!a.mask_bytes || ((uintptr_t)a.mask_in & 3) == 0);
+  a.attention_words = ((uintptr_t)a.attention & 3) == 0;
+  const dim3 grid((unsigned)p.bs);
+  if (p.L <= kShortRow)
+    hipLaunchKernelGGL(k_advantage_rows<256>, grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_advantage_rows<512>, grid, dim3(512), 0, st, a);
   if (p.norm) launch_norm_apply(a.norm, a.stats, p.advantages, st);
   return launch_status();
 }

@@ -1,6 +1,7 @@
 """GPU parity of the advantage pipeline (GAE scan, Normalization, masked moments) against the CPU oracle and the
 reference's own known-answer cases."""
 import itertools
+import math
 import json
 from pathlib import Path
 
@@ -364,6 +365,55 @@ def test_advantage_rows_agree_with_the_separate_kernels(device, bs, L, variant):
             assert float((a - b).abs().max()) <= 4 * 2.0 ** -23 * max(float(b.abs().max()), 1.0), k
         else:
             assert torch.equal(a, b), k
+
+
+@pytest.mark.parametrize("bs,L,offset", [(5, 1021, 0), (5, 1022, 0), (3, 1025, 0), (5, 2045, 0), (5, 2047, 0), (4, 2048, 0),
+                                         (3, 2051, 0), (3, 6143, 0), (1030, 5, 0), (2050, 1022, 0), (5, 61, 1), (3, 2049, 3)])
+@pytest.mark.parametrize("gamma,lam", [(1.0, 0.95), (1.0, 1.0)])
+def test_advantage_rows_at_the_edges_of_their_blocks(device, bs, L, offset, gamma, lam):
+    """Rows around the sizes of a block of 1024 and of 2048 positions, at every place in a 16-byte piece, more rows than the
+    last workgroup holds, and arrays that do not start on 16 bytes (``offset`` elements into a larger one): advantages and
+    returns against the recurrence in float64.  A float32 scan of the same maps keeps each state to one rounding per step
+    it is composed over, 2^-24 of the largest state, and there are log2(L) + 8 of those behind a state."""
+    from areal_amd import engine_glue
+
+    g = torch.Generator().manual_seed(bs + L)
+    lens = torch.randint((L + 1) // 2, L + 1, (bs, 1), generator=g)
+    at = torch.arange(L)[None]
+    attention = at < lens
+    mask = attention & (torch.rand(bs, L, generator=g) < 0.8)
+    logp = -2.0 * torch.rand(bs, L, generator=g)
+    base = dict(attention_mask=attention, loss_mask=mask, logprobs=logp, rewards=torch.randn(bs, generator=g),
+                ref_logp=logp + 0.05 * torch.randn(bs, L, generator=g), prox_logp=logp.clone(),
+                values=torch.randn(bs, L, generator=g))
+
+    def placed(t):
+        if offset == 0 or t.dim() != 2:
+            return t.clone().to(device)
+        flat = torch.empty(t.numel() + offset, dtype=t.dtype, device=device)
+        flat[offset:] = t.flatten().to(device)
+        return flat[offset:].view(t.shape)
+
+    kw = dict(kl_ctl=0.1, kl_estimator="k1", discount=gamma, gae_lambda=lam, use_decoupled_loss=True)
+    out = engine_glue.compute_advantages({k: placed(v) for k, v in base.items()}, **kw)
+    norm = Normalization(NormConfig(mean_level="batch", std_level="batch"))
+    normed = engine_glue.compute_advantages({k: placed(v) for k, v in base.items()}, adv_norm=norm, **kw)
+    m, v, r = out["loss_mask"].cpu().double(), base["values"].double(), out["tot_rewards"].cpu().double()
+    no_eos = (lens[:, 0] == L)
+    nv, lg = torch.where(no_eos, v[:, -1], 0.0), torch.zeros(bs, dtype=torch.float64)
+    adv, biggest = torch.zeros(bs, L, dtype=torch.float64), 1.0
+    for t in range(L - 2, -1, -1):
+        new = r[:, t] + gamma * nv - v[:, t] + gamma * lam * lg
+        nv, lg = torch.where(m[:, t] > 0, v[:, t], nv), torch.where(m[:, t] > 0, new, lg)
+        adv[:, t] = lg
+        biggest = max(biggest, float(lg.abs().max()))
+    bound = 2.0 ** -24 * biggest * (math.log2(L) + 8) * (1 if lam < 1 else math.sqrt(L))  # lam = 1: roundings add up along a row
+    assert float((out["advantages"].cpu().double() - adv).abs().max()) <= bound
+    ret = adv + v
+    assert float((out["returns"].cpu().double() - ret).abs().max()) <= bound + 2.0 ** -24 * float(ret.abs().max())
+    # the separate two-pass normalisation of the same advantages: float64 sums in another order, then one rounding to float32
+    want = norm(out["advantages"], out["loss_mask"])
+    assert float((normed["advantages"] - want).abs().max()) <= 4 * 2.0 ** -23 * max(float(want.abs().max()), 1.0)
 
 
 @pytest.mark.parametrize("shared", ["ref_logp is logprobs", "ref_logp is values", "prox_logp is values"])
