@@ -214,6 +214,7 @@ SIGNATURES = {
     "aa_kl_estimate": (_i, [_p, _p, _i64, _i, _i, _p, _p]),
     "aa_overlong_penalty": (_i, [_p, _p, _i64, _i64, _i, _f, _i64, _p]),
     "aa_kd_terms": (_i, [_p, _p, _p, _p, _i64, _i, _p, _p, _p]),
+    "aa_sft_sequence_stats": (_i, [_p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p]),
     "aa_sft_loss": (_i, [_p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     "aa_dpo_seq_sums": (_i, [_p, _p, _p, _p, _i64, _i64, _p, _p, _p, _p]),
     "aa_dpo_seq_sums_bwd": (_i, [_p, _p, _p, _p, _i64, _i64, _p, _p]),

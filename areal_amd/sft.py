@@ -82,12 +82,8 @@ class _SftLoss(torch.autograd.Function):
         return out, None, None, None, None, None
 
 
-def _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs, extra=None):
-    stat = dict(loss=stat_loss, seqlogp=seq_logp[:n_seqs], n_seqs=seq_count[:n_seqs] > 0, ppl=seq_ppl,
-                valid_tokens_per_seq=seq_count[:n_seqs])
-    if extra:
-        stat.update(extra)
-    return stat
+def _stat(stat_loss, seq_logp, seq_count, selected, seq_ppl):
+    return dict(loss=stat_loss, seqlogp=seq_logp, n_seqs=selected, ppl=seq_ppl, valid_tokens_per_seq=seq_count)
 
 
 def _scale_tensor(loss_scale, dev):
@@ -112,7 +108,8 @@ def sft_loss_fn(logprobs: torch.Tensor, loss_mask: torch.Tensor, cu_seqlens: tor
     cu, n_seqs = _cu_i32(cu_seqlens, dev)
     loss, stat_loss, seq_logp, seq_count, seq_ppl = _SftLoss.apply(lp, m8, cu, n_seqs, _count_nonzero(m8),
                                                                    _scale_tensor(loss_scale, dev))
-    return loss, _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs)
+    seq_logp, seq_count = seq_logp[:n_seqs], seq_count[:n_seqs]
+    return loss, _stat(stat_loss, seq_logp, seq_count, seq_count > 0, seq_ppl)
 
 
 def _nll_step(dev, T, T_active, loss_mask, loss_scale):
@@ -123,11 +120,20 @@ def _nll_step(dev, T, T_active, loss_mask, loss_scale):
 def _step_stat(step, cu, n_seqs, extrema):
     """The stat dict of a fused step: that of ``sft_loss_fn`` plus the per-token outputs."""
     logp, entropy, vmax, vmin, stat_loss, _ratio = step.rows()
-    _, _, _, seq_logp, seq_count, seq_ppl = _launch(logp, step.mask, cu, n_seqs, step.counts_address, None, False, False)
-    extra = dict(logprobs=logp, entropy=entropy)
+    dev = step.device
+    seq_logp = torch.empty(n_seqs, dtype=torch.float64, device=dev)
+    seq_count = torch.empty(n_seqs, dtype=torch.int32, device=dev)
+    selected = torch.empty(n_seqs, dtype=torch.bool, device=dev)
+    seq_ppl = torch.empty(n_seqs, dtype=torch.float32, device=dev)
+    with _on(dev):
+        N.check(N.load().aa_sft_sequence_stats(_ptr(logp), _ptr(step.mask), step.T_active, _ptr(cu), n_seqs, _ptr(seq_logp),
+                                               _ptr(seq_count), _ptr(selected), _ptr(seq_ppl), _stream(dev)),
+                "aa_sft_sequence_stats")
+    stat = _stat(stat_loss, seq_logp, seq_count, selected, seq_ppl)
+    stat.update(logprobs=logp, entropy=entropy)
     if extrema:
-        extra.update(vocab_min_logits=vmin, vocab_max_logits=vmax)
-    return _stat(stat_loss, seq_logp, seq_count, seq_ppl, n_seqs, extra)
+        stat.update(vocab_min_logits=vmin, vocab_max_logits=vmax)
+    return stat
 
 
 def _check_fused_inputs(rows: torch.Tensor, labels: torch.Tensor, loss_mask: torch.Tensor, what: str) -> int:

@@ -531,6 +531,16 @@ int aa_sft_loss(const float* logp, const uint8_t* mask, int64_t T,
                 int32_t* seq_count, float* seq_ppl, void* stream);
 
 /*
+ * The per-sequence part of aa_sft_loss alone, for a step whose loss is known:
+ * seq_logp, seq_count, seq_ppl (nullable) as there but with n_seqs entries,
+ * and seq_selected[b] = seq_count[b] > 0 as a byte (nullable).  Same bits.
+ */
+int aa_sft_sequence_stats(const float* logp, const uint8_t* mask, int64_t T,
+                          const int32_t* cu_seqlens, int64_t n_seqs,
+                          double* seq_logp, int32_t* seq_count,
+                          uint8_t* seq_selected, float* seq_ppl, void* stream);
+
+/*
  * Direct preference optimisation over a packed batch whose sequences are
  * interleaved [chosen_0, rejected_0, chosen_1, rejected_1, ...].
  *

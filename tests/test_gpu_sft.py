@@ -210,3 +210,29 @@ def test_full_size_supervised_lm_head_step(device):
     assert cosine(dh1.float().cpu(), h.grad.float().cpu()) > 0.9999
     assert cosine(dw1.float().cpu(), w.grad.float().cpu()) > 0.9999
     assert not dh1[~case.loss_mask.bool()].any()
+
+
+@pytest.mark.parametrize("T,cuts", [(1, [0, 1]), (300, [0, 0, 1, 65, 299]), (5000, [7, 1031, 1032, 3000, 3000, 5000]), (40, [0])])
+def test_sequence_stats_alone_are_those_of_the_loss(device, T, cuts):
+    """``aa_sft_sequence_stats`` against ``aa_sft_loss``, bit for bit: empty sequences, sequences without a selected token,
+    tokens outside every sequence, no sequence at all."""
+    from areal_amd import _native as N
+    from areal_amd.functional import _count_nonzero
+    from areal_amd.sft import _launch
+
+    g = torch.Generator().manual_seed(T)
+    logp = (-3.0 * torch.rand(T, generator=g)).to(device)
+    mask = (torch.rand(T, generator=g) < 0.5)
+    mask[cuts[0]:cuts[min(1, len(cuts) - 1)]] = False
+    mask = mask.to(device)
+    cu, n = torch.tensor(cuts, dtype=torch.int32, device=device), len(cuts) - 1
+    n_valid = _count_nonzero(mask.view(torch.uint8))
+    _, _, _, want_logp, want_count, want_ppl = _launch(logp, mask, cu, n, n_valid.data_ptr(), None, False, False)
+    got_logp = torch.full((n,), 7.0, dtype=torch.float64, device=device)
+    got_count, got_ppl = torch.full((n,), 7, dtype=torch.int32, device=device), torch.full((n,), 7.0, device=device)
+    selected = torch.zeros(n, dtype=torch.bool, device=device)
+    N.check(N.load().aa_sft_sequence_stats(logp.data_ptr(), mask.data_ptr(), T, cu.data_ptr(), n, got_logp.data_ptr(),
+                                           got_count.data_ptr(), selected.data_ptr(), got_ppl.data_ptr(),
+                                           torch.cuda.current_stream().cuda_stream), "aa_sft_sequence_stats")
+    assert torch.equal(got_logp, want_logp[:n]) and torch.equal(got_count, want_count[:n]) and torch.equal(got_ppl, want_ppl)
+    assert torch.equal(selected, want_count[:n] > 0)
