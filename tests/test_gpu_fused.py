@@ -981,3 +981,21 @@ def test_work_buffer_keeps_nothing_between_the_launches_of_a_step(device):
         loss, _ = engine_glue.compute_logprobs_and_loss(x, {"rolled_input_ids": ids}, mb, 0, 977.0, 0.2, rejection_sampling=rs)
         assert float(loss.detach()) != 0.0
         assert not F._work_words(device)[:48].any()  # 16 words of counters, 32 of the moments table
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,lead", [(1, 0), (7, 1), (8, 0), (9, 3), (1000, 5), (1024 * 256 * 8 + 13, 1), (3 * 1024 * 256 * 8, 0)])
+def test_upstream_factor_in_place(device, dtype, n, lead):
+    """``aa_scale_inplace``: 16-byte pieces, what lies ahead of the first and behind the last, more of them than one round of
+    workgroups takes; a factor of one leaves the array alone.  One product in float32 and one rounding: exact."""
+    from areal_amd import _native as N
+    from areal_amd.functional import _DTYPES
+
+    flat = torch.randn(lead + n + 5, device=device).to(dtype)
+    want = flat.clone()
+    want[lead:lead + n] = (flat[lead:lead + n].float() * 0.37).to(dtype)
+    for f, expected in ((1.0, flat.clone()), (0.37, want)):
+        factor = torch.tensor([f], device=device)
+        N.check(N.load().aa_scale_inplace(flat[lead:].data_ptr(), _DTYPES[dtype], n, factor.data_ptr(),
+                                          torch.cuda.current_stream().cuda_stream), "aa_scale_inplace")
+        assert torch.equal(flat, expected)
