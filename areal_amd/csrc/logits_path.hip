@@ -229,9 +229,7 @@ struct GradCoef {
 // has a NaN gradient in the reference as well (the entropy itself is NaN there).
 __device__ __forceinline__ float grad_weight(const GradCoef& g, float x) { return g.B == 0.f ? g.A : fmaf(g.B, x, g.A); }
 
-// STREAM: the row and its gradient pass through once (`nt` policy on loads and stores); fp32 rows then go in 16-byte
-// pieces, so that every load and store instruction of a wave covers 1 KB of consecutive addresses.
-template <int DT, int NT, bool STREAM = false>
+template <int DT, int NT>
 __device__ __forceinline__ void row_grad_generic(const void* row, void* out, int V, bool vec_ok, const GradCoef& g) {
   const RowSplit sp = split_row<DT>(row, V, vec_ok);
   const int tid = threadIdx.x;
@@ -242,29 +240,10 @@ __device__ __forceinline__ void row_grad_generic(const void* row, void* out, int
     Elem<DT>::store1(out, j, o);
   };
   for (int j = tid; j < sp.head; j += NT) one(j);
-  if constexpr (STREAM && DT == AA_F32) {
-    const int n4 = sp.nvec * 2;
-    for (int v = tid; v < n4; v += NT) {
-      const int e0 = sp.head + (v << 2);
-      float x[4], o[4];
-      load4_stream((const float*)row + e0, x);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = fast_exp2(fmaf(x[i], g.c, -g.lse2)) * grad_weight(g, x[i]);
-      if ((unsigned)(g.label - e0) < 4u) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (e0 + i == g.label) o[i] += g.lab_add;
-      }
-      store4_stream((float*)out + e0, o);
-    }
-    for (int j = sp.tail0 + tid; j < V; j += NT) one(j);
-    return;
-  }
   for (int v = tid; v < sp.nvec; v += NT) {
     const int e0 = sp.head + (v << 3);
     float x[8], o[8];
-    if constexpr (STREAM) load8_stream<DT>(row, e0, x);
-    else load8<DT>(row, e0, x);
+    load8<DT>(row, e0, x);
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = fast_exp2(fmaf(x[i], g.c, -g.lse2)) * grad_weight(g, x[i]);
     if ((unsigned)(g.label - e0) < 8u) {
@@ -272,8 +251,77 @@ __device__ __forceinline__ void row_grad_generic(const void* row, void* out, int
       for (int i = 0; i < 8; ++i)
         if (e0 + i == g.label) o[i] += g.lab_add;
     }
-    if constexpr (STREAM && DT != AA_F32) store8_stream16<DT>(out, e0, o);
-    else store8<DT>(out, e0, o);
+    store8<DT>(out, e0, o);
+  }
+  for (int j = sp.tail0 + tid; j < V; j += NT) one(j);
+}
+
+constexpr int kBufferFlags = 0x00020000;  // raw buffer, 32-bit data format
+constexpr int kAuxStream = 2;  // cache-policy bit 'nt': data is touched once, do not keep it in the caches
+
+// The same, the row and its gradient passing through once (STREAM: with the `nt` policy on loads and stores), with up to U
+// 16-byte pieces of the row read by every thread before the first of their gradients is written: the
+// memory system sees runs of U * NT * 16 bytes in one direction and then in the other.  (A piece at a time, 256 threads a
+// row, the two are mixed at the finest grain; at 4 096 x 128 256 fp32 with 30 % of the rows masked, us: 256 threads, 1 / 16
+// pieces: 711 / 687, 512 threads, 16 / 32: 676 / 645, 1 024 threads, 4 / 8 / 16 / 24: 645 / 639 / 614 / 592.)  The backward of
+// the log-prob op, us before / so: 4 096 x 128 256 fp32 747 / 599, 4 096 x 128 263 864 / 733, 8 192 x 151 936 bf16 852 / 714,
+// 8 192 x 151 943 956 / 857, 4 096 x 50 257 168 / 150, 30 000 x 16 000 310 / 297; the same bits.
+template <int DT, int NT, int U, bool STREAM>
+__device__ __forceinline__ void row_grad_bursts(const void* row, void* out, int V, bool vec_ok, const GradCoef& g) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  constexpr int E = 16 / Elem<DT>::kBytes;
+  const RowSplit sp = split_row<DT>(row, V, vec_ok);
+  const int tid = threadIdx.x;
+  auto one = [&](int j) {
+    const float x = Elem<DT>::load1(row, j);
+    float o = fast_exp2(fmaf(x, g.c, -g.lse2)) * grad_weight(g, x);
+    if (j == g.label) o += g.lab_add;
+    Elem<DT>::store1(out, j, o);
+  };
+  for (int j = tid; j < sp.head; j += NT) one(j);
+  const char* src = (const char*)row + (int64_t)sp.head * Elem<DT>::kBytes;
+  char* dst = (char*)out + (int64_t)sp.head * Elem<DT>::kBytes;
+  const int64_t n = (int64_t)sp.nvec * (8 / E);
+  constexpr int kAux = STREAM ? kAuxStream : 0;
+  auto value = [&](float x) { return fast_exp2(fmaf(x, g.c, -g.lse2)) * grad_weight(g, x); };
+  auto grad = [&](u32x4_t w, int at) {  // at: place of the label in the piece, if it lies there
+    u32x4_t r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (DT == AA_F32) r[i] = __float_as_uint(value(__uint_as_float(w[i])));
+      else r[i] = Elem<DT>::pack(value(Elem<DT>::lo(w[i])), value(Elem<DT>::hi(w[i])));
+    }
+    if ((unsigned)at < (unsigned)E) {  // one piece of a row: the word of the label again
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (DT == AA_F32) {
+          if (at == i) r[i] = __float_as_uint(value(__uint_as_float(w[i])) + g.lab_add);
+        } else {
+          if (at / 2 == i)
+            r[i] = Elem<DT>::pack(value(Elem<DT>::lo(w[i])) + (at & 1 ? 0.f : g.lab_add), value(Elem<DT>::hi(w[i])) + (at & 1 ? g.lab_add : 0.f));
+        }
+      }
+    }
+    return r;
+  };
+  for (int64_t v0 = 0; v0 < n; v0 += U * NT) {
+    // pieces past the row's last come as zeros and are not written
+    const int bytes = (int)(n - v0 < U * NT ? n - v0 : U * NT) * 16;
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc((void*)(src + v0 * 16), 0, bytes, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc((void*)(dst + v0 * 16), 0, bytes, kBufferFlags);
+    const int64_t first = g.label - sp.head - v0 * E;
+    const int at = first < 0 || first >= U * NT * E ? -1 - U * NT * E : (int)first - tid * E;  // in the thread's first piece
+    u32x4_t x[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) x[q] = __builtin_amdgcn_raw_buffer_load_b128(from, tid * 16, q * NT * 16, kAux);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      x[q] = grad(x[q], at - q * NT * E);
+      __builtin_amdgcn_sched_barrier(0);  // piece by piece: there are no registers for the intermediate values of several
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) __builtin_amdgcn_raw_buffer_store_b128(x[q], to, tid * 16 + q * NT * 16, 0, kAux);
   }
   for (int j = sp.tail0 + tid; j < V; j += NT) one(j);
 }
@@ -351,8 +399,9 @@ struct OutPtr<true, T> {
 // -----------------------------------------------------------------------------
 // STREAM: `nt` loads and stores (the host asks for them when the rows start on 128-byte lines: with rows that do
 // not, the pieces that two waves write into one line are no longer merged in the cache, and the pass is slower).
-template <int DT, int NT, bool ALIAS, bool STREAM>
-__global__ __launch_bounds__(NT) void k_logits_bwd(typename InPtr<ALIAS, void>::type logits, int V, int64_t stride,
+// U: pieces of a thread in a burst (row_grad_bursts).
+template <int DT, int NT, int U, bool ALIAS, bool STREAM>
+__global__ __launch_bounds__(NT, U > 8 ? 4 : (NT > 256 ? 8 : 4)) void k_logits_bwd(typename InPtr<ALIAS, void>::type logits, int V, int64_t stride,
                                                    const int64_t* __restrict__ labels, float inv_t, int vec_ok,
                                                    const float* __restrict__ row_lse,
                                                    const float* __restrict__ row_ez,
@@ -377,7 +426,7 @@ __global__ __launch_bounds__(NT) void k_logits_bwd(typename InPtr<ALIAS, void>::
   g.B = -gh * inv_t * inv_t;
   g.lab_add = gl * inv_t;
   g.label = (y >= 0 && y < V) ? (int)y : -1;
-  row_grad_generic<DT, NT, STREAM>(row, out, V, vec_ok != 0, g);
+  row_grad_bursts<DT, NT, U, STREAM>(row, out, V, vec_ok != 0, g);
 }
 
 // -----------------------------------------------------------------------------
@@ -566,8 +615,6 @@ __global__ __launch_bounds__(NT) void k_fused_generic(typename InPtr<ALIAS, void
 // is one.  Needs V % 8 == 0, 16-byte aligned rows and rows below 2 GB.
 // -----------------------------------------------------------------------------
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-constexpr int kBufferFlags = 0x00020000;  // raw buffer, 32-bit data format
-constexpr int kAuxStream = 2;  // cache-policy bit 'nt': data is touched once, do not keep it in the caches
 constexpr int kHoldChunk = 8 * 1024;  // values per chunk: 8 per thread
 constexpr int kHoldChunkBytes = kHoldChunk * 4;
 constexpr int kHoldStageRegs = 32;  // VGPRs for chunks in flight plus chunks held in registers, while that binds
@@ -1693,26 +1740,38 @@ extern "C" int aa_logits_bwd(const void* logits, int dtype, int64_t T, int64_t V
   if (T_active < 0 || T_active > T || !(inv_temperature > 0.f)) return AA_ERR_INVALID_ARGUMENT;
   hipStream_t st = (hipStream_t)stream;
   const int vec_ok = rows_vec_ok(logits, dlogits, dtype) ? 1 : 0;
-  constexpr int NT = 256;
   // rows on 128-byte lines take the streaming cache policy
   const int64_t row_bytes = row_stride * (dtype == AA_F32 ? 4 : 2);
   const bool streaming = vec_ok && row_bytes % 128 == 0 && ((((uintptr_t)logits | (uintptr_t)dlogits) & 127) == 0);
-#define AA_LAUNCH_AS(DT, ALIAS, STREAM)                                                                               \
-  hipLaunchKernelGGL((k_logits_bwd<DT, NT, ALIAS, STREAM>), dim3((unsigned)T), dim3(NT), 0, st, logits, (int)V,      \
+  // Bursts of 24 pieces of 1 024 threads (393 KB) for rows that 8 of them do not hold: 4 096 x 128 256 fp32 639 us with 8,
+  // 592 with 24, 8 192 x 151 936 bf16 767 and 733; a shorter row leaves most of the registers of 24 idle, and half as many
+  // workgroups fit a compute unit: 4 096 x 50 304 bf16 107 and 151.  Up to 64 KB 512 threads with 4 (30 000 x 16 000 bf16 297
+  // us; 256 with 8 306, 1 024 with 8 662), up to 16 KB 256 with one, which is no burst (20 000 x 5 000: 73 us, 512 with 4 78).
+  const int64_t bytes = V * (dtype == AA_F32 ? 4 : 2);
+#define AA_LAUNCH_AS(DT, NT, U, ALIAS, STREAM)                                                                        \
+  hipLaunchKernelGGL((k_logits_bwd<DT, NT, U, ALIAS, STREAM>), dim3((unsigned)T), dim3(NT), 0, st, logits, (int)V,   \
                      row_stride, labels, inv_temperature, vec_ok, row_lse, row_ez, g_logp, g_entropy, T_active, dlogits)
-#define AA_LAUNCH(DT)                                                \
+#define AA_LAUNCH_U(DT, NT, U)                                       \
   do {                                                               \
     if (dlogits == logits) {                                         \
-      if (streaming) AA_LAUNCH_AS(DT, true, true);                    \
-      else AA_LAUNCH_AS(DT, true, false);                            \
+      if (streaming) AA_LAUNCH_AS(DT, NT, U, true, true);            \
+      else AA_LAUNCH_AS(DT, NT, U, true, false);                     \
     } else {                                                         \
-      if (streaming) AA_LAUNCH_AS(DT, false, true);                    \
-      else AA_LAUNCH_AS(DT, false, false);                           \
+      if (streaming) AA_LAUNCH_AS(DT, NT, U, false, true);           \
+      else AA_LAUNCH_AS(DT, NT, U, false, false);                    \
     }                                                                \
+  } while (0)
+#define AA_LAUNCH(DT)                                                \
+  do {                                                               \
+    if (bytes > 8 * 1024 * 16) AA_LAUNCH_U(DT, 1024, 24);            \
+    else if (bytes > 65536) AA_LAUNCH_U(DT, 1024, 8);                \
+    else if (bytes > 16384) AA_LAUNCH_U(DT, 512, 4);                 \
+    else AA_LAUNCH_U(DT, 256, 1);                                    \
   } while (0)
   if (dtype == AA_BF16) AA_LAUNCH(AA_BF16);
   else if (dtype == AA_F16) AA_LAUNCH(AA_F16);
   else AA_LAUNCH(AA_F32);
+#undef AA_LAUNCH_U
 #undef AA_LAUNCH
 #undef AA_LAUNCH_AS
   return launch_status();

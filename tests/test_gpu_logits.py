@@ -345,3 +345,46 @@ def test_hbm_stream_probe_moves_what_it_says(device):
     assert lib.aa_hbm_stream_probe(3, 0, F._ptr(src), None, n, 3, st) == 1      # unknown kind
     assert lib.aa_hbm_stream_probe(2, 0, F._ptr(src), None, n, 3, st) == 1      # a copy needs a destination
     assert lib.aa_hbm_stream_probe(0, 0, F._ptr(src), None, n + 8, 3, st) == 1  # not a multiple of 16
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("row_bytes", [16, 16384, 16400, 32768 + 16, 65536, 65536 + 16, 131072, 131072 + 16, 393216, 393216 + 32])
+@pytest.mark.parametrize("extra", [0, 1])  # rows on 16-byte boundaries, and one value more: at every place inside a piece
+@pytest.mark.parametrize("inplace", [False, True])
+def test_backward_at_the_edges_of_its_bursts(device, dtype, row_bytes, extra, inplace):
+    """Rows around one and two bursts of every form of the backward kernel, the label in the first and last value, around
+    the end of the first burst and in between, rows without a gradient, with and without one through the entropy.  Against
+    the closed form in float64: the exponent is one fma from exact, 2^-24 of values up to 40, and 2^x and the products add
+    a few ulps: 4e-6 of the entry, then one rounding to the type of the logits."""
+    size = torch.finfo(dtype).bits // 8
+    V = row_bytes // size + extra
+    g = torch.Generator().manual_seed(V)
+    T = 9
+    x = (3.0 * torch.randn(T, V, generator=g)).to(dtype)
+    edge = min(V - 1, 512 * 4 * 16 // size)
+    labels = torch.tensor([0, V - 1, V // 2, max(edge - 1, 0), edge, min(edge + 1, V - 1), V // 3, min(7, V - 1), min(8, V - 1)])
+    gl = torch.randn(T, generator=g)
+    gl[6] = 0.0
+    gh = 0.3 * torch.randn(T, generator=g)
+    for with_entropy in (False, True):
+        xd = x.clone().to(device).requires_grad_(True)
+        lp, ent = areal_amd.gather_logprobs_entropy(xd * 1.0 if inplace else xd, labels.to(device), 0.8, inplace_backward=inplace)
+        obj = (lp * gl.to(device)).sum()
+        if with_entropy:
+            obj = obj + (ent * (gh * (gl != 0)).to(device)).sum()
+        obj.backward()
+        z = x.double() / 0.8
+        p = torch.softmax(z, 1)
+        onehot = torch.zeros_like(z).scatter_(1, labels[:, None], 1.0)
+        want = gl.double()[:, None] * (onehot - p)
+        scale = gl.double().abs()[:, None] * (onehot + p)
+        if with_entropy:
+            h = (gh * (gl != 0)).double()[:, None]
+            ez = (p * z).sum(1, keepdim=True)
+            want = want - h * p * (z - ez)
+            scale = scale + h.abs() * p * (z.abs() + ez.abs())
+        got = xd.grad.double().cpu()
+        ulp = 0.0 if dtype is torch.float32 else 2.0 ** (-8 if dtype is torch.bfloat16 else -11)
+        tiny = 2.0 ** -25 if dtype is torch.float16 else 0.0  # half a step of the subnormal values
+        assert bool(((got - want / 0.8).abs() <= (ulp * want.abs() + 8e-6 * scale) / 0.8 + tiny + 1e-30).all())
+        assert float(got[6].abs().max()) == 0.0
