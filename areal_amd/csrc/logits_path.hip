@@ -156,7 +156,8 @@ __device__ __forceinline__ RowStats block_stats(const ThreadStats& t, float* sme
   return r;
 }
 
-template <int DT, int NT, bool STREAM = false, bool WANT_U = true, bool WANT_MM = true>
+// AHEAD: groups of eight values that a thread has on their way together (rows read once, STREAM)
+template <int DT, int NT, bool STREAM = false, bool WANT_U = true, bool WANT_MM = true, int AHEAD = 1>
 __device__ __forceinline__ RowStats row_stats_generic(const void* row, int V, bool vec_ok, float c, float* smem) {
   ThreadStats a{kNegBig, 0.f, 0.f, -FLT_MAX, FLT_MAX};
   const RowSplit sp = split_row<DT>(row, V, vec_ok);
@@ -169,11 +170,23 @@ __device__ __forceinline__ RowStats row_stats_generic(const void* row, int V, bo
     const int n4 = sp.nvec * 2;  // 16-byte pieces of the vector body
     const float* body = (const float*)row + sp.head;
     int v = tid;
-    for (; v + NT < n4; v += 2 * NT) {
-      float x[8];
-      load4_stream(body + ((int64_t)v << 2), x);
-      load4_stream(body + ((int64_t)(v + NT) << 2), x + 4);
-      stats_add8_sel<WANT_U, WANT_MM>(a, x, c);
+    for (; v + (2 * AHEAD - 1) * NT < n4; v += 2 * AHEAD * NT) {
+      float x[AHEAD][8];
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q) {
+        load4_stream(body + ((int64_t)(v + 2 * q * NT) << 2), x[q]);
+        load4_stream(body + ((int64_t)(v + (2 * q + 1) * NT) << 2), x[q] + 4);
+      }
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q) stats_add8_sel<WANT_U, WANT_MM>(a, x[q], c);
+    }
+    if constexpr (AHEAD > 1) {
+      for (; v + NT < n4; v += 2 * NT) {
+        float x[8];
+        load4_stream(body + ((int64_t)v << 2), x);
+        load4_stream(body + ((int64_t)(v + NT) << 2), x + 4);
+        stats_add8_sel<WANT_U, WANT_MM>(a, x, c);
+      }
     }
     if (v < n4) {
       float x[4];
@@ -182,7 +195,27 @@ __device__ __forceinline__ RowStats row_stats_generic(const void* row, int V, bo
       for (int i = 0; i < 4; ++i) stats_add1(a, x[i], c);
     }
   } else {
-    for (int v = tid; v < sp.nvec; v += NT) {
+    int v = tid;
+    if constexpr (AHEAD > 1) {
+      typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+      const u32x4_t* body = (const u32x4_t*)((const uint16_t*)row + sp.head);
+      for (; v + (AHEAD - 1) * NT < sp.nvec; v += AHEAD * NT) {
+        u32x4_t w[AHEAD];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) w[q] = __builtin_nontemporal_load(body + v + q * NT);
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+          float x[8];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            x[2 * i] = Elem<DT == AA_F32 ? AA_BF16 : DT>::lo(w[q][i]);
+            x[2 * i + 1] = Elem<DT == AA_F32 ? AA_BF16 : DT>::hi(w[q][i]);
+          }
+          stats_add8_sel<WANT_U, WANT_MM>(a, x, c);
+        }
+      }
+    }
+    for (; v < sp.nvec; v += NT) {
       float x[8];
       if constexpr (STREAM) load8_stream<DT>(row, sp.head + ((int64_t)v << 3), x);  // the row is not read again
       else load8<DT>(row, sp.head + ((int64_t)v << 3), x);
@@ -349,7 +382,7 @@ __device__ __forceinline__ const void* row_ptr(const void* base, int64_t t, int6
 // -----------------------------------------------------------------------------
 // Forward: logp, entropy, row statistics.  grid = T rows, NT threads.
 // -----------------------------------------------------------------------------
-template <int DT, int NT, bool WANT_U, bool WANT_MM>
+template <int DT, int NT, int AHEAD, bool WANT_U, bool WANT_MM>
 __global__ __launch_bounds__(NT) void k_logits_fwd(const void* __restrict__ logits, int V, int64_t stride,
                                                    const int64_t* __restrict__ labels, float inv_t, int vec_ok,
                                                    float* __restrict__ logp, float* __restrict__ entropy,
@@ -362,7 +395,7 @@ __global__ __launch_bounds__(NT) void k_logits_fwd(const void* __restrict__ logi
   const int64_t y = labels[t];
   const bool y_ok = (y >= 0) && (y < V);
   const float xy = y_ok ? Elem<DT>::load1(row, y) : 0.f;
-  const RowStats rs = row_stats_generic<DT, NT, true, WANT_U, WANT_MM>(row, V, vec_ok != 0, c, smem);
+  const RowStats rs = row_stats_generic<DT, NT, true, WANT_U, WANT_MM, AHEAD>(row, V, vec_ok != 0, c, smem);
   if (threadIdx.x == 0) {
     const RowOut ro = finish_row(rs);
     logp[t] = y_ok ? label_logp(xy, c, rs, ro) : __builtin_nanf("");
@@ -1710,22 +1743,36 @@ extern "C" int aa_logits_fwd(const void* logits, int dtype, int64_t T, int64_t V
   if (!(inv_temperature > 0.f)) return AA_ERR_INVALID_ARGUMENT;
   hipStream_t st = (hipStream_t)stream;
   const int vec_ok = rows_vec_ok(logits, nullptr, dtype) ? 1 : 0;
-  constexpr int NT = 256;
   // the entropy sum and the extrema are left out of the pass when no output asks for them
   const bool want_u = entropy || row_ez, want_mm = vmax || vmin;
-#define AA_LAUNCH_AS(DT, U, MM)                                                                                      \
-  hipLaunchKernelGGL((k_logits_fwd<DT, NT, U, MM>), dim3((unsigned)T), dim3(NT), 0, st, logits, (int)V, row_stride, \
-                     labels, inv_temperature, vec_ok, logp, entropy, row_lse, row_ez, vmax, vmin)
-#define AA_LAUNCH(DT)                                        \
-  do {                                                       \
-    if (want_u && want_mm) AA_LAUNCH_AS(DT, true, true);     \
-    else if (want_u) AA_LAUNCH_AS(DT, true, false);          \
-    else if (want_mm) AA_LAUNCH_AS(DT, false, true);         \
-    else AA_LAUNCH_AS(DT, false, false);                     \
+  // Four groups of eight values a thread on their way together, and 1 024 threads for rows of more than 256 KB: few of them do
+  // not fill the chip otherwise.  us, 256 threads with one group / 256 with four / 1 024 with four: 200 x 151 936 bf16 43.9 /
+  // 22.9 / 16.7, 700 x 151 936 57.1 / 40.4 / 40.2, 16 384 x 151 936 712.5 / 715.7 / 702.4, 4 096 x 128 256 fp32 312 / 308 / 306;
+  // shorter rows: 400 x 60 001 fp32 26.3 / 19.3 / 20.4, 4 000 x 50 257 bf16 67.4 / 66.0 / 76.0, 20 000 x 20 001 131 / 120 / 222.
+  // Many 16-bit rows with the entropy or the extrema are bound by their arithmetic and stay with one group of 256 threads
+  // (16 384 x 151 936 bf16 729 us; 256 with four 739, 1 024 with four 740; 4 000 rows 191 / 190 / 185).
+  const bool long_row = V * (dtype == AA_F32 ? 4 : 2) > 256 * 1024;
+  const bool arithmetic = dtype != AA_F32 && (want_u || want_mm) && T >= 8192;
+#define AA_LAUNCH_AS(DT, NT, AHEAD, U, MM)                                                                           \
+  hipLaunchKernelGGL((k_logits_fwd<DT, NT, AHEAD, U, MM>), dim3((unsigned)T), dim3(NT), 0, st, logits, (int)V,          \
+                     row_stride, labels, inv_temperature, vec_ok, logp, entropy, row_lse, row_ez, vmax, vmin)
+#define AA_LAUNCH_NT(DT, NT, AHEAD)                                 \
+  do {                                                              \
+    if (want_u && want_mm) AA_LAUNCH_AS(DT, NT, AHEAD, true, true); \
+    else if (want_u) AA_LAUNCH_AS(DT, NT, AHEAD, true, false);      \
+    else if (want_mm) AA_LAUNCH_AS(DT, NT, AHEAD, false, true);     \
+    else AA_LAUNCH_AS(DT, NT, AHEAD, false, false);                 \
+  } while (0)
+#define AA_LAUNCH(DT)                              \
+  do {                                             \
+    if (long_row && arithmetic) AA_LAUNCH_NT(DT, 256, 1); \
+    else if (long_row) AA_LAUNCH_NT(DT, 1024, 4);  \
+    else AA_LAUNCH_NT(DT, 256, 4);                 \
   } while (0)
   if (dtype == AA_BF16) AA_LAUNCH(AA_BF16);
   else if (dtype == AA_F16) AA_LAUNCH(AA_F16);
   else AA_LAUNCH(AA_F32);
+#undef AA_LAUNCH_NT
 #undef AA_LAUNCH
 #undef AA_LAUNCH_AS
   return launch_status();

@@ -388,3 +388,27 @@ def test_backward_at_the_edges_of_its_bursts(device, dtype, row_bytes, extra, in
         tiny = 2.0 ** -25 if dtype is torch.float16 else 0.0  # half a step of the subnormal values
         assert bool(((got - want / 0.8).abs() <= (ulp * want.abs() + 8e-6 * scale) / 0.8 + tiny + 1e-30).all())
         assert float(got[6].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("row_bytes", [16, 4096, 16384, 16384 + 48, 32768, 262144, 262144 + 16, 262144 + 65536, 400000])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_forward_at_the_edges_of_its_rounds(device, dtype, row_bytes, extra):
+    """Rows around one and two rounds of what the threads have on their way together, and around the length from which more
+    threads take a row: every output against float64.  fp32 sums of at most 131 073 terms over 256 threads or more, each
+    to a few ulps: 2e-6 of values around 12."""
+    size = torch.finfo(dtype).bits // 8
+    V, T = row_bytes // size + extra, 5
+    g = torch.Generator().manual_seed(V)
+    x = (3.0 * torch.randn(T, V, generator=g)).to(dtype)
+    labels = torch.tensor([0, V - 1, V // 2, V // 3, min(8, V - 1)])
+    z = x.double() / 0.7
+    lse = torch.logsumexp(z, 1)
+    want_lp = z.gather(1, labels[:, None]).squeeze(1) - lse
+    want_ent = lse - (torch.softmax(z, 1) * z).sum(1)
+    xd, y = x.to(device), labels.to(device)
+    lp, ent, vmin, vmax = areal_amd.gather_logprobs_entropy_stats(xd, y, 0.7)
+    alone = areal_amd.gather_logprobs(xd, y, 0.7)
+    assert float((lp.cpu().double() - want_lp).abs().max()) < 2e-5 and float((ent.cpu().double() - want_ent).abs().max()) < 2e-5
+    assert torch.equal(vmax.cpu(), x.float().max(1).values) and torch.equal(vmin.cpu(), x.float().min(1).values)
+    assert float((alone.cpu().double() - want_lp).abs().max()) < 2e-5
