@@ -999,3 +999,25 @@ def test_upstream_factor_in_place(device, dtype, n, lead):
         N.check(N.load().aa_scale_inplace(flat[lead:].data_ptr(), _DTYPES[dtype], n, factor.data_ptr(),
                                           torch.cuda.current_stream().cuda_stream), "aa_scale_inplace")
         assert torch.equal(flat, expected)
+
+
+@pytest.mark.parametrize("total", [1, 3, 40000.0, 123457.0, 0.37, "tensor", 0])
+@pytest.mark.parametrize("multiplier", [1.0, 0.25, 3, 1e-3])
+def test_a_loss_times_the_weight_the_host_has_read(device, total, multiplier):
+    """``_times_weight`` gives the bits of the tensor expression, whatever form the total has, and its gradient."""
+    if total == "tensor":
+        total = torch.tensor(40000.0, device=device)
+    for n in (1, 7, 8191, 122433, 2 ** 24 + 3):
+        w = torch.tensor(n, device=device)
+        weight = engine_glue._weight_is_zero(w)
+        assert not weight[0]() and weight[2]() == n
+        for dtype in (torch.float32, torch.float64, torch.bfloat16):
+            x = torch.tensor(-1.2345, dtype=dtype, device=device, requires_grad=True)
+            y = x.detach().clone().requires_grad_(True)
+            got, want = engine_glue._times_weight(x, w, weight[2], total, multiplier), y * (w / total * multiplier)
+            assert got.dtype == want.dtype and torch.equal(got, want)
+            got.backward()
+            want.backward()
+            assert torch.equal(x.grad, y.grad)
+        one = torch.tensor([n], device=device)  # a weight of shape [1] keeps its shape
+        assert engine_glue._times_weight(torch.ones((), device=device), one, engine_glue._weight_is_zero(one)[2], 2.0, 1.0).shape == (1,)
