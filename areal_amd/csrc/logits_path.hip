@@ -1542,8 +1542,18 @@ __global__ __launch_bounds__(256) void k_copy16(const uint4* __restrict__ src, u
 }
 
 // The upstream factor of a backward pass on a gradient that is there already: one, almost always, and then the launch is all
-// there is (1 024 workgroups that read the factor and return, 3.2 to 4.4 us, instead of 4 096, 3.6 to 4.7).  In 16-byte
-// pieces; what lies ahead of the first and behind the last whole piece goes element by element.
+// there is (1 024 workgroups that read the factor and return: 2.15 us in a row of launches, 4 096 took 2.47).  In 16-byte
+// pieces; what lies ahead of the first and behind the last whole piece goes element by element.  Float16 products are
+// rounded once, from the exact product, one value at a time: a packed conversion rounds to float32 first, and values next
+// to a tie come out a unit off (2.5 % of them at 0.7).
+// x, a float16 value, times f with one rounding (v_fma_mixlo_f16, as for the single elements).  The empty asm keeps the
+// compiler from pairing the conversions of two values, which would round each product to float32 first.
+__device__ __forceinline__ uint32_t scale_f16(float x, float f) {
+  uint32_t w = __builtin_bit_cast(uint16_t, (_Float16)(x * f));
+  asm("" : "+v"(w));
+  return w;
+}
+
 constexpr int kScaleGroups = 1024;
 template <int DT>
 __global__ __launch_bounds__(256) void k_scale(void* __restrict__ data, int64_t n, const float* __restrict__ factor) {
@@ -1558,9 +1568,17 @@ __global__ __launch_bounds__(256) void k_scale(void* __restrict__ data, int64_t 
   for (int64_t i = first; i < pieces; i += step) {
     float x[8];
     load8<DT>(body, 8 * i, x);
+    if constexpr (DT == AA_F16) {
+      uint32_t w[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) x[q] *= f;
-    store8<DT>(body, 8 * i, x);
+      for (int q = 0; q < 8; ++q) w[q] = scale_f16(x[q], f);
+      *(uint4*)((uint16_t*)body + 8 * i) =
+          make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) x[q] *= f;
+      store8<DT>(body, 8 * i, x);
+    }
   }
   for (int64_t i = first; i < head; i += step) Elem<DT>::store1(data, i, Elem<DT>::load1(data, i) * f);
   for (int64_t i = tail + first; i < n; i += step) Elem<DT>::store1(data, i, Elem<DT>::load1(data, i) * f);

@@ -987,18 +987,28 @@ def test_work_buffer_keeps_nothing_between_the_launches_of_a_step(device):
 @pytest.mark.parametrize("n,lead", [(1, 0), (7, 1), (8, 0), (9, 3), (1000, 5), (1024 * 256 * 8 + 13, 1), (3 * 1024 * 256 * 8, 0)])
 def test_upstream_factor_in_place(device, dtype, n, lead):
     """``aa_scale_inplace``: 16-byte pieces, what lies ahead of the first and behind the last, more of them than one round of
-    workgroups takes; a factor of one leaves the array alone.  One product in float32 and one rounding: exact."""
+    workgroups takes; a factor of one leaves the array alone.  Every type rounds the exact product once: it has 35 bits at
+    most for float16 values (32 for bfloat16), float64 holds it, and numpy goes from there to float16 in one rounding.  At
+    0.7 one float16 value in forty lies where rounding to float32 first would give its neighbour; the bfloat16 products
+    of these factors have no such ties."""
+    import numpy as np
+
     from areal_amd import _native as N
     from areal_amd.functional import _DTYPES
 
-    flat = torch.randn(lead + n + 5, device=device).to(dtype)
-    want = flat.clone()
-    want[lead:lead + n] = (flat[lead:lead + n].float() * 0.37).to(dtype)
-    for f, expected in ((1.0, flat.clone()), (0.37, want)):
+    start = torch.randn(lead + n + 5, device=device).to(dtype)
+    for f in (1.0, 0.37, 0.7, -1.7):
         factor = torch.tensor([f], device=device)
+        flat, want = start.clone(), start.clone()
+        part = start[lead:lead + n]
+        if dtype == torch.float16:
+            exact = part.cpu().numpy().astype(np.float64) * np.float64(np.float32(f))
+            want[lead:lead + n] = torch.from_numpy(exact.astype(np.float16)).to(device)
+        else:
+            want[lead:lead + n] = (part.float() * factor).to(dtype)
         N.check(N.load().aa_scale_inplace(flat[lead:].data_ptr(), _DTYPES[dtype], n, factor.data_ptr(),
                                           torch.cuda.current_stream().cuda_stream), "aa_scale_inplace")
-        assert torch.equal(flat, expected)
+        assert torch.equal(flat, want), f
 
 
 @pytest.mark.parametrize("total", [1, 3, 40000.0, 123457.0, 0.37, "tensor", 0])
