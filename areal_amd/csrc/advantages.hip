@@ -567,7 +567,7 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // longer rows go block by block from the end.  The first block's loads are queued ahead of the count of the attention
 // bytes.  The maps of the recurrence are composed per thread, scanned over the wave in the lanes themselves (DPP) and over
 // the waves by every wave alike.  256 threads where a block of theirs holds a row, 512 otherwise (1 024 have half the
-// registers and spill: 512 x 4096 takes 37 us; two pieces a thread spill too: 38).
+// registers and spill: 512 x 4096 takes 37 us instead of 28).
 // With byte masks and a reference policy 10 bytes in per token (14 with values) and 28 out (24 without a reference policy):
 // 88 MB at 512 x 4096 with values, 14 us at the rate of an even mix of reads and writes.  us, with one-element memory
 // instructions and the row in LDS / so: 512 x 4096: 35.8 / 27.8, 1024 x 4096: 63.5 / 47.7, 1024 x 1001: 47.8 / 27.6,

@@ -408,8 +408,8 @@ __device__ __forceinline__ Side16 make_side16(const Operand& X, int x0, int wq, 
 //
 // NT = kNarrow: a tile of 256 x 128 for a last column of tiles with at most 128 columns of D in use.  B units hold 128
 // rows (two loads in half 0, two in half 3), a half is 16 MFMAs; A units, ring, waits and order are the same.  It needs
-// 48 B/clk of loads at full MFMA rate, near what a compute unit sustains, and takes about 0.7 of a wide tile's time (a 17th
-// column of 594 tiles at K = 1 536: 65 us narrow, 90 us wide).
+// 48 B/clk of loads at full MFMA rate, near what a compute unit sustains (4 160 x 1 536 x 151 936, a 17th column of 594
+// tiles: 1 626 us with wide tiles throughout, 1 576 with narrow ones and the panel's strips).
 template <int NT>
 __device__ __forceinline__ void mainloop16(const Operand& A, const Operand& B, int K, int m0, int n0, Acc16<NT>& acc, char* lds) {
   static_assert(NT == kWide || NT == kNarrow, "a wave's block is 128 or 64 columns wide");

@@ -1287,7 +1287,7 @@ class _FusedLmHeadPpo(torch.autograd.Function):
         V = weight.shape[0]
         dev = step.device
         # Batch padding has no outputs and a zero gradient: it stays out of the tiles where that makes them fewer (tiles
-        # end at multiples of 128 tokens).  4 096 + 56 tokens x 1 536 x 151 936: 4 112 us a step with, 3 973 without the
+        # end at multiples of 128 tokens).  4 096 + 56 tokens x 1 536 x 151 936: 4 112 us a step with, 3 999 without the
         # padding; elsewhere clearing its gradient rows in a launch of their own would only cost, about 4 us.
         if 0 < step.T_active and (step.T_active + 127) // 128 < (T + 127) // 128:
             T = step.struct.T = step.T_active
