@@ -394,9 +394,8 @@ def test_backward_at_the_edges_of_its_bursts(device, dtype, row_bytes, extra, in
 @pytest.mark.parametrize("row_bytes", [16, 4096, 16384, 16384 + 48, 32768, 262144, 262144 + 16, 262144 + 65536, 400000])
 @pytest.mark.parametrize("extra", [0, 1])
 def test_forward_at_the_edges_of_its_rounds(device, dtype, row_bytes, extra):
-    """Rows around one and two rounds of what the threads have on their way together, and around the length from which more
-    threads take a row: every output against float64.  fp32 sums of at most 131 073 terms over 256 threads or more, each
-    to a few ulps: 2e-6 of values around 12."""
+    """Rows around one and two rounds of what the 256 threads have on their way together, and long ones: every output against
+    float64.  fp32 sums of at most 200 001 terms over 256 threads, each to a few ulps: 2e-6 of values around 12."""
     size = torch.finfo(dtype).bits // 8
     V, T = row_bytes // size + extra, 5
     g = torch.Generator().manual_seed(V)
@@ -412,3 +411,28 @@ def test_forward_at_the_edges_of_its_rounds(device, dtype, row_bytes, extra):
     assert float((lp.cpu().double() - want_lp).abs().max()) < 2e-5 and float((ent.cpu().double() - want_ent).abs().max()) < 2e-5
     assert torch.equal(vmax.cpu(), x.float().max(1).values) and torch.equal(vmin.cpu(), x.float().min(1).values)
     assert float((alone.cpu().double() - want_lp).abs().max()) < 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("V", [16001, 65536, 131080, 140001])
+def test_log_probs_have_the_same_bits_in_every_call(device, dtype, V):
+    """A row is summed in one order, whatever its neighbours and whichever outputs are asked for: the log-probs that a loss
+    is formed from and those that a policy was asked for beforehand agree to the last bit, so an importance ratio of the
+    same policy is 1, and means of differences of log-probs, which cancel, are those of any other call.  Few rows and more than 8 192 of them, log-probs alone, with entropy, with the extrema as well."""
+    g = torch.Generator(device=device).manual_seed(V)
+    few, many = 64, 8192 + 64  # the same places inside a 16-byte piece in both
+    head = (3.0 * torch.randn(few, V, generator=g, device=device)).to(dtype)
+    y = torch.randint(0, V, (few,), generator=g, device=device)
+    alone = areal_amd.gather_logprobs(head, y, 0.9)
+    x = torch.zeros(many, V, dtype=dtype, device=device)
+    x[-few:] = head
+    labels = torch.zeros(many, dtype=torch.int64, device=device)
+    labels[-few:] = y
+    for rows, at in ((head, y), (x, labels)):
+        entropies = []
+        for call in (areal_amd.gather_logprobs, areal_amd.gather_logprobs_entropy, areal_amd.gather_logprobs_entropy_stats):
+            out = call(rows, at, 0.9)
+            out = out if isinstance(out, tuple) else (out,)
+            assert torch.equal(out[0][-few:], alone), (rows.shape, call.__name__)
+            entropies += [t[-few:] for t in out[1:2]]
+        assert torch.equal(*entropies)
