@@ -65,10 +65,13 @@ def _weight_is_zero(local_weight):
 def _times_weight(loss, local_weight, host_weight, total_loss_weight, multiplier):
     """``loss * (local_weight / total_loss_weight * multiplier)``.  A count that the host has read already is scaled there,
     in the float32 steps that torch takes on the device (a division by a number is a product with its reciprocal): the same
-    bits, one launch behind the loss instead of three."""
+    bits, one launch behind the loss instead of three.  Only for a loss on the device of the weight: a Python number or a
+    loss on the host takes type and device of the result from the weight tensor, or is refused with it."""
     if (host_weight is not None and local_weight.dim() == 0 and local_weight.dtype in (torch.int32, torch.int64)
-            and loss.dtype in (torch.float32, torch.float64) and type(total_loss_weight) in (int, float) and type(multiplier) in (int, float)
-            and torch.get_default_dtype() is torch.float32 and 1e-30 < abs(total_loss_weight) < 1e30):
+            and isinstance(loss, torch.Tensor) and loss.device == local_weight.device
+            and loss.dtype in (torch.float32, torch.float64) and type(total_loss_weight) in (int, float)
+            and type(multiplier) in (int, float) and torch.get_default_dtype() is torch.float32
+            and 1e-30 < abs(total_loss_weight) < 1e30 and abs(multiplier) < 1e30):
         f32 = lambda x: ctypes.c_float(x).value
         return loss * f32(f32(f32(host_weight()) * f32(1.0 / f32(total_loss_weight))) * f32(multiplier))
     return loss * (local_weight / total_loss_weight * multiplier)

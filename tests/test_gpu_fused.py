@@ -943,6 +943,40 @@ def test_padding_only_with_a_weight_of_its_own(device, lm_head):
         assert float(grad.float().abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("lm_head", [False, True])
+@pytest.mark.parametrize("kind", ["number", "0-d on the host", "0-d float64 on the host", "vector on the host", "whole number", "on the device"])
+def test_what_a_loss_function_may_return(device, kind, lm_head):
+    """The result of ``loss_fn`` times the weight as torch forms it, ``out * (weight / total * multiplier)`` with the 0-d
+    weight on the device: value, type and device; what torch refuses is refused."""
+    hidden, weight, logits, ids, mb = _glue_inputs(device)
+    mb["loss_mask"][:37] = True
+    made = {"number": lambda lp: 0.7, "0-d on the host": lambda lp: torch.tensor(0.7),
+            "0-d float64 on the host": lambda lp: torch.tensor(0.7, dtype=torch.float64),
+            "vector on the host": lambda lp: torch.tensor([0.7, 0.3]), "whole number": lambda lp: torch.tensor(3, device=device),
+            "on the device": lambda lp: lp.sum()}[kind]
+    seen = []
+    loss_fn = lambda logp, entropy, mb, **kw: seen.append(made(logp)) or (seen[-1], dict(tag=1))
+    count = lambda mb: mb["loss_mask"].count_nonzero()
+
+    def call():
+        inputs = {"rolled_input_ids": ids}
+        if lm_head:
+            return engine_glue.compute_lm_head_loss_with(hidden, weight, inputs, mb, 9, loss_fn, count, 977.0, loss_multiplier=0.3)
+        return engine_glue.compute_loss_with(logits, inputs, mb, 9, loss_fn, count, 977.0, loss_multiplier=0.3)
+
+    scale = mb["loss_mask"].count_nonzero() / 977.0 * 0.3
+    if kind == "vector on the host":
+        with pytest.raises(RuntimeError):
+            torch.tensor([0.7, 0.3]) * scale
+        with pytest.raises(RuntimeError):
+            call()
+        return
+    got, stat = call()
+    want = seen[-1] * scale
+    assert stat == dict(tag=1) and got.dtype == want.dtype and got.device == want.device and got.shape == want.shape
+    assert torch.equal(got.detach(), want.detach())
+
+
 @pytest.mark.parametrize("call", ["ppo", "sft", "lm_head ppo", "any", "lm_head any"])
 def test_long_forward_of_a_micro_batch_of_weight_zero_is_not_queued(device, monkeypatch, call):
     """Past the bound on what is queued ahead the weight is asked for first; up to it the forward runs at most once."""
