@@ -846,8 +846,8 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   };
   constexpr int kRowsHeld = 4;
   if (n.n_groups == 0 && a.bs <= kRowsHeld * THREADS) {
-    // The whole batch is one segment: a thread's rows are fetched at once and stay in its registers (the loads go past the
-    // caches: one after the other they were half of this tail)
+    // The whole batch is one segment (no group levels, or no full group): a thread's rows are fetched at once and stay in its
+    // registers (the loads go past the caches: one after the other they were half of this tail)
     RowSums held[kRowsHeld];
     double bf[2] = {0.0, 0.0}, z[1] = {0.0};
 #pragma unroll
@@ -865,7 +865,9 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
       bf[1] += held[k].F;
     }
     block_sums<2, kWaves>(bf, smem);
-    const double mean = n.mean_level == 0 || bf[1] == 0.0 ? 0.0 : bf[0] / bf[1];
+    // a mean of the group is none here: with fewer rows than a group holds there is no full group, and rows outside the full
+    // groups are centred on zero (row_mean)
+    const double mean = n.mean_level == 1 && bf[1] != 0.0 ? bf[0] / bf[1] : 0.0;
 #pragma unroll
     for (int k = 0; k < kRowsHeld; ++k)
       if (tid + k * THREADS < a.bs) z[0] += squares_about(held[k], mean);

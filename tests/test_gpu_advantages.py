@@ -416,6 +416,36 @@ def test_advantage_rows_at_the_edges_of_their_blocks(device, bs, L, offset, gamm
     assert float((normed["advantages"] - want).abs().max()) <= 4 * 2.0 ** -23 * max(float(want.abs().max()), 1.0)
 
 
+@pytest.mark.parametrize("bs,L", [(1, 64), (3, 33), (3, 1025), (3, 4097)])
+@pytest.mark.parametrize("levels", [("group", "batch"), ("group", None), ("group", "group"), (None, "group"), ("batch", "group"),
+                                    (None, "batch"), ("batch", "batch")])
+def test_normalised_advantage_rows_of_a_batch_smaller_than_a_group(device, bs, L, levels):
+    """No group is full, so a mean of the group is no mean (0), in the squares of a batch-wide deviation as well.  The
+    one-pass kernel against the separate two-pass normalisation and against the oracle, with advantages far from their
+    mean: float64 sums in another order, then one rounding to float32, 4 ulps of the largest."""
+    from areal_amd import engine_glue
+
+    g = torch.Generator().manual_seed(bs + L)
+    mask = torch.rand(bs, L, generator=g) < 0.8
+    data = dict(attention_mask=torch.ones(bs, L, dtype=torch.bool), loss_mask=mask, logprobs=-torch.rand(bs, L, generator=g),
+                values=-4.0 + torch.rand(bs, L, generator=g), rewards=torch.rand(bs, generator=g))
+    cfg = dict(mean_level=levels[0], std_level=levels[1], group_size=4)
+    norm = Normalization(NormConfig(**cfg))
+
+    def run(adv_norm):
+        d = {k: v.clone().to(device) for k, v in data.items()}
+        return engine_glue.compute_advantages(d, adv_norm=adv_norm, discount=0.0, gae_lambda=0.0, use_decoupled_loss=True)
+
+    plain, got, want = run(None), run(norm)["advantages"], run(lambda x, m: norm(x, m))["advantages"]
+    counted = plain["advantages"][plain["loss_mask"].bool()]
+    assert counted.numel() > L // 4 and float(counted[counted != 0].abs().min()) > 1.0
+    bound = 4 * 2.0 ** -23 * max(float(want.abs().max()), 1.0)
+    assert float(want.abs().max()) > 0.5 and float((got - want).abs().max()) <= bound
+    by_oracle = O.normalization(plain["advantages"].cpu(), plain["loss_mask"].cpu(), mean_leave1out=False, std_unbiased=True,
+                                eps=1e-5, **cfg)
+    assert float((got.cpu() - by_oracle).abs().max()) <= 2e-6 * (float(by_oracle.abs().max()) + 1.0)
+
+
 @pytest.mark.parametrize("shared", ["ref_logp is logprobs", "ref_logp is values", "prox_logp is values"])
 def test_advantages_of_arrays_that_share_memory(device, shared):
     """Log-probs are masked in place: with a second role for the same memory the result is that of separate kernels that
