@@ -1803,11 +1803,17 @@ extern "C" int aa_logits_bwd(const void* logits, int dtype, int64_t T, int64_t V
   // rows on 128-byte lines take the streaming cache policy
   const int64_t row_bytes = row_stride * (dtype == AA_F32 ? 4 : 2);
   const bool streaming = vec_ok && row_bytes % 128 == 0 && ((((uintptr_t)logits | (uintptr_t)dlogits) & 127) == 0);
-  // Bursts of 24 pieces of 1 024 threads (393 KB) for rows that 8 of them do not hold: 4 096 x 128 256 fp32 639 us with 8,
-  // 592 with 24, 8 192 x 151 936 bf16 767 and 733; a shorter row leaves most of the registers of 24 idle, and half as many
-  // workgroups fit a compute unit: 4 096 x 50 304 bf16 107 and 151.  Up to 64 KB 512 threads with 4 (30 000 x 16 000 bf16 297
-  // us; 256 with 8 306, 1 024 with 8 662), up to 16 KB 256 with one, which is no burst (20 000 x 5 000: 73 us, 512 with 4 78).
+  // Bursts of 24 pieces of 1 024 threads (393 KB) for long rows: 4 096 x 128 256 fp32 639 us with 8, 592 with 24, 8 192 x 151 936
+  // bf16 767 and 733.  A shorter row leaves most of the registers of 24 idle, and half as many workgroups fit a compute unit.
+  // Where the two meet, 1 GB of rows, us with 8 / 24 pieces, rows on 128-byte lines and not: fp32 130 KB 328 / 335 and 390 / 391,
+  // 136 KB 332 / 330 and 390 / 379, 180 KB 333 / 328 and 400 / 370; 16-bit rows, which turn twice the values a piece, bf16 100 KB
+  // 327 / 512 and 382 / 580, 130 KB 331 / 420 and 389 / 460, 165 KB 340 / 358 and 402 / 399, 180 KB 335 / 350 and 401 / 383, 200 KB
+  // 335 / 338 and 395 / 377, 240 KB 330 / 332 and 407 / 382.  12 and 16 pieces lie between them, 2 to 4 % below both from 130 to 165 KB
+  // off the lines; 512 threads with 16 or 24 are 4 to 7 % behind 8.
+  // Up to 64 KB 512 threads with 4 (30 000 x 16 000 bf16 297 us; 256 with 8 306, 1 024 with 8 662), up to 16 KB 256 with one, which
+  // is no burst (20 000 x 5 000: 73 us, 512 with 4 78).
   const int64_t bytes = V * (dtype == AA_F32 ? 4 : 2);
+  const int64_t long_row = (dtype == AA_F32 ? 132 : streaming ? 192 : 160) * 1024;
 #define AA_LAUNCH_AS(DT, NT, U, ALIAS, STREAM)                                                                        \
   hipLaunchKernelGGL((k_logits_bwd<DT, NT, U, ALIAS, STREAM>), dim3((unsigned)T), dim3(NT), 0, st, logits, (int)V,   \
                      row_stride, labels, inv_temperature, vec_ok, row_lse, row_ez, g_logp, g_entropy, T_active, dlogits)
@@ -1823,7 +1829,7 @@ extern "C" int aa_logits_bwd(const void* logits, int dtype, int64_t T, int64_t V
   } while (0)
 #define AA_LAUNCH(DT)                                                \
   do {                                                               \
-    if (bytes > 8 * 1024 * 16) AA_LAUNCH_U(DT, 1024, 24);            \
+    if (bytes > long_row) AA_LAUNCH_U(DT, 1024, 24);                 \
     else if (bytes > 65536) AA_LAUNCH_U(DT, 1024, 8);                \
     else if (bytes > 16384) AA_LAUNCH_U(DT, 512, 4);                 \
     else AA_LAUNCH_U(DT, 256, 1);                                    \

@@ -348,7 +348,8 @@ def test_hbm_stream_probe_moves_what_it_says(device):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("row_bytes", [16, 16384, 16400, 32768 + 16, 65536, 65536 + 16, 131072, 131072 + 16, 393216, 393216 + 32])
+@pytest.mark.parametrize("row_bytes", [16, 16384, 16400, 32768 + 16, 65536, 65536 + 16, 131072, 131072 + 16, 135168 + 16,
+                                       163840 + 16, 196608, 196608 + 16, 393216, 393216 + 32])
 @pytest.mark.parametrize("extra", [0, 1])  # rows on 16-byte boundaries, and one value more: at every place inside a piece
 @pytest.mark.parametrize("inplace", [False, True])
 def test_backward_at_the_edges_of_its_bursts(device, dtype, row_bytes, extra, inplace):
