@@ -1,6 +1,8 @@
 // Advantage pipeline of the PPO actor on gfx950: the GAE reverse scan, reward / advantage normalisation, and the
 // masked moments the statistics logger asks for.  Reference: areal/trainer/ppo/actor.py:209-236 (GAE, a Python
 // loop over max_seqlen), areal/utils/data.py:1378-1596 (Normalization), areal/utils/stats_tracker.py:227-285.
+#include <type_traits>
+
 #include "device_utils.h"
 #include "ppo_step.h"
 
@@ -121,27 +123,33 @@ __device__ __forceinline__ void enter(const Affine& mine, Affine* wave_tot, floa
   lg = (float)fma(before.c, (double)nv0, fma(before.d, (double)lg0, before.f));
 }
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
+// 16 bytes of an array that starts anywhere (on its own elements), four of a byte array
+typedef float f32x4_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u8x4_t __attribute__((aligned(1)));
 
-// A row in pieces of four positions that share 16 bytes of every array, blocks of one piece a thread from the end of the
-// row: the front of a block lies up to three positions before the row where that is what it takes, and inside it positions
-// are counted from there.  Thread 0 has the end of the block.
+// A row in pieces of four positions, blocks of one piece a thread from the end of the row.  The pieces share 16 bytes of every
+// array that starts on 16 (elsewhere a piece costs a line more now and then: 4 000 x 1 024 40 us and 46, element by element 81),
+// and the end of the last block lies up to three positions behind the row for that, unless this takes a block more (RowPlan).
+// What lies outside the row at either end is skipped; places inside a block are counted from its front.  Thread 0 has its end.
 constexpr int kOwn = 4;
 template <int THREADS>
 struct Block {
   static constexpr int kPositions = THREADS * kOwn;
   int own;          // place of the thread's first position
   int lo_in, hi_in; // the row's part of the block
-  bool whole;       // the thread's piece is inside the row, and the arrays start on 16 bytes
+  bool whole;       // the thread's piece is inside the row
   int64_t at;       // position of the row at the block's front
 
-  __device__ __forceinline__ static int64_t first(int64_t r0, int64_t L) { return ((r0 + L + 3) & ~(int64_t)3) - r0 - kPositions; }
-  __device__ __forceinline__ Block(int64_t at_, int64_t L, bool aligned) {
+  // shift: 3, or 0 for blocks that end with the row wherever that is
+  __device__ __forceinline__ static int64_t first(int64_t r0, int64_t L, int shift) {
+    return ((r0 + L + shift) & ~(int64_t)shift) - r0 - kPositions;
+  }
+  __device__ __forceinline__ Block(int64_t at_, int64_t L) {
     at = at_;
     own = (THREADS - 1 - (int)threadIdx.x) * kOwn;
     lo_in = at < 0 ? (int)-at : 0;
     hi_in = L - at < kPositions ? (int)(L - at) : kPositions;
-    whole = aligned && own >= lo_in && own + kOwn <= hi_in;
+    whole = own >= lo_in && own + kOwn <= hi_in;
   }
   __device__ __forceinline__ bool in(int o) const { return o >= lo_in && o < hi_in; }
   __device__ __forceinline__ int place(int64_t t) const { return t >= at && t < at + kPositions ? (int)(t - at) : -1; }
@@ -168,13 +176,49 @@ struct Block {
   }
 };
 
-constexpr int kShortRow = Block<256>::kPositions - 3;  // a block of 256 threads holds the row, whatever its place in a piece
+// Threads of a row.  A compute unit holds four workgroups of 256 or two of 512, and a block takes either about as long, so
+// the one that has its share of the rows through in fewer blocks one after the other is the faster one (the rounds of a launch
+// counted half as whole ones, half as they fill up: its workgroups drift apart).  Where that is the same, 512 have a row through
+// sooner; 256 are the better ones for rows that a block of theirs holds, and of those that a block of 512 holds for very many, or
+// without the sums of a normalisation.  us of a whole call, 256 / 512, with a normalisation: 1 024 x 2 050 50 / 57, 4 000 x 3 000
+// 228 / 255, 6 000 x 1 023 156 / 191, 1 333 x 9 000 231 / 200, 512 x 9 000 69 / 61; equal by that count: 2 048 x 2 044 81 / 73
+// (without 41 / 44), 2 048 x 1 279 78 / 71 (39 / 43), 2 048 x 4 096 148 / 135, 5 870 x 2 044 251 / 258.  Numbers of waves between
+// the two lose (3 000 x 1 600 with seven of them 108, with eight 104; 3 000 x 1 279 with five 114, with eight 105: they do not
+// divide over the four SIMDs).
+struct RowPlan {
+  bool wide;  // 512 threads, otherwise 256
+  int shift;  // see Block::first
+};
+static RowPlan row_plan(int64_t bs, int64_t L, bool sums) {
+  constexpr int64_t kUnits = 256;
+  auto blocks = [&](int64_t threads, int64_t more) { return (L + more + kOwn * threads - 1) / (kOwn * threads); };
+  auto chain = [&](int64_t threads) {  // in 2048ths of a block
+    const int64_t at_once = kUnits * 1024 / threads, rounds = (bs + at_once - 1) / at_once;
+    return (rounds * at_once + (bs > at_once ? bs : at_once)) * (threads / 256) * blocks(threads, 0);
+  };
+  const int64_t narrow = chain(256), wide = chain(512);
+  const bool few_blocks = blocks(256, 0) == 1 || (blocks(512, 0) == 1 && (bs >= 4096 || !sums));
+  RowPlan p;
+  p.wide = wide < narrow || (wide == narrow && !few_blocks);
+  p.shift = blocks(p.wide ? 512 : 256, kOwn - 1) == blocks(p.wide ? 512 : 256, 0) || L % kOwn == 0 ? kOwn - 1 : 0;
+  return p;
+}
+
+// launch(number of threads at compile time, shift)
+template <typename F>
+static void with_row_plan(int64_t bs, int64_t L, bool sums, F launch) {
+  const RowPlan p = row_plan(bs, L, sums);
+  if (p.wide)
+    launch(std::integral_constant<int, 512>{}, p.shift);
+  else
+    launch(std::integral_constant<int, 256>{}, p.shift);
+}
 
 // One workgroup per row: a block's inputs are read once and held in registers until its results are written.
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void k_gae(const float* __restrict__ rewards, const float* __restrict__ values,
                                                  const float* __restrict__ mask, const uint8_t* __restrict__ no_eos,
-                                                 int64_t L, float gamma, float lam, int aligned, float* adv, float* returns) {
+                                                 int64_t L, float gamma, float lam, int shift, float* adv, float* returns) {
   constexpr int kWaves = THREADS / kWave;
   __shared__ Affine wave_tot[kWaves];
   __shared__ float carry[2];
@@ -182,8 +226,8 @@ __global__ __launch_bounds__(THREADS) void k_gae(const float* __restrict__ rewar
   const float v_end = values ? values[r0 + L - 1] : 0.f;
   const float gl = gamma * lam;
   float nv0 = (no_eos && no_eos[row]) ? v_end : 0.f, lg0 = 0.f;  // nextvalues = values[:, L-1] * seq_no_eos_mask
-  for (int64_t at = Block<THREADS>::first(r0, L);; at -= Block<THREADS>::kPositions) {
-    const Block<THREADS> b(at, L, aligned != 0);
+  for (int64_t at = Block<THREADS>::first(r0, L, shift);; at -= Block<THREADS>::kPositions) {
+    const Block<THREADS> b(at, L);
     const int64_t front = r0 + at;
     const int p_end = b.place(L - 1);
     float m[kOwn], r[kOwn], v[kOwn] = {0.f, 0.f, 0.f, 0.f}, out[kOwn], ret[kOwn];
@@ -561,13 +605,13 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // ------------------------------------------------------------------------------------------------------------------
 // The advantage pipeline of a padded batch (PPOActor._compute_advantages, actor.py:172-236) in one pass per row: mask and
 // log-probs rolled and masked, KL-regularised rewards, the GAE scan, and the sums that the normalisation of the
-// advantages needs.  One workgroup per row, a thread per four positions that share 16 bytes of every array, so that each
-// array is read and written in 16-byte pieces whatever the length of the rows (the pieces at the two ends of a row are
-// taken one element at a time).  A block of 4 THREADS positions is held in registers, from its one read to its one write;
+// advantages needs.  One workgroup per row, a thread per four positions, so that each array is read and written in 16-byte
+// pieces whatever the length of the rows and wherever the arrays start (the pieces at the two ends of a row are taken one
+// element at a time).  A block of 4 THREADS positions is held in registers, from its one read to its one write;
 // longer rows go block by block from the end.  The first block's loads are queued ahead of the count of the attention
 // bytes.  The maps of the recurrence are composed per thread, scanned over the wave in the lanes themselves (DPP) and over
-// the waves by every wave alike.  256 threads where a block of theirs holds a row, 512 otherwise (1 024 have half the
-// registers and spill: 512 x 4096 takes 37 us instead of 28).
+// the waves by every wave alike.  256 threads or 512 (row_plan; 1 024 have half the registers and spill: 512 x 4096 takes 37
+// us instead of 28).
 // With byte masks and a reference policy 10 bytes in per token (14 with values) and 28 out (24 without a reference policy):
 // 88 MB at 512 x 4096 with values, 14 us at the rate of an even mix of reads and writes.  us, with one-element memory
 // instructions and the row in LDS / so: 512 x 4096: 35.8 / 27.8, 1024 x 4096: 63.5 / 47.7, 1024 x 1001: 47.8 / 27.6,
@@ -579,8 +623,8 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // ------------------------------------------------------------------------------------------------------------------
 
 // Per row: sums for the normalisation.  F = sum m, S = sum x m; A = sum m^2, B = sum m^2 (x - c), C = sum m^2 (x - c)^2
-// about a centre c of the row's own (its mean in the first super-block with a token that counts), from which the sum of squares about any mean
-// follows without cancellation.
+// about a centre c of the row's own (its mean in the first blocks up to one with a token that counts), from which the sum of
+// squares about any mean follows without cancellation.
 struct RowSums {
   double F, S, A, B, C, c;
 };
@@ -605,8 +649,7 @@ struct RowArgs {
   int64_t bs, L;
   float kl_ctl, gamma, lam;
   int estimator, mask_no_eos_with_zero, mask_bytes, roll;
-  int whole_pieces;         // the arrays start on 16 bytes (byte masks on four)
-  int attention_words;      // the attention bytes start on four
+  int shift;                // of the blocks (RowPlan)
   NormArgs norm;            // levels and groups of the normalisation (no leave-one-out)
 };
 
@@ -654,19 +697,19 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x, L = a.L, r0 = row * L;
   const float gl = a.gamma * a.lam;
-  int64_t at = Block<THREADS>::first(r0, L);
+  int64_t at = Block<THREADS>::first(r0, L, a.shift);
   struct Inputs {
     float m[kOwn + 1], lo[kOwn + 1], lr[kOwn], v[kOwn];  // mask and log-prob: one more (torch.roll(x, -1))
   };
   // what lies outside the row comes as zeros; position L, behind the last, is position 0
   auto fetch = [&](int64_t at, Inputs& x) {
-    const Block<THREADS> b(at, L, a.whole_pieces != 0);
+    const Block<THREADS> b(at, L);
     const int64_t front = r0 + at;  // (the arrays are addressed from the front of the block, by 32-bit places)
     const uint8_t* mask_b = (const uint8_t*)a.mask_in + front;
     const float *mask_f = (const float*)a.mask_in + front, *logp = a.logp + front;
     auto mask_of = [&](int o) { return a.mask_bytes ? (mask_b[o] ? 1.f : 0.f) : mask_f[o]; };
     if (b.whole && a.mask_bytes) {
-      const uint32_t w = *(const uint32_t*)(mask_b + b.own);
+      const uint32_t w = *(const u8x4_t*)(mask_b + b.own);
 #pragma unroll
       for (int q = 0; q < kOwn; ++q) x.m[q] = (w >> (8 * q)) & 0xffu ? 1.f : 0.f;
     } else if (!a.mask_bytes) {
@@ -700,22 +743,18 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   int64_t sl;
   if (a.attention) {
     uint32_t n = 0;
-    if (a.attention_words) {
-      const int lead = (int)(r0 & 3);
-      const int64_t words = (lead + L + 3) >> 2;
+    const uint8_t* attention = a.attention + r0;
+    const int lead = (int)((uintptr_t)attention & 3);  // words as they lie
+    const int64_t words = (lead + L + 3) >> 2;
 #pragma unroll 2
-      for (int64_t j = tid; j < words; j += THREADS) {
-        const int64_t t0 = 4 * j - lead;
-        if (t0 >= 0 && t0 + 4 <= L) {
-          n = __builtin_amdgcn_sad_u8(*(const uint32_t*)(a.attention + r0 + t0), 0u, n);
-        } else {
-          for (int q = 0; q < 4; ++q)
-            if (t0 + q >= 0 && t0 + q < L) n += a.attention[r0 + t0 + q];
-        }
+    for (int64_t j = tid; j < words; j += THREADS) {
+      const int64_t t0 = 4 * j - lead;
+      if (t0 >= 0 && t0 + 4 <= L) {
+        n = __builtin_amdgcn_sad_u8(*(const uint32_t*)(attention + t0), 0u, n);
+      } else {
+        for (int q = 0; q < 4; ++q)
+          if (t0 + q >= 0 && t0 + q < L) n += attention[t0 + q];
       }
-    } else {
-#pragma unroll 8
-      for (int64_t t = tid; t < L; t += THREADS) n += a.attention[r0 + t];
     }
     sl = block_sum<int>((int)n, smem_i);
   } else {
@@ -731,7 +770,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   bool first = true;
   float nv0 = no_eos ? v_end : 0.f, lg0 = 0.f;  // the state that enters the block
   for (;; at -= kBlock) {
-    const Block<THREADS> b(at, L, a.whole_pieces != 0);
+    const Block<THREADS> b(at, L);
     const int64_t front = r0 + at;
     const int p_last = b.place(at_last), p_put = b.place(put), p_end = b.place(L - 1);
     float m[kOwn], r[kOwn], v[kOwn];
@@ -1050,14 +1089,11 @@ extern "C" int aa_gae(const float* rewards, const float* values, const float* lo
   if (bs < 0 || L < 1) return AA_ERR_INVALID_ARGUMENT;
   if (bs == 0) return AA_OK;
   if (!rewards || !loss_mask || !advantages) return AA_ERR_INVALID_ARGUMENT;
-  const uintptr_t arrays = (uintptr_t)rewards | (uintptr_t)values | (uintptr_t)loss_mask | (uintptr_t)advantages | (uintptr_t)returns;
-  const int aligned = (arrays & 15) == 0;
-  if (L <= kShortRow)  // as in aa_advantages: the two are one scan
-    hipLaunchKernelGGL(k_gae<256>, dim3((unsigned)bs), dim3(256), 0, (hipStream_t)stream, rewards, values, loss_mask,
-                       seq_no_eos, L, discount, gae_lambda, aligned, advantages, returns);
-  else
-    hipLaunchKernelGGL(k_gae<512>, dim3((unsigned)bs), dim3(512), 0, (hipStream_t)stream, rewards, values, loss_mask,
-                       seq_no_eos, L, discount, gae_lambda, aligned, advantages, returns);
+  with_row_plan(bs, L, true, [&](auto threads, int shift) {
+    constexpr int kT = decltype(threads)::value;
+    hipLaunchKernelGGL(k_gae<kT>, dim3((unsigned)bs), dim3(kT), 0, (hipStream_t)stream, rewards, values, loss_mask, seq_no_eos,
+                       L, discount, gae_lambda, shift, advantages, returns);
+  });
   return launch_status();
 }
 
@@ -1189,16 +1225,11 @@ extern "C" int aa_advantages(const aa_advantage_step* step, void* stream) {
     a.work = (StepWork*)p.work;
   }
   hipStream_t st = (hipStream_t)stream;
-  const uintptr_t arrays = (uintptr_t)a.logp | (uintptr_t)a.ref | (uintptr_t)a.values | (uintptr_t)a.mask_out |
-                           (uintptr_t)a.old_out | (uintptr_t)a.kl_rewards | (uintptr_t)a.rewards | (uintptr_t)a.adv |
-                           (uintptr_t)a.returns | (uintptr_t)(a.mask_bytes ? nullptr : a.mask_in);
-  a.whole_pieces = (arrays & 15) == 0 && (!a.mask_bytes || ((uintptr_t)a.mask_in & 3) == 0);
-  a.attention_words = ((uintptr_t)a.attention & 3) == 0;
-  const dim3 grid((unsigned)p.bs);
-  if (p.L <= kShortRow)
-    hipLaunchKernelGGL(k_advantage_rows<256>, grid, dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL(k_advantage_rows<512>, grid, dim3(512), 0, st, a);
+  with_row_plan(p.bs, p.L, a.sums != nullptr, [&](auto threads, int shift) {
+    a.shift = shift;
+    constexpr int kT = decltype(threads)::value;
+    hipLaunchKernelGGL(k_advantage_rows<kT>, dim3((unsigned)p.bs), dim3(kT), 0, st, a);
+  });
   if (p.norm) launch_norm_apply(a.norm, a.stats, p.advantages, st);
   return launch_status();
 }
