@@ -1766,26 +1766,30 @@ extern "C" int aa_logits_fwd(const void* logits, int dtype, int64_t T, int64_t V
   const bool want_u = entropy || row_ez, want_mm = vmax || vmin;
   // 256 threads for every row, whatever its length, the number of rows and the outputs asked for: the order of the sums, and
   // with it the last bit of a log-prob, is the same in every call of this entry (for rows at the same place in a 16-byte piece),
-  // so that the ratio of a policy to itself is one there, and means of differences of log-probs, which cancel, do not move.  (1 024 threads for rows of more than 256 KB change a third of the
-  // log-probs by an ulp; they are faster where rows are few and 1 to 4 % otherwise: 200 x 151 936 bf16 16.5 us, 16 384 x 151 936
-  // 731, 4 096 x 128 256 fp32 317.)  Four groups of eight values a thread on their way together leave the order as it is.  us,
-  // one group / two / four, log-probs alone: 200 x 151 936 bf16 41.6 / 28.2 / 22.1, 1 000 64.9 / 52.5 / 52.3, 4 000 195 / 198 / 193,
-  // 16 384 755 / 757 / 752, 500 x 50 257 21.1 / 16.0 / 13.4, 4 000 69.7 / 70.3 / 69.2, 4 096 x 128 256 fp32 327 / 328 / 326; with
-  // entropy and extrema, which bind 16-bit rows by their arithmetic, 200 x 151 936 44.4 / 30.6 / 24.4, 4 000 199 / 200 / 199,
-  // 8 192 387 / 389 / 394, 12 000 564 / 568 / 560, 16 384 762 / 770 / 771.
-#define AA_LAUNCH_AS(DT, U, MM)                                                                                      \
-  hipLaunchKernelGGL((k_logits_fwd<DT, NT, 4, U, MM>), dim3((unsigned)T), dim3(NT), 0, st, logits, (int)V, row_stride, \
-                     labels, inv_temperature, vec_ok, logp, entropy, row_lse, row_ez, vmax, vmin)
-#define AA_LAUNCH(DT)                                        \
-  do {                                                       \
-    if (want_u && want_mm) AA_LAUNCH_AS(DT, true, true);     \
-    else if (want_u) AA_LAUNCH_AS(DT, true, false);          \
-    else if (want_mm) AA_LAUNCH_AS(DT, false, true);         \
-    else AA_LAUNCH_AS(DT, false, false);                     \
+  // so that the ratio of a policy to itself is one there, and means of differences of log-probs, which cancel, do not move.
+  // (1 024 threads for rows of more than 256 KB change a third of the log-probs by an ulp; they are faster where rows are few
+  // and 1 to 4 % otherwise: 200 x 151 936 bf16 16.5 us, 16 384 x 151 936 731, 4 096 x 128 256 fp32 317.)
+  // Four groups of eight values a thread on their way together, or one, leave the order as it is.  us, one group / two / four,
+  // log-probs alone: 200 x 151 936 bf16 41.6 / 28.2 / 22.1, 1 000 64.9 / 52.5 / 52.3, 4 000 195 / 198 / 193, 500 x 50 257 21.1 /
+  // 16.0 / 13.4, 4 000 69.7 / 70.3 / 69.2, 4 096 x 128 256 fp32 327 / 328 / 326.  Many 16-bit rows, which are bound by their
+  // arithmetic, have nothing to wait for: 16 384 x 151 936 715 / - / 720; with entropy and extrema 8 192 rows 387 / 389 / 394,
+  // 16 384 762 / 770 / 771, but 6 000 295 / 292 / 290.
+  const bool many = dtype != AA_F32 && T >= 8192;
+#define AA_LAUNCH_AS(DT, AHEAD, U, MM)                                                                               \
+  hipLaunchKernelGGL((k_logits_fwd<DT, NT, AHEAD, U, MM>), dim3((unsigned)T), dim3(NT), 0, st, logits, (int)V,       \
+                     row_stride, labels, inv_temperature, vec_ok, logp, entropy, row_lse, row_ez, vmax, vmin)
+#define AA_LAUNCH(DT, AHEAD)                                    \
+  do {                                                          \
+    if (want_u && want_mm) AA_LAUNCH_AS(DT, AHEAD, true, true); \
+    else if (want_u) AA_LAUNCH_AS(DT, AHEAD, true, false);      \
+    else if (want_mm) AA_LAUNCH_AS(DT, AHEAD, false, true);     \
+    else AA_LAUNCH_AS(DT, AHEAD, false, false);                 \
   } while (0)
-  if (dtype == AA_BF16) AA_LAUNCH(AA_BF16);
-  else if (dtype == AA_F16) AA_LAUNCH(AA_F16);
-  else AA_LAUNCH(AA_F32);
+  if (dtype == AA_BF16 && many) AA_LAUNCH(AA_BF16, 1);
+  else if (dtype == AA_BF16) AA_LAUNCH(AA_BF16, 4);
+  else if (dtype == AA_F16 && many) AA_LAUNCH(AA_F16, 1);
+  else if (dtype == AA_F16) AA_LAUNCH(AA_F16, 4);
+  else AA_LAUNCH(AA_F32, 4);
 #undef AA_LAUNCH
 #undef AA_LAUNCH_AS
   return launch_status();
