@@ -1541,11 +1541,6 @@ __global__ __launch_bounds__(256) void k_copy16(const uint4* __restrict__ src, u
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) dst[i] = src[i];
 }
 
-// The upstream factor of a backward pass on a gradient that is there already: one, almost always, and then the launch is all
-// there is (1 024 workgroups that read the factor and return: 2.15 us in a row of launches, 4 096 took 2.47).  In 16-byte
-// pieces; what lies ahead of the first and behind the last whole piece goes element by element.  Float16 products are
-// rounded once, from the exact product, one value at a time: a packed conversion rounds to float32 first, and values next
-// to a tie come out a unit off (2.5 % of them at 0.7).
 // x, a float16 value, times f with one rounding (v_fma_mixlo_f16, as for the single elements).  The empty asm keeps the
 // compiler from pairing the conversions of two values, which would round each product to float32 first.
 __device__ __forceinline__ uint32_t scale_f16(float x, float f) {
@@ -1554,6 +1549,11 @@ __device__ __forceinline__ uint32_t scale_f16(float x, float f) {
   return w;
 }
 
+// The upstream factor of a backward pass on a gradient that is there already: one, almost always, and then the launch is all
+// there is (1 024 workgroups that read the factor and return: 2.15 us in a row of launches, 4 096 took 2.47).  In 16-byte
+// pieces; what lies ahead of the first and behind the last whole piece goes element by element.  Float16 products are
+// rounded once, from the exact product, one value at a time: a packed conversion rounds to float32 first, and values next
+// to a tie come out a unit off (2.5 % of them at 0.7).
 constexpr int kScaleGroups = 1024;
 template <int DT>
 __global__ __launch_bounds__(256) void k_scale(void* __restrict__ data, int64_t n, const float* __restrict__ factor) {
@@ -2088,7 +2088,7 @@ extern "C" int aa_copy_bytes(const void* src, void* dst, int64_t nbytes, void* s
 extern "C" int aa_scale_inplace(void* data, int dtype, int64_t n, const float* factor, void* stream) {
   if (!data || !factor || n < 0) return AA_ERR_INVALID_ARGUMENT;
   if (n == 0) return AA_OK;
-  int64_t blocks = (n + 255) / 256;
+  int64_t blocks = ((n + 7) / 8 + 255) / 256;  // a thread for eight values at first
   if (blocks > kScaleGroups) blocks = kScaleGroups;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == AA_BF16) hipLaunchKernelGGL(k_scale<AA_BF16>, dim3((unsigned)blocks), dim3(256), 0, st, data, n, factor);
