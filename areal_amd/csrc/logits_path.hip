@@ -1812,7 +1812,7 @@ extern "C" int aa_logits_bwd(const void* logits, int dtype, int64_t T, int64_t V
   // Where the two meet, 1 GB of rows, us with 8 / 24 pieces, rows on 128-byte lines and not: fp32 130 KB 328 / 335 and 390 / 391,
   // 136 KB 332 / 330 and 390 / 379, 180 KB 333 / 328 and 400 / 370; 16-bit rows, which turn twice the values a piece, bf16 100 KB
   // 327 / 512 and 382 / 580, 130 KB 331 / 420 and 389 / 460, 165 KB 340 / 358 and 402 / 399, 180 KB 335 / 350 and 401 / 383, 200 KB
-  // 335 / 338 and 395 / 377, 240 KB 330 / 332 and 407 / 382.  12 and 16 pieces lie between them, 2 to 4 % below both from 130 to 165 KB
+  // 335 / 338 and 395 / 377, 240 KB 330 / 332 and 407 / 382.  12 and 16 pieces are 2 to 5 % below both from 130 to 165 KB
   // off the lines; 512 threads with 16 or 24 are 4 to 7 % behind 8.
   // Up to 64 KB 512 threads with 4 (30 000 x 16 000 bf16 297 us; 256 with 8 306, 1 024 with 8 662), up to 16 KB 256 with one, which
   // is no burst (20 000 x 5 000: 73 us, 512 with 4 78).
