@@ -45,6 +45,13 @@ static_assert(strip_bytes(32) % 16 == 0 && 4 * strip_bytes(32) <= kLdsBytes, "th
 
 __host__ __device__ __forceinline__ int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
+// Pitch of the panel in elements: V rounded up to whole 128-byte lines, so that every row starts on one (the array itself
+// does, see plan()).  The panel's strips are stored, and read again by both gradient products, in pieces of 128 bytes and
+// more; with a pitch that is only a multiple of 16 bytes each of them touches a line more.  us, V = 50 264 at its own pitch / on
+// lines: forward tiles, d_hidden, d_weight of 8 000 x 2 048 1 436 / 1 371, 971 / 882, 952 / 931.  Next to 2^22 only the multiple of
+// 8 that the pieces need: 256 rows stay below the 32-bit byte offsets of a tile.
+static int64_t panel_pitch(int64_t V) { return round_up(V, 64) < ((int64_t)1 << 22) ? round_up(V, 64) : round_up(V, 8); }
+
 enum { kModeStats = 0, kModeStatsCarry = 1, kModeRecompute = 2 };
 
 // ---- the row count of a chunk, when only the device knows it -------------------------------------------------------
@@ -66,8 +73,8 @@ struct TileArgs {
   const int64_t* labels;  // labels of the chunk
   int64_t pitch_t;
   float c;                // log2(e) / temperature
-  // panel [rows, panel_ld] bf16, panel_ld = V rounded up to 8 (the entries past V are written as zeros): row
-  // out_rows[token] (or the token itself when out_rows is null); negative: no row
+  // panel [rows, panel_ld] bf16 (panel_pitch; the entries from V up to a multiple of 8 are written as zeros, those behind
+  // them by nobody): row out_rows[token] (or the token itself when out_rows is null); negative: no row
   uint16_t* panel;
   int64_t panel_ld;
   const int32_t* out_rows;
@@ -1094,7 +1101,7 @@ __global__ __launch_bounds__(256) void k_f32_to_bf16(const f32x4_t* __restrict__
 struct Workspace {
   int64_t chunk, blocks;                // tokens per chunk, 128-row vocabulary blocks
   int64_t off_pk, off_ps, off_pu;       // block partials [blocks][chunk]
-  int64_t panel_ld;                     // pitch of the panel: V rounded up to 8 elements
+  int64_t panel_ld;                     // pitch of the panel (panel_pitch)
   int64_t off_xy, off_g, off_lse;       // per token of the chunk: label logit, g, logsumexp
   int64_t fwd_bytes;                    // what the forward alone needs
   int64_t off_pn;                       // smallest logit per block [blocks][chunk] (only when the extrema are asked for)
@@ -1130,7 +1137,7 @@ static Workspace plan(int64_t T, int64_t H, int64_t V, bool external_panel = fal
   w.off_flag = off;    off += 256;              // the chunk's "redo by recompute" flag
   w.off_total = off;   off += 256;
   w.off_rows = off;    off += up(2 * w.chunk * 4);
-  w.panel_ld = round_up(V, 8);
+  w.panel_ld = panel_pitch(V);
   w.off_panel = off;   off += external_panel ? 0 : up(w.chunk * w.panel_ld * 2);
   w.off_hc = off;      off += up(w.chunk * H * 2);
   w.off_dw = off;      off += T > w.chunk ? up(V * H * 4) : 0;
@@ -1569,7 +1576,7 @@ extern "C" int64_t aa_lmhead_carry_workspace_bytes(int64_t T, int64_t H, int64_t
   return plan(T, H, V, true).bytes;
 }
 
-extern "C" int64_t aa_lmhead_panel_pitch(int64_t V) { return round_up(V, 8); }
+extern "C" int64_t aa_lmhead_panel_pitch(int64_t V) { return panel_pitch(V); }
 
 // rows of the panel that the chunks before chunk `upto` take: the tokens named by the host's counts, or all of them
 static int64_t panel_rows_before(const int64_t* kept_per_chunk, int64_t chunk, int64_t T, int64_t upto) {

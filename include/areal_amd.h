@@ -778,7 +778,7 @@ int aa_moments_table(const void* const* values, const uint8_t* const* masks,
 
 /* Bytes of workspace aa_lmhead_bwd / aa_lmhead_ppo_fused need for these sizes.
  * With C = min(T, aa_lmhead_chunk_tokens()): 2 * C * V (the bf16 d(logits)
- * rows of one token chunk; their pitch is V rounded up to 8), 32 * (V / 256) *
+ * rows of one token chunk; their pitch is V rounded up to 64), 32 * (V / 256) *
  * C (softmax partials and smallest logit per 128 vocabulary rows and token), 2 * C * H (the hidden rows of the tokens with a
  * gradient, closed up), 16 * C * H (four fp32 planes of d_hidden rows: the
  * product that forms them has few tiles and is cut along the vocabulary into

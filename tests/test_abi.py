@@ -121,3 +121,13 @@ def test_argument_validation_of_the_sibling_entry_points_without_gpu():
                                    p, p, p, p, z, z) == bad                             # SAPO gate temperature of zero
     params = _native.PpoParams(clip_lo=0.8, clip_hi=1.2, loss_kind=1)
     assert lib.aa_ppo_loss(p, p, p, p, z, 4, z, 0, 0, ctypes.byref(params), p, p, p, p, p, z) == 2   # unsupported
+
+
+@pytest.mark.parametrize("V", [1, 8, 64, 65, 50257, 151936, (1 << 22) - 64, (1 << 22) - 63, (1 << 22) - 8, (1 << 22) - 1])
+def test_panel_pitch(V):
+    """Whole 128-byte lines of bf16, except next to 2^22: 256 rows of the panel stay below the byte offsets of a tile, or
+    reach them where the multiple of 8 does."""
+    pitch = int(_native.load().aa_lmhead_panel_pitch(V))
+    eight = (V + 7) // 8 * 8
+    assert pitch >= V and pitch % 8 == 0
+    assert pitch == (V + 63) // 64 * 64 if V <= (1 << 22) - 64 else pitch == eight

@@ -1008,3 +1008,24 @@ def test_workspace_of_a_small_step_follows_its_size(device):
     chunk, H, V = 256, 64, 1024
     partials, panel, rows, vectors = 4 * 2 * (V // 256) * chunk * 4, chunk * V * 2, chunk * H * 2, 1 << 16
     assert lib.aa_lmhead_workspace_bytes(chunk, H, V) <= partials + panel + rows + vectors + 32 * chunk * H * 4
+
+
+@pytest.mark.parametrize("V", [56, 65, 127, 648, 1001, 4152])
+def test_panel_rows_that_end_inside_a_line(device, V):
+    """The rows of the panel start on 128-byte lines: what lies between the end of a row and the next line is written by
+    nobody and must not be read.  The step over a workspace of NaN patterns against the oracle (bounds as above)."""
+    lib = _native.load()
+    assert V <= int(lib.aa_lmhead_panel_pitch(V)) < V + 64 and int(lib.aa_lmhead_panel_pitch(V)) % 64 == 0
+    T, H = 300, 72
+    hidden, weight, labels, prox, old, adv, mask = _inputs(T, T, H, V, seed=V)
+    h = hidden.to(device).requires_grad_(True)
+    w = weight.to(device).requires_grad_(True)
+    _poison_the_allocator_cache(device, int(lib.aa_lmhead_workspace_bytes(T, H, V)))
+    loss, _ = areal_amd.fused_lm_head_ppo_loss(h, w, *(t.to(device) for t in (labels, prox, old, adv)), eps_clip=0.2,
+                                               loss_mask=mask.to(device))
+    loss.backward()
+    o_loss, _, _, _, o_dh, o_dw = _oracle_step(hidden, weight, labels, prox, old, adv, mask, 1.0, 1.0, eps_clip=0.2)
+    assert float(loss.detach()) == pytest.approx(o_loss, rel=1e-3)
+    for got, want in ((h.grad, o_dh), (w.grad, o_dw)):
+        assert cosine(got.cpu().float(), want) > 0.9999
+        assert_same_magnitude(got, want)
