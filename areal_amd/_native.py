@@ -157,6 +157,21 @@ class AdvantageStep(C.Structure):
     ]
 
 
+SCORE_GROUP = 64  # AA_SCORE_GROUP
+
+
+class ScoreStep(C.Structure):
+    """``aa_score_step``"""
+
+    _fields_ = [
+        ("rewards", C.c_void_p),
+        ("bias", C.c_float),
+        ("scaling", C.c_float),
+        ("clip", C.c_float),
+        ("norm", C.POINTER(NormParams)),
+    ]
+
+
 _p = C.c_void_p
 _i64 = C.c_int64
 _f = C.c_float
@@ -231,6 +246,7 @@ SIGNATURES = {
     "aa_reward_scores": (_i, [_p, _i64, _f, _f, _f, C.POINTER(NormParams), _p, _p]),
     "aa_advantages_scratch_bytes": (_i64, [_i64]),
     "aa_advantages": (_i, [C.POINTER(AdvantageStep), _p]),
+    "aa_advantages_scored": (_i, [C.POINTER(AdvantageStep), C.POINTER(ScoreStep), _p]),
     "aa_kl_rewards": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _f, _i, _i, _p, _p, _p]),
     "aa_gae": (_i, [_p, _p, _p, _p, _i64, _i64, _f, _f, _p, _p, _p]),
     "aa_normalize_scratch_bytes": (_i64, [_i64, _i64, _i64]),

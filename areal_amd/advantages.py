@@ -130,16 +130,37 @@ def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
     return pa < pb + b.numel() * b.element_size() and pb < pa + a.numel() * a.element_size()
 
 
+def _scorable(rewards, bias, scaling, clip, norm) -> bool:
+    if not all(isinstance(v, Real) for v in (bias, scaling, clip)):
+        return False
+    if norm is not None and not (type(norm) is Normalization and _one_process() and rewards.numel() <= 8192):
+        return False
+    return (_plain(rewards, rewards.shape, rewards.device) and rewards.ndim == 1 and rewards.is_cuda
+            and rewards.numel() != 0)
+
+
+def score_step(rewards: torch.Tensor, bias: float, scaling: float, clip: float, norm) -> N.ScoreStep | None:
+    """``reward_scores`` for ``advantage_rows`` to form in its own launch; None when the rewards ask for one ahead of it (a
+    level over the batch, groups of more rows than a wave) or for the general way."""
+    if not _scorable(rewards, bias, scaling, clip, norm):
+        return None
+    step = N.ScoreStep(_ptr(rewards), float(bias), float(scaling), float(clip))
+    if norm is not None:
+        params = norm._params()
+        if 1 in (params.mean_level, params.std_level):
+            return None
+        if 2 in (params.mean_level, params.std_level) and not 1 <= params.group_size <= N.SCORE_GROUP:
+            return None
+        step.norm = C.pointer(params)
+    return step
+
+
 @torch.no_grad()
 def reward_scores(rewards: torch.Tensor, bias: float, scaling: float, clip: float, norm) -> torch.Tensor | None:
     """``norm(clip((rewards + bias) * scaling, -clip, clip))`` (actor.py:166-172) in one launch; None when the inputs ask
     for the general way (``norm`` another callable than ``Normalization``, more rewards than one launch takes, tensors for
     numbers)."""
-    if not all(isinstance(v, Real) for v in (bias, scaling, clip)):
-        return None
-    if norm is not None and not (type(norm) is Normalization and _one_process() and rewards.numel() <= 8192):
-        return None
-    if not _plain(rewards, rewards.shape, rewards.device) or rewards.ndim != 1 or not rewards.is_cuda or rewards.numel() == 0:
+    if not _scorable(rewards, bias, scaling, clip, norm):
         return None
     out = torch.empty_like(rewards)
     dev = rewards.device
@@ -152,10 +173,11 @@ def reward_scores(rewards: torch.Tensor, bias: float, scaling: float, clip: floa
 
 @torch.no_grad()
 def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, values, kl_ctl, kl_estimator, discount,
-                   gae_lambda, mask_no_eos_with_zero, norm):
+                   gae_lambda, mask_no_eos_with_zero, norm, scores=None):
     """Masks, rewards, GAE and the normalisation of the advantages in one pass per row (``aa_advantages``): returns
     ``(mask, logp, kl_rewards, rewards, advantages, returns)``, ``ref_logp`` (and, without ``roll``, ``logp``) masked in
-    place; None when the inputs ask for the general way."""
+    place; None when the inputs ask for the general way.  ``scores`` (``score_step``): ``score`` holds the rewards, and the
+    scores are formed on the way."""
     if loss_mask.ndim != 2 or not loss_mask.is_cuda or loss_mask.numel() == 0 or kl_estimator not in _KL_IDS:
         return None
     shape, dev = loss_mask.shape, loss_mask.device
@@ -171,6 +193,8 @@ def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, value
         return None
     if not roll and values is not None and _overlap(logp, values):
         return None
+    if scores is not None and any(t is not None and _overlap(score, t) for t in (ref_logp, None if roll else logp)):
+        return None  # a row reads the rewards of its group
     if attention_mask.shape != shape or attention_mask.device != dev or score.shape != (bs,) or not _plain(score, (bs,), dev):
         return None
     if loss_mask.dtype is torch.bool:
@@ -189,7 +213,9 @@ def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, value
     a = N.AdvantageStep()
     a.bs, a.L = bs, L
     a.loss_mask, a.loss_mask_bytes, a.roll_logp = _ptr(mask), is_bytes, int(roll)
-    a.logp, a.ref_logp, a.values, a.reward_score = _ptr(logp), _ptr(ref_logp), _ptr(values), _ptr(score)
+    a.logp, a.ref_logp, a.values = _ptr(logp), _ptr(ref_logp), _ptr(values)
+    if scores is None:
+        a.reward_score = _ptr(score)
     a.attention_mask, a.seqlens = _ptr(attention), _ptr(seqlens)
     a.kl_ctl, a.discount, a.gae_lambda = float(kl_ctl), float(discount), float(gae_lambda)
     a.kl_estimator, a.mask_no_eos_with_zero = _KL_IDS[kl_estimator], int(bool(mask_no_eos_with_zero))
@@ -201,7 +227,10 @@ def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, value
         a.norm = C.pointer(params)
         a.scratch, a.scratch_bytes, a.work = _ptr(scratch), scratch.numel() * 8, _ptr(_work_words(dev))
     with _on(dev):
-        N.check(lib.aa_advantages(a, _stream(dev)), "aa_advantages")
+        if scores is None:
+            N.check(lib.aa_advantages(a, _stream(dev)), "aa_advantages")
+        else:
+            N.check(lib.aa_advantages_scored(a, scores, _stream(dev)), "aa_advantages_scored")
     for t in (ref_logp, None if roll else logp):  # written through a raw pointer: autograd is told
         if t is not None:
             torch.autograd.graph.increment_version(t)

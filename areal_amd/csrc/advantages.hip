@@ -376,6 +376,7 @@ __global__ __launch_bounds__(kWave) void k_norm_finish(const double2* __restrict
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int64_t kSmallNorm = 8192;  // values
 constexpr int kSmallThreads = 256;
+static_assert(AA_SCORE_GROUP == kWave, "a group of the scores is one wave (row_score)");
 
 struct Scores {
   int on;
@@ -560,6 +561,34 @@ static bool one_launch(const NormArgs& a) {
   return reads <= (a.mask ? 15360 : 18432);
 }
 
+// Score of one row by a wave, normalised by its group when `a` names levels (0 or 2, groups of at most kWave rows): a lane
+// has one value of the group, so the two sums are those of k_norm_small in the same order and the result its bits.  Its loads
+// and sums lie behind the loads of the row's first block; a launch ahead of it was 5 us on the stream and 7 on the host (whole calls,
+// us, a launch / so: 512 x 4096 41.2 / 35.1, 32 x 300 42.1 / 35.7).  Groups of more rows, and levels over the batch, which every
+// row would have to read, keep the launch.
+__device__ __forceinline__ float row_score(const Scores& sc, const NormArgs& a, const float* __restrict__ rewards, int64_t row) {
+  const float xi = score_of(sc, rewards[row]);
+  if (a.mean_level == 0 && a.std_level == 0) return xi;
+  const int64_t g = row / a.group_size;
+  const bool grouped = g < a.n_groups;
+  double4 group = make_double4(0.0, 0.0, 0.0, 0.0);
+  if (grouped) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool on = lane < (int)a.group_size;
+    const float x = on ? score_of(sc, rewards[g * a.group_size + lane]) : 0.f;
+    group.x = wave_sum((double)x);
+    group.y = (double)a.group_size;
+    if (a.std_level == 2) {
+      double mean = 0.0;
+      if (a.mean_level == 2 && !(a.group_size == 1 && a.mean_leave1out))
+        mean = (double)(float)level_mean(group.x, group.y, a.mean_leave1out != 0, false, x, 1.0);
+      const double d = on ? (double)x - mean : 0.0;
+      group.z = wave_sum(d * d);
+    }
+  }
+  return norm_element(a, make_double4(0.0, 0.0, 0.0, 0.0), group, grouped, false, xi, 1.f);
+}
+
 // without a normalisation: the scores themselves
 __global__ __launch_bounds__(256) void k_scores(const float* __restrict__ x, int64_t n, Scores sc, float* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -635,7 +664,8 @@ struct RowArgs {
   float* ref;               // nullable; masked in place
   const uint8_t* attention; // nullable: [bs, L], one byte per token ...
   const int64_t* seqlens;   // ... or the lengths [bs]
-  const float* score;       // [bs]
+  const float* score;       // [bs]; or null and ...
+  const float* reward;      // ... [bs], the scores formed here (row_score)
   const float* values;      // nullable
   float* mask_out;
   float* old_out;           // may be logp itself when it is not rolled
@@ -651,6 +681,8 @@ struct RowArgs {
   int estimator, mask_no_eos_with_zero, mask_bytes, roll;
   int shift;                // of the blocks (RowPlan)
   NormArgs norm;            // levels and groups of the normalisation (no leave-one-out)
+  Scores sc;                // with reward
+  NormArgs score_norm;      // with reward: levels none or group
 };
 
 __device__ __forceinline__ float mask_at(const RowArgs& a, int64_t i) {
@@ -694,6 +726,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   __shared__ double smem[kWaves * 5];
   __shared__ int smem_i[kWaves];
   __shared__ int last;
+  __shared__ float row_reward;
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x, L = a.L, r0 = row * L;
   const float gl = a.gamma * a.lam;
@@ -740,6 +773,10 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   Inputs x;
   fetch(at, x);
   const float v_end = a.values ? a.values[r0 + L - 1] : 0.f;
+  if (a.reward && tid < kWave) {  // one wave, behind the others' loads; there is a barrier before anyone needs it
+    const float v = row_score(a.sc, a.score_norm, a.reward, row);
+    if (tid == 0) row_reward = v;
+  }
   int64_t sl;
   if (a.attention) {
     uint32_t n = 0;
@@ -759,13 +796,14 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
     sl = block_sum<int>((int)n, smem_i);
   } else {
     sl = a.seqlens[row];
+    if (a.reward) __syncthreads();
   }
   int64_t at_last = sl - 1;
   if (at_last < 0) at_last += L;  // Python's negative index, as the reference's fancy indexing does
   int64_t put = sl - 2;
   if (put < 0) put = 0;
   const bool no_eos = sl == L;
-  const float score = (a.mask_no_eos_with_zero && no_eos) ? 0.f : a.score[row];
+  const float score = (a.mask_no_eos_with_zero && no_eos) ? 0.f : (a.reward ? row_reward : a.score[row]);
   double F = 0.0, S = 0.0, A = 0.0, B = 0.0, C = 0.0, c = 0.0;
   bool first = true;
   float nv0 = no_eos ? v_end : 0.f, lg0 = 0.f;  // the state that enters the block
@@ -1177,12 +1215,12 @@ extern "C" int64_t aa_advantages_scratch_bytes(int64_t bs) {
   return (1 + bs) * (int64_t)sizeof(double4) + bs * (int64_t)sizeof(RowSums);
 }
 
-extern "C" int aa_advantages(const aa_advantage_step* step, void* stream) {
+static int advantages(const aa_advantage_step* step, const aa_score_step* scores, void* stream) {
   if (!step) return AA_ERR_INVALID_ARGUMENT;
   const aa_advantage_step& p = *step;
   if (p.bs < 0 || p.L < 1 || p.bs > 0x7fffffff || p.kl_estimator < 0 || p.kl_estimator > 2) return AA_ERR_INVALID_ARGUMENT;
   if (p.bs == 0) return AA_OK;
-  if (!p.loss_mask || !p.logp || !p.reward_score || (!p.attention_mask && !p.seqlens) || !p.mask_out || !p.logp_out ||
+  if (!p.loss_mask || !p.logp || !(scores ? scores->rewards : p.reward_score) || (!p.attention_mask && !p.seqlens) || !p.mask_out || !p.logp_out ||
       !p.kl_rewards || !p.rewards || !p.advantages || !p.returns)
     return AA_ERR_INVALID_ARGUMENT;
   if (p.roll_logp && p.logp_out == p.logp) return AA_ERR_INVALID_ARGUMENT;
@@ -1192,7 +1230,22 @@ extern "C" int aa_advantages(const aa_advantage_step* step, void* stream) {
   a.ref = p.ref_logp;
   a.attention = p.attention_mask;
   a.seqlens = p.seqlens;
-  a.score = p.reward_score;
+  a.score = scores ? nullptr : p.reward_score;
+  if (scores) {
+    a.reward = scores->rewards;
+    a.sc = Scores{1, scores->bias, scores->scaling, scores->clip};
+    if (scores->norm) {
+      const aa_norm_params& q = *scores->norm;
+      if (q.mean_level < 0 || q.mean_level > 2 || q.std_level < 0 || q.std_level > 2) return AA_ERR_INVALID_ARGUMENT;
+      if (q.mean_level == 1 || q.std_level == 1) return AA_ERR_UNSUPPORTED;
+      const bool grouped = q.mean_level == 2 || q.std_level == 2;
+      if (grouped && q.group_size < 1) return AA_ERR_INVALID_ARGUMENT;
+      if (grouped && q.group_size > AA_SCORE_GROUP) return AA_ERR_UNSUPPORTED;
+      const int64_t gs = grouped ? q.group_size : p.bs;
+      a.score_norm = NormArgs{scores->rewards, nullptr, p.bs, gs, grouped ? p.bs / gs : 0, gs, q.mean_level, q.mean_leave1out,
+                              q.std_level, q.std_unbiased, q.eps};
+    }
+  }
   a.values = p.values;
   a.mask_out = p.mask_out;
   a.old_out = p.logp_out;
@@ -1232,6 +1285,12 @@ extern "C" int aa_advantages(const aa_advantage_step* step, void* stream) {
   });
   if (p.norm) launch_norm_apply(a.norm, a.stats, p.advantages, st);
   return launch_status();
+}
+
+extern "C" int aa_advantages(const aa_advantage_step* step, void* stream) { return advantages(step, nullptr, stream); }
+
+extern "C" int aa_advantages_scored(const aa_advantage_step* step, const aa_score_step* scores, void* stream) {
+  return scores ? advantages(step, scores, stream) : AA_ERR_INVALID_ARGUMENT;
 }
 
 extern "C" int aa_kl_rewards(const float* old_logp, const float* ref_logp, const float* loss_mask,

@@ -14,7 +14,7 @@ from typing import Any
 
 import torch
 
-from .advantages import advantage_rows, gae_advantages, kl_regularized_rewards, reward_scores
+from .advantages import advantage_rows, gae_advantages, kl_regularized_rewards, reward_scores, score_step
 from .functional import (
     COUNT_ON_DEVICE_BYTES,
     _HostCounts,
@@ -325,16 +325,23 @@ def compute_advantages(
 
         assert overlong_penalty_factor is not None and max_new_tokens is not None
         data = reward_overlong_penalty(data, overlong_tokens, overlong_penalty_factor, max_new_tokens)
-    reward_score = reward_scores(data["rewards"], reward_bias, reward_scaling, reward_clip, reward_norm)
-    if reward_score is None:
-        reward_score = (data["rewards"] + reward_bias) * reward_scaling      # actor.py:166-170
-        reward_score = torch.clip(reward_score, max=reward_clip, min=-reward_clip)
-        if reward_norm is not None:
-            reward_score = reward_norm(reward_score)
     recomputed = not use_decoupled_loss and recompute_logprob
-    rows = advantage_rows(data["loss_mask"], data["prox_logp"] if recomputed else data["logprobs"], not recomputed,
-                          data.get("ref_logp"), data["attention_mask"], reward_score, data.get("values"), kl_ctl,
-                          kl_estimator, discount, gae_lambda, mask_no_eos_with_zero, adv_norm)
+
+    def one_pass(reward_score, scores=None):
+        return advantage_rows(data["loss_mask"], data["prox_logp"] if recomputed else data["logprobs"], not recomputed,
+                              data.get("ref_logp"), data["attention_mask"], reward_score, data.get("values"), kl_ctl,
+                              kl_estimator, discount, gae_lambda, mask_no_eos_with_zero, adv_norm, scores)
+
+    scores = score_step(data["rewards"], reward_bias, reward_scaling, reward_clip, reward_norm)
+    rows = None if scores is None else one_pass(data["rewards"], scores)
+    if rows is None:
+        reward_score = reward_scores(data["rewards"], reward_bias, reward_scaling, reward_clip, reward_norm)
+        if reward_score is None:
+            reward_score = (data["rewards"] + reward_bias) * reward_scaling      # actor.py:166-170
+            reward_score = torch.clip(reward_score, max=reward_clip, min=-reward_clip)
+            if reward_norm is not None:
+                reward_score = reward_norm(reward_score)
+        rows = one_pass(reward_score)
     if rows is not None:  # the whole of what follows in one pass per row
         loss_mask, old_logp, kl_rewards, rewards, advantages, returns = rows
         if not use_decoupled_loss and not recomputed:

@@ -1122,6 +1122,23 @@ typedef struct {
 int64_t aa_advantages_scratch_bytes(int64_t bs);
 int aa_advantages(const aa_advantage_step* step, void* stream);
 
+/*
+ * The same from the rewards themselves (step->reward_score is not read): the
+ * scores clip((rewards + bias) * scaling, -clip, clip), normalised when norm is
+ * given, are formed by the launch that uses them, with the bits that
+ * aa_reward_scores writes.  rewards [bs] must not overlap what the step writes.
+ * norm: levels none or group, groups of at most AA_SCORE_GROUP rows
+ * (AA_ERR_UNSUPPORTED otherwise: aa_reward_scores, then aa_advantages).
+ */
+#define AA_SCORE_GROUP 64
+typedef struct {
+  const float* rewards;
+  float bias, scaling, clip;
+  const aa_norm_params* norm; /* nullable */
+} aa_score_step;
+int aa_advantages_scored(const aa_advantage_step* step,
+                         const aa_score_step* scores, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -367,6 +367,46 @@ def test_advantage_rows_agree_with_the_separate_kernels(device, bs, L, variant):
             assert torch.equal(a, b), k
 
 
+@pytest.mark.parametrize("bs,group", [(1, 1), (7, 3), (12, 1), (32, 16), (130, 64), (64, 65), (5, 8)])
+@pytest.mark.parametrize("levels", [None, ("group", False, "group", False), ("group", True, "group", True), ("group", False, None, False),
+                                    (None, False, "group", True), (None, False, None, False)])
+@pytest.mark.parametrize("lengths", [False, True])
+def test_scores_formed_by_the_advantage_rows(device, bs, group, levels, lengths):
+    """The reward scores of the one-pass kernel against those of a launch of their own (``reward_scores``): the same sums in
+    the same order, so the same bits; rows past the last full group, groups up to a wave and one row more (which takes the
+    other way); lengths from an attention mask of bytes or as numbers."""
+    from areal_amd import engine_glue
+    from areal_amd.advantages import advantage_rows, reward_scores, score_step
+
+    g = torch.Generator().manual_seed(bs * 100 + group)
+    L = 37
+    attention = (torch.arange(L)[None] < torch.randint(1, L + 1, (bs, 1), generator=g)).to(device)
+    attention = attention.long() if lengths else attention
+    mask = (torch.rand(bs, L, generator=g) < 0.7).to(device)
+    logp = (-2.0 * torch.rand(bs, L, generator=g)).to(device)
+    rewards = (3.0 * torch.randn(bs, generator=g)).to(device)
+    norm = None
+    if levels is not None:
+        norm = Normalization(NormConfig(mean_level=levels[0], mean_leave1out=levels[1], std_level=levels[2],
+                                        std_unbiased=levels[3], group_size=group))
+    args = (rewards, -0.5, 2.0, 5.0, norm)
+    scores = score_step(*args)
+    grouped = levels is not None and "group" in levels
+    assert (scores is None) == (grouped and group > 64)
+
+    def rows(score, step=None):
+        return advantage_rows(mask, logp, True, None, attention, score, None, 0.1, "k1", 1.0, 0.95, False, None, step)
+
+    want = rows(reward_scores(*args))
+    data = dict(attention_mask=attention, loss_mask=mask, logprobs=logp, rewards=rewards)
+    out = engine_glue.compute_advantages(data, kl_ctl=0.1, gae_lambda=0.95, reward_bias=-0.5, reward_scaling=2.0,
+                                         reward_clip=5.0, reward_norm=norm)
+    assert torch.equal(out["tot_rewards"], want[3]) and torch.equal(out["advantages"], want[4])
+    if scores is not None:
+        for a, b in zip(rows(rewards, scores), want):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("bs,L,offset", [(5, 1021, 0), (5, 1022, 0), (3, 1025, 0), (5, 2045, 0), (5, 2047, 0), (4, 2048, 0),
                                          (3, 2051, 0), (3, 6143, 0), (1030, 5, 0), (2050, 1022, 0), (5, 61, 1), (3, 2049, 3),
                                          (3, 1024, 0), (3, 1028, 1), (3, 1277, 0), (3, 1278, 2), (3, 1533, 0), (3, 1534, 0),
