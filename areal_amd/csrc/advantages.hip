@@ -647,7 +647,7 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // 1024 x 300: 42.3 / 25.2 (maps composed in 32 bits: 24.7, 41.3, 26.2, 24.2, at two to seven times the error: 512 x 4096
 // against 64 bits, gamma lambda = 0.95: 1.7e-7 then and before, 6.8e-8 so).  A quarter to a half of it is the sums of a
 // normalisation: 64-bit arithmetic, and three trips past the caches at the end of the launch (sums out, counter, sums in).
-// The sums of a row are published past the caches for the last workgroup to fold: with a __threadfence() in every
+// Where the last workgroup folds the sums of the rows (not k_norm_rows) they are published past the caches: with a __threadfence() in every
 // workgroup (a write-back of its XCD's L2, full of the outputs' lines) 512 x 4096 took 4 us more.
 // ------------------------------------------------------------------------------------------------------------------
 
@@ -657,6 +657,12 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 struct RowSums {
   double F, S, A, B, C, c;
 };
+
+__device__ __forceinline__ double squares_about(const RowSums& q, double mean) {
+  const double d = mean - q.c;
+  if (isinf(q.C) && isfinite(d)) return q.C;  // (the terms below are infinities of both signs)
+  return q.C - 2.0 * d * q.B + d * d * q.A;
+}
 
 struct RowArgs {
   const void* mask_in;      // [bs, L] loss mask: one byte (mask_bytes) or one float per token
@@ -675,7 +681,7 @@ struct RowArgs {
   float* returns;
   RowSums* sums;            // nullable: no normalisation
   double4* stats;           // with sums: one per segment of the normalisation (see k_norm_partial)
-  StepWork* work;           // with sums
+  StepWork* work;           // with sums; null: k_norm_rows folds them, `stats` is not written
   int64_t bs, L;
   float kl_ctl, gamma, lam;
   int estimator, mask_no_eos_with_zero, mask_bytes, roll;
@@ -716,6 +722,79 @@ __device__ __forceinline__ void block_sums(double (&v)[N], double* smem) {
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) v[q] += smem[w * N + q];
   }
+}
+
+// The segment of a whole batch (no group levels, or no full group) from the sums of its rows, the same in every thread: a
+// thread's rows are fetched at once and stay in its registers.  smem [waves][2].  load(row): its sums.
+constexpr int kRowsHeld = 4;
+template <int THREADS>
+__host__ __device__ __forceinline__ bool folds_at_once(int64_t n_groups, int64_t bs) {
+  return n_groups == 0 && bs <= kRowsHeld * THREADS;
+}
+template <int THREADS, typename Load>
+__device__ __forceinline__ double4 fold_rows(bool centred, int64_t bs, double* smem, Load load) {
+  constexpr int kWaves = THREADS / kWave;
+  RowSums held[kRowsHeld];
+  double bf[2] = {0.0, 0.0}, z[1] = {0.0};
+#pragma unroll
+  for (int k = 0; k < kRowsHeld; ++k) {
+    const int64_t r = threadIdx.x + k * THREADS;
+    held[k] = r < bs ? load(r) : RowSums{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  }
+#pragma unroll
+  for (int k = 0; k < kRowsHeld; ++k) {
+    bf[0] += held[k].S;
+    bf[1] += held[k].F;
+  }
+  block_sums<2, kWaves>(bf, smem);
+  // a mean of the group is none here: with fewer rows than a group holds there is no full group, and rows outside the full
+  // groups are centred on zero (row_mean)
+  const double mean = centred && bf[1] != 0.0 ? bf[0] / bf[1] : 0.0;
+#pragma unroll
+  for (int k = 0; k < kRowsHeld; ++k)
+    if (threadIdx.x + k * THREADS < bs) z[0] += squares_about(held[k], mean);
+  block_sums<1, kWaves>(z, smem);
+  return make_double4(bf[0], bf[1], z[0] < 0.0 ? 0.0 : z[0], 0.0);
+}
+
+// k_norm_apply<true> straight from the sums of the rows: every workgroup folds them for itself while its first elements are on
+// their way, in the order in which the last workgroup of k_advantage_rows folds them elsewhere (the same bits).  That launch
+// then ends with a plain store of its sums, without three trips past the caches one after the other, and the elements go
+// in 16-byte pieces.  Bound by memory, behind the latency of the sums.  us a call, the last workgroup / so: 1 024 x 2 048
+// 44.3 / 38.0, 1 024 x 4 096 59.2 / 54.2, 512 x 8 192 51.9 / 48.2, 800 x 4 097 58.2 / 53.0; up to kFoldRows rows: the sums of
+// 2 000 rows, 96 KB to every workgroup, cost more than the tail (2 000 x 1 024 61.2 / 64.4, 2 048 x 1 000 62.1 / 65.3).
+constexpr int64_t kFoldRows = 1024;
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_norm_rows(NormArgs a, const RowSums* __restrict__ sums, int64_t bs, float* out) {
+  __shared__ double smem[THREADS / kWave * 2];
+  constexpr int kHeld = 2;  // pieces of four elements on their way per thread
+  const int64_t pieces = a.n / kOwn, step = (int64_t)gridDim.x * THREADS, first = (int64_t)blockIdx.x * THREADS + threadIdx.x;
+  f32x4_t x[kHeld], m[kHeld];
+  auto fetch = [&](int64_t p) {
+#pragma unroll
+    for (int h = 0; h < kHeld; ++h) {
+      const int64_t at = p + h * step < pieces ? p + h * step : p;
+      x[h] = *(const f32x4_t*)(a.x + kOwn * at);
+      m[h] = *(const f32x4_t*)(a.mask + kOwn * at);
+    }
+  };
+  if (first < pieces) fetch(first);
+  const double4 st = fold_rows<THREADS>(true, bs, smem, [&](int64_t r) { return sums[r]; });
+  if (st.y == 0.0) return;  // nothing counts: the elements stay as they are
+  const double mean = st.x / st.y;
+  const double inv = 1.0 / (level_std(st.z, st.y, a.std_unbiased != 0) + (double)a.eps);
+  auto one = [&](float xi, float mi) { return (float)(((double)xi - mean) * (double)mi * inv); };
+  for (int64_t p = first; p < pieces; p += kHeld * step) {
+    if (p != first) fetch(p);
+#pragma unroll
+    for (int h = 0; h < kHeld; ++h) {
+      f32x4_t o;
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q) o[q] = one(x[h][q], m[h][q]);
+      if (p + h * step < pieces) *(f32x4_t*)(out + kOwn * (p + h * step)) = o;
+    }
+  }
+  for (int64_t i = kOwn * pieces + first; i < a.n; i += step) out[i] = one(a.x[i], a.mask[i]);  // up to three at the end
 }
 
 template <int THREADS>
@@ -901,6 +980,10 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   {
     double v[5] = {F, S, A, B, C};
     block_sums<5, kWaves>(v, smem);
+    if (!a.work) {  // the kernel that normalises folds the rows itself
+      if (tid == 0) a.sums[row] = RowSums{v[0], v[1], v[2], v[3], v[4], c};
+      return;
+    }
     if (tid == 0) {
       RowSums* o = a.sums + row;
       publish(&o->F, v[0]);
@@ -916,41 +999,14 @@ __global__ __launch_bounds__(THREADS, 4) void k_advantage_rows(RowArgs a) {
   if (!last) return;
   // The last workgroup: the segments of the normalisation from the sums of their rows.
   const NormArgs& n = a.norm;
-  auto squares_about = [&](const RowSums& q, double mean) {
-    const double d = mean - q.c;
-    if (isinf(q.C) && isfinite(d)) return q.C;  // (the terms below are infinities of both signs)
-    return q.C - 2.0 * d * q.B + d * d * q.A;
-  };
-  constexpr int kRowsHeld = 4;
-  if (n.n_groups == 0 && a.bs <= kRowsHeld * THREADS) {
-    // The whole batch is one segment (no group levels, or no full group): a thread's rows are fetched at once and stay in its
-    // registers (the loads go past the caches: one after the other they were half of this tail)
-    RowSums held[kRowsHeld];
-    double bf[2] = {0.0, 0.0}, z[1] = {0.0};
-#pragma unroll
-    for (int k = 0; k < kRowsHeld; ++k) {
-      const int64_t r = tid + k * THREADS;
-      held[k] = RowSums{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-      if (r < a.bs) {
-        const RowSums* q = a.sums + r;
-        held[k] = RowSums{published(&q->F), published(&q->S), published(&q->A), published(&q->B), published(&q->C), published(&q->c)};
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kRowsHeld; ++k) {
-      bf[0] += held[k].S;
-      bf[1] += held[k].F;
-    }
-    block_sums<2, kWaves>(bf, smem);
-    // a mean of the group is none here: with fewer rows than a group holds there is no full group, and rows outside the full
-    // groups are centred on zero (row_mean)
-    const double mean = n.mean_level == 1 && bf[1] != 0.0 ? bf[0] / bf[1] : 0.0;
-#pragma unroll
-    for (int k = 0; k < kRowsHeld; ++k)
-      if (tid + k * THREADS < a.bs) z[0] += squares_about(held[k], mean);
-    block_sums<1, kWaves>(z, smem);
+  if (folds_at_once<THREADS>(n.n_groups, a.bs)) {
+    // (the loads go past the caches: one after the other they were half of this tail)
+    const double4 st = fold_rows<THREADS>(n.mean_level == 1, a.bs, smem, [&](int64_t r) {
+      const RowSums* q = a.sums + r;
+      return RowSums{published(&q->F), published(&q->S), published(&q->A), published(&q->B), published(&q->C), published(&q->c)};
+    });
     if (tid == 0) {
-      a.stats[0] = make_double4(bf[0], bf[1], z[0] < 0.0 ? 0.0 : z[0], 0.0);
+      a.stats[0] = st;
       a.work->finished = 0;
     }
     return;
@@ -1281,9 +1337,19 @@ static int advantages(const aa_advantage_step* step, const aa_score_step* scores
   with_row_plan(p.bs, p.L, a.sums != nullptr, [&](auto threads, int shift) {
     a.shift = shift;
     constexpr int kT = decltype(threads)::value;
+    const bool fold = p.norm && a.norm.mean_level == 1 && a.norm.std_level == 1 && folds_at_once<kT>(a.norm.n_groups, p.bs) &&
+                      p.bs <= kFoldRows;
+    if (fold) a.work = nullptr;
     hipLaunchKernelGGL(k_advantage_rows<kT>, dim3((unsigned)p.bs), dim3(kT), 0, st, a);
+    if (fold) {
+      constexpr int64_t kGroups = 512 * 512 / kT;  // what the chip holds at a time
+      const int64_t groups = (a.norm.n + 2 * kOwn * kT - 1) / (2 * kOwn * kT);
+      hipLaunchKernelGGL(k_norm_rows<kT>, dim3((unsigned)(groups < kGroups ? groups : kGroups)), dim3(kT), 0, st, a.norm,
+                         (const RowSums*)a.sums, p.bs, p.advantages);
+    } else if (p.norm) {
+      launch_norm_apply(a.norm, a.stats, p.advantages, st);
+    }
   });
-  if (p.norm) launch_norm_apply(a.norm, a.stats, p.advantages, st);
   return launch_status();
 }
 

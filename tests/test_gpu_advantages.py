@@ -465,6 +465,31 @@ def test_advantage_rows_at_the_edges_of_their_blocks(device, bs, L, offset, gamm
     assert float((normed["advantages"] - want).abs().max()) <= 4 * 2.0 ** -23 * max(float(want.abs().max()), 1.0)
 
 
+@pytest.mark.parametrize("bs,L", [(1, 1), (1, 3), (3, 2047), (257, 5), (513, 9), (700, 2051), (1024, 33), (1025, 33), (9, 4097)])
+@pytest.mark.parametrize("std_unbiased", [True, False])
+@pytest.mark.parametrize("masked", [0.0, 0.6, 1.0])
+def test_batch_normalisation_from_the_sums_of_the_rows(device, bs, L, std_unbiased, masked):
+    """Up to 1 024 rows the kernel that normalises folds their sums itself: sizes either side of a thread's rows, of a piece of
+    four elements and of that limit, with nothing and everything under the mask, against the separate two-pass normalisation of
+    the same advantages.  float64 sums in another order, then one rounding to float32: 4 ulps of the largest."""
+    from areal_amd import engine_glue
+
+    g = torch.Generator().manual_seed(bs * 101 + L)
+    mask = torch.rand(bs, L, generator=g) >= masked if masked < 1.0 else torch.zeros(bs, L, dtype=torch.bool)
+    data = dict(attention_mask=torch.ones(bs, L, dtype=torch.bool), loss_mask=mask, logprobs=-torch.rand(bs, L, generator=g),
+                values=torch.randn(bs, L, generator=g) + 2.0, rewards=torch.rand(bs, generator=g))
+    norm = Normalization(NormConfig(mean_level="batch", std_level="batch", std_unbiased=std_unbiased))
+
+    def run(adv_norm):
+        d = {k: v.clone().to(device) for k, v in data.items()}
+        return engine_glue.compute_advantages(d, adv_norm=adv_norm, discount=0.99, gae_lambda=0.95, use_decoupled_loss=True)
+
+    plain, got, again = run(None), run(norm)["advantages"], run(norm)["advantages"]
+    want = norm(plain["advantages"], plain["loss_mask"])
+    assert torch.equal(got, again)
+    assert float((got - want).abs().max()) <= 4 * 2.0 ** -23 * max(float(want.abs().max()), 1.0)
+
+
 @pytest.mark.parametrize("bs,L", [(1, 64), (3, 33), (3, 1025), (3, 4097)])
 @pytest.mark.parametrize("levels", [("group", "batch"), ("group", None), ("group", "group"), (None, "group"), ("batch", "group"),
                                     (None, "batch"), ("batch", "batch")])
