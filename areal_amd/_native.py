@@ -10,6 +10,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libareal_amd.so"
+HOST_PATH = LIB_PATH.with_name("_host.so")
 
 AA_OK = 0
 AA_ERR_INVALID_ARGUMENT = 1
@@ -288,6 +289,26 @@ def load() -> C.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+def host():
+    """The native host side of the steps (``csrc/host.cpp``), behind the library that it calls."""
+    if _host is None:
+        load()
+        _load_host()
+    return _host
+
+
+_host = None
+
+
+def _load_host() -> None:
+    global _host
+    try:
+        from . import _host as module
+    except ImportError as e:
+        raise NativeLibraryError(f"cannot load {HOST_PATH}: build it with `python -m areal_amd.build` ({e})") from e
+    _host = module
 
 
 def check(status: int, what: str) -> None:

@@ -42,9 +42,12 @@ class Normalization:
                 f"group_size must be a positive integer when using group normalization, got {self.group_size}"
             )
 
+    def _fields(self) -> tuple:
+        return (_LEVELS[self.mean_level], int(bool(self.mean_leave1out)), _LEVELS[self.std_level],
+                int(bool(self.std_unbiased)), float(self.eps), int(self.group_size))
+
     def _params(self) -> N.NormParams:
-        return N.NormParams(_LEVELS[self.mean_level], int(bool(self.mean_leave1out)), _LEVELS[self.std_level],
-                            int(bool(self.std_unbiased)), float(self.eps), int(self.group_size))
+        return N.NormParams(*self._fields())
 
     @torch.no_grad()
     def __call__(self, x: torch.Tensor, loss_mask: torch.Tensor | None = None, high_precision: bool = True,
@@ -124,12 +127,6 @@ def _plain(t: torch.Tensor | None, shape, dev) -> bool:
                          and not t.requires_grad and (not t.is_inference() or torch.is_inference_mode_enabled()))
 
 
-def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
-    """Whether two contiguous arrays share memory."""
-    pa, pb = a.data_ptr(), b.data_ptr()
-    return pa < pb + b.numel() * b.element_size() and pb < pa + a.numel() * a.element_size()
-
-
 def _scorable(rewards, bias, scaling, clip, norm) -> bool:
     if not all(isinstance(v, Real) for v in (bias, scaling, clip)):
         return False
@@ -139,20 +136,17 @@ def _scorable(rewards, bias, scaling, clip, norm) -> bool:
             and rewards.numel() != 0)
 
 
-def score_step(rewards: torch.Tensor, bias: float, scaling: float, clip: float, norm) -> N.ScoreStep | None:
+def score_step(rewards: torch.Tensor, bias: float, scaling: float, clip: float, norm) -> tuple | None:
     """``reward_scores`` for ``advantage_rows`` to form in its own launch; None when the rewards ask for one ahead of it (a
     level over the batch, groups of more rows than a wave) or for the general way."""
     if not _scorable(rewards, bias, scaling, clip, norm):
         return None
-    step = N.ScoreStep(_ptr(rewards), float(bias), float(scaling), float(clip))
-    if norm is not None:
-        params = norm._params()
-        if 1 in (params.mean_level, params.std_level):
+    fields = None if norm is None else norm._fields()
+    if fields is not None:
+        levels, group_size = (fields[0], fields[2]), fields[5]
+        if 1 in levels or (2 in levels and not 1 <= group_size <= N.SCORE_GROUP):
             return None
-        if 2 in (params.mean_level, params.std_level) and not 1 <= params.group_size <= N.SCORE_GROUP:
-            return None
-        step.norm = C.pointer(params)
-    return step
+    return float(bias), float(scaling), float(clip), fields
 
 
 @torch.no_grad()
@@ -180,61 +174,25 @@ def advantage_rows(loss_mask, logp, roll, ref_logp, attention_mask, score, value
     scores are formed on the way."""
     if loss_mask.ndim != 2 or not loss_mask.is_cuda or loss_mask.numel() == 0 or kl_estimator not in _KL_IDS:
         return None
-    shape, dev = loss_mask.shape, loss_mask.device
-    bs, L = shape
     if norm is not None and not (type(norm) is Normalization and _one_process()
                                  and not (norm.mean_leave1out and _LEVELS[norm.mean_level] != 0)):
         return None
-    if logp is None or not all(_plain(t, shape, dev) for t in (logp, ref_logp, values)):
-        return None
-    # what is masked in place is an array of its own: the kernel reads a neighbour's log-prob after that has been masked,
-    # and one array as both policies is masked twice
-    if ref_logp is not None and any(t is not None and _overlap(ref_logp, t) for t in (logp, values)):
-        return None
-    if not roll and values is not None and _overlap(logp, values):
-        return None
-    if scores is not None and any(t is not None and _overlap(score, t) for t in (ref_logp, None if roll else logp)):
-        return None  # a row reads the rewards of its group
-    if attention_mask.shape != shape or attention_mask.device != dev or score.shape != (bs,) or not _plain(score, (bs,), dev):
+    host = N.host()
+    if logp is None or not host.advantages_plain(loss_mask, logp, roll, ref_logp, attention_mask, score, values, scores is not None):
         return None
     if loss_mask.dtype is torch.bool:
-        mask, is_bytes = (loss_mask if loss_mask.is_contiguous() else loss_mask.contiguous()), 1
+        mask = loss_mask if loss_mask.is_contiguous() else loss_mask.contiguous()
     else:
-        mask, is_bytes = _f32(loss_mask), 0
+        mask = _f32(loss_mask)
     attention = seqlens = None
     if attention_mask.dtype is torch.bool and attention_mask.is_contiguous():
         attention = attention_mask
     else:
         seqlens = attention_mask.sum(-1).long()
-    lib = N.load()
-    new = lambda: torch.empty(shape, dtype=torch.float32, device=dev)
-    mask_out, kl_rewards, rewards, adv, returns = new(), new(), new(), new(), new()
-    logp_out = new() if roll else logp
-    a = N.AdvantageStep()
-    a.bs, a.L = bs, L
-    a.loss_mask, a.loss_mask_bytes, a.roll_logp = _ptr(mask), is_bytes, int(roll)
-    a.logp, a.ref_logp, a.values = _ptr(logp), _ptr(ref_logp), _ptr(values)
-    if scores is None:
-        a.reward_score = _ptr(score)
-    a.attention_mask, a.seqlens = _ptr(attention), _ptr(seqlens)
-    a.kl_ctl, a.discount, a.gae_lambda = float(kl_ctl), float(discount), float(gae_lambda)
-    a.kl_estimator, a.mask_no_eos_with_zero = _KL_IDS[kl_estimator], int(bool(mask_no_eos_with_zero))
-    a.mask_out, a.logp_out, a.kl_rewards, a.rewards = _ptr(mask_out), _ptr(logp_out), _ptr(kl_rewards), _ptr(rewards)
-    a.advantages, a.returns = _ptr(adv), _ptr(returns)
-    if norm is not None:
-        params = norm._params()
-        scratch = torch.empty(lib.aa_advantages_scratch_bytes(bs) // 8, dtype=torch.float64, device=dev)
-        a.norm = C.pointer(params)
-        a.scratch, a.scratch_bytes, a.work = _ptr(scratch), scratch.numel() * 8, _ptr(_work_words(dev))
-    with _on(dev):
-        if scores is None:
-            N.check(lib.aa_advantages(a, _stream(dev)), "aa_advantages")
-        else:
-            N.check(lib.aa_advantages_scored(a, scores, _stream(dev)), "aa_advantages_scored")
-    for t in (ref_logp, None if roll else logp):  # written through a raw pointer: autograd is told
-        if t is not None:
-            torch.autograd.graph.increment_version(t)
-    return mask_out, logp_out, kl_rewards, rewards, adv, returns
+    return host.advantages(mask, logp, roll, ref_logp, attention, seqlens, score, values, float(kl_ctl), _KL_IDS[kl_estimator],
+                           float(discount), float(gae_lambda), bool(mask_no_eos_with_zero),
+                           None if norm is None else norm._fields(), scores,
+                           None if norm is None else _work_words(loss_mask.device))
 
 
 _MOMENT_KEYS = ("sum", "min", "max", "count", "avg")

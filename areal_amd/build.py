@@ -72,6 +72,31 @@ def build_library(verbose: bool = True, jobs: int = 4) -> Path:
     return LIB_PATH
 
 
+def build_host(verbose: bool = True) -> Path:
+    """Compile ``csrc/host.cpp`` (host code, against torch's C++ headers) into ``areal_amd/_host.so``, next to the library that
+    it is linked to."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    out = PKG_DIR / "_host.so"
+    tmp = out.with_suffix(".so.tmp")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    if verbose:
+        print("[areal_amd.build] g++ host.cpp", flush=True)
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f"-I{root}/include",
+          f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}", f"-I{rocm}/include",
+          f"-I{PKG_DIR.parent}/include", str(CSRC / "host.cpp"), "-o", str(tmp), f"-L{root}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu",
+          "-ltorch", "-ltorch_python", f"-L{PKG_DIR}", "-lareal_amd", "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, out)
+    if verbose:
+        print(f"[areal_amd.build] wrote {out}", flush=True)
+    return out
+
+
 if __name__ == "__main__":
     build_library()
+    build_host()
     sys.exit(0)

@@ -107,15 +107,8 @@ def _rows(logits: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
 
 
 def _empty_rows_like(logits2d: torch.Tensor, stride: int) -> torch.Tensor:
-    """An uninitialised [T, V] array for the gradient of ``logits2d``: the same row stride, and the same place inside
-    a 16-byte piece of memory, so that the kernels walk both arrays alike (the fused kernel's fast path for rows that
-    do not start on 16-byte boundaries asks for that)."""
-    T, V = logits2d.shape
-    lead = (logits2d.data_ptr() % 16) // logits2d.element_size()
-    if stride == V and lead == 0:
-        return torch.empty_like(logits2d, memory_format=torch.contiguous_format)
-    flat = torch.empty(lead + (T - 1) * stride + V, dtype=logits2d.dtype, device=logits2d.device)
-    return flat.as_strided((T, V), (stride, 1), lead)
+    """An uninitialised [T, V] array for the gradient of ``logits2d``, laid out like it (``csrc/host.cpp``)."""
+    return N.host().empty_rows_like(logits2d, stride)
 
 
 def _check_tp(tp_group: Any) -> None:
@@ -575,44 +568,20 @@ class _Step:
     The outputs are rows of two arrays (float32 and bytes), so that a step allocates three times and not sixteen; an entry
     of the stat dict that is kept keeps all of them (45 bytes a token, a clone its own four)."""
 
-    # floats: logp, entropy, vmax, vmin, stat_loss, ratio, approx_kl, behave_kl, behave_w, (counts)
-    # bools: (flags), mask_out, clip_mask, dual_clip_mask, behave_mask
     __slots__ = ("T", "T_active", "device", "floats", "bools", "loss", "mask", "slot", "struct", "rs", "_keep")
 
     def __init__(self, dev, T, T_active, mask, prox, old, adv, params, rs=None, cu=None, n_segments=0, scale=None,
                  derived=True, host_counts=False, behave_w=None, counts=None):
         self.T, self.T_active, self.device, self.rs, self.mask = T, T_active, dev, rs, mask
-        pitch = max(64, (T + 63) & ~63)
-        f = self.floats = torch.empty(10, pitch, dtype=torch.float32, device=dev)
-        b = self.bools = torch.empty(5, pitch, dtype=torch.bool, device=dev)
-        self.loss = torch.empty((), dtype=torch.float32, device=dev)
         work = _work_words(dev)
         scale_c, scale_t = _scale_struct(scale, dev)
         self.slot = _HostSlot(dev) if (rs is not None or host_counts or isinstance(scale, _PerValidToken)) else None
-        f0, b0, row = f.data_ptr(), b.data_ptr(), pitch * 4
         c = self.struct = N.PpoStep()
-        c.T, c.T_active = T, T_active
-        c.prox_logp, c.old_logp, c.adv, c.mask = _ptr(prox), _ptr(old), _ptr(adv), _ptr(mask)
-        c.cu_seqlens, c.n_segments = _ptr(cu), n_segments
         c.params, c.rs, c.scale = params, _rs_struct(rs), scale_c
-        c.logp, c.entropy, c.vmax, c.vmin = f0, f0 + row, f0 + 2 * row, f0 + 3 * row
-        c.stat_loss, c.ratio, c.flags = f0 + 4 * row, f0 + 5 * row, b0
-        if derived:
-            c.approx_kl, c.clip_mask, c.dual_clip_mask = f0 + 6 * row, b0 + 2 * pitch, b0 + 3 * pitch
-            if rs is not None:
-                c.behave_mask, c.behave_kl = b0 + 4 * pitch, f0 + 7 * row
-        if rs is not None:
-            c.mask_out, c.behave_w = b0 + pitch, f0 + 8 * row
-        elif behave_w is not None:
-            c.behave_w = behave_w.data_ptr()
-        if counts is not None:
-            c.counts, c.counts_given = counts.data_ptr(), 1
-        else:
-            c.counts = f0 + 9 * row
-        c.loss = self.loss.data_ptr()
         if self.slot is not None:
             c.host_counts, c.host_tag = self.slot.address, self.slot.tag
-        c.work = work.data_ptr()
+        self.floats, self.bools, self.loss = N.host().make_step(
+            C.addressof(c), T, T_active, mask, prox, old, adv, cu, n_segments, derived, rs is not None, behave_w, counts, work, dev)
         self._keep = (prox, old, adv, mask, cu, scale_t, behave_w, counts, work)
 
     @property
@@ -622,21 +591,13 @@ class _Step:
 
     def rows(self) -> list:
         """logp, entropy, vmax, vmin, stat_loss, ratio: ``[T_active]`` each."""
-        return list(self.floats[:6, : self.T_active].unbind(0))
+        return N.host().step_rows(self.floats, self.T_active)
 
     def stats(self, rows: bool, shape=None) -> dict:
         """The stat dict of ``ppo_actor_loss_fn`` (functional.py:505-558); ``rows``: with the per-row outputs as well."""
-        n = self.T_active
-        f = self.floats[:, :n].unbind(0)
-        b = self.bools[:, :n].unbind(0)
+        stat = N.host().step_stats(self.floats, self.bools, self.T_active, rows, self.rs is not None)
         if shape is not None and len(shape) != 1:
-            f = [v.view(shape) for v in f]
-            b = [v.view(shape) for v in b]
-        stat = dict(loss=f[4], importance_weight=f[5], approx_kl=f[6], clip_mask=b[2], dual_clip_mask=b[3])
-        if rows:
-            stat.update(logprobs=f[0], entropy=f[1], vocab_min_logits=f[3], vocab_max_logits=f[2])
-        if self.rs is not None:
-            stat.update(behave_approx_kl=f[7], behave_imp_weight=f[8], behave_mask=b[4])
+            stat = {k: v.view(shape) for k, v in stat.items()}
         return stat
 
     def finish(self, stat: dict) -> dict:
@@ -768,48 +729,9 @@ def _hand_out_once(ctx) -> None:
     ctx.handed_out = True
 
 
-class _FusedLogitsPpo(torch.autograd.Function):
-    """The step on logits; its per-token outputs are in ``step``."""
-
-    @staticmethod
-    def forward(ctx, logits2d, step, labels1d, stride, temperature, inplace):
-        dev = step.device
-        T, V = logits2d.shape
-        if inplace:
-            # the gradient takes the place of the logits: every kernel reads an element for the last time before it
-            # writes it, so the two arrays of the C entry point may be one
-            dlogits = logits2d.detach()
-        else:
-            dlogits = _empty_rows_like(logits2d, stride)
-        with _on(dev):
-            N.check(
-                N.load().aa_logits_ppo_step(step.struct, _ptr(logits2d), _DTYPES[logits2d.dtype], V, stride, _ptr(labels1d),
-                                            1.0 / temperature, _ptr(dlogits), _stream(dev)),
-                "aa_logits_ppo_step",
-            )
-        if inplace:
-            # written through a raw pointer: tell autograd, so that an operation that saved the logits for its own
-            # backward fails loudly instead of reading gradients
-            torch.autograd.graph.increment_version(logits2d)
-        ctx.save_for_backward(dlogits)
-        return step.loss
-
-    @staticmethod
-    def backward(ctx, g_loss):
-        _hand_out_once(ctx)
-        (dlogits,) = ctx.saved_tensors
-        dev = dlogits.device
-        g = _f32_values(g_loss)
-        # d(logits) was written with the loss; an upstream factor other than 1 is
-        # applied in place (the kernel returns at once when the factor is 1).
-        T, V = dlogits.shape
-        with _on(dev):
-            N.check(
-                N.load().aa_scale_rows_inplace(_ptr(dlogits), _DTYPES[dlogits.dtype], T, V,
-                                               dlogits.stride(0) if T > 1 else V, _ptr(g), _stream(dev)),
-                "aa_scale_rows_inplace",
-            )
-        return dlogits, None, None, None, None, None
+def _fused_logits(logits2d, step, labels1d, stride, temperature, inplace):
+    """The loss of the step on logits, differentiable in them; its per-token outputs are in ``step``."""
+    return N.host().fused_logits(logits2d, C.addressof(step.struct), step.loss, labels1d, stride, temperature, inplace)
 
 
 def _scaled(loss, scale, loss_mask):
@@ -917,7 +839,7 @@ def fused_logprobs_ppo_loss(
     x, T, V, stride = _rows(logits)
     step = _ppo_step(dev, T, T_active, loss_mask, proximal_logprobs, old_logprobs, advantages, eps_clip, eps_clip_higher,
                      c_clip, rejection_sampling, cu_seqlens, loss_scale)
-    loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
+    loss = _fused_logits(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
     stat = step.finish(step.stats(rows=True))
     _note_valid_tokens(loss_scale, step)
     return loss, stat

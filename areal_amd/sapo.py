@@ -11,7 +11,7 @@ import torch
 from . import _native as N
 from .functional import (
     _FusedLmHeadPpo,
-    _FusedLogitsPpo,
+    _fused_logits,
     _Step,
     _f32_values,
     _labels_i64,
@@ -84,7 +84,7 @@ def fused_logprobs_sapo_loss(logits: torch.Tensor, labels: torch.Tensor, old_log
     x, T, V, stride = _rows(logits)
     old, adv = _f32_values(old_logprobs), _f32_values(advantages)
     step = _Step(dev, T, T_active, _mask_bytes(loss_mask.to(dev)), old, None, adv, params, scale=loss_scale, derived=False)
-    loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
+    loss = _fused_logits(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
     return loss, _step_stat(step, old, adv, tau_pos, tau_neg)
 
 

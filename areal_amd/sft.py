@@ -11,7 +11,7 @@ from . import _native as N
 from .functional import (
     _DTYPES,
     _FusedLmHeadPpo,
-    _FusedLogitsPpo,
+    _fused_logits,
     _Step,
     _count_nonzero,
     _f32,
@@ -168,7 +168,7 @@ def fused_logprobs_sft_loss(logits: torch.Tensor, labels: torch.Tensor, loss_mas
         return loss, stat
     x, T, V, stride = _rows(logits)
     step = _nll_step(dev, T, T_active, loss_mask, loss_scale)
-    loss = _FusedLogitsPpo.apply(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
+    loss = _fused_logits(x, step, _labels_i64(labels, dev), stride, float(temperature), bool(inplace_backward))
     stat = _step_stat(step, cu, n_seqs, extrema=True)
     _note_valid_tokens(loss_scale, step)
     return loss, stat

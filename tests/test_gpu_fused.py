@@ -1065,3 +1065,55 @@ def test_a_loss_times_the_weight_the_host_has_read(device, total, multiplier):
             assert torch.equal(x.grad, y.grad)
         one = torch.tensor([n], device=device)  # a weight of shape [1] keeps its shape
         assert engine_glue._times_weight(torch.ones((), device=device), one, engine_glue._weight_is_zero(one)[2], 2.0, 1.0).shape == (1,)
+
+
+@pytest.mark.parametrize("T,pad", [(1, 0), (63, 1), (65, 0)])
+def test_node_of_the_fused_step(device, T, pad):
+    """The autograd node of the fused step: its saved gradient goes through the hooks for saved tensors, forward and backward
+    run on the stream that is current (with an upstream factor other than one), what it does not support raises, and so does
+    a description that the library refuses.  The same bits in every way."""
+    from areal_amd import _native as N
+    from areal_amd import functional as F
+
+    g = torch.Generator().manual_seed(T)
+    V = 4099
+    x = torch.randn(T + pad, V, generator=g).to(device, torch.bfloat16).requires_grad_()
+    y = torch.randint(0, V, (T + pad,), generator=g).to(device)
+    lp = areal_amd.gather_logprobs(x.detach(), y)[:T]
+    adv = torch.randn(T, generator=g).to(device)
+    mask = torch.ones(T, dtype=torch.bool, device=device)
+
+    def step():
+        return areal_amd.fused_logprobs_ppo_loss(x, y, lp, lp, adv, 0.2, mask, loss_scale=0.5)
+
+    loss, stat = step()
+    (want,) = torch.autograd.grad(loss * 3.0, x)
+    assert float(want[:T].float().abs().max()) > 0 and not bool(want[T:].any())
+    for k, v in stat.items():
+        assert v.shape == (T,) and v.stride() == (1,), k
+    packed = []
+
+    def pack(t):
+        packed.append(t.shape)
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(device)):
+        loss, _ = step()
+    (got,) = torch.autograd.grad(loss * 3.0, x)
+    assert x.shape in packed and torch.equal(got, want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        loss, _ = step()
+        (got,) = torch.autograd.grad(loss * 3.0, x)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(got, want)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda a: areal_amd.fused_logprobs_ppo_loss(a, y, lp, lp, adv, 0.2, mask)[0])(x.detach()[None].requires_grad_())
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        areal_amd.fused_logprobs_ppo_loss(dual, y, lp, lp, adv, 0.2, mask)
+    s = F._ppo_step(torch.device(device), T + pad, T, mask, lp, lp, adv, 0.2, None, None, None, None, None)
+    s.struct.T_active = T + pad + 1
+    with pytest.raises(N.NativeLibraryError, match="aa_logits_ppo_step failed"):
+        F._fused_logits(x, s, y, V, 1.0, False)

@@ -139,6 +139,42 @@ def test_gradient_array_is_laid_out_like_the_logits(V, stride, lead):
     assert float(out.float().sum()) == T * V
 
 
+def test_arrays_that_the_advantage_rows_take_as_they_are():
+    """The native check against the rule in words: float32, contiguous, of the shape and on the device of the mask, without a
+    gradient, not made in inference mode; what is masked in place shares no memory with another input."""
+    from areal_amd import _native as N
+
+    bs, L = 4, 6
+    flat = torch.zeros(4 * bs * L)
+    good = lambda i=0: flat[i * bs * L : (i + 1) * bs * L].view(bs, L)
+    with torch.inference_mode():
+        inferred = torch.zeros(bs, L)
+    mask, score = torch.ones(bs, L, dtype=torch.bool), torch.zeros(bs)
+
+    def takes(logp=good(0), roll=True, ref=good(1), attention=mask, score=score, values=good(2), scored=False):
+        return N.host().advantages_plain(mask, logp, roll, ref, attention, score, values, scored)
+
+    assert takes() and takes(ref=None, values=None) and takes(roll=False) and takes(scored=True)
+    others = [good().double(), good().half(), torch.zeros(L, bs).t(), torch.zeros(bs, 2 * L)[:, ::2], torch.zeros(bs, L + 1)[:, :L],
+              torch.zeros(bs + 1, L), torch.zeros(bs * L), torch.zeros(bs, L, requires_grad=True), inferred,
+              torch.zeros(bs, L, device="meta")]
+    for x in others:
+        assert not takes(logp=x) and not takes(ref=x) and not takes(values=x)
+    with torch.inference_mode():
+        assert takes(logp=inferred) and takes(ref=inferred)
+    for x in (torch.zeros(bs + 1), torch.zeros(bs, 1), torch.zeros(2 * bs)[::2], torch.zeros(bs).double()):
+        assert not takes(score=x)
+    assert not takes(attention=mask[:, 1:]) and takes(attention=mask.long())
+    shifted = flat[bs * L - 1 : 2 * bs * L - 1].view(bs, L)  # its first element is the last one of good(0)
+    for x in (good(0), shifted):
+        assert not takes(ref=x) and not takes(values=x, roll=False) and takes(values=x, ref=None)
+    assert not takes(ref=good(1), values=good(1))
+    inside = flat[bs * L : bs * L + bs]
+    assert takes(score=inside) and not takes(score=inside, scored=True)
+    inside = flat[:bs]
+    assert takes(score=inside, scored=True) and not takes(score=inside, scored=True, roll=False)
+
+
 def test_moments_of_a_mask_in_host_memory_are_refused(monkeypatch):
     """Every mask is asked for its device before its address goes to a kernel: the supervised loss function takes a mask
     from anywhere, and its statistics used to refuse one in host memory."""
