@@ -58,8 +58,9 @@ __device__ __forceinline__ Affine compose(const Affine& first, const Affine& sec
 
 // ---- lanes of a wave without LDS ---------------------------------------------------------------------------------
 // DPP controls: row_shr:n moves a value n lanes up inside its row of 16, row_bcast15 / 31 hand the last lane of a row / of
-// the lower half on to the rows named by the mask.  Lanes that are sent nothing get `old`.
-constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+// the lower half on to the rows named by the mask, wave_shr:1 moves a value one lane up in the whole wave.  Lanes that are sent
+// nothing get `old`.
+constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143, kWaveShr1 = 0x138;
 template <int CTRL, int ROWS>
 __device__ __forceinline__ float dpp(float old, float x) {
   return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp((int)__float_as_uint(old), (int)__float_as_uint(x), CTRL, ROWS, 0xf, false));
@@ -93,34 +94,56 @@ __device__ __forceinline__ Affine scan_step(const Affine& x) {
   p.f = dpp<CTRL, ROWS>(0.0, x.f);
   return compose(p, x);
 }
-__device__ __forceinline__ Affine scan_row(Affine x) {  // over each row of 16 lanes
+// over each row of 16 lanes, of which the first LANES hold maps
+template <int LANES = 16>
+__device__ __forceinline__ Affine scan_row(Affine x) {
   x = scan_step<kRowShr + 1, 0xf>(x);
-  x = scan_step<kRowShr + 2, 0xf>(x);
-  x = scan_step<kRowShr + 4, 0xf>(x);
-  return scan_step<kRowShr + 8, 0xf>(x);
+  if constexpr (LANES > 2) x = scan_step<kRowShr + 2, 0xf>(x);
+  if constexpr (LANES > 4) x = scan_step<kRowShr + 4, 0xf>(x);
+  if constexpr (LANES > 8) x = scan_step<kRowShr + 8, 0xf>(x);
+  return x;
 }
-__device__ __forceinline__ Affine shfl(const Affine& x, int from) {
-  return {__shfl(x.a, from, kWave), __shfl(x.e, from, kWave), __shfl(x.c, from, kWave), __shfl(x.d, from, kWave),
-          __shfl(x.f, from, kWave)};
+__device__ __forceinline__ void apply(const Affine& m, float& nv, double& lg) {
+  lg = fma(m.c, (double)nv, fma(m.d, lg, m.f));
+  nv = fmaf(m.a, nv, m.e);
+}
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), lane));
+}
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  uint2 b = __builtin_bit_cast(uint2, x);
+  b.x = (uint32_t)__builtin_amdgcn_readlane((int)b.x, lane);
+  b.y = (uint32_t)__builtin_amdgcn_readlane((int)b.y, lane);
+  return __builtin_bit_cast(double, b);
 }
 
 // The state (nv, lg) that enters a thread's positions: (nv0, lg0) through the maps of the threads before it.  One barrier;
-// `wave_tot` (LDS, one per wave) may be written again behind another one.
+// `wave_tot` (LDS, one per wave) may be written again behind another one.  Behind the scan of the wave it is states that are
+// handed on, not maps: three numbers instead of five, and nothing to compose.  us a call, maps shuffled through LDS and composed / so:
+// 512 x 4 096 32.5 / 31.0, 1 024 x 4 096 54.1 / 50.5, 2 048 x 2 048 77.2 / 71.3, 1 500 x 4 097 105.4 / 93.2.
 template <int WAVES>
 __device__ __forceinline__ void enter(const Affine& mine, Affine* wave_tot, float nv0, float lg0, float& nv, float& lg) {
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   Affine inc = scan_row(mine);
   inc = scan_step<kRowBcast15, 0xa>(inc);
   inc = scan_step<kRowBcast31, 0xc>(inc);
   if (lane == kWave - 1) wave_tot[wave] = inc;
   __syncthreads();
-  // the maps of the waves before this one: every wave scans the totals in its first lanes
-  const Affine tot = scan_row(lane < WAVES ? wave_tot[lane] : identity());
-  Affine before = wave > 0 ? shfl(tot, wave - 1) : identity();
-  const Affine up = shfl(inc, lane > 0 ? lane - 1 : 0);
-  before = compose(before, lane > 0 ? up : identity());
-  nv = fmaf(before.a, nv0, before.e);
-  lg = (float)fma(before.c, (double)nv0, fma(before.d, (double)lg0, before.f));
+  // the state that enters this wave: every wave scans the totals in its first lanes
+  const Affine tot = scan_row<WAVES>(lane < WAVES ? wave_tot[lane] : identity());
+  float nv_in = nv0;
+  double lg_in = (double)lg0;
+  if (wave > 0) {
+    apply(tot, nv_in, lg_in);
+    nv_in = lane_value(nv_in, wave - 1);
+    lg_in = lane_value(lg_in, wave - 1);
+  }
+  // through the lanes below
+  const Affine up = {dpp<kWaveShr1, 0xf>(1.f, inc.a), dpp<kWaveShr1, 0xf>(0.f, inc.e), dpp<kWaveShr1, 0xf>(0.0, inc.c),
+                     dpp<kWaveShr1, 0xf>(1.0, inc.d), dpp<kWaveShr1, 0xf>(0.0, inc.f)};
+  apply(up, nv_in, lg_in);
+  nv = nv_in;
+  lg = (float)lg_in;
 }
 
 // 16 bytes of an array that starts anywhere (on its own elements), four of a byte array
