@@ -84,6 +84,38 @@ __device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int& 
   tile_at(xcd_contiguous(pid, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn, group_m);
 }
 
+// A grid whose last round of tiles would fill at most half of the compute units runs that round as half tiles, two workgroups
+// to a tile: it is over in little more than half the time.  XCD by XCD, since a workgroup stays on the XCD that its id names; a
+// workgroup without a tile returns.  half: 0 or 1, or -1 for a whole tile.  units: compute units of the device; 0: whole tiles
+// throughout.  us, whole tiles / so: TODO
+__host__ __device__ __forceinline__ int whole_tiles(int count, int units) {  // of the `count` tiles of an XCD
+  const int per = units >> 3, rest = per > 0 ? count % per : 0;
+  return 2 * rest <= per ? count - rest : count;
+}
+__device__ __forceinline__ bool tile_or_half_of(int pid, int tiles_m, int tiles_n, int units, int& tm, int& tn, int& half) {
+  const int total = tiles_m * tiles_n;
+  const int x = pid & 7, i = pid >> 3, rem = total & 7;
+  const int count = (total >> 3) + (x < rem ? 1 : 0), whole = whole_tiles(count, units);
+  int q = i;
+  half = -1;
+  if (i >= whole) {
+    q = whole + ((i - whole) >> 1);
+    half = (i - whole) & 1;
+  }
+  if (q >= count) return false;
+  tile_at(x * (total >> 3) + (x < rem ? x : rem) + q, tiles_m, tiles_n, tm, tn);
+  return true;
+}
+// workgroups of such a grid
+inline int64_t grid_with_halves(int64_t tiles, int units) {
+  int most = 0;
+  for (int64_t count = tiles >> 3; count <= (tiles + 7) >> 3; ++count) {
+    const int n = 2 * (int)count - whole_tiles((int)count, units);
+    most = n > most ? n : most;
+  }
+  return 8 * (int64_t)most;
+}
+
 // One operand.  K-contiguous: element (x, k) at ptr[x * ld + k], `rows` = number of valid x.  K-major: element (x, k)
 // at ptr[k * ld + x], `rows` = number of valid x (the columns of the array).  ld and rows are multiples of 8 (16-byte
 // pieces never straddle an edge); 256 array rows must stay below 2^30 elements (32-bit byte offsets inside a tile).

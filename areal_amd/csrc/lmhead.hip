@@ -783,7 +783,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_store(Operand A, Operand B, i
                                                          OutT* __restrict__ C, int64_t ldc,
                                                          const int32_t* __restrict__ c_rows,
                                                          const float* __restrict__ n_scale,
-                                                         const int32_t* __restrict__ bounds) {
+                                                         const int32_t* __restrict__ bounds, int units) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   if constexpr (BOUND == kBoundN) {
     const int live = bounds[kRowsLive];
@@ -791,9 +791,14 @@ __global__ __launch_bounds__(kThreads) void k_gemm_store(Operand A, Operand B, i
     // the same decision in every thread of the workgroup
     if (bounds[kRowsSplits] != 1 || (int)blockIdx.x >= tiles_m * tiles_n) return;
   }
-  int tm, tn;
-  tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  int tm, tn, half = -1;
+  if constexpr (BKM) {  // d_weight: half tiles are halves along m
+    if (!tile_or_half_of(blockIdx.x, tiles_m, tiles_n, units, tm, tn, half)) return;
+  } else {
+    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  }
+  const int m0 = tm * BM + (half == 1 ? BM / 2 : 0), n0 = tn * BN;
+  if (half == 1 && m0 >= A.rows) return;
   if constexpr (BOUND == kBoundK) {
     const int kb = bounds[kRowsSliced];
     K = kb < K ? kb : K;
@@ -801,7 +806,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_store(Operand A, Operand B, i
   // A last row or column of tiles with at most 128 in use is one of narrow tiles, as in the forward.  Both gradients
   // together with a hidden size that ends in such a row of tiles, whole steps, us wide / narrow: 2 000 x 600 x 64 000:
   // 583 / 536, 700 x 3 584 x 100 000 (490 rows with a gradient): 1 390 / 1 311, 1 000 x 2 696 x 90 000: 1 377 / 1 335.
-  const bool narrow_m = A.rows - m0 <= BM / 2;
+  const bool narrow_m = half >= 0 || A.rows - m0 <= BM / 2;
   int columns = B.rows;
   if constexpr (BOUND == kBoundN) columns = bounds[kRowsTotal] < columns ? bounds[kRowsTotal] : columns;
   if constexpr (!BKM) {  // a K-major B is the panel as d_weight reads it: its columns are the vocabulary
@@ -1222,8 +1227,10 @@ static void launch_gemm(hipStream_t st, const uint16_t* A, int64_t lda, int64_t 
                         const float* n_scale = nullptr, const int32_t* bounds = nullptr) {
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
   Operand a{A, lda, (int)M}, b{B, ldb, (int)N};
-  hipLaunchKernelGGL((k_gemm_store<AKM, BKM, OutT, ACCUM, BOUND>), dim3((unsigned)(tiles_m * tiles_n)), dim3(kThreads),
-                     kLdsBytes, st, a, b, (int)K, tiles_m, tiles_n, C, ldc, c_rows, n_scale, bounds);
+  const int units = BKM ? compute_units() : 0;
+  const int64_t grid = BKM ? grid_with_halves(tiles_m * tiles_n, units) : tiles_m * tiles_n;
+  hipLaunchKernelGGL((k_gemm_store<AKM, BKM, OutT, ACCUM, BOUND>), dim3((unsigned)grid), dim3(kThreads), kLdsBytes, st, a, b,
+                     (int)K, tiles_m, tiles_n, C, ldc, c_rows, n_scale, bounds, units);
 }
 
 // d_weight (+)= ds^T . hidden rows in the dtype and mode asked for; with `bounds` the contraction stops at the rows in use

@@ -630,3 +630,30 @@ def test_sequence_level_step_reads_nothing_back(device):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
     assert cosine(a[2].float().cpu(), b[2].float().cpu()) > 0.9999999
     assert float(a[1].float().abs().sum()) > 0.0
+
+
+@pytest.mark.parametrize("V,H", [(256 * 128, 256), (256 * 136, 256), (256 * 264, 256), (256 * 259 + 8, 256), (256 * 129, 392),
+                                 (1000, 136), (9, 8)])
+def test_weight_gradient_with_a_last_round_of_half_tiles(device, V, H):
+    """A grid whose last round fills at most half of the chip runs it as half tiles: sizes either side of that (16 and 17 tiles
+    an XCD, 33, an uneven number), a last row of tiles that is narrow by itself, one tile.  Every element is written (the memory
+    held NaN), and the gradient is that of fp32 to the rounding of the bf16 rows that it is formed from."""
+    T = 40
+    g = torch.Generator().manual_seed(V + H)
+    h = torch.randn(T, H, generator=g).to(device, torch.bfloat16).requires_grad_()
+    w = (0.05 * torch.randn(V, H, generator=g)).to(device, torch.bfloat16).requires_grad_()
+    y = torch.randint(0, V, (T,), generator=g).to(device)
+    up = torch.randn(T, generator=g).to(device)
+    grads = []
+    for _ in range(2):
+        logp, _ = areal_amd.lm_head_logprobs_entropy(h, w, y)
+        nan = torch.full((V, H), float("nan"), dtype=torch.bfloat16, device=device)
+        del nan
+        grads.append(torch.autograd.grad((logp * up).sum(), [h, w]))
+    z = h.detach().float() @ w.detach().float().t()
+    d = -torch.softmax(z, 1)
+    d[torch.arange(T, device=device), y] += 1.0
+    want = (d * up[:, None]).t() @ h.detach().float()
+    got = grads[0][1].float()
+    assert torch.equal(grads[0][1], grads[1][1]) and bool(torch.isfinite(got).all())
+    assert float((got - want).norm()) <= 2.0 ** -7 * float(want.norm())
