@@ -668,8 +668,9 @@ __global__ __launch_bounds__(256) void k_kl_rewards(const float* __restrict__ ol
 // 88 MB at 512 x 4096 with values, 14 us at the rate of an even mix of reads and writes.  us, with one-element memory
 // instructions and the row in LDS / so: 512 x 4096: 35.8 / 27.8, 1024 x 4096: 63.5 / 47.7, 1024 x 1001: 47.8 / 27.6,
 // 1024 x 300: 42.3 / 25.2 (maps composed in 32 bits: 24.7, 41.3, 26.2, 24.2, at two to seven times the error: 512 x 4096
-// against 64 bits, gamma lambda = 0.95: 1.7e-7 then and before, 6.8e-8 so).  A quarter to a half of it is the sums of a
-// normalisation: 64-bit arithmetic, and three trips past the caches at the end of the launch (sums out, counter, sums in).
+// against 64 bits, gamma lambda = 0.95: 1.7e-7 then and before, 6.8e-8 so).  Half of its time is vector instructions, some
+// 1 600 a wave at 512 x 4096: the states that go from wave to wave (enter) and the sums in pairs (half_sums) have it at 24.8 us.
+// Where k_norm_rows does not fold the sums, three trips past the caches end the launch (sums out, counter, sums in).
 // Where the last workgroup folds the sums of the rows (not k_norm_rows) they are published past the caches: with a __threadfence() in every
 // workgroup (a write-back of its XCD's L2, full of the outputs' lines) 512 x 4096 took 4 us more.
 // ------------------------------------------------------------------------------------------------------------------
