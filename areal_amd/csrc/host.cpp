@@ -54,9 +54,10 @@ enum { kLogp, kEntropy, kVmax, kVmin, kStatLoss, kRatio, kApproxKl, kBehaveKl, k
 enum { kFlags, kMaskOut, kClip, kDual, kBehaveMask, kBoolRows };
 
 // Allocates (floats, bools, loss) and enters them and the arrays that the caller brought in the aa_ppo_step at `address`.
-py::tuple make_step(int64_t address, int64_t T, int64_t T_active, const Tensor& mask, const OptTensor& prox, const OptTensor& old,
-                    const OptTensor& adv, const OptTensor& cu, int64_t n_segments, bool derived, bool sampled,
-                    const OptTensor& behave_w, const OptTensor& counts, const Tensor& work, const at::Device& device) {
+std::tuple<Tensor, Tensor, Tensor> make_step(int64_t address, int64_t T, int64_t T_active, const Tensor& mask, const OptTensor& prox, const OptTensor& old,
+                                             const OptTensor& adv, const OptTensor& cu, int64_t n_segments, bool derived, bool sampled,
+                                             const OptTensor& behave_w, const OptTensor& counts, const Tensor& work,
+                                             const at::Device& device) {
   const int64_t pitch = std::max<int64_t>(64, (T + 63) & ~(int64_t)63);
   const auto options = at::TensorOptions().device(device);
   Tensor floats = at::empty({kFloatRows, pitch}, options.dtype(at::kFloat));
@@ -99,7 +100,7 @@ py::tuple make_step(int64_t address, int64_t T, int64_t T_active, const Tensor& 
   s.counts_given = counts.has_value() ? 1 : 0;
   s.loss = (float*)loss.data_ptr();
   s.work = work.data_ptr();
-  return py::make_tuple(floats, bools, loss);
+  return {floats, bools, loss};
 }
 
 Tensor row(const Tensor& rows, int i, int64_t n) {
@@ -235,10 +236,11 @@ using Scoring = std::tuple<double, double, double, std::optional<Norm>>;  // bia
 
 // (mask, logp, kl_rewards, rewards, advantages, returns).  mask: bool or float32; attention (bool) or seqlens (int64); with
 // `scoring` the scores are formed on the way and `score` holds the rewards; work: with a normalisation.
-py::tuple advantages(const Tensor& mask, const Tensor& logp, bool roll, const OptTensor& ref_logp, const OptTensor& attention,
-                     const OptTensor& seqlens, const Tensor& score, const OptTensor& values, double kl_ctl, int kl_estimator,
-                     double discount, double gae_lambda, bool mask_no_eos_with_zero, const std::optional<Norm>& norm,
-                     const std::optional<Scoring>& scoring, const OptTensor& work) {
+using SixTensors = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
+SixTensors advantages(const Tensor& mask, const Tensor& logp, bool roll, const OptTensor& ref_logp, const OptTensor& attention,
+                      const OptTensor& seqlens, const Tensor& score, const OptTensor& values, double kl_ctl, int kl_estimator,
+                      double discount, double gae_lambda, bool mask_no_eos_with_zero, const std::optional<Norm>& norm,
+                      const std::optional<Scoring>& scoring, const OptTensor& work) {
   const int64_t bs = mask.size(0), L = mask.size(1);
   const auto device = mask.device();
   const auto options = at::TensorOptions().device(device).dtype(at::kFloat);
@@ -298,17 +300,21 @@ py::tuple advantages(const Tensor& mask, const Tensor& logp, bool roll, const Op
   // written through a raw pointer: autograd is told
   if (ref_logp.has_value() && !ref_logp->is_inference()) ref_logp->unsafeGetTensorImpl()->bump_version();
   if (!roll && !logp.is_inference()) logp.unsafeGetTensorImpl()->bump_version();
-  return py::make_tuple(mask_out, logp_out, kl_rewards, rewards, adv, returns);
+  return {mask_out, logp_out, kl_rewards, rewards, adv, returns};
 }
 
 }  // namespace
 
+// What allocates or launches does so without the GIL, as torch's own bindings and ctypes do: an allocation may wait for the device, a
+// launch for room in the queue, and neither may stop the other threads of a trainer (one of them may have to queue the work that
+// is waited for).
 PYBIND11_MODULE(_host, m) {
-  m.def("make_step", &make_step);
+  using without_gil = py::call_guard<py::gil_scoped_release>;
+  m.def("make_step", &make_step, without_gil());
   m.def("step_rows", &step_rows);
   m.def("step_stats", &step_stats);
-  m.def("empty_rows_like", &empty_rows_like);
-  m.def("fused_logits", &fused_logits);
+  m.def("empty_rows_like", &empty_rows_like, without_gil());
+  m.def("fused_logits", &fused_logits, without_gil());
   m.def("advantages_plain", &advantages_plain);
-  m.def("advantages", &advantages);
+  m.def("advantages", &advantages, without_gil());
 }

@@ -1,4 +1,8 @@
 """Shared comparison helpers for the parity tests."""
+import sys
+import threading
+import time
+
 import torch
 
 
@@ -70,3 +74,32 @@ class Cfg:
         self.level, self.action, self.metric, self.agg, self.upper, self.lower = level, action, metric, agg, upper, lower
         if action == "clamp" and lower is None:
             self.lower = 0.0
+
+
+def lets_other_threads_run(call, tries: int = 1000) -> bool:
+    """Whether ``call`` gives up the GIL.  With a switch interval of 1 000 s another thread runs only when this one hands the
+    GIL over by itself; what ``call`` returns is kept meanwhile, because freeing a tensor hands it over too.  A call that
+    gives it up for a moment may take it again before the other thread is awake, hence the tries."""
+    beats, stop, kept = [0], [False], []
+
+    def beat():
+        while not stop[0]:
+            beats[0] += 1
+            time.sleep(0)
+
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    thread = threading.Thread(target=beat)
+    try:
+        thread.start()
+        time.sleep(0.01)
+        before = beats[0]
+        for _ in range(tries):
+            kept.append(call())
+            if beats[0] != before:
+                return True
+        return False
+    finally:
+        stop[0] = True
+        sys.setswitchinterval(interval)
+        thread.join()

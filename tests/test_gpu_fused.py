@@ -8,7 +8,7 @@ import torch
 import areal_amd
 import oracle
 from areal_amd import RejectionSamplingConfig, engine_glue, synth
-from helpers import assert_same_magnitude, cosine
+from helpers import assert_same_magnitude, cosine, lets_other_threads_run
 
 pytestmark = pytest.mark.gpu
 
@@ -1117,3 +1117,26 @@ def test_node_of_the_fused_step(device, T, pad):
     s.struct.T_active = T + pad + 1
     with pytest.raises(N.NativeLibraryError, match="aa_logits_ppo_step failed"):
         F._fused_logits(x, s, y, V, 1.0, False)
+
+
+def test_native_calls_that_launch_let_other_threads_run(device):
+    """A launch can wait for room in the queue: the native host side makes it without the GIL (the fused step, and the
+    advantage rows with scores given and with scores formed on the way)."""
+    import ctypes as C
+
+    from areal_amd import _native as N
+    from areal_amd import functional as F
+
+    host, T, V = N.host(), 3, 64
+    x = torch.randn(T, V, device=device).requires_grad_()
+    y = torch.zeros(T, dtype=torch.int64, device=device)
+    lp = torch.zeros(T, device=device)
+    mask = torch.ones(T, dtype=torch.bool, device=device)
+    step = F._ppo_step(torch.device(device), T, T, mask, lp, lp, lp, 0.2, None, None, None, None, None)
+    assert lets_other_threads_run(lambda: host.fused_logits(x, C.addressof(step.struct), step.loss.detach(), y, V, 1.0, False))
+    bs, L = 2, 5
+    mask, logp = torch.ones(bs, L, dtype=torch.bool, device=device), torch.zeros(bs, L, device=device)
+    score = torch.zeros(bs, device=device)
+    for scoring in (None, (0.0, 1.0, 5.0, None)):
+        assert lets_other_threads_run(lambda: host.advantages(mask, logp, True, None, mask, None, score, None, 0.0, 0, 1.0, 1.0,
+                                                              False, None, scoring, None))

@@ -4,6 +4,7 @@ import torch
 
 import areal_amd
 from areal_amd import RejectionSamplingConfig, synth
+from helpers import lets_other_threads_run
 
 
 # config validation: the cases of tests/test_rejection_sampling.py:8-41 and :806-839 of the reference
@@ -173,6 +174,20 @@ def test_arrays_that_the_advantage_rows_take_as_they_are():
     assert takes(score=inside) and not takes(score=inside, scored=True)
     inside = flat[:bs]
     assert takes(score=inside, scored=True) and not takes(score=inside, scored=True, roll=False)
+
+
+def test_native_calls_that_allocate_let_other_threads_run():
+    """An allocation can wait for the device: the native host side makes it without the GIL."""
+    import ctypes as C
+
+    from areal_amd import _native as N
+
+    host, step, T = N.host(), N.PpoStep(), 400
+    mask, rows = torch.ones(T, dtype=torch.bool), torch.zeros(10, 448)
+    assert not lets_other_threads_run(lambda: host.step_rows(rows, T))  # (views only: the measure itself)
+    assert lets_other_threads_run(lambda: host.make_step(C.addressof(step), T, T, mask, None, None, None, None, 0, True, False,
+                                                         None, None, mask, torch.device("cpu")))
+    assert lets_other_threads_run(lambda: host.empty_rows_like(rows, 448))
 
 
 def test_moments_of_a_mask_in_host_memory_are_refused(monkeypatch):
