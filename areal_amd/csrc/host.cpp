@@ -195,8 +195,8 @@ struct FusedLogits : torch::autograd::Function<FusedLogits> {
 };
 
 Tensor fused_logits(const Tensor& logits, int64_t address, const Tensor& loss, const Tensor& labels, int64_t stride,
-                    double temperature, bool inplace) {
-  const FusedLaunch a{(const aa_ppo_step*)address, loss, labels, stride, (float)(1.0 / temperature), inplace};
+                    double inv_temperature, bool inplace) {
+  const FusedLaunch a{(const aa_ppo_step*)address, loss, labels, stride, (float)inv_temperature, inplace};
   return FusedLogits::apply(logits, &a);
 }
 

@@ -731,7 +731,7 @@ def _hand_out_once(ctx) -> None:
 
 def _fused_logits(logits2d, step, labels1d, stride, temperature, inplace):
     """The loss of the step on logits, differentiable in them; its per-token outputs are in ``step``."""
-    return N.host().fused_logits(logits2d, C.addressof(step.struct), step.loss, labels1d, stride, temperature, inplace)
+    return N.host().fused_logits(logits2d, C.addressof(step.struct), step.loss, labels1d, stride, 1.0 / temperature, inplace)
 
 
 def _scaled(loss, scale, loss_mask):

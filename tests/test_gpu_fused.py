@@ -1119,6 +1119,23 @@ def test_node_of_the_fused_step(device, T, pad):
         F._fused_logits(x, s, y, V, 1.0, False)
 
 
+@pytest.mark.parametrize("grad", [True, False])
+def test_temperature_zero_is_refused(device, grad):
+    """By every fused step on logits, with a gradient (one pass) and without (the forward kernel)."""
+    T, V = 3, 64
+    x = torch.randn(T, V, device=device).requires_grad_(grad)
+    y = torch.zeros(T, dtype=torch.int64, device=device)
+    lp = torch.zeros(T, device=device)
+    mask = torch.ones(T, dtype=torch.bool, device=device)
+    cu = torch.tensor([0, T], dtype=torch.int32, device=device)
+    for call in (lambda t: areal_amd.fused_logprobs_ppo_loss(x, y, lp, lp, lp, 0.2, mask, temperature=t),
+                 lambda t: areal_amd.fused_logprobs_sapo_loss(x, y, lp, lp, 1.0, 1.05, mask, temperature=t),
+                 lambda t: areal_amd.fused_logprobs_sft_loss(x, y, mask, cu, temperature=t)):
+        with pytest.raises(ZeroDivisionError):
+            call(0.0)
+        assert bool(torch.isfinite(call(2.0)[0]))
+
+
 def test_native_calls_that_launch_let_other_threads_run(device):
     """A launch can wait for room in the queue: the native host side makes it without the GIL (the fused step, and the
     advantage rows with scores given and with scores formed on the way)."""

@@ -176,6 +176,19 @@ def test_arrays_that_the_advantage_rows_take_as_they_are():
     assert takes(score=inside, scored=True) and not takes(score=inside, scored=True, roll=False)
 
 
+def test_temperature_zero_is_refused_before_the_native_step():
+    """A temperature of zero is a division by zero, as on every other path, not an infinite factor for the kernels."""
+    from types import SimpleNamespace
+
+    from areal_amd import _native as N
+    from areal_amd import functional as F
+
+    x = torch.zeros(2, 8, requires_grad=True)
+    step = SimpleNamespace(struct=N.PpoStep(), loss=torch.zeros(()))
+    with pytest.raises(ZeroDivisionError):
+        F._fused_logits(x, step, torch.zeros(2, dtype=torch.int64), 8, 0.0, False)
+
+
 def test_native_calls_that_allocate_let_other_threads_run():
     """An allocation can wait for the device: the native host side makes it without the GIL."""
     import ctypes as C
