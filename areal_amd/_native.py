@@ -182,6 +182,7 @@ _d = C.c_double
 # name -> (restype, argtypes); must list every function of include/areal_amd.h
 SIGNATURES = {
     "aa_version": (_i, []),
+    "aa_layout": (C.c_uint64, []),
     "aa_status_string": (C.c_char_p, [_i]),
     "aa_logits_fwd": (_i, [_p, _i, _i64, _i64, _i64, _p, _f, _p, _p, _p, _p, _p, _p, _p]),
     "aa_logits_bwd": (_i, [_p, _i, _i64, _i64, _i64, _p, _f, _p, _p, _p, _p, _i64, _p, _p]),
@@ -259,6 +260,33 @@ SIGNATURES = {
     "aa_hbm_stream_probe": (_i, [_i, _i, _p, _p, _i64, _i, _p]),
 }
 
+_SHARED_STRUCTS = (PpoParams, RsParams, LossScale, PpoStep, NormParams, AdvantageStep, ScoreStep)
+
+
+def _layout(structs=_SHARED_STRUCTS) -> int:
+    """The number of ``csrc/layout.h`` for the structs as they are written down here."""
+    h = 0xCBF29CE484222325
+
+    def mix(name: str, size: int, place: int) -> None:
+        nonlocal h
+        for n in (*name.encode(), size, place):
+            h = (h ^ n) * 0x100000001B3 % 2**64
+
+    for struct in structs:
+        mix(struct.__doc__.strip("`"), C.sizeof(struct), 0)
+        for name, *_ in struct._fields_:
+            field = getattr(struct, name)
+            mix(name, field.size, field.offset)
+    return h
+
+
+def _check_layout(path: Path, found: int | None) -> None:
+    """Three binaries fill in and read the same structs; one of another header would write past them without a word."""
+    if found != _layout():
+        raise NativeLibraryError(f"{path} was built from another include/areal_amd.h than this package: build both libraries "
+                                 "with `python -m areal_amd.build`")
+
+
 _lib = None
 _lock = threading.Lock()
 
@@ -287,6 +315,7 @@ def load() -> C.CDLL:
                 raise NativeLibraryError(f"{LIB_PATH} does not export {name}") from e
             fn.restype = res
             fn.argtypes = args
+        _check_layout(LIB_PATH, lib.aa_layout())
         _lib = lib
     return _lib
 
@@ -308,6 +337,7 @@ def _load_host() -> None:
         from . import _host as module
     except ImportError as e:
         raise NativeLibraryError(f"cannot load {HOST_PATH}: build it with `python -m areal_amd.build` ({e})") from e
+    _check_layout(HOST_PATH, getattr(module, "layout", None))
     _host = module
 
 

@@ -14,6 +14,7 @@
 #include <torch/extension.h>
 
 #include "areal_amd.h"
+#include "layout.h"
 
 namespace py = pybind11;
 using at::Tensor;
@@ -310,6 +311,7 @@ SixTensors advantages(const Tensor& mask, const Tensor& logp, bool roll, const O
 // is waited for).
 PYBIND11_MODULE(_host, m) {
   using without_gil = py::call_guard<py::gil_scoped_release>;
+  m.attr("layout") = aa::layout();
   m.def("make_step", &make_step, without_gil());
   m.def("step_rows", &step_rows);
   m.def("step_stats", &step_stats);

@@ -1,7 +1,10 @@
 // Library identification for the C ABI.
 #include "../../include/areal_amd.h"
+#include "layout.h"
 
 extern "C" int aa_version(void) { return 100; /* 0.1.0 */ }
+
+extern "C" uint64_t aa_layout(void) { return aa::layout(); }
 
 extern "C" const char* aa_status_string(int status) {
   switch (status) {

@@ -149,6 +149,10 @@ typedef struct {
 /* Library version (major * 10000 + minor * 100 + patch). */
 int aa_version(void);
 
+/* A number for the layout of the structs that the library was compiled with:
+ * differs where a field has another name, size or place. */
+uint64_t aa_layout(void);
+
 /* Text for an aa_status value (static storage). */
 const char* aa_status_string(int status);
 

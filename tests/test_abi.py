@@ -39,6 +39,47 @@ def test_binding_covers_header_and_loads():
     assert lib.aa_status_string(1) == b"invalid argument"
 
 
+@pytest.mark.parametrize("load", [_native.load, _native.host])
+@pytest.mark.parametrize("struct,field", [("PpoStep", "work"), ("PpoStep", "mask"), ("AdvantageStep", "bs"), ("ScoreStep", "norm")])
+def test_binaries_of_another_header_are_refused(monkeypatch, load, struct, field):
+    """The library and the native host side say which layout of the shared structs they were compiled with: one that lacks a
+    field of the binding, or has it elsewhere, is not used."""
+    load()
+    known = getattr(_native, struct)
+    fields = [f for f in known._fields_ if f[0] != field]
+    other = type(struct, (ctypes.Structure,), {"__doc__": known.__doc__, "_fields_": fields})
+    moved = type(struct, (ctypes.Structure,), {"__doc__": known.__doc__, "_fields_": known._fields_[1:] + known._fields_[:1]})
+    for new in (other, moved):
+        structs = tuple(new if s is known else s for s in _native._SHARED_STRUCTS)
+        monkeypatch.setattr(_native._layout, "__defaults__", (structs,))
+        monkeypatch.setattr(_native, "_lib" if load is _native.load else "_host", None)
+        with pytest.raises(_native.NativeLibraryError, match="another include/areal_amd.h"):
+            load()
+        monkeypatch.undo()
+    load()
+
+
+def test_shared_structs_are_those_of_the_header(tmp_path):
+    """Name, size and place of every field of the binding's structs, asked of a C compiler."""
+    import shutil
+    import subprocess
+
+    gcc = shutil.which("gcc")
+    if gcc is None:
+        pytest.skip("no gcc")
+    lines = ["#include <stddef.h>", f'#include "{HEADER}"']
+    for struct in _native._SHARED_STRUCTS:
+        name = struct.__doc__.strip("`")
+        lines.append(f"_Static_assert(sizeof({name}) == {ctypes.sizeof(struct)}, \"{name}\");")
+        for field, *_ in struct._fields_:
+            at = getattr(struct, field)
+            lines.append(f"_Static_assert(offsetof({name}, {field}) == {at.offset} && "
+                         f"sizeof((({name}*)0)->{field}) == {at.size}, \"{name}.{field}\");")
+    src = tmp_path / "t.c"
+    src.write_text("\n".join(lines) + "\n")
+    subprocess.run([gcc, "-std=c11", "-Wall", "-Werror", "-fsyntax-only", str(src)], check=True)
+
+
 def test_header_is_plain_c(tmp_path):
     import shutil
     import subprocess
