@@ -85,9 +85,17 @@ __device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int& 
 }
 
 // A grid whose last round of tiles would fill at most half of the compute units runs that round as half tiles, two workgroups
-// to a tile: it is over in little more than half the time.  XCD by XCD, since a workgroup stays on the XCD that its id names; a
-// workgroup without a tile returns.  half: 0 or 1, or -1 for a whole tile.  units: compute units of the device; 0: whole tiles
-// throughout.  us, whole tiles / so: TODO
+// to a tile.  A half tile has half of the matrix products but reads all of one operand: it takes 0.7 to 0.95 of the time of a
+// whole one.  XCD by XCD, since a workgroup stays on the XCD that its id names; a workgroup without a tile returns.  half: 0 or
+// 1, or -1 for a whole tile.  units: compute units of the device; 0: whole tiles throughout.
+// us of d_weight, whole tiles / so, hidden size 512, rows 256, 1 024, 4 096, 8 192 for a vocabulary of
+//   1 024   (8 tiles)   11.1 / 8.8    22.5 / 16.5   68.6 / 49.7    129 / 96
+//   8 192   (64)        11.8 / 9.5    24.3 / 18.1   68.7 / 49.7    129 / 92
+//   16 384  (128)       12.4 / 10.4   24.0 / 19.4   70.3 / 59.9    148 / 139     (the largest grid that is half tiles throughout)
+//   33 792  (264)       24.9 / 22.3   51.8 / 46.7   172 / 161
+//   49 152  (384)       25.8 / 23.8   58.2 / 53.7   195 / 190      370 / 361     (a whole round, then half of one)
+// and past the line, where the half tiles would be two rounds themselves: 17 408 (136) 12.5 / 16.8, 25.4 / 35.6, 84 / 114, 178 / 257;
+// 50 176 (392) 25.9 / 30.4, 58.4 / 67.7, 195 / 243, 373 / 483.
 __host__ __device__ __forceinline__ int whole_tiles(int count, int units) {  // of the `count` tiles of an XCD
   const int per = units >> 3, rest = per > 0 ? count % per : 0;
   return 2 * rest <= per ? count - rest : count;

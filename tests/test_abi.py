@@ -164,6 +164,32 @@ def test_argument_validation_of_the_sibling_entry_points_without_gpu():
     assert lib.aa_ppo_loss(p, p, p, p, z, 4, z, 0, 0, ctypes.byref(params), p, p, p, p, p, z) == 2   # unsupported
 
 
+def test_scores_of_advantage_rows_are_validated_without_gpu():
+    """``aa_advantages_scored`` takes no level over the batch and no group of more than AA_SCORE_GROUP rows (``aa_reward_scores``
+    does), and refuses null scores, levels out of range and groups of nothing, before any launch."""
+    lib, address = _native.load(), 256  # (never dereferenced on the host)
+    step = _native.AdvantageStep(bs=4, L=8)
+    for name in ("loss_mask", "logp", "attention_mask", "mask_out", "logp_out", "kl_rewards", "rewards", "advantages", "returns"):
+        setattr(step, name, address)
+    step.logp_out = 2 * address
+
+    def status(*norm, rewards=address):
+        scores = _native.ScoreStep(rewards, 0.0, 1.0, 5.0)
+        if norm:
+            scores.norm = ctypes.pointer(_native.NormParams(norm[0], 0, norm[1], 0, 1e-5, norm[2]))
+        return lib.aa_advantages_scored(step, scores, None)
+
+    assert lib.aa_advantages_scored(step, None, None) == 1 and status(rewards=None) == 1
+    for levels in ((3, 0), (0, 3), (-1, 2)):
+        assert status(*levels, 4) == 1
+    assert status(2, 0, 0) == 1 and status(0, 2, -4) == 1
+    for levels in ((1, 1), (1, 0), (2, 1)):
+        assert status(*levels, 4) == 2
+    assert status(2, 2, _native.SCORE_GROUP + 1) == 2
+    step.bs = 0
+    assert status(2, 2, 4) == 0
+
+
 @pytest.mark.parametrize("V", [1, 8, 64, 65, 50257, 151936, (1 << 22) - 64, (1 << 22) - 63, (1 << 22) - 8, (1 << 22) - 1])
 def test_panel_pitch(V):
     """Whole 128-byte lines of bf16, except next to 2^22: 256 rows of the panel stay below the byte offsets of a tile, or

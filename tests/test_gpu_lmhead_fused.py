@@ -1029,3 +1029,49 @@ def test_panel_rows_that_end_inside_a_line(device, V):
     for got, want in ((h.grad, o_dh), (w.grad, o_dw)):
         assert cosine(got.cpu().float(), want) > 0.9999
         assert_same_magnitude(got, want)
+
+
+@pytest.mark.parametrize("V", [65, 1001])
+@pytest.mark.parametrize("T", [300, CHUNK + 200])
+@pytest.mark.parametrize("counted", ["host", "device", "none"])
+def test_rows_of_a_panel_of_its_own_that_end_inside_a_line(device, V, T, counted):
+    """The same for the stand-alone op, whose panel is an array of its own (with two chunks the second one's rows start behind
+    those of the first): panel and workspaces of NaN, some tokens without a row.  The tiles write nothing behind the last
+    multiple of 8 of a row (the backward clears rows without a token, whole), and the gradients are those of fp32 (bounds as
+    above)."""
+    import ctypes as C
+
+    lib, H = _native.load(), 72
+    g = torch.Generator().manual_seed(V + T)
+    hidden = torch.randn(T, H, generator=g).bfloat16().to(device)
+    weight = (0.3 * torch.randn(V, H, generator=g)).bfloat16().to(device)
+    labels = torch.randint(0, V, (T,), generator=g).to(device)
+    has_row = torch.rand(T, generator=g).to(device) < 0.7 if counted != "none" else torch.ones(T, dtype=torch.bool, device=device)
+    g_logp = torch.randn(T, generator=g).to(device) * has_row
+    per_chunk = [int(has_row[a : a + CHUNK].sum()) for a in range(0, T, CHUNK)]
+    rows, kept, mask = T, None, None
+    if counted == "host":
+        rows, kept, mask = sum(per_chunk), (C.c_int64 * len(per_chunk))(*per_chunk), has_row.data_ptr()
+    elif counted == "device":
+        kept, mask = (C.c_int64 * len(per_chunk))(*[_native.AA_LMHEAD_COUNT_ON_DEVICE] * len(per_chunk)), has_row.data_ptr()
+    pitch, size = int(lib.aa_lmhead_panel_pitch(V)), int(lib.aa_lmhead_carry_workspace_bytes(T, H, V))
+    panel = torch.full((rows, pitch), float("nan"), dtype=torch.bfloat16, device=device)
+    workspaces = [torch.full((size,), 0xFF, dtype=torch.uint8, device=device) for _ in range(2)]  # (0xffff...: NaN in every format)
+    logp, lse = torch.empty(T, device=device), torch.empty(T, device=device)
+    dh, dw = torch.full_like(hidden, float("nan")), torch.full_like(weight, float("nan"))
+    stream = torch.cuda.current_stream(device).cuda_stream
+    common = (hidden.data_ptr(), weight.data_ptr(), T, H, V, labels.data_ptr(), 1.0)
+    _native.check(lib.aa_lmhead_fwd_carry(*common, mask, kept, logp.data_ptr(), None, lse.data_ptr(), None, None, None,
+                                          panel.data_ptr(), rows, workspaces[0].data_ptr(), size, stream), "aa_lmhead_fwd_carry")
+    assert bool(torch.isnan(panel[:, (V + 7) // 8 * 8 :]).all())
+    _native.check(lib.aa_lmhead_bwd_carry(*common, logp.data_ptr(), lse.data_ptr(), g_logp.data_ptr(), mask, kept, panel.data_ptr(),
+                                          rows, dh.data_ptr(), dw.data_ptr(), _native.AA_BF16, workspaces[1].data_ptr(), size,
+                                          stream), "aa_lmhead_bwd_carry")
+    z = hidden.float() @ weight.float().t()
+    d = -torch.softmax(z, 1)
+    d[torch.arange(T, device=device), labels] += 1.0
+    d *= g_logp[:, None]
+    for got, want in ((dh, d @ weight.float()), (dw, d.t() @ hidden.float())):
+        assert cosine(got.float().cpu(), want.cpu()) > 0.9999
+        assert_same_magnitude(got.float(), want)
+    assert float(dh[~has_row].float().abs().sum()) == 0.0
