@@ -1031,17 +1031,19 @@ def test_panel_rows_that_end_inside_a_line(device, V):
         assert_same_magnitude(got, want)
 
 
-@pytest.mark.parametrize("V", [65, 1001])
-@pytest.mark.parametrize("T", [300, CHUNK + 200])
+@pytest.mark.parametrize("T,H,V", [(300, 72, 65), (300, 72, 1001), (CHUNK + 200, 72, 65), (CHUNK + 200, 72, 1001),
+                                   # d(weight) of 16 and 17 tiles an XCD (half tiles, whole tiles), and one round and a little
+                                   (300, 72, 256 * 128 - 3), (300, 72, 256 * 136 - 3), (300, 72, 256 * 264 + 5),
+                                   (300, 392, 256 * 129 - 5)])
 @pytest.mark.parametrize("counted", ["host", "device", "none"])
-def test_rows_of_a_panel_of_its_own_that_end_inside_a_line(device, V, T, counted):
+def test_rows_of_a_panel_of_its_own_that_end_inside_a_line(device, T, H, V, counted):
     """The same for the stand-alone op, whose panel is an array of its own (with two chunks the second one's rows start behind
-    those of the first): panel and workspaces of NaN, some tokens without a row.  The tiles write nothing behind the last
-    multiple of 8 of a row (the backward clears rows without a token, whole), and the gradients are those of fp32 (bounds as
-    above)."""
+    those of the first): panel, workspaces and gradients held NaN, some tokens have no row.  The tiles write nothing behind the
+    last multiple of 8 of a row (the backward clears rows without a token, whole), every entry of the gradients is written, and
+    they are those of fp32 (bounds as above)."""
     import ctypes as C
 
-    lib, H = _native.load(), 72
+    lib = _native.load()
     g = torch.Generator().manual_seed(V + T)
     hidden = torch.randn(T, H, generator=g).bfloat16().to(device)
     weight = (0.3 * torch.randn(V, H, generator=g)).bfloat16().to(device)
