@@ -1,4 +1,5 @@
 """Shared comparison helpers for the parity tests."""
+import gc
 import sys
 import threading
 import time
@@ -76,10 +77,11 @@ class Cfg:
             self.lower = 0.0
 
 
-def lets_other_threads_run(call, tries: int = 1000) -> bool:
+def lets_other_threads_run(call, tries: int = 1000, rounds: int = 10) -> bool:
     """Whether ``call`` gives up the GIL.  With a switch interval of 1 000 s another thread runs only when this one hands the
-    GIL over by itself; what ``call`` returns is kept meanwhile, because freeing a tensor hands it over too.  A call that
-    gives it up for a moment may take it again before the other thread is awake, hence the tries."""
+    GIL over by itself; what ``call`` returns is kept meanwhile, because freeing a tensor hands it over too (so may a
+    collection of garbage).  A call that gives it up for a moment may take it again before the other thread is awake, hence
+    the tries, and the rounds on a busy machine."""
     beats, stop, kept = [0], [False], []
 
     def beat():
@@ -87,19 +89,25 @@ def lets_other_threads_run(call, tries: int = 1000) -> bool:
             beats[0] += 1
             time.sleep(0)
 
-    interval = sys.getswitchinterval()
+    interval, collects = sys.getswitchinterval(), gc.isenabled()
+    gc.collect()
+    gc.disable()
     sys.setswitchinterval(1000.0)
     thread = threading.Thread(target=beat)
     try:
         thread.start()
-        time.sleep(0.01)
-        before = beats[0]
-        for _ in range(tries):
-            kept.append(call())
-            if beats[0] != before:
-                return True
+        for _ in range(rounds):
+            kept.clear()
+            time.sleep(0.01)
+            before = beats[0]
+            for _ in range(tries):
+                kept.append(call())
+                if beats[0] != before:
+                    return True
         return False
     finally:
         stop[0] = True
         sys.setswitchinterval(interval)
         thread.join()
+        if collects:
+            gc.enable()
